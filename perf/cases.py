@@ -373,7 +373,7 @@ def lengths(case):
     rng = random.Random(zlib.crc32(json.dumps({k: v for k, v in case.items() if k != "name"}, sort_keys=True).encode()))
 
     def some(count, longest):
-        if not case["ragged"]:
+        if not count or not case["ragged"]:
             return [longest] * count
         return [longest] + [rng.randint(max(1, longest // 32), longest) for _ in range(count - 1)]
 
