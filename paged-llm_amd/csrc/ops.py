@@ -9,6 +9,7 @@ is no CPU fallback, and a missing or unbuildable library raises at the first cal
 from __future__ import annotations
 
 import ctypes
+import functools
 import logging
 from ctypes import c_float, c_int, c_long, c_longlong, c_ulonglong, c_void_p
 
@@ -75,7 +76,9 @@ _SIGNATURES = {
     "pllm_rope_scatter": [c_int, c_void_p, c_int, c_void_p, c_void_p, c_void_p, c_void_p, c_void_p, c_void_p,
                           c_int, c_int, c_int, c_int, c_int, c_int, c_int, c_int, c_void_p],
     "pllm_copy_pages": [c_int, c_void_p, c_void_p, c_void_p, c_int, c_long, c_void_p],
-    "pllm_gemm_nt": [c_int, c_int, c_void_p, c_int, c_void_p, c_int, c_void_p, c_int, c_int, c_int, c_int, c_void_p],
+    "pllm_gemm_nt": [c_int, c_void_p, c_int, c_void_p, c_int, c_void_p, c_int, c_int, c_int, c_int, c_void_p],
+    "pllm_gemm_float": [c_void_p, c_int, c_long, c_void_p, c_int, c_long, c_void_p, c_int, c_long, c_int, c_int, c_int, c_int,
+                        c_int, c_int, c_void_p],
     "pllm_paged_attention_generic": [c_int, c_void_p, c_int, c_void_p, c_void_p, c_void_p, c_int, c_void_p, c_int,
                                      c_void_p, c_void_p, c_int, c_int, c_int, c_int, c_int, c_int, c_float, c_int,
                                      c_float, c_void_p, c_void_p, c_int, c_int, c_void_p, c_void_p],
@@ -276,8 +279,35 @@ def copy_pages(pages: torch.Tensor, src: torch.Tensor, dst: torch.Tensor) -> Non
 
 
 # ------------------------------------------------------------------------------------------- products
+# The float product's tiles (in sixteens of rows and of weight rows): the time of one round of workgroups, one on every
+# compute unit, at K = 2048, and what a launch takes beside its rounds (microseconds, fitted to 1 to 2048 rows of matrices of
+# 1024 to 32000 weight rows; a round is in proportion to K).  Small tiles give a step of few rows enough workgroups, large
+# ones use the matrix cores better; the products of one round or two are decided by how full the rounds are (301 rows x
+# 2048 x 2048: tiles of 48 x 64 in one round 36 us, 64 x 64 47 us, 32 x 32 47 us; 301 x 2560 x 2048: 48 x 64 in two rounds 65 us,
+# 64 x 64 in one 48 us).
+FLOAT_GEMM_TILES = {(1, 1): (7.0, 4.0), (1, 2): (10.4, 4.0), (2, 2): (16.0, 4.0), (3, 4): (33.2, 3.0), (4, 4): (43.0, 3.0)}
+
+
+@functools.lru_cache(maxsize=4096)
+def float_gemm_plan(M: int, N: int, K: int, batch: int, compute_units: int) -> tuple[int, int]:
+    """The tile of a float product: the one whose rounds of workgroups take the least time.  The result of the product does
+    not depend on it."""
+    def cost(tile):
+        per_round, fixed = FLOAT_GEMM_TILES[tile]
+        workgroups = -(-M // (16 * tile[0])) * -(-N // (16 * tile[1])) * batch
+        return fixed + -(-workgroups // compute_units) * per_round * K / 2048
+    return min(FLOAT_GEMM_TILES, key=cost)
+
+
+def _gemm_float(a_ptr, lda, a_batch, w_ptr, ldw, w_batch, out_ptr, ldc, c_batch, M, N, K, batch, device, what) -> None:
+    tile = float_gemm_plan(M, N, K, batch, _num_compute_units(device))
+    _check(_fn("gemm_float.hip", "pllm_gemm_float")(a_ptr, lda, a_batch, w_ptr, ldw, w_batch, out_ptr, ldc, c_batch, M, N, K, batch,
+                                                    *tile, _stream()), what)
+
+
 def gemm_generic(a: torch.Tensor, w: torch.Tensor, out_dtype: torch.dtype | None = None) -> torch.Tensor:
-    """a [M, K] times w [N, K] transposed, float accumulation in ascending k, any sizes."""
+    """a [M, K] times w [N, K] transposed with float accumulation, any sizes: float32 on the float matrix cores (the order of
+    the additions depends on K alone), bfloat16 on the plain kernel (ascending k)."""
     _on_gpu(a, w)
     _need(a.dim() == 2 and w.dim() == 2 and a.shape[1] == w.shape[1], f"gemm shapes {tuple(a.shape)} x {tuple(w.shape)}^T")
     _need(a.stride(1) == 1 and w.stride(1) == 1, "gemm operands need unit inner stride")
@@ -286,8 +316,13 @@ def gemm_generic(a: torch.Tensor, w: torch.Tensor, out_dtype: torch.dtype | None
     M, K = a.shape
     N = w.shape[0]
     out = torch.empty((M, N), dtype=out_dtype, device=a.device)
-    _check(_fn("gemm_generic.hip", "pllm_gemm_nt")(dtype_code(a.dtype), dtype_code(out_dtype), _ptr(a), a.stride(0),
-                                                    _ptr(w), w.stride(0), _ptr(out), N, M, N, K, _stream()), "gemm_generic")
+    if a.dtype == torch.float32:
+        _need(out_dtype == torch.float32, "float32 operands give float32 results")
+        _gemm_float(_ptr(a), a.stride(0), 0, _ptr(w), w.stride(0), 0, _ptr(out), N, 0, M, N, K, 1, a.device, "gemm_generic")
+    else:
+        _need(a.dtype == torch.bfloat16, f"kernels take float32 or bfloat16, not {a.dtype}")
+        _check(_fn("gemm_generic.hip", "pllm_gemm_nt")(dtype_code(out_dtype), _ptr(a), a.stride(0), _ptr(w), w.stride(0), _ptr(out), N,
+                                                       M, N, K, _stream()), "gemm_generic")
     return out
 
 
@@ -1329,10 +1364,8 @@ def gemm_heads(a: torch.Tensor, w: HeadMatrices, out: torch.Tensor | None = None
         # the output's rows through views with the heads in front
         torch.bmm(a.transpose(0, 1), w.data, out=out.transpose(0, 1))
         return out
-    sig = [c_int, c_int, c_void_p, c_int, c_long, c_void_p, c_int, c_long, c_void_p, c_int, c_long, c_int, c_int, c_int, c_int, c_void_p]
-    _check(_fn("gemm_generic.hip", "pllm_gemm_nt_batched", signature=sig)(
-        dtype_code(a.dtype), dtype_code(out.dtype), _ptr(a), a.stride(0), a.stride(1), _ptr(w.data), K, N * K, _ptr(out), out.stride(0), out.stride(1),
-        T, N, K, heads, _stream()), "gemm_heads")
+    _gemm_float(_ptr(a), a.stride(0), a.stride(1), _ptr(w.data), K, N * K, _ptr(out), out.stride(0), out.stride(1), T, N, K, heads,
+                a.device, "gemm_heads")
     return out
 
 
