@@ -143,7 +143,7 @@ def load_library(source: str, defines: dict | None = None) -> ctypes.CDLL:
 
 
 # Sources every model needs, and the specialised ones per head size.
-COMMON_SOURCES = ["elementwise.hip", "gemm_generic.hip", "gemm_float.hip", "attention_generic.hip", "sampling.hip", "decode_linear.hip",
+COMMON_SOURCES = ["elementwise.hip", "gemm_generic.hip", "gemm_float.hip", "attention_generic.hip", "attention_float.hip", "sampling.hip", "decode_linear.hip",
                   "attention_noalloc.hip", "stream_linear.hip", "float_stream.hip", "recurrent.hip", "latent_attention.hip", "attention_prepare.hip", "moe.hip",
                   "selective_scan.hip", "delta_rule.hip"]
 # Head sizes whose attention library a full build makes (others are compiled at first use).

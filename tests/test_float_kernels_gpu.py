@@ -1,10 +1,12 @@
 """The kernels of the true 32-bit path on the float matrix cores, at the edges of their tiles: products in every form of the
-kernel."""
+kernel, attention with every mask, term and weighting, and values that are no numbers where nobody may see them."""
+
+import math
 
 import pytest
 import torch
 
-from tests.test_kernels_gpu import rnd
+from tests.test_kernels_gpu import dense_attention, paged_case, rnd
 
 pytestmark = pytest.mark.gpu
 
@@ -45,3 +47,70 @@ def test_float_product_batches():
     o.gemm_heads(a.cuda(), o.HeadMatrices(w.cuda()), out=out[:, :, :40])
     want = torch.einsum("thk,hnk->thn", a.double(), w.double())
     assert float((out[:, :, :40].cpu().double() - want).abs().max() / want.abs().max()) <= 1e-6 and bool((out[:, :, 40:] == 0).all())
+
+
+CASES = [([1], [1]), ([40, 9, 64], [8, 1, 3]), ([129, 300, 17], [129, 300, 17]), ([1000, 33, 2048, 5], [1, 1, 1, 1]), ([577, 64, 77], [37, 2, 12])]
+SHAPES = [(32, 4, 64, 16), (3, 1, 48, 32), (5, 5, 16, 16), (6, 2, 128, 16), (40, 1, 144, 16), (2, 1, 256, 64)]
+
+
+@pytest.mark.parametrize("heads,kv_heads,d,bs", SHAPES)
+@pytest.mark.parametrize("lens,num_q", CASES)
+def test_float_attention(heads, kv_heads, d, bs, lens, num_q):
+    """Against the plain kernel in float32 (both within 2e-5 of dense attention in the tests of that kernel)."""
+    o = ops()
+    if sum(lens) * heads * d > 3_000_000 and heads != 32:
+        pytest.skip("long case kept for one shape")
+    q, kp, vp, tables, cu, sl = paged_case(lens, num_q, heads, kv_heads, d, bs, torch.float32, seed=1)
+    args = (q.cuda(), kp.cuda(), vp.cuda(), tables.cuda(), cu.cuda(), sl.cuda(), heads, kv_heads, d, 1 / math.sqrt(d))
+    g = torch.Generator().manual_seed(5)
+    slopes, sinks = (torch.randn(heads, generator=g).mul(0.05).cuda() for _ in range(2))
+    for window, terms, weights in ((0, None, None), (19, None, None), (-64, o.ScoreTerms(sinks=sinks), None), (100, o.ScoreTerms(cap=3.0, slopes=slopes, sinks=sinks), None),
+                                   (70, None, o.KeyWeights(keep_first=4)), (33, o.ScoreTerms(cap=5.0), o.KeyWeights(keep_first=20, sigmoid=True, head_bias=sinks)),
+                                   (0, None, o.KeyWeights(sigmoid=True))):
+        got = o.paged_attention_float(*args, window, terms=terms, weights=weights)
+        want = o.paged_attention_generic(*args, window, terms=terms, weights=weights)
+        assert float((got - want).abs().max() / want.abs().max()) <= 4e-5, (window, terms, weights)
+    want = dense_attention(q, kp, vp, tables, cu, sl, heads, kv_heads, d, 1 / math.sqrt(d))
+    got = o.paged_attention_float(*args).cpu()
+    assert float((got - want).abs().max() / want.abs().max()) <= 2e-5
+
+
+def test_float_attention_does_not_depend_on_the_cut():
+    """The same positions as one prompt, in portions and beside other requests: the same bits."""
+    o = ops()
+    heads, kv_heads, d, bs = 8, 2, 64, 16
+    q, kp, vp, tables, cu, sl = paged_case([530], [530], heads, kv_heads, d, bs, torch.float32, seed=2)
+    rest = (kp.cuda(), vp.cuda())
+    for window, weights in ((0, None), (100, None), (90, o.KeyWeights(keep_first=5)), (100, o.KeyWeights(sigmoid=True))):
+        tail = (heads, kv_heads, d, 0.125, window)
+        whole = o.paged_attention_float(q.cuda(), *rest, tables.cuda(), cu.cuda(), sl.cuda(), *tail, weights=weights).cpu()
+        for lo, hi in ((0, 1), (3, 70), (64, 128), (529, 530), (200, 467)):
+            two = torch.cat([q[lo:hi], q[hi - 1:hi]]).cuda()
+            part = o.paged_attention_float(two, *rest, tables.repeat(2, 1).cuda(), torch.tensor([0, hi - lo, hi - lo + 1], dtype=torch.int32, device="cuda"),
+                                           torch.tensor([hi, hi], dtype=torch.int32, device="cuda"), *tail, weights=weights).cpu()
+            assert torch.equal(part[:hi - lo], whole[lo:hi]) and torch.equal(part[hi - lo:], whole[hi - 1:hi]), (window, lo, hi)
+
+
+def test_float_attention_leaves_unseen_slots_alone():
+    """Garbage past the context, in table entries past it and in front of a window changes nothing; an infinite value reaches
+    the queries that see its key and no other."""
+    o = ops()
+    heads, kv_heads, d, bs = 4, 2, 32, 16
+    q, kp, vp, tables, cu, sl = paged_case([37, 5], [20, 1], heads, kv_heads, d, bs, torch.float32, seed=3)
+    def run(kp, vp, tables, window):
+        return o.paged_attention_float(q.cuda(), kp.cuda(), vp.cuda(), tables.cuda(), cu.cuda(), sl.cuda(), heads, kv_heads, d, 0.3, window).cpu()
+    t2, kp2, vp2 = tables.clone(), kp.clone(), vp.clone()
+    t2[1, 1:] = 999_999
+    kp2[tables[1, 0], :, 5:, :] = float("nan")
+    vp2[tables[1, 0], :, :, 5:] = float("inf")
+    kp2[tables[0, 2], :, 5:, :] = float("nan")
+    vp2[tables[0, 2], :, :, 5:] = float("nan")
+    assert torch.equal(run(kp, vp, tables, 0), run(kp2, vp2, t2, 0))
+    vp2[tables[0, 0], :, :, :14] = float("nan")                 # (positions that a window of 4 has passed before the first query, at 17)
+    assert torch.equal(run(kp, vp, tables, 4), run(kp2, vp2, t2, 4))
+    vp3 = vp.clone()
+    vp3[tables[0, 1], :, 7, 13] = float("inf")                  # position 29 of the first request, channel 7
+    plain, odd = run(kp, vp, tables, 0), run(kp, vp3, tables, 0)
+    seen = torch.zeros(21, heads, d, dtype=torch.bool)
+    seen[29 - 17:20, :, 7] = True
+    assert bool(torch.isinf(odd.view(21, heads, d)[seen]).all()) and torch.equal(odd.view(21, heads, d)[~seen], plain.view(21, heads, d)[~seen])
