@@ -469,7 +469,7 @@ def paged_attention_float(q: torch.Tensor, k_pages: torch.Tensor, v_pages: torch
 def _paged_attention_plain(q, k_pages, v_pages, block_tables, cu_seqlens_q, seq_lens_k, num_heads, num_kv_heads, head_dim, scale, window,
                            terms, weights=None) -> torch.Tensor:
     """Float32 attention, and whatever the bfloat16 kernels refuse.  (301 tokens, 32 heads of 64 on 4: 253 us with the plain
-    kernel, 23 us on the matrix cores; decoding 8 requests at contexts to 700: 186 and 21 us.)"""
+    kernel, 30 us on the matrix cores; decoding 8 requests at contexts to 700: 186 and 19 us.)"""
     kernel = paged_attention_float if float_attention_takes(q, k_pages, v_pages, head_dim, k_pages.shape[2]) else paged_attention_generic
     return kernel(q, k_pages, v_pages, block_tables, cu_seqlens_q, seq_lens_k, num_heads, num_kv_heads, head_dim, scale, window, terms=terms,
                   weights=weights)
@@ -1488,17 +1488,44 @@ RECURRENCE_CHUNKS_FROM = 128      # tokens of the longest sequence of a step fro
 
 
 def recurrence_chunk(max_q_len: int, num_tokens: int) -> int:
-    """Tokens per chunk for a step's recurrences (0: every sequence token by token in one workgroup per head).  Chunks
-    spread a long portion over the GPU at the price of a workspace of one state per chunk, so they grow with the step."""
+    """Tokens per chunk for a step's recurrences whose states are too tall for the matrix form (0: every sequence token by token
+    in one workgroup per head).  Chunks spread a long portion over the GPU at the price of a workspace of one state per chunk,
+    so they grow with the step."""
     if max_q_len < RECURRENCE_CHUNKS_FROM:
         return 0
-    # (short steps: more, shorter chunks, or most of the GPU stays idle.  Measured at width 2,048, a prompt of 256 / 512 /
-    #  1,024 / 2,048 tokens in ms: chunks of 16: 2.39 / 3.09 / 4.73 / 8.46; of 32: 2.54 / 3.09 / 4.34 / 7.29; of 64: 3.11 /
-    #  3.55 / 4.65 / 6.92; of 128: 4.60 / 4.81 / 5.71 / 7.80)
+    # (short steps: more, shorter chunks, or most of the GPU stays idle)
     for limit, chunk in ((384, 16), (1536, 32), (4096, 64), (16384, 128)):
         if num_tokens <= limit:
             return chunk
     return 256
+
+
+RECURRENCE_PIECE = 32             # tokens that the matrix form of a long portion works off at a time
+
+
+def recurrence_form(max_q_len: int, num_tokens: int, num_seqs: int, heads: int, rows: int, columns: int, by_row: bool, compute_units: int) -> int:
+    """How a step's recurrences run: 0, every sequence token by token in one workgroup per head and block of columns; -1, every
+    sequence in one workgroup likewise, in pieces of 32 tokens; else the tokens per chunk of the three passes over chunks, which
+    spread a long portion over the GPU at the price of a workspace of one state per chunk and two passes over every sequence."""
+    if max_q_len <= 1:
+        return 0
+    if rows <= (128 if by_row else 256):
+        # What each takes, in us, from 1 to 2,048 tokens of 64 heads of 128 x 64 rows and columns, of 8 of 128 x 257 and 256 x 512, of
+        # 16 of 128 x 128 with a decay per row, alone and beside 32 single tokens.  Single tokens stay token by token (64 heads: 17
+        # us), portions beside many of them in pieces (64 tokens and 32 single ones: token by token 110, pieces 74, chunks 330),
+        # long portions in chunks (2,048: pieces 460, chunks 142) of so many pieces that their workgroups fill the GPU once:
+        # chunks of 1 / 2 / 4 / 8 pieces take 200 / 159 / 152 / 142, and at 512 tokens 62 / 53 / 64 / 101.
+        wide = by_row or rows > 128                     # workgroups of eight wavefronts, one to a compute unit; else of four, two
+        slots = compute_units * (1 if wide else 2)
+        groups = heads * -(-columns // (128 if wide else 64))
+        pieces, fill = -(-max_q_len // RECURRENCE_PIECE), max(1.0, num_seqs * groups / slots)
+        chunk = -(-(-(-num_tokens // RECURRENCE_PIECE) * groups) // slots)
+        by_token = 6.0 + 1.25 * max_q_len + 5.0 * fill
+        in_pieces = 25.0 * fill + 12.5 * (pieces - 1) if wide else 16.0 * fill + 7.0 * (pieces - 1)
+        beside = (num_seqs - 1) * groups / slots
+        in_chunks = 36.0 + 25.0 * (chunk - 1) + 100.0 * beside if wide else 30.0 + 14.0 * (chunk - 1) + 75.0 * beside
+        return min((by_token, 0), (in_pieces, -1), (in_chunks, RECURRENCE_PIECE * chunk))[1]
+    return recurrence_chunk(max_q_len, num_tokens)
 
 
 def linear_recurrence(q: torch.Tensor, k: torch.Tensor, v: torch.Tensor, decay: torch.Tensor, state: torch.Tensor, state_offset: int,
@@ -1548,10 +1575,10 @@ def linear_recurrence(q: torch.Tensor, k: torch.Tensor, v: torch.Tensor, decay: 
     _check_sequences(state, state_slots, seq_starts, cu_seqlens, num_seqs)
     _need(0 <= state_offset and state_offset + H * N * P <= state.shape[1], "the recurrence's state does not fit the state slot")
     out = torch.empty((T, H * P), dtype=torch.float32, device=v.device)
-    chunk = recurrence_chunk(max_q_len, T)
-    max_chunks = T // chunk + num_seqs if chunk else 0
-    ws_state = torch.empty((max_chunks, H * N * P), dtype=torch.float32, device=v.device) if chunk else None
-    ws_decay = torch.empty((max_chunks, H * (N if row_decay is not None else 1)), dtype=torch.float32, device=v.device) if chunk else None
+    chunk = recurrence_form(max_q_len, T, num_seqs, H, N, P, row_decay is not None, _num_compute_units(v.device))
+    max_chunks = T // chunk + num_seqs if chunk > 0 else 0
+    ws_state = torch.empty((max_chunks, H * N * P), dtype=torch.float32, device=v.device) if chunk > 0 else None
+    ws_decay = torch.empty((max_chunks, H * (N if row_decay is not None else 1)), dtype=torch.float32, device=v.device) if chunk > 0 else None
     sig = [c_void_p, c_void_p, c_int, c_int, c_void_p, c_int, c_int, c_void_p, c_int, c_void_p, c_int, c_void_p, c_void_p,
            c_void_p, c_int, c_int, c_void_p, c_void_p,
            c_void_p, c_long, c_void_p, c_void_p,

@@ -465,9 +465,444 @@ static void launch_recurrence(const RecurrenceArgs& a, const ChunkArgs& ca, dim3
   else hipLaunchKernelGGL((linear_recurrence_kernel<64, 256, MODE>), grid, block, 0, stream, a, ca);
 }
 
+// ---------------------------------------------------------------------------------------------
+// The first and the third pass as matrix products in float (v_mfma_f32_16x16x4_f32), for heads of up to 256 rows (128 with a
+// decay per row): a workgroup walks its chunk in pieces of 32 tokens.  With D[t, j] the product of the decays of tokens
+// j + 1 .. t of a piece, G_t that of its tokens up to t and S the state in front of it,
+//   Y = (G Q) S + M V + skip V,   M[t, j] = D[t, j] g_j (q_t . k_j) for j <= t,
+//   S <- G_32 S + K^T (g_j D[32, j] V)
+// (every product of decays is built by multiplication, none from a difference of logarithms: as many roundings as token by
+// token).  A decay per row stands inside the sums over the rows: there (G Q) and K^T carry it element by element; M's tile of
+// late queries and early keys takes both from the tiles' border (no factor is above 1), and its two tiles on the diagonal are
+// summed by vector instructions, a thread walking the queries behind one key with the key's rows times their decays at hand.
+//
+// A wavefront owns 16 columns of S and all of its rows in registers.  A result's lane (g, c) = (lane >> 4, lane & 15) holds
+// rows 4 g .. 4 g + 3 of column c, and such a fragment of S is the operand of Y^T = S^T Q^T as it stands; so is one of M.
+// K and V lie in LDS by rows of S and columns (tokens in fours, in an order that spreads the banks).  The next piece's rows
+// travel while this one is worked off.
+//
+// What bounds it: the float matrix cores (a third to half busy) beside a piece's barriers and its way through LDS.  A prompt
+// of 2,048 tokens, one layer, states + carry + outputs: 64 heads of 128 x 64 452 us token by token in chunks of 64 -> 142 us (58 + 9 +
+// 102 under the profiler); 8 heads of 256 x 512 758 -> 210 us; 16 heads of 128 x 128 with a decay per row 232 -> 131 us.  Errors
+// against 64 bits over 1 to 2,048 tokens: outputs 2.6e-8 to 1.5e-6 as before or below, the last states below (1.1e-7 against
+// 2.0e-7, 2.1e-6 against 6.3e-6).
+constexpr int kPiece = 32, kPieceLd = kPiece + 4;
+
+typedef float f32x4 __attribute__((ext_vector_type(4)));
+
+__device__ __forceinline__ f32x4 mfma16(const f32x4 a, const f32x4 b, f32x4 acc) {
+#pragma unroll
+  for (int i = 0; i < 4; ++i) acc = __builtin_amdgcn_mfma_f32_16x16x4f32(a[i], b[i], acc, 0, 0, 0);
+  return acc;
+}
+// The products of sixteen rows of one operand and sixteen of the other over 16 NT elements, in four sums: a chain of
+// roundings as short as the token-by-token kernel's.
+template <int NT>
+__device__ __forceinline__ f32x4 dot_rows(const float* a, const float* b) {
+  f32x4 part[4];
+#pragma unroll
+  for (int i = 0; i < 4; ++i) part[i] = f32x4{0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+  for (int i = 0; i < NT; ++i) part[i & 3] = mfma16(*reinterpret_cast<const f32x4*>(a + 16 * i), *reinterpret_cast<const f32x4*>(b + 16 * i), part[i & 3]);
+  return (part[0] + part[1]) + (part[2] + part[3]);
+}
+// Where four tokens 4 f .. 4 f + 3 of row n stand in an array of rows over the tokens of a piece.
+__device__ __forceinline__ int token_quad(int n, int f) { return n * kPiece + ((f ^ n ^ (n >> 3)) & 7) * 4; }
+__device__ __forceinline__ f32x4 lds_quad(const float* p) { return *reinterpret_cast<const f32x4*>(p); }
+
+// Elements n .. n + 3 of a row that holds `count`, zeros past it.  vec: they can be read at once and never straddle the end.
+__device__ __forceinline__ f32x4 row_quad(const void* base, int dtype, size_t at, int n, int count, bool vec) {
+  f32x4 v = {0.f, 0.f, 0.f, 0.f};
+  if (n >= count) return v;
+  if (!vec) {
+    v[0] = load_as_f32(base, dtype, at);
+    if (n + 1 < count) v[1] = load_as_f32(base, dtype, at + 1);
+    if (n + 2 < count) v[2] = load_as_f32(base, dtype, at + 2);
+    if (n + 3 < count) v[3] = load_as_f32(base, dtype, at + 3);
+    return v;
+  }
+  if (dtype == PLLM_F32) return *reinterpret_cast<const f32x4*>(reinterpret_cast<const float*>(base) + at);
+  const uint2 w = *reinterpret_cast<const uint2*>(reinterpret_cast<const uint16_t*>(base) + at);
+  v[0] = __uint_as_float(w.x << 16); v[1] = __uint_as_float(w.x & 0xffff0000u);
+  v[2] = __uint_as_float(w.y << 16); v[3] = __uint_as_float(w.y & 0xffff0000u);
+  return v;
+}
+
+constexpr int kVecRows = 1, kVecValues = 2, kVecOut = 4, kVecDecay = 8;
+
+// Floats of LDS, in the order the kernel lays them out.
+template <int NT, int WAVES, int MODE, bool ROW> constexpr int piece_lds_floats() {
+  constexpr int NP = 16 * NT, rows = kPiece * (NP + 4), half = (kPiece / 2) * (NP + 4);
+  int n = NP * kPiece + 16 * WAVES * kPiece;                                     // K^T, V^T
+  if (MODE != kChunkState) n += 2 * rows + kPiece * kPieceLd;                      // Q, K, M
+  if (ROW) n += rows + NP + kPiece + (MODE != kChunkState ? 2 * half : rows);      // decays, G_32, g; late queries, early keys (first pass: K)
+  else n += 2 * (kPiece * kPieceLd + kPiece);                                    // D with G behind it and g, of this piece and of the next
+  return n;
+}
+
+template <int NT, int WAVES, int MODE, bool ROW>
+__global__ __launch_bounds__(64 * WAVES, 2) void recurrence_piece_kernel(RecurrenceArgs a, ChunkArgs ca, int vec) {
+  constexpr int NP = 16 * NT, LD = NP + 4, kThreads = 64 * WAVES, kQuads = (kPiece * NP / 4 + kThreads - 1) / kThreads;
+  constexpr bool kOut = MODE != kChunkState;                           // (kWhole: a sequence from the slot's state to the slot's state)
+  extern __shared__ __attribute__((aligned(16))) unsigned char piece_lds[];
+  float* KT = reinterpret_cast<float*>(piece_lds);                     // [NP][32]
+  float* VT = KT + NP * kPiece;                                        // [16 WAVES][32]
+  float* Q = VT + 16 * WAVES * kPiece;                                 // [32][LD]  (ROW: q, then G q)
+  float* K = kOut ? Q + kPiece * LD : Q;                               // [32][LD]
+  float* M = K + kPiece * LD;                                          // [32][kPieceLd]
+  float* rest = kOut ? M + kPiece * kPieceLd : ROW ? M : Q;
+  float* DR = rest;                                                    // ROW: [32][LD] decays
+  float* gC = DR + kPiece * LD;                                        // ROW: [NP]
+  float* gs = gC + NP;                                                 // ROW: [32] g
+  float* Q2 = gs + kPiece;                                             // ROW: [16][LD] late queries, decayed from token 16 on
+  float* K2 = Q2 + (kPiece / 2) * LD;                                  // ROW: [16][LD] early keys, decayed up to token 15
+  const int tid = threadIdx.x, lane = tid & 63, c16 = lane & 15, quad = lane >> 4;
+  const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+  const int head = blockIdx.x / a.pblocks, pb = blockIdx.x % a.pblocks;
+  int seq = blockIdx.y, local = 0;
+  if (MODE != kWhole && !find_chunk(a.cu_seqlens, ca.num_seqs, ca.chunk, blockIdx.y, seq, local)) return;
+  const int q_begin = a.cu_seqlens[seq], q_len = a.cu_seqlens[seq + 1] - q_begin;
+  if (q_len <= 0) return;
+  const int t_first = MODE == kWhole ? 0 : local * ca.chunk, t_last = MODE == kWhole ? q_len : min(t_first + ca.chunk, q_len);
+  const int kh = head / (a.heads / a.key_heads), ld = a.ld, p0 = pb * 16 * WAVES;
+  const int p = p0 + 16 * wave + c16;                                  // this lane's column of S
+  float* st = MODE == kWhole ? a.state + (size_t)a.state_slots[seq] * a.slot_stride + (size_t)head * a.N * ld
+                             : ca.ws_state + ((size_t)blockIdx.y * a.heads + head) * a.N * ld;
+  const bool from_state = MODE == kChunkOut || (MODE == kWhole && a.seq_starts[seq] > 0);
+  const bool live = p0 + 16 * wave < ld;                               // (the wavefront has columns)
+
+  f32x4 S[NT];
+#pragma unroll
+  for (int i = 0; i < NT; ++i)
+#pragma unroll
+    for (int r = 0; r < 4; ++r) {
+      const int n = 16 * i + 4 * quad + r;
+      S[i][r] = from_state && p < ld && n < a.N ? st[(size_t)n * ld + p] : 0.f;
+    }
+  const float skip = a.skip ? a.skip[head] : 0.f;
+  const float rate = a.raw ? expf(a.a_log[head]) : 0.f, raw_bias = a.raw ? a.raw_bias[head] : 0.f;
+
+  // D, G and g of a piece, by the last wavefront: lane j < 32 walks the tokens behind token j, lane 32 all of them.  What the
+  // walk reads is asked for a piece ahead.
+  float raw_a = 1.f, raw_g = 0.f;
+  auto ask_decays = [&](int t0) {
+    const bool in = lane < min(kPiece, t_last - t0);
+    const size_t row = (size_t)(q_begin + t0 + (in ? lane : 0));
+    if (a.raw) {
+      raw_a = in ? load_as_f32(a.raw, a.raw_dtype, row * a.raw_stride + head) : 0.f;
+      raw_g = in ? 1.f : 0.f;
+    } else {
+      raw_a = in ? a.decay[row * a.decay_stride + head] : 1.f;
+      raw_g = !in ? 0.f : a.vscale ? a.vscale[row * a.heads + head] : 1.f;
+    }
+  };
+  auto walk_decays = [&](float* D) {
+    float at = raw_a, gt = raw_g;
+    if (a.raw) {
+      const float z = raw_a + raw_bias, step = z > 20.f ? z : log1pf(expf(z));
+      at = raw_g == 0.f ? 1.f : expf(-rate * step);
+      gt *= step;
+    }
+    float d = lane == kPiece ? 1.f : 0.f;
+#pragma unroll 8
+    for (int t = 0; t < kPiece; ++t) {
+      d = lane == t ? 1.f : d * row_lane(at, t);
+      if (lane <= kPiece) D[t * kPieceLd + lane] = d;
+    }
+    if (lane < kPiece) D[kPiece * kPieceLd + lane] = gt;
+  };
+  float* D = rest;                                                     // !ROW
+  if (!ROW && wave == WAVES - 1) ask_decays(t_first);
+
+  f32x4 rq[kOut ? kQuads : 1], rk[kQuads], rd[ROW ? kQuads : 1], rv[2];
+  float rg = 1.f;                                                      // ROW: g of token tid
+  auto fetch = [&](int t0) {
+#pragma unroll
+    for (int e = 0; e < kQuads; ++e) {
+      const int at = tid + e * kThreads, t = at / (NP / 4), n = at % (NP / 4) * 4;
+      const bool in = t < kPiece && t0 + t < t_last;
+      const size_t row = (size_t)(q_begin + (in ? t0 + t : t_first));
+      const int most = in ? a.N : 0;
+      rk[e] = row_quad(a.k, a.qk_dtype, row * a.qk_stride + (size_t)kh * a.N + n, n, most, vec & kVecRows);
+      if (kOut) rq[e] = row_quad(a.q, a.qk_dtype, row * a.qk_stride + (size_t)kh * a.N + n, n, most, vec & kVecRows);
+      if (ROW) {
+        rd[e] = row_quad(a.row_decay, PLLM_F32, row * a.row_decay_stride + (size_t)head * a.N + n, n, most, vec & kVecDecay);
+        if (!in) rd[e] = f32x4{1.f, 1.f, 1.f, 1.f};
+      }
+    }
+#pragma unroll
+    for (int e = 0; e < 2; ++e) {
+      const int at = tid + e * kThreads, t = at / (4 * WAVES), col = p0 + at % (4 * WAVES) * 4;
+      const bool in = t0 + t < t_last;
+      const size_t row = (size_t)(q_begin + (in ? t0 + t : t_first));
+      rv[e] = row_quad(a.v, a.v_dtype, row * a.v_stride + (size_t)head * a.P + col, col, in ? a.P : 0, vec & kVecValues);
+#pragma unroll
+      for (int i = 0; i < 4; ++i)
+        if (in && ld > a.P && col + i == a.P) rv[e][i] = 1.f;          // the normaliser's column
+    }
+    if (ROW && tid < kPiece) rg = a.vscale && t0 + tid < t_last ? a.vscale[(size_t)(q_begin + t0 + tid) * a.heads + head] : 1.f;
+  };
+  fetch(t_first);
+  if (!ROW && wave == WAVES - 1) walk_decays(D);
+  float total = 1.f;                                                   // first pass: the product of the chunk's decays
+
+  for (int t0 = t_first; t0 < t_last; t0 += kPiece) {
+    const bool last = t0 + kPiece >= t_last;
+    __syncthreads();                                                   // the piece before is done with LDS
+    bool odd = false;                                                  // a value that is no number (see below)
+#pragma unroll
+    for (int e = 0; e < kQuads; ++e) {
+      const int at = tid + e * kThreads, t = at / (NP / 4), n = at % (NP / 4) * 4;
+      if (kPiece * NP / 4 % kThreads && t >= kPiece) break;
+      if (kOut) *reinterpret_cast<f32x4*>(Q + t * LD + n) = rq[e];
+      if (kOut || ROW) *reinterpret_cast<f32x4*>(K + t * LD + n) = rk[e];
+      if (ROW) *reinterpret_cast<f32x4*>(DR + t * LD + n) = rd[e];
+      if (!ROW) {
+#pragma unroll
+        for (int i = 0; i < 4; ++i) KT[token_quad(n + i, t >> 2) + (t & 3)] = rk[e][i];
+      }
+    }
+#pragma unroll
+    for (int e = 0; e < 2; ++e) {
+      const int at = tid + e * kThreads, t = at / (4 * WAVES), col = at % (4 * WAVES) * 4;
+#pragma unroll
+      for (int i = 0; i < 4; ++i) {
+        const float x = rv[e][i];
+        VT[token_quad(col + i, t >> 2) + (t & 3)] = x;
+        odd = odd || !(fabsf(x) < INFINITY);
+      }
+    }
+    if (ROW && tid < kPiece) gs[tid] = rg;
+    odd = kOut && __syncthreads_or(odd);
+    if (!kOut) __syncthreads();
+    if (!last) fetch(t0 + kPiece);
+    if (!ROW && wave == WAVES - 1 && !last) ask_decays(t0 + kPiece);
+
+    if constexpr (ROW) {
+      // Thread n < NP walks the tokens forward (queries), thread NP + n backward (keys).
+      for (int who = tid; who < 2 * NP; who += kThreads) {
+        const int n = who % NP;
+        if (who < NP) {
+          if (kOut) {
+            float from16 = 1.f;
+#pragma unroll 4
+            for (int t = kPiece / 2; t < kPiece; ++t) {
+              from16 *= DR[t * LD + n];
+              Q2[(t - kPiece / 2) * LD + n] = Q[t * LD + n] * from16;
+            }
+          }
+          float all = 1.f;
+#pragma unroll 4
+          for (int t = 0; t < kPiece; ++t) all *= DR[t * LD + n];
+          gC[n] = all;
+        } else {
+          float behind = 1.f;
+#pragma unroll 4
+          for (int t = kPiece - 1; t >= 0; --t) {
+            KT[token_quad(n, t >> 2) + (t & 3)] = K[t * LD + n] * behind * gs[t];
+            behind *= DR[t * LD + n];
+          }
+          if (kOut) {
+            float to15 = 1.f;
+#pragma unroll 4
+            for (int t = kPiece / 2 - 1; t >= 0; --t) {
+              K2[t * LD + n] = K[t * LD + n] * to15;
+              to15 *= DR[t * LD + n];
+            }
+          }
+        }
+      }
+      if constexpr (kOut) {
+        // The tiles of M on the diagonal: sixteen lanes share a key, NT of its rows each.
+        for (int who = tid; who < 512; who += kThreads) {
+          const int j = who >> 4, n = (who & 15) * NT, stop = (j & 16) + 16;
+          float w[NT];
+#pragma unroll
+          for (int i = 0; i < NT; ++i) w[i] = K[j * LD + n + i];
+          for (int t = j & 16; t < stop; ++t) {
+            float dot = 0.f;
+            if (t >= j) {
+#pragma unroll
+              for (int i = 0; i < NT; ++i) {
+                if (t > j) w[i] *= DR[t * LD + n + i];
+                dot = fmaf(w[i], Q[t * LD + n + i], dot);
+              }
+            }
+            dot += dpp_move<kDppSwap1>(dot);
+            dot += dpp_move<kDppSwap2>(dot);
+            dot += dpp_move<kDppHalfMirror>(dot);
+            dot += dpp_move<kDppMirror>(dot);
+            if ((who & 15) == 0) M[t * kPieceLd + j] = dot * gs[j];
+          }
+        }
+        __syncthreads();
+        for (int n = tid; n < NP; n += kThreads) {                     // (the diagonal is done with the plain queries)
+          float all = 1.f;
+#pragma unroll 4
+          for (int t = 0; t < kPiece; ++t) {
+            all *= DR[t * LD + n];
+            Q[t * LD + n] *= all;
+          }
+        }
+        if (wave == WAVES - 1) {                                       // late queries, early keys
+          const f32x4 m = dot_rows<NT>(K2 + c16 * LD + 4 * quad, Q2 + c16 * LD + 4 * quad);
+          *reinterpret_cast<f32x4*>(M + (16 + c16) * kPieceLd + 4 * quad) = m * lds_quad(gs + 4 * quad);
+        }
+      }
+      __syncthreads();
+    } else if constexpr (kOut) {
+      if (wave < 3) {
+        const int tt = wave > 0, jt = wave > 1;                        // tiles of M: (0, 0), (1, 0), (1, 1)
+        f32x4 m = dot_rows<NT>(K + (16 * jt + c16) * LD + 4 * quad, Q + (16 * tt + c16) * LD + 4 * quad);
+        const int t = 16 * tt + c16, j = 16 * jt + 4 * quad;
+        const f32x4 d = lds_quad(D + t * kPieceLd + j), g = lds_quad(D + kPiece * kPieceLd + j);
+#pragma unroll
+        for (int r = 0; r < 4; ++r) {
+          m[r] = j + r <= t ? m[r] * d[r] * g[r] : 0.f;
+        }
+        *reinterpret_cast<f32x4*>(M + t * kPieceLd + j) = m;
+      }
+    }
+    float* D_next = D == rest ? rest + kPiece * kPieceLd + kPiece : rest;
+    f32x4 v[2], y[2], carried[2];
+#pragma unroll
+    for (int f = 0; f < 2; ++f) {
+      v[f] = lds_quad(VT + token_quad(16 * wave + c16, 4 * f + quad));
+      y[f] = f32x4{0.f, 0.f, 0.f, 0.f};
+    }
+    if (kOut && live) {
+      f32x4 part[4][2];                                                // (four sums, as in dot_rows)
+#pragma unroll
+      for (int f = 0; f < 2; ++f) part[0][f] = part[1][f] = part[2][f] = part[3][f] = y[f];
+#pragma unroll
+      for (int i = 0; i < NT; ++i)
+#pragma unroll
+        for (int f = 0; f < 2; ++f) part[i & 3][f] = mfma16(S[i], lds_quad(Q + (16 * f + c16) * LD + 16 * i + 4 * quad), part[i & 3][f]);
+#pragma unroll
+      for (int f = 0; f < 2; ++f) {
+        carried[f] = (part[0][f] + part[1][f]) + (part[2][f] + part[3][f]);
+        if (!ROW) carried[f] *= D[(16 * f + c16) * kPieceLd + kPiece];
+      }
+    }
+    if ((MODE != kChunkOut || !last) && live) {
+      f32x4 vs[2];
+#pragma unroll
+      for (int f = 0; f < 2; ++f) {
+        vs[f] = v[f];
+        if (!ROW) vs[f] *= lds_quad(D + (kPiece - 1) * kPieceLd + 16 * f + 4 * quad) * lds_quad(D + kPiece * kPieceLd + 16 * f + 4 * quad);
+      }
+      const float g_all = ROW ? 1.f : D[(kPiece - 1) * kPieceLd + kPiece];
+#pragma unroll
+      for (int i = 0; i < NT; ++i) {
+        if (ROW) S[i] *= lds_quad(gC + 16 * i + 4 * quad);
+        else S[i] *= g_all;
+#pragma unroll
+        for (int f = 0; f < 2; ++f) S[i] = mfma16(lds_quad(KT + token_quad(16 * i + c16, 4 * f + quad)), vs[f], S[i]);
+      }
+    }
+    if (!ROW && wave == WAVES - 1 && !last) walk_decays(D_next);
+    if (!kOut) {
+      if (ROW) {
+        if (pb == 0 && tid < a.N) {
+          total *= gC[tid];
+          if (last) ca.ws_decay[((size_t)blockIdx.y * a.heads + head) * a.N + tid] = total;
+        }
+      } else if (pb == 0 && tid == 0) {
+        total *= D[(kPiece - 1) * kPieceLd + kPiece];
+        if (last) ca.ws_decay[(size_t)blockIdx.y * a.heads + head] = total;
+      }
+    }
+    if constexpr (kOut) {
+      if (!ROW) __syncthreads();                                       // M is whole
+      if (live) {
+        // (A weight of zero must not meet a value that is no number: such a value reaches its own token and later ones only.)
+        f32x4 fine[2] = {v[0], v[1]};
+        if (odd) {
+#pragma unroll
+          for (int f = 0; f < 2; ++f)
+#pragma unroll
+            for (int r = 0; r < 4; ++r)
+              if (!(fabsf(fine[f][r]) < INFINITY)) fine[f][r] = 0.f;
+#pragma unroll 1
+          for (int j = 0; j < kPiece; ++j)
+#pragma unroll
+            for (int r = 0; r < 4; ++r) {
+              const float x = VT[token_quad(16 * wave + 4 * quad + r, j >> 2) + (j & 3)];
+              if (fabsf(x) < INFINITY) continue;
+#pragma unroll
+              for (int f = 0; f < 2; ++f)
+                if (j <= 16 * f + c16) y[f][r] = fmaf(M[(16 * f + c16) * kPieceLd + j], x, y[f][r]);
+            }
+        }
+        y[0] = mfma16(fine[0], lds_quad(M + c16 * kPieceLd + 4 * quad), y[0]);
+        y[1] = mfma16(fine[0], lds_quad(M + (16 + c16) * kPieceLd + 4 * quad), y[1]);
+        y[1] += mfma16(fine[1], lds_quad(M + (16 + c16) * kPieceLd + 16 + 4 * quad), f32x4{0.f, 0.f, 0.f, 0.f});
+        const int col = p0 + 16 * wave + 4 * quad;
+#pragma unroll
+        for (int f = 0; f < 2; ++f) {
+          const int t = t0 + 16 * f + c16;
+          if (t >= t_last) continue;
+          y[f] += carried[f];
+          if (a.skip) {
+#pragma unroll
+            for (int r = 0; r < 4; ++r)
+              if (col + r < a.P) y[f][r] = fmaf(skip, VT[token_quad(16 * wave + 4 * quad + r, 4 * f + (c16 >> 2)) + (c16 & 3)], y[f][r]);
+          }
+          float* o = a.out + (size_t)(q_begin + t) * ((size_t)a.heads * ld) + (size_t)head * ld + col;
+          if ((vec & kVecOut) && col + 4 <= ld) {
+            *reinterpret_cast<f32x4*>(o) = y[f];
+          } else {
+#pragma unroll
+            for (int r = 0; r < 4; ++r)
+              if (col + r < ld) o[r] = y[f][r];
+          }
+        }
+      }
+    }
+    D = D_next;
+  }
+  if (MODE != kChunkOut && p < ld) {
+#pragma unroll
+    for (int i = 0; i < NT; ++i)
+#pragma unroll
+      for (int r = 0; r < 4; ++r) {
+        const int n = 16 * i + 4 * quad + r;
+        if (n < a.N) st[(size_t)n * ld + p] = S[i][r];
+      }
+  }
+}
+
+template <int NT, int WAVES, int MODE, bool ROW>
+static int launch_pieces(RecurrenceArgs a, const ChunkArgs& ca, int max_chunks, int vec, hipStream_t stream) {
+  constexpr size_t lds = (size_t)piece_lds_floats<NT, WAVES, MODE, ROW>() * sizeof(float);
+  auto kernel = recurrence_piece_kernel<NT, WAVES, MODE, ROW>;
+  if (lds > 64 * 1024) {
+    hipError_t e = hipFuncSetAttribute(reinterpret_cast<const void*>(kernel), hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds);
+    if (e != hipSuccess) return (int)e;
+  }
+  a.pblocks = (a.ld + 16 * WAVES - 1) / (16 * WAVES);
+  hipLaunchKernelGGL(kernel, dim3(a.heads * a.pblocks, max_chunks), dim3(64 * WAVES), lds, stream, a, ca, vec);
+  return (int)hipGetLastError();
+}
+
+// Wavefronts (tiles of 16 columns) of a workgroup: eight for tall states and for a decay per row, whose work per piece that
+// all columns share is large and whose LDS leaves room for one workgroup; else four, two workgroups to a compute unit (257
+// columns, a normaliser's: 55 us as four and one tile over, 75 us in workgroups of five, which do not pair up; 777 tokens).
+template <int MODE>
+static int launch_piece_pass(const RecurrenceArgs& a, const ChunkArgs& ca, int max_chunks, int vec, hipStream_t stream) {
+  const int tiles = (a.ld + 15) / 16;
+  if (a.row_decay) {
+    if (a.N <= 64) return tiles <= 4 ? launch_pieces<4, 4, MODE, true>(a, ca, max_chunks, vec, stream) : launch_pieces<4, 8, MODE, true>(a, ca, max_chunks, vec, stream);
+    return tiles <= 4 ? launch_pieces<8, 4, MODE, true>(a, ca, max_chunks, vec, stream) : launch_pieces<8, 8, MODE, true>(a, ca, max_chunks, vec, stream);
+  }
+  if (a.N > 128) return launch_pieces<16, 8, MODE, false>(a, ca, max_chunks, vec, stream);
+  return a.N > 64 ? launch_pieces<8, 4, MODE, false>(a, ca, max_chunks, vec, stream) : launch_pieces<4, 4, MODE, false>(a, ca, max_chunks, vec, stream);
+}
+
 // v_cols: P, or P - 1 for a recurrence with a normaliser (v holds P - 1 columns per head; column P - 1 of S holds
 // n_t = a_t n_(t-1) + g_t k_t, and the last element of a head's output n_t . q_t).
-// chunk == 0: every sequence token by token in one workgroup per (head, block of channels).  chunk > 0: the three passes
+// chunk == 0: every sequence token by token in one workgroup per (head, block of channels).  chunk < 0: the same in pieces of
+// 32 tokens, for states of up to 256 rows (128 with a decay per row).  chunk > 0: the three passes
 // over chunks of that many tokens; ws_state holds max_chunks * heads * N * P floats and ws_decay max_chunks * heads, with
 // max_chunks >= sum over the sequences of ceil(q_len / chunk) (total tokens / chunk + num_seqs is enough).
 PLLM_API int pllm_linear_recurrence(const void* q, const void* k, int qk_dtype, int qk_stride, const void* v, int v_dtype,
@@ -480,7 +915,7 @@ PLLM_API int pllm_linear_recurrence(const void* q, const void* k, int qk_dtype, 
   if (num_seqs <= 0) return 0;
   if (heads <= 0 || key_heads <= 0 || heads % key_heads || N <= 0 || N > 1024 || P <= 0 || (v_cols != P && v_cols != P - 1)) return -2;
   if ((raw && (!raw_bias || !a_log)) || (!raw && !decay && !row_decay) || (row_decay && (raw || decay || heads != key_heads))) return -2;
-  if (chunk < 0 || (chunk > 0 && (max_chunks <= 0 || max_chunks > 65535 || !ws_state || !ws_decay)) || num_seqs > 65535) return -2;
+  if ((chunk > 0 && (max_chunks <= 0 || max_chunks > 65535 || !ws_state || !ws_decay)) || num_seqs > 65535) return -2;
   RecurrenceArgs a;
   a.q = q; a.k = k; a.v = v; a.decay = decay; a.row_decay = row_decay; a.row_decay_stride = row_decay_stride; a.vscale = vscale; a.skip = skip; a.state = state;
   a.state_slots = state_slots; a.seq_starts = seq_starts; a.cu_seqlens = cu_seqlens; a.out = out;
@@ -489,13 +924,32 @@ PLLM_API int pllm_linear_recurrence(const void* q, const void* k, int qk_dtype, 
   a.decay_stride = decay_stride; a.heads = heads; a.key_heads = key_heads; a.N = N; a.P = v_cols; a.ld = P; a.pblocks = (v_cols + 63) / 64;
   ChunkArgs ca{ws_state, ws_decay, chunk, num_seqs};
   const int waves = (N + 63) / 64, need = (N + waves - 1) / waves;   // rows of S per wave
+  const bool pieces = N <= (row_decay ? 128 : 256);
+  auto wide = [](const void* p, int dtype, long stride) { return (reinterpret_cast<uintptr_t>(p) & (dtype == PLLM_F32 ? 15 : 7)) == 0 && stride % 4 == 0; };
+  const int vec = (N % 4 == 0 && wide(q, qk_dtype, qk_stride) && wide(k, qk_dtype, qk_stride) ? kVecRows : 0) |
+                  (v_cols % 4 == 0 && wide(v, v_dtype, v_stride) ? kVecValues : 0) | (P % 4 == 0 && wide(out, PLLM_F32, 0) ? kVecOut : 0) |
+                  (row_decay && N % 4 == 0 && wide(row_decay, PLLM_F32, row_decay_stride) ? kVecDecay : 0);
+  if (chunk < 0) {
+    if (!pieces) return -2;
+    return launch_piece_pass<kWhole>(a, ca, num_seqs, vec, stream);
+  }
   if (chunk == 0) {
     launch_recurrence<kWhole>(a, ca, dim3(heads * a.pblocks, num_seqs), waves, need, stream);
   } else {
-    launch_recurrence<kChunkState>(a, ca, dim3(heads * a.pblocks, max_chunks), waves, need, stream);
+    if (pieces) {
+      const int code = launch_piece_pass<kChunkState>(a, ca, max_chunks, vec, stream);
+      if (code) return code;
+    } else {
+      launch_recurrence<kChunkState>(a, ca, dim3(heads * a.pblocks, max_chunks), waves, need, stream);
+    }
     const size_t per_seq = (size_t)heads * N * P;     // (P: all columns of a row of S, the normaliser's among them)
     hipLaunchKernelGGL(recurrence_carry_kernel, dim3((unsigned)((per_seq + 255) / 256), num_seqs), dim3(256), 0, stream, a, ca);
-    launch_recurrence<kChunkOut>(a, ca, dim3(heads * a.pblocks, max_chunks), waves, need, stream);
+    if (pieces) {
+      const int code = launch_piece_pass<kChunkOut>(a, ca, max_chunks, vec, stream);
+      if (code) return code;
+    } else {
+      launch_recurrence<kChunkOut>(a, ca, dim3(heads * a.pblocks, max_chunks), waves, need, stream);
+    }
   }
   PLLM_RETURN_LAST_ERROR();
 }
