@@ -949,6 +949,13 @@ def attention_plan(num_seqs: int, num_kv_heads: int, max_q_len: int, max_k_len: 
     # fewer, longer work items are faster than many short ones plus a larger merge.
     items = num_seqs * num_kv_heads
     want_parts = max(1, compute_units // items)
+    # Up to 512 keys and 16 query columns eight wavefronts take everything in one piece, a block of 64 keys each: a merge by a
+    # second kernel costs more than half the keys to a workgroup give (1 / 8 sequences x 4 kv heads at head size 64, context 182:
+    # 6.5 / 6.6 us against 9.0 / 9.2 in two partitions of 256; context 500 8.4 against 9.5; at head size 128 13.3 against 13.7).
+    # From a bound of 1,024 on the partitions are ahead (context 1,000: 9.3 / 10.3 against 12.9 / 13.5), and so they are with more
+    # columns or larger heads, whose blocks are more work (5 rows at head size 128: 20.4 against 25.0).
+    if 256 < max_k_len <= 512 and cols <= 16 and max_waves == 8 and items <= compute_units:
+        return 8, 0, 1
     size = 256                                        # at least four blocks of 64 keys per workgroup
     while (max_k_len + size - 1) // size > want_parts:
         size *= 2
