@@ -54,6 +54,8 @@ struct StreamLinearParams {
   int ksteps;                 // K / 32
   int num_stages;             // stages of 256 columns that K has
   int stages_per_split;
+  int n_blocks, m_blocks;     // the tiled kernel: blocks of weight rows, blocks of input rows
+  int weights_once;           // the tiled kernel: the weights need not stay in the caches
   // SL_ROPE_KV: W = [q; k; v] rows tiled in units of 8 lower-half elements of a head and their 8 partners
   const int* positions; const float* cos_t; const float* sin_t; const int* slots;
   bf16* k_pages; bf16* v_pages;
@@ -364,22 +366,29 @@ PLLM_API int pllm_stream_linear(int epi, const void* x, int ldx, const void* wt,
 }
 
 // ---------------------------------------------------------------------------------------------
-// The same products for a few hundred rows (steps that hold a prompt portion, short prompts): tiles of up to 128 input
-// rows x 128 weight rows per workgroup, along x the blocks of weight rows, along y the blocks of input rows, along z
-// ranges of K.  With this many rows every workgroup of the kernel above would read all of them for its 32 weight rows;
+// The same products for a few hundred rows (steps that hold a prompt portion, short prompts): tiles of up to 160 input
+// rows x 128 weight rows per workgroup, along x the blocks of weight rows and of input rows, along z ranges of K.  With this many rows every workgroup of the kernel above would read all of them for its 32 weight rows;
 // here both operands of a stage (64 columns of K) come into LDS once per workgroup, brought by the four loader
 // wavefronts (the weights' tiles are 1 KB of contiguous memory each and land in operand order; the rows as above), and
 // the eight compute wavefronts, as 2 x 4 over the tile (MTW tiles of 16 input rows x 2 blocks of 16 weight rows each),
 // only read LDS and multiply.  No sums across wavefronts: each owns its outputs.  Epilogues as above.
 constexpr int kTileBlocksN = 8;                      // blocks of 16 weight rows per workgroup, at most (NB: 8 or 4)
 constexpr int kTileStageSteps = 2;                   // steps of 32 columns per stage
+constexpr int kReadOnce = 2;                         // a load's cache policy: nt, the line is the first to leave the caches
 
 // MT: tiles of 16 input rows per workgroup (the upper row of wavefronts takes the larger half).
-// What bounds a workgroup is what its compute unit can draw from the L2 (about 28 bytes a cycle when all compute units
-// draw: cycle stamps show the loaders' requests queueing, a stage of 34 KB taking 1,250 cycles, whatever the number of
-// stages in flight, with or without the products; four compute wavefronts as 2 x 2 with a third less LDS traffic took the
-// same time), so a tile is as large as registers and LDS allow, and matrices of many rows and few hundred input rows,
-// whose tiles cannot be large in both directions, stay with the library, which meets the same bound.
+// What bounds it is what the chiplets fetch from behind their L2s: about 7 TB/s for all of them, from the Infinity Cache as from
+// HBM, whatever is in flight (a kernel of loads alone), where lines that hit the L2 come at 35.  With the LDS reads and the products
+// taken out the kernel takes as long as with them (256 x 28672 x 4096: 88 us of 90), and so it does with the next stage's
+// operands read during the products.  Hence:
+//   * workgroups that read the same weights (the blocks of input rows of one block of weight rows) follow each other on one
+//     chiplet (workgroup i runs on chiplet i % 8): groups of 8 blocks of weight rows x all blocks of input rows.  With the
+//     blocks of input rows a whole grid apart, 264 rows x 28672 x 4096 drew its 235 MB of weights twice: 102 us against 92;
+//   * an input row's 128 bytes of a stage are one line of one load (8 rows to a load, their eight pieces XOR-ed by the row so that
+//     operand reads meet no bank twice): with 64 bytes of 16 rows to a load every line was asked for twice (777 x 2048 x 2080:
+//     16.2 against 14.3 us, 512 x 2560 x 2048 14.7 and 12.9, 264 x 4096 x 4096 18.7 and 17.5);
+//   * weights of large matrices leave the L2 first (kReadOnce), so that they do not push out the rows that all
+//     workgroups share (24 x 28672 x 4096: 49.4 against 43.7 us, 264 x 4096 x 4096 17.5 and 17.1).
 template <int EPI, int MT, int R, int NB>
 __global__ __launch_bounds__(kStreamThreads) void tile_linear_kernel(const StreamLinearParams p) {
   constexpr int CW = kComputeWaves;
@@ -389,14 +398,16 @@ __global__ __launch_bounds__(kStreamThreads) void tile_linear_kernel(const Strea
   constexpr int kWBlocks = NB * kTileStageSteps, kXBlocks = MT * kTileStageSteps;
   constexpr int kSlotBytes = (kWBlocks + kXBlocks) * 1024;
   const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
-  const int nb = blockIdx.x, row0 = blockIdx.y * (MT * 16), split = blockIdx.z;
+  // (the last group has fewer than 8 blocks of weight rows where their number is no multiple of 8)
+  const int group = blockIdx.x / (8 * p.m_blocks), in_group = blockIdx.x - group * 8 * p.m_blocks, across = min(8, p.n_blocks - group * 8);
+  const int nb = group * 8 + in_group % across, row0 = in_group / across * (MT * 16), split = blockIdx.z;
   const int first_stage = split * p.stages_per_split;           // (stages of 64 columns here)
   const int nstages = min(p.stages_per_split, p.num_stages - first_stage);
   floatx4 acc[MTW][NTW];
 
   if (wave >= CW) {
     const int l = wave - CW;
-    const int xr = lane >> 2, xg = (lane & 3) ^ (xr >> 2);
+    const int xr = lane >> 3, xg = (lane & 7) ^ xr;
     constexpr int kBlocks = kWBlocks + kXBlocks, kPerLoader = (kBlocks + kLoaderWaves - 1) / kLoaderWaves;
     static_assert(kWBlocks % kLoaderWaves == 0, "a loader's i-th block is a weight tile for all loaders or for none");
     // A loader's i-th block of a stage is the same block in every stage, kAdvance further along K: the addresses of the
@@ -411,11 +422,23 @@ __global__ __launch_bounds__(kStreamThreads) void tile_linear_kernel(const Strea
         const int u = bb / kTileStageSteps, st = bb - u * kTileStageSteps;
         base[i] = p.wt + (((size_t)(nb * NB + u) * p.ksteps + first_stage * kTileStageSteps + st) * 64 + lane) * 8;
       } else {
-        const int bx = bb - kWBlocks, t = bx / kTileStageSteps, st = bx - t * kTileStageSteps;
-        const int row = min(row0 + t * 16 + xr, p.M - 1);        // rows past M repeat the last one: never stored
-        base[i] = p.x + (size_t)row * p.ldx + (first_stage * kTileStageSteps + st) * kChunkK + xg * 8;
+        const int row = min(row0 + (bb - kWBlocks) * 8 + xr, p.M - 1);   // rows past M repeat the last one: never stored
+        base[i] = p.x + (size_t)row * p.ldx + first_stage * kTileStageSteps * kChunkK + xg * 8;
       }
     }
+    auto issue_blocks = [&](int s, unsigned char* slot, bool once) {        // (called with constants: two loops without a condition)
+      constexpr int kTileAdvance = kTileStageSteps * kTileElems, kRowAdvance = kTileStageSteps * kChunkK;
+#pragma unroll
+      for (int i = 0; i < kPerLoader; ++i) {
+        const int bb = min(l + i * kLoaderWaves, kBlocks - 1);
+        const bool weight = i * kLoaderWaves < kWBlocks;
+        const bf16* src = base[i] + (size_t)s * (weight ? kTileAdvance : kRowAdvance);
+        if (weight && once) __builtin_amdgcn_global_load_lds((const __attribute__((address_space(1))) void*)src,
+                                                             (__attribute__((address_space(3))) void*)(slot + bb * 1024), 16, 0, kReadOnce);
+        else __builtin_amdgcn_global_load_lds((const __attribute__((address_space(1))) void*)src,
+                                              (__attribute__((address_space(3))) void*)(slot + bb * 1024), 16, 0, 0);
+      }
+    };
     const bool odd_steps = p.ksteps & 1;                         // K no multiple of 64: the last stage has one step only
     auto issue = [&](int s) {
       unsigned char* slot = sl_lds + (s % R) * kSlotBytes;
@@ -427,20 +450,14 @@ __global__ __launch_bounds__(kStreamThreads) void tile_linear_kernel(const Strea
           const int bb = min(l + i * kLoaderWaves, kBlocks - 1);
           const bf16* src;
           if (bb < kWBlocks) src = p.wt + (((size_t)(nb * NB + bb / kTileStageSteps) * p.ksteps + ks0) * 64 + lane) * 8;
-          else src = p.x + (size_t)min(row0 + ((bb - kWBlocks) / kTileStageSteps) * 16 + xr, p.M - 1) * p.ldx + ks0 * kChunkK + xg * 8;
+          else src = p.x + (size_t)min(row0 + (bb - kWBlocks) * 8 + xr, p.M - 1) * p.ldx + ks0 * kChunkK + (xg & 3) * 8;
           __builtin_amdgcn_global_load_lds((const __attribute__((address_space(1))) void*)src,
                                            (__attribute__((address_space(3))) void*)(slot + bb * 1024), 16, 0, 0);
         }
         return;
       }
-#pragma unroll
-      for (int i = 0; i < kPerLoader; ++i) {
-        const int bb = min(l + i * kLoaderWaves, kBlocks - 1);
-        constexpr int kTileAdvance = kTileStageSteps * kTileElems, kRowAdvance = kTileStageSteps * kChunkK;
-        const bf16* src = base[i] + (size_t)s * (i * kLoaderWaves < kWBlocks ? kTileAdvance : kRowAdvance);
-        __builtin_amdgcn_global_load_lds((const __attribute__((address_space(1))) void*)src,
-                                         (__attribute__((address_space(3))) void*)(slot + bb * 1024), 16, 0, 0);
-      }
+if (p.weights_once) issue_blocks(s, slot, true);
+      else issue_blocks(s, slot, false);
     };
 #pragma unroll
     for (int s = 0; s < R - 1; ++s) {
@@ -465,7 +482,8 @@ __global__ __launch_bounds__(kStreamThreads) void tile_linear_kernel(const Strea
     const int my_tiles = wm == 0 ? MTW : MT - MTW;               // (the same for the whole wavefront)
     const int r = lane & 15, g = lane >> 4;
     const unsigned char* my_w = sl_lds + (wn * NTW * kTileStageSteps) * 1024 + lane * 16;
-    const unsigned char* my_x = sl_lds + (kWBlocks + wm * MTW * kTileStageSteps) * 1024 + (r * 4 + (g ^ (r >> 2))) * 16;
+    const unsigned char* my_x = sl_lds + (kWBlocks + wm * MTW * kTileStageSteps) * 1024 + r * 128;
+    const int my_piece[kTileStageSteps] = {(g ^ (r & 7)) * 16, ((4 + g) ^ (r & 7)) * 16};
     int slot = 0;
     for (int s = 0; s < nstages; ++s) {
       stage_barrier();
@@ -480,7 +498,7 @@ __global__ __launch_bounds__(kStreamThreads) void tile_linear_kernel(const Strea
         for (int u = 0; u < NTW; ++u) wf[st][u] = *reinterpret_cast<const bf16x8*>(my_w + slot * kSlotBytes + (u * kTileStageSteps + st) * 1024);
         // (the lower row of wavefronts may have a tile less: it reads its last tile again and leaves the product out)
 #pragma unroll
-        for (int t = 0; t < MTW; ++t) xf[st][t] = *reinterpret_cast<const bf16x8*>(my_x + slot * kSlotBytes + (min(t, my_tiles - 1) * kTileStageSteps + st) * 1024);
+        for (int t = 0; t < MTW; ++t) xf[st][t] = *reinterpret_cast<const bf16x8*>(my_x + slot * kSlotBytes + min(t, my_tiles - 1) * kTileStageSteps * 1024 + my_piece[st]);
       }
       asm volatile("" ::: "memory");
 #pragma unroll
@@ -701,8 +719,12 @@ PLLM_API int pllm_tile_linear(int epi, const void* x, int ldx, const void* wt, v
   const int rows = (M + m_blocks - 1) / m_blocks, mt = tile_rows_compiled(rows);     // tiles of 16 rows per workgroup: 2 to 10
   m_blocks = (M + mt * 16 - 1) / (mt * 16);                                     // (blocks are filled to whole tiles, the last one may be short)
   const int n_blocks = ((rows_of_w + 15) / 16 + nb_per - 1) / nb_per;
-  if (m_blocks > 65535 || splits > 65535) return -2;
-  const dim3 grid(n_blocks, m_blocks, splits);
+  if ((long)n_blocks * m_blocks > 0x7fffffffL / kStreamThreads || splits > 65535) return -2;
+  p.n_blocks = n_blocks; p.m_blocks = m_blocks;
+  // Weights are read once and let go from 32 MB a matrix on: a model of such matrices does not fit the Infinity Cache's 256 MB
+  // anyway.  Smaller ones may stay there from step to step (33 x 2048 x 5632, two matrices in turn: 18.8 us kept, 21.3 let go).
+  p.weights_once = (long)rows_of_w * K >= (16L << 20);
+  const dim3 grid(n_blocks * m_blocks, 1, splits);
   // (the kernel's row offset of a block along y is MT * 16: blocks are filled to whole tiles, the last one may be short)
 #define PLLM_TL(EPI_, MT_)                                                                       \
   do {                                                                                           \

@@ -1115,6 +1115,19 @@ def test_tile_linear_plain_float_and_partial(m, n, k):
     assert torch.equal(alone.cpu(), o.tile_linear(x.cuda(), tiled, o.SL_F32)[m // 2:m // 2 + 5].cpu())     # a row's sums do not depend on the others
 
 
+@pytest.mark.parametrize("m", [24, 161, 481])
+def test_tile_linear_many_blocks_of_a_large_matrix(m):
+    """66 blocks of weight rows (no multiple of the eight that a group holds) x one to four blocks of input rows, a K that ends
+    within a stage, and weights large enough to be let go by the caches."""
+    o = ops()
+    n, k = 8330, 2080
+    x, w = rnd(m, k, seed=74, dtype=torch.bfloat16), rnd(n, k, seed=75, dtype=torch.bfloat16)
+    tiled = o.tile_weight(w.cuda())
+    want = x.double() @ w.double().T
+    assert rel_err(o.tile_linear(x.cuda(), tiled, o.SL_F32), want) <= 2e-5
+    assert rel_err(o.tile_linear(x.cuda(), tiled, o.SL_PARTIAL, splits=3).double().sum(0), want) <= 2e-5
+
+
 def test_tile_shapes_of_the_tiled_kernel():
     """A product in one range of K takes the tile shape with the most workgroups in one round of the compute units; the
     largest tiles when none fits; blocks of rows always cover the rows."""
