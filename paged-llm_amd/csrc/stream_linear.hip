@@ -56,6 +56,7 @@ struct StreamLinearParams {
   int stages_per_split;
   int n_blocks, m_blocks;     // the tiled kernel: blocks of weight rows, blocks of input rows
   int weights_once;           // the tiled kernel: the weights need not stay in the caches
+  int weight_blocks;          // the tiled kernel: blocks of 16 weight rows there are (a multiple of 8)
   // SL_ROPE_KV: W = [q; k; v] rows tiled in units of 8 lower-half elements of a head and their 8 partners
   const int* positions; const float* cos_t; const float* sin_t; const int* slots;
   bf16* k_pages; bf16* v_pages;
@@ -372,7 +373,7 @@ PLLM_API int pllm_stream_linear(int epi, const void* x, int ldx, const void* wt,
 // wavefronts (the weights' tiles are 1 KB of contiguous memory each and land in operand order; the rows as above), and
 // the eight compute wavefronts, as 2 x 4 over the tile (MTW tiles of 16 input rows x 2 blocks of 16 weight rows each),
 // only read LDS and multiply.  No sums across wavefronts: each owns its outputs.  Epilogues as above.
-constexpr int kTileBlocksN = 8;                      // blocks of 16 weight rows per workgroup, at most (NB: 8 or 4)
+constexpr int kTileBlocksN = 8;                      // blocks of 16 weight rows per workgroup (NB: 8, 4, or 16 for gated products)
 constexpr int kTileStageSteps = 2;                   // steps of 32 columns per stage
 constexpr int kReadOnce = 2;                         // a load's cache policy: nt, the line is the first to leave the caches
 
@@ -419,8 +420,8 @@ __global__ __launch_bounds__(kStreamThreads) void tile_linear_kernel(const Strea
       const int bb = min(l + i * kLoaderWaves, kBlocks - 1);     // (every loader issues the same number of loads per stage: the waits
                                                                  //  below count them; a loader whose share is one short repeats its last block)
       if (bb < kWBlocks) {
-        const int u = bb / kTileStageSteps, st = bb - u * kTileStageSteps;
-        base[i] = p.wt + (((size_t)(nb * NB + u) * p.ksteps + first_stage * kTileStageSteps + st) * 64 + lane) * 8;
+        const int u = bb / kTileStageSteps, st = bb - u * kTileStageSteps;       // (NB 16: blocks past the last repeat it, never stored)
+        base[i] = p.wt + (((size_t)min(nb * NB + u, p.weight_blocks - 1) * p.ksteps + first_stage * kTileStageSteps + st) * 64 + lane) * 8;
       } else {
         const int row = min(row0 + (bb - kWBlocks) * 8 + xr, p.M - 1);   // rows past M repeat the last one: never stored
         base[i] = p.x + (size_t)row * p.ldx + first_stage * kTileStageSteps * kChunkK + xg * 8;
@@ -449,7 +450,7 @@ __global__ __launch_bounds__(kStreamThreads) void tile_linear_kernel(const Strea
         for (int i = 0; i < kPerLoader; ++i) {
           const int bb = min(l + i * kLoaderWaves, kBlocks - 1);
           const bf16* src;
-          if (bb < kWBlocks) src = p.wt + (((size_t)(nb * NB + bb / kTileStageSteps) * p.ksteps + ks0) * 64 + lane) * 8;
+          if (bb < kWBlocks) src = p.wt + (((size_t)min(nb * NB + bb / kTileStageSteps, p.weight_blocks - 1) * p.ksteps + ks0) * 64 + lane) * 8;
           else src = p.x + (size_t)min(row0 + (bb - kWBlocks) * 8 + xr, p.M - 1) * p.ldx + ks0 * kChunkK + (xg & 3) * 8;
           __builtin_amdgcn_global_load_lds((const __attribute__((address_space(1))) void*)src,
                                            (__attribute__((address_space(3))) void*)(slot + bb * 1024), 16, 0, 0);
@@ -677,7 +678,19 @@ static void tile_shape(int M, int weight_blocks16, int cus, int* m_blocks_out, i
   }
 }
 
-// What `tile_shape` chooses for M input rows and a matrix of `weight_rows` rows on `compute_units` compute units: rows per
+// A gated product whose tiles of 128 weight rows need more than one round of the compute units takes tiles of 256 where those need
+// one: a compute unit draws a stage at the same rate whatever its tile, and the tile of 144 x 256 draws 50 KB for twice the
+// products of the 34 KB of 144 x 128 (200 / 264 / 320 rows x 28672 x 4096:
+// 78 / 81 / 83 us against 92 / 93 / 97, where the library takes 72 / 78 / 77 and 6 more for the activation; 264 x 24576 x 2048 43
+// against 50).  Three stages of it fill the LDS, and its wavefronts' sums and operands 160 registers.  Where tiles of 256 need a second
+// round they gain nothing (264 x 36864 x 2048: 76.3 and 76.4), and blocks of up to 96 rows stay with 128, of which more run at once.
+static bool wide_takes(int m_blocks, int mt, int weight_blocks16, int cus) {
+  const long tiles = (long)m_blocks * ((weight_blocks16 + kTileBlocksN - 1) / kTileBlocksN);
+  const long wide_tiles = (long)m_blocks * ((weight_blocks16 + 2 * kTileBlocksN - 1) / (2 * kTileBlocksN));
+  return mt >= 8 && tiles > cus && wide_tiles <= cus;
+}
+
+// What `tile_shape` chooses, before `wide_takes` doubles a gated product's tiles, for M input rows and a matrix of `weight_rows` rows on `compute_units` compute units: rows per
 // block of input rows (a multiple of 16) and weight rows per tile (128 or 64); returns the number of workgroups.
 PLLM_API int pllm_tile_linear_shape(int M, int weight_rows, int compute_units, int* block_rows, int* tile_weight_rows) {
   if (M <= 0 || weight_rows <= 0 || compute_units <= 0) return -2;
@@ -718,9 +731,11 @@ PLLM_API int pllm_tile_linear(int epi, const void* x, int ldx, const void* wt, v
   const bool narrow = nb_per != kTileBlocksN;
   const int rows = (M + m_blocks - 1) / m_blocks, mt = tile_rows_compiled(rows);     // tiles of 16 rows per workgroup: 2 to 10
   m_blocks = (M + mt * 16 - 1) / (mt * 16);                                     // (blocks are filled to whole tiles, the last one may be short)
+  const bool wide = epi == SL_GATED && wide_takes(m_blocks, mt, (rows_of_w + 15) / 16, num_compute_units());
+  if (wide) nb_per = 2 * kTileBlocksN;
   const int n_blocks = ((rows_of_w + 15) / 16 + nb_per - 1) / nb_per;
   if ((long)n_blocks * m_blocks > 0x7fffffffL / kStreamThreads || splits > 65535) return -2;
-  p.n_blocks = n_blocks; p.m_blocks = m_blocks;
+  p.n_blocks = n_blocks; p.m_blocks = m_blocks; p.weight_blocks = weight_blocks;
   // Weights are read once and let go from 32 MB a matrix on: a model of such matrices does not fit the Infinity Cache's 256 MB
   // anyway.  Smaller ones may stay there from step to step (33 x 2048 x 5632, two matrices in turn: 18.8 us kept, 21.3 let go).
   p.weights_once = (long)rows_of_w * K >= (16L << 20);
@@ -728,6 +743,9 @@ PLLM_API int pllm_tile_linear(int epi, const void* x, int ldx, const void* wt, v
   // (the kernel's row offset of a block along y is MT * 16: blocks are filled to whole tiles, the last one may be short)
 #define PLLM_TL(EPI_, MT_)                                                                       \
   do {                                                                                           \
+    if constexpr ((MT_) >= 8 && (EPI_) == SL_GATED) {                                            \
+      if (wide) return launch_tile<EPI_, MT_, 3, 2 * kTileBlocksN>(p, grid, stream);             \
+    }                                                                                            \
     if constexpr ((MT_) <= 8) {                                                                  \
       if (narrow) return launch_tile<EPI_, MT_, 4, kTileBlocksN / 2>(p, grid, stream);           \
     }                                                                                            \

@@ -1128,6 +1128,20 @@ def test_tile_linear_many_blocks_of_a_large_matrix(m):
     assert rel_err(o.tile_linear(x.cuda(), tiled, o.SL_PARTIAL, splits=3).double().sum(0), want) <= 2e-5
 
 
+@pytest.mark.parametrize("m", [100, 250, 264, 300])
+def test_tile_linear_gated_in_wide_tiles(m):
+    """Matrices whose tiles of 128 weight rows need a second round take tiles of 256; the last of them reaches past the padded
+    matrix (1,080 blocks of 16 rows, no multiple of 16).  (100 rows: one block of rows, and tiles of 128 as before.)"""
+    o = ops()
+    inter, k = 8600, 96
+    assert (o.tile_linear_shape(m, 2 * inter, 256)[2] > 256) == (m > 160)
+    x, w = rnd(m, k, seed=76, dtype=torch.bfloat16), rnd(2 * inter, k, seed=77, dtype=torch.bfloat16, scale=k ** -0.5)
+    tiled = o.tile_weight(w.cuda(), "gated")
+    assert tiled.blocks == 1080
+    want = torch.nn.functional.silu(x.double() @ w[:inter].double().T) * (x.double() @ w[inter:].double().T)
+    assert rel_err(o.tile_linear(x.cuda(), tiled, o.SL_GATED), want) <= 1e-2
+
+
 def test_tile_shapes_of_the_tiled_kernel():
     """A product in one range of K takes the tile shape with the most workgroups in one round of the compute units; the
     largest tiles when none fits; blocks of rows always cover the rows."""
