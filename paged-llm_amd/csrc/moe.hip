@@ -592,7 +592,7 @@ __global__ __launch_bounds__(256) void moe_expert_splitk_kernel(const bf16* __re
   }
 }
 
-// Prompt steps with 128 pairs or more per expert: a workgroup is a tile of 128 rows of one expert times 128 weight rows
+// Prompt steps whose tiles have 128 rows, for K that are no multiple of 64 (the kernel below takes the others): a workgroup is a tile of 128 rows of one expert times 128 weight rows
 // (gated: 64 of the gate's and the 64 of the up product that belong to them), staged through LDS in k-steps of 64, two
 // buffers deep: every thread fetches eight pieces of 16 bytes of the steps ahead into registers while the matrix cores
 // work on this one, and stores a step's pieces behind the products of the step before; one barrier a step, which waits
@@ -759,14 +759,186 @@ __global__ __launch_bounds__(256) void moe_expert_tile_kernel(const bf16* __rest
   }
 }
 
+// The same prompt steps where K is a multiple of 64: a tile of 128 rows of one expert times NB blocks of 16 weight rows (gated: a
+// gate's block and its up block in turn), eight wavefronts that multiply and four that bring the operands: stages of 64 columns
+// go from memory straight into LDS, R stages deep, a load taking the whole 128-byte lines of eight rows, whose eight pieces
+// lie XOR-ed by the row so that operand reads meet no bank twice.  Workgroups that follow each other on a chiplet
+// (i, i + 8, ...) take the tiles of one block of weight rows in turn, so that the tiles of an expert find its weights in their L2.
+// The kernel above draws half lines through registers, in an order that spreads an expert's tiles over all chiplets (both
+// products together, us, above / here: 1,178 tokens with 2 of 8 plain experts of 4,096 at width 2,048 225 / 143; 777 with 2 of 8 gated
+// ones of 2,048 157 / 73; 2,048 with 4 of 30 gated ones of 1,408 370 / 236; 300 with 2 of 8 plain ones of 4,096 145 / 82).
+// What bounds it is the drawing of the operands, as in the tiled products of whole steps: the compute unit's rate is the same
+// whatever the tile, so a tile of 256 weight rows (48 KB a stage) takes the place of two of 128 (64 KB) where that needs no more
+// rounds.  The sums run over ascending k in one accumulator per output, as in the kernels above, and give the same bits.
+constexpr int kStageThreads = 768;
+
+template <int N_>
+__device__ __forceinline__ void wait_loads_but() {            // until at most N_ of this wavefront's loads are still under way
+  static_assert(N_ >= 0 && N_ < 64, "vmcnt has six bits");
+  __builtin_amdgcn_s_waitcnt((N_ & 0xf) | ((N_ >> 4) << 14) | 0x0f70);
+}
+
+template <int FORM, int NB>
+__global__ __launch_bounds__(kStageThreads) void moe_expert_stage_kernel(const bf16* __restrict__ rows_in, int ld_in, const bf16* __restrict__ w,
+                                                                         const int* __restrict__ tiles, int max_tiles, const int* __restrict__ sorted_pair, int top,
+                                                                         int n_out, int K, void* __restrict__ out_, int ld_out, int act,
+                                                                         const float* __restrict__ pair_scale) {
+  constexpr bool GATED = FORM == kFormGated, FIRST = FORM != kFormDown;      // FIRST: from the tokens' rows, activated
+  constexpr int kOutputs = GATED ? NB * 8 : NB * 16, R = NB > 8 ? 3 : 4, NTW = NB / 4, MTW = 4;
+  constexpr int kWLoads = NB * 2, kLoads = kWLoads + kBigRows / 8, kPerLoader = kLoads / 4, kSlotBytes = kLoads * 1024;
+  static_assert(kLoads % 4 == 0 && kWLoads % 4 == 0, "the loaders' shares are equal");
+  extern __shared__ __attribute__((aligned(16))) unsigned char stages_lds[];
+  const int n_blocks = (n_out + kOutputs - 1) / kOutputs;
+  const int group = blockIdx.x / (8 * max_tiles), in_group = blockIdx.x - group * 8 * max_tiles, across = min(8, n_blocks - group * 8);
+  const int tile = in_group / across, n0 = (group * 8 + in_group - tile * across) * kOutputs;
+  const int expert = tiles[3 * tile], row0 = tiles[3 * tile + 1], nrows = tiles[3 * tile + 2];
+  if (nrows <= 0) return;                                    // the whole workgroup: no barrier is left behind
+  const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  const int nstages = K >> 6;
+  if (wave >= 8) {
+    const int l = wave - 8, lr = lane >> 3, lp = ((lane & 7) ^ lr) * 8;
+    const bf16* we = w + (size_t)expert * (GATED ? 2 : 1) * n_out * K;
+    const bf16* base[kPerLoader];
+#pragma unroll
+    for (int i = 0; i < kPerLoader; ++i) {
+      const int b = l + 4 * i;
+      if (4 * i < kWLoads) {
+        const int u = b >> 1, in_block = (b & 1) * 8 + lr;
+        const int row = GATED ? min(n0 + (u >> 1) * 16 + in_block, n_out - 1) + (u & 1) * n_out : min(n0 + u * 16 + in_block, n_out - 1);
+        base[i] = we + (size_t)row * K + lp;                 // (outputs past the last repeat it: never stored)
+      } else {
+        const int rr = row0 + min((b - kWLoads) * 8 + lr, nrows - 1);        // rows past the tile's last repeat it: never stored
+        base[i] = rows_in + (size_t)(FIRST ? sorted_pair[rr] / top : rr) * ld_in + lp;
+      }
+    }
+    auto issue = [&](int s) {
+      unsigned char* slot = stages_lds + (s % R) * kSlotBytes;
+#pragma unroll
+      for (int i = 0; i < kPerLoader; ++i)
+        __builtin_amdgcn_global_load_lds((const __attribute__((address_space(1))) void*)(base[i] + (size_t)s * 64),
+                                         (__attribute__((address_space(3))) void*)(slot + (l + 4 * i) * 1024), 16, 0, 0);
+    };
+#pragma unroll
+    for (int s = 0; s < R - 1; ++s) {
+      if (s < nstages) issue(s);
+    }
+    for (int s = 0; s < nstages; ++s) {
+      // stage s has landed when at most the loads of the stages behind it are under way (fewer near the end)
+      const int behind = min(R - 2, nstages - 1 - s);
+      if (behind >= 2) wait_loads_but<2 * kPerLoader>();
+      else if (behind == 1) wait_loads_but<kPerLoader>();
+      else wait_loads_but<0>();
+      asm volatile("s_barrier" ::: "memory");                // everybody is done with stage s - 1: its slot is free
+      if (s + R - 1 < nstages) issue(s + R - 1);
+    }
+    return;
+  }
+  const int r = lane & 15, g = lane >> 4, wm = wave >> 2, wn = wave & 3;
+  const int my_tiles = min(MTW, max(0, (nrows - wm * 64 + 15) >> 4));        // tiles of 16 rows this wavefront has (the same for all its lanes)
+  const unsigned char* my_w = stages_lds + wn * NTW * 2048 + r * 128;
+  const unsigned char* my_x = stages_lds + kWLoads * 1024 + wm * MTW * 2048 + r * 128;
+  const int piece[2] = {(g ^ (r & 7)) * 16, ((4 + g) ^ (r & 7)) * 16};
+  moe_floatx4 acc[MTW][NTW];
+#pragma unroll
+  for (int t = 0; t < MTW; ++t)
+#pragma unroll
+    for (int u = 0; u < NTW; ++u) acc[t][u] = moe_floatx4{0.f, 0.f, 0.f, 0.f};
+  int slot = 0;
+  for (int s = 0; s < nstages; ++s) {
+    asm volatile("s_barrier" ::: "memory");
+    moe_bf16x8 b[2][NTW], a[2][MTW];
+#pragma unroll
+    for (int st = 0; st < 2; ++st) {
+#pragma unroll
+      for (int u = 0; u < NTW; ++u) b[st][u] = *reinterpret_cast<const moe_bf16x8*>(my_w + slot * kSlotBytes + u * 2048 + piece[st]);
+#pragma unroll
+      for (int t = 0; t < MTW; ++t) a[st][t] = *reinterpret_cast<const moe_bf16x8*>(my_x + slot * kSlotBytes + t * 2048 + piece[st]);
+    }
+    // (an operand of rows the tile does not have is used by nobody: it need not be back when the slot is filled anew)
+    asm volatile("" ::: "memory");
+#pragma unroll
+    for (int st = 0; st < 2; ++st) {
+#pragma unroll
+      for (int t = 0; t < MTW; ++t) {
+        if (t < my_tiles) {
+#pragma unroll
+          for (int u = 0; u < NTW; ++u) acc[t][u] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(b[st][u], a[st][t], acc[t][u], 0, 0, 0);
+        }
+      }
+    }
+    slot = slot + 1 == R ? 0 : slot + 1;
+  }
+  // a lane's four sums: outputs 4 g .. 4 g + 3 of a weights' block, for row r of a rows' block
+#pragma unroll
+  for (int t = 0; t < MTW; ++t) {
+    const int row = wm * 64 + t * 16 + r;
+    if (row >= nrows) continue;
+    const float ps = (FIRST && pair_scale) ? pair_scale[sorted_pair[row0 + row]] : 1.f;       // a factor on the pair's input row
+#pragma unroll
+    for (int u = 0; u < NTW; u += GATED ? 2 : 1) {
+      const int col = n0 + (GATED ? (wn * NTW + u) / 2 : wn * NTW + u) * 16 + 4 * g;
+      if (col >= n_out) continue;
+      if (FIRST) {
+        bf16* o = reinterpret_cast<bf16*>(out_) + (size_t)(row0 + row) * ld_out + col;
+        struct alignas(8) { bf16 v[4]; } y;
+#pragma unroll
+        for (int i = 0; i < 4; ++i)
+          y.v[i] = from_f32<bf16>(GATED ? gate_activation(acc[t][u][i] * ps, act) * (acc[t][u + GATED][i] * ps) : row_activation_for_bf16(acc[t][u][i] * ps, act));
+        if (col + 3 < n_out && (ld_out & 3) == 0) {
+          *reinterpret_cast<decltype(y)*>(o) = y;
+        } else {
+#pragma unroll
+          for (int i = 0; i < 4; ++i)
+            if (col + i < n_out) o[i] = y.v[i];
+        }
+      } else {
+        float* o = reinterpret_cast<float*>(out_) + (size_t)(row0 + row) * ld_out + col;
+        if (col + 3 < n_out && (ld_out & 3) == 0) {
+          *reinterpret_cast<float4*>(o) = make_float4(acc[t][u][0], acc[t][u][1], acc[t][u][2], acc[t][u][3]);
+        } else {
+#pragma unroll
+          for (int i = 0; i < 4; ++i)
+            if (col + i < n_out) o[i] = acc[t][u][i];
+        }
+      }
+    }
+  }
+}
+
+template <int FORM, int NB>
+static int launch_moe_stage(int max_tiles, const bf16* rows_in, int ld_in, const bf16* w, const int* tiles, const int* sorted_pair, int top, int n_out,
+                            int K, void* out, int ld_out, int act, const float* pair_scale, hipStream_t stream) {
+  constexpr int kOutputs = FORM == kFormGated ? NB * 8 : NB * 16, R = NB > 8 ? 3 : 4;
+  constexpr size_t lds = (size_t)R * (NB * 2 + kBigRows / 8) * 1024;
+  static_assert(lds <= 160 * 1024, "LDS of one compute unit");
+  auto kernel = moe_expert_stage_kernel<FORM, NB>;
+  hipError_t e = hipFuncSetAttribute(reinterpret_cast<const void*>(kernel), hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds);
+  if (e != hipSuccess) return (int)e;
+  const long n_blocks = (n_out + kOutputs - 1) / kOutputs;
+  if (n_blocks * max_tiles > 0x7fffffffL / kStageThreads) return -2;
+  hipLaunchKernelGGL(kernel, dim3((unsigned)(n_blocks * max_tiles)), dim3(kStageThreads), lds, stream, rows_in, ld_in, w, tiles, max_tiles, sorted_pair, top, n_out, K, out,
+                     ld_out, act, pair_scale);
+  return (int)hipGetLastError();
+}
+
 constexpr int kSplitBelowWorkgroups = 256;                   // the compute units of the GPU this is written for
 
 template <int FORM>
-static void launch_moe_mfma(int tile_rows, int max_tiles, int pairs, const bf16* rows_in, int ld_in, const bf16* w, const int* tiles,
+static int launch_moe_mfma(int tile_rows, int max_tiles, int pairs, const bf16* rows_in, int ld_in, const bf16* w, const int* tiles,
                             const int* sorted_pair, int top, int n_out, int K, void* out, int ld_out, int act, const float* pair_scale,
                             hipStream_t stream) {
   constexpr bool GATED = FORM == kFormGated;
   const int blocks = (n_out + 15) / 16;
+  if (tile_rows >= kBigRows && (K & 63) == 0) {
+    // tiles of 256 weight rows where their rounds of 256 compute units, at 48 KB a stage, cost less than those of 128 at 32 KB (about
+    // half of the experts end in a tile that is not full): 777 tokens' gated products of 2,048 with 2 of 8 experts 47 us against 59 in tiles of
+    // 128, their down products 35 against 26; 1,178 tokens' down products of 4,096 60 against 75, their plain products 88 against 82
+    const long tiles_used = pairs / kBigRows + max(1, (max_tiles - pairs / kBigRows) / 2), rows_of_w = (long)(GATED ? 2 : 1) * n_out;
+    const long rounds8 = (tiles_used * ((rows_of_w + 127) / 128) + 255) / 256, rounds16 = (tiles_used * ((rows_of_w + 255) / 256) + 255) / 256;
+    if (rounds16 * 48 < rounds8 * 32)
+      return launch_moe_stage<FORM, 16>(max_tiles, rows_in, ld_in, w, tiles, sorted_pair, top, n_out, K, out, ld_out, act, pair_scale, stream);
+    return launch_moe_stage<FORM, 8>(max_tiles, rows_in, ld_in, w, tiles, sorted_pair, top, n_out, K, out, ld_out, act, pair_scale, stream);
+  }
   if (tile_rows >= kBigRows) {
     dim3 grid(max_tiles, GATED ? (n_out + 63) / 64 : (n_out + 127) / 128);
     hipLaunchKernelGGL((moe_expert_tile_kernel<FORM>), grid, dim3(256), 0, stream, rows_in, ld_in, w, tiles, sorted_pair, top, n_out, K, out, ld_out, act, pair_scale);
@@ -782,6 +954,7 @@ static void launch_moe_mfma(int tile_rows, int max_tiles, int pairs, const bf16*
     dim3 grid(max_tiles, (blocks + 3) / 4);
     hipLaunchKernelGGL((moe_expert_mfma_kernel<FORM, 1, 1>), grid, dim3(256), 0, stream, rows_in, ld_in, w, tiles, sorted_pair, top, n_out, K, out, ld_out, act, pair_scale);
   }
+  return (int)hipGetLastError();
 }
 
 // form: kFormDown, kFormGated or kFormPlain.
@@ -799,13 +972,12 @@ PLLM_API int pllm_moe_expert_gemm(int dtype, int form, const void* rows_in, int 
   if (tile_rows != kMoeTileRows && !(matrix_cores && (tile_rows == 64 || tile_rows == kMoeMaxTileRows))) return -2;
   if (matrix_cores) {
 #define PLLM_MOE_MFMA(F)                                                                                                          \
-  launch_moe_mfma<F>(tile_rows, max_tiles, pairs, (const bf16*)rows_in, ld_in, (const bf16*)w, tiles, sorted_pair, top, n_out, K, out, \
+  return launch_moe_mfma<F>(tile_rows, max_tiles, pairs, (const bf16*)rows_in, ld_in, (const bf16*)w, tiles, sorted_pair, top, n_out, K, out, \
                      ld_out, act, pair_scale, stream)
     if (form == kFormGated) PLLM_MOE_MFMA(kFormGated);
     else if (form == kFormPlain) PLLM_MOE_MFMA(kFormPlain);
     else PLLM_MOE_MFMA(kFormDown);
 #undef PLLM_MOE_MFMA
-    PLLM_RETURN_LAST_ERROR();
   }
   dim3 grid(max_tiles, (n_out + kMoeCols - 1) / kMoeCols), block(256);
 #define PLLM_MOE(T, G)                                                                                                         \

@@ -1,0 +1,36 @@
+"""The experts' products of prompt steps for inner sizes that are multiples of 64 (tiles of 128 rows x 128 or 256 weight rows, both
+operands through LDS in stages): bit for bit what the kernel for tiles of 64 rows gives, which sums in the same order and is tested
+against float64 elsewhere."""
+import pytest
+import torch
+
+pytestmark = pytest.mark.gpu
+
+
+# inner size: one stage, fewer and more than the stages under way; outputs: no multiple of 16 or of a tile, one and several groups of 8
+# tiles; tokens: experts with tiles of 1 to 128 rows; the last two take tiles of 256 weight rows for gated and down products
+@pytest.mark.parametrize("tokens,top,experts,inner,outputs", [(300, 2, 8, 128, 192), (517, 2, 3, 192, 328), (260, 4, 5, 64, 72), (131, 1, 1, 448, 40),
+                                                              (64, 3, 3, 320, 1100), (777, 2, 8, 192, 2040), (1178, 2, 8, 64, 2048)])
+def test_staged_products_give_the_smaller_tiles_bits(tokens, top, experts, inner, outputs):
+    from paged_llm_amd.csrc import ops
+    gen = torch.Generator().manual_seed(tokens)
+    h = torch.randn((tokens, inner), generator=gen).to(torch.bfloat16).cuda()
+    w = (torch.randn((experts, 2 * outputs, inner), generator=gen) * inner ** -0.5).to(torch.bfloat16).cuda()
+    ids = torch.stack([torch.randperm(experts + 1, generator=gen)[:top] for _ in range(tokens)]).to(torch.int32).cuda()    # (expert `experts`: passed through)
+    scale = torch.rand((tokens * top,), generator=gen).cuda()
+    count = int((ids < experts).sum())
+    for form in ("gated", "plain", "down"):
+        got = {}
+        for rows in (ops.MOE_MID_TILE_ROWS, ops.MOE_MAX_TILE_ROWS):
+            sorted_pair, row_of_pair, tiles = ops.moe_align(ids, experts, rows)
+            place = row_of_pair.long()
+            if form == "down":          # the rows of the pairs, each at the place this alignment gives it
+                x = torch.zeros((tokens * top, inner), dtype=torch.bfloat16, device="cuda")
+                x[place[place >= 0]] = h[torch.nonzero(place >= 0)[:, 0] // top] * scale[place >= 0, None].to(torch.bfloat16)
+                out = ops.moe_expert_gemm(x, w, tiles, sorted_pair, top, False, tile_rows=rows)
+            else:
+                weights = w if form == "gated" else w[:, :outputs].contiguous()
+                out = ops.moe_expert_gemm(h, weights, tiles, sorted_pair, top, form == "gated", "silu" if form == "gated" else "relu2", tile_rows=rows,
+                                          pair_scale=scale if form == "gated" else None, plain=form == "plain")
+            got[rows] = out[place[place >= 0]]
+        assert got[128].shape[0] == count and torch.isfinite(got[128].float()).all() and torch.equal(got[64], got[128]), form
