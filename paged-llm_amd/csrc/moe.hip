@@ -759,18 +759,23 @@ __global__ __launch_bounds__(256) void moe_expert_tile_kernel(const bf16* __rest
   }
 }
 
-// The same prompt steps where K is a multiple of 64: a tile of 128 rows of one expert times NB blocks of 16 weight rows (gated: a
-// gate's block and its up block in turn), eight wavefronts that multiply and four that bring the operands: stages of 64 columns
+// The products where K is a multiple of 64: a tile of MT blocks of 16 rows of one expert times NB blocks of 16 weight rows (gated: a
+// gate's block and its up block in turn), for prompt steps eight wavefronts that multiply and four that bring the operands: stages of 64 columns
 // go from memory straight into LDS, R stages deep, a load taking the whole 128-byte lines of eight rows, whose eight pieces
 // lie XOR-ed by the row so that operand reads meet no bank twice.  Workgroups that follow each other on a chiplet
 // (i, i + 8, ...) take the tiles of one block of weight rows in turn, so that the tiles of an expert find its weights in their L2.
 // The kernel above draws half lines through registers, in an order that spreads an expert's tiles over all chiplets (both
 // products together, us, above / here: 1,178 tokens with 2 of 8 plain experts of 4,096 at width 2,048 225 / 143; 777 with 2 of 8 gated
 // ones of 2,048 157 / 73; 2,048 with 4 of 30 gated ones of 1,408 370 / 236; 300 with 2 of 8 plain ones of 4,096 145 / 82).
-// What bounds it is the drawing of the operands, as in the tiled products of whole steps: the compute unit's rate is the same
+// In steps of few tokens (MT 1: tiles of 16 rows, which are bound by the experts' bytes) the same form streams tiles of 64 weight rows seven
+// stages deep, two workgroups to a compute unit; the kernel for 16 rows above reads its weights a quarter of a line at a time
+// (first and down product, us, above / here: 8 tokens with 4 of 30 gated experts of 1,408 at width 2,048 63 + 30 / 44 + 21, 33 with 2
+// of 8 gated ones of 2,048 46 + 26 / 30 + 18, 64 with 2 of 8 plain ones of 4,096 62 + 59 / 33 + 40; 4.0 to 5.8 TB/s).
+// What bounds large tiles is the drawing of the operands, as in the tiled products of whole steps: the compute unit's rate is the same
 // whatever the tile, so a tile of 256 weight rows (48 KB a stage) takes the place of two of 128 (64 KB) where that needs no more
 // rounds.  The sums run over ascending k in one accumulator per output, as in the kernels above, and give the same bits.
-constexpr int kStageThreads = 768;
+
+constexpr int kReadOnce = 2;                                 // a load's cache policy: nt, the line is the first to leave the caches
 
 template <int N_>
 __device__ __forceinline__ void wait_loads_but() {            // until at most N_ of this wavefront's loads are still under way
@@ -778,15 +783,23 @@ __device__ __forceinline__ void wait_loads_but() {            // until at most N
   __builtin_amdgcn_s_waitcnt((N_ & 0xf) | ((N_ >> 4) << 14) | 0x0f70);
 }
 
-template <int FORM, int NB>
-__global__ __launch_bounds__(kStageThreads) void moe_expert_stage_kernel(const bf16* __restrict__ rows_in, int ld_in, const bf16* __restrict__ w,
-                                                                         const int* __restrict__ tiles, int max_tiles, const int* __restrict__ sorted_pair, int top,
+template <int FORM, int NB, int MT>
+struct StageShape {
+  static constexpr int WM = MT > 1 ? 2 : 1, WN = MT == 1 && NB == 4 && FORM == kFormGated ? 2 : 4, CW = WM * WN;      // compute wavefronts: along the rows, the weight rows
+  static constexpr int kThreads = (CW + 4) * 64, kLoads = (NB + MT) * 2, R = NB == 4 ? 7 : NB == 8 ? 4 : 3;
+  static constexpr size_t kLds = (size_t)R * kLoads * 1024;
+};
+
+template <int FORM, int NB, int MT>
+__global__ __launch_bounds__((StageShape<FORM, NB, MT>::kThreads)) void moe_expert_stage_kernel(const bf16* __restrict__ rows_in, int ld_in, const bf16* __restrict__ w,
+                                                                         const int* __restrict__ tiles, int max_tiles, int weights_once, const int* __restrict__ sorted_pair, int top,
                                                                          int n_out, int K, void* __restrict__ out_, int ld_out, int act,
                                                                          const float* __restrict__ pair_scale) {
   constexpr bool GATED = FORM == kFormGated, FIRST = FORM != kFormDown;      // FIRST: from the tokens' rows, activated
-  constexpr int kOutputs = GATED ? NB * 8 : NB * 16, R = NB > 8 ? 3 : 4, NTW = NB / 4, MTW = 4;
-  constexpr int kWLoads = NB * 2, kLoads = kWLoads + kBigRows / 8, kPerLoader = kLoads / 4, kSlotBytes = kLoads * 1024;
-  static_assert(kLoads % 4 == 0 && kWLoads % 4 == 0, "the loaders' shares are equal");
+  constexpr int kOutputs = GATED ? NB * 8 : NB * 16, R = StageShape<FORM, NB, MT>::R, CW = StageShape<FORM, NB, MT>::CW;
+  constexpr int NTW = NB / StageShape<FORM, NB, MT>::WN, MTW = MT / StageShape<FORM, NB, MT>::WM;
+  constexpr int kWLoads = NB * 2, kLoads = StageShape<FORM, NB, MT>::kLoads, kPerLoader = (kLoads + 3) / 4, kSlotBytes = kLoads * 1024;
+  static_assert(kWLoads % 4 == 0, "a loader's i-th load is of weights for all loaders or for none");
   extern __shared__ __attribute__((aligned(16))) unsigned char stages_lds[];
   const int n_blocks = (n_out + kOutputs - 1) / kOutputs;
   const int group = blockIdx.x / (8 * max_tiles), in_group = blockIdx.x - group * 8 * max_tiles, across = min(8, n_blocks - group * 8);
@@ -795,13 +808,13 @@ __global__ __launch_bounds__(kStageThreads) void moe_expert_stage_kernel(const b
   if (nrows <= 0) return;                                    // the whole workgroup: no barrier is left behind
   const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
   const int nstages = K >> 6;
-  if (wave >= 8) {
-    const int l = wave - 8, lr = lane >> 3, lp = ((lane & 7) ^ lr) * 8;
+  if (wave >= CW) {
+    const int l = wave - CW, lr = lane >> 3, lp = ((lane & 7) ^ lr) * 8;
     const bf16* we = w + (size_t)expert * (GATED ? 2 : 1) * n_out * K;
     const bf16* base[kPerLoader];
 #pragma unroll
     for (int i = 0; i < kPerLoader; ++i) {
-      const int b = l + 4 * i;
+      const int b = min(l + 4 * i, kLoads - 1);              // (every loader issues the same number of loads: the waits count them)
       if (4 * i < kWLoads) {
         const int u = b >> 1, in_block = (b & 1) * 8 + lr;
         const int row = GATED ? min(n0 + (u >> 1) * 16 + in_block, n_out - 1) + (u & 1) * n_out : min(n0 + u * 16 + in_block, n_out - 1);
@@ -811,12 +824,22 @@ __global__ __launch_bounds__(kStageThreads) void moe_expert_stage_kernel(const b
         base[i] = rows_in + (size_t)(FIRST ? sorted_pair[rr] / top : rr) * ld_in + lp;
       }
     }
-    auto issue = [&](int s) {
+    auto issue_loads = [&](int s, bool once) {               // (called with constants: two loops without a condition)
       unsigned char* slot = stages_lds + (s % R) * kSlotBytes;
 #pragma unroll
-      for (int i = 0; i < kPerLoader; ++i)
-        __builtin_amdgcn_global_load_lds((const __attribute__((address_space(1))) void*)(base[i] + (size_t)s * 64),
-                                         (__attribute__((address_space(3))) void*)(slot + (l + 4 * i) * 1024), 16, 0, 0);
+      for (int i = 0; i < kPerLoader; ++i) {
+        unsigned char* to = slot + min(l + 4 * i, kLoads - 1) * 1024;
+        if (once && 4 * i < kWLoads)
+          __builtin_amdgcn_global_load_lds((const __attribute__((address_space(1))) void*)(base[i] + (size_t)s * 64),
+                                           (__attribute__((address_space(3))) void*)to, 16, 0, kReadOnce);
+        else
+          __builtin_amdgcn_global_load_lds((const __attribute__((address_space(1))) void*)(base[i] + (size_t)s * 64),
+                                           (__attribute__((address_space(3))) void*)to, 16, 0, 0);
+      }
+    };
+    auto issue = [&](int s) {
+      if (weights_once) issue_loads(s, true);
+      else issue_loads(s, false);
     };
 #pragma unroll
     for (int s = 0; s < R - 1; ++s) {
@@ -825,7 +848,8 @@ __global__ __launch_bounds__(kStageThreads) void moe_expert_stage_kernel(const b
     for (int s = 0; s < nstages; ++s) {
       // stage s has landed when at most the loads of the stages behind it are under way (fewer near the end)
       const int behind = min(R - 2, nstages - 1 - s);
-      if (behind >= 2) wait_loads_but<2 * kPerLoader>();
+      if (behind == R - 2) wait_loads_but<(R - 2) * kPerLoader>();
+      else if (behind >= 2) wait_loads_but<2 * kPerLoader>();
       else if (behind == 1) wait_loads_but<kPerLoader>();
       else wait_loads_but<0>();
       asm volatile("s_barrier" ::: "memory");                // everybody is done with stage s - 1: its slot is free
@@ -833,8 +857,8 @@ __global__ __launch_bounds__(kStageThreads) void moe_expert_stage_kernel(const b
     }
     return;
   }
-  const int r = lane & 15, g = lane >> 4, wm = wave >> 2, wn = wave & 3;
-  const int my_tiles = min(MTW, max(0, (nrows - wm * 64 + 15) >> 4));        // tiles of 16 rows this wavefront has (the same for all its lanes)
+  const int r = lane & 15, g = lane >> 4, wm = wave / StageShape<FORM, NB, MT>::WN, wn = wave - wm * StageShape<FORM, NB, MT>::WN;
+  const int my_tiles = min(MTW, max(0, (nrows - wm * MTW * 16 + 15) >> 4));        // tiles of 16 rows this wavefront has (the same for all its lanes)
   const unsigned char* my_w = stages_lds + wn * NTW * 2048 + r * 128;
   const unsigned char* my_x = stages_lds + kWLoads * 1024 + wm * MTW * 2048 + r * 128;
   const int piece[2] = {(g ^ (r & 7)) * 16, ((4 + g) ^ (r & 7)) * 16};
@@ -871,7 +895,7 @@ __global__ __launch_bounds__(kStageThreads) void moe_expert_stage_kernel(const b
   // a lane's four sums: outputs 4 g .. 4 g + 3 of a weights' block, for row r of a rows' block
 #pragma unroll
   for (int t = 0; t < MTW; ++t) {
-    const int row = wm * 64 + t * 16 + r;
+    const int row = (wm * MTW + t) * 16 + r;
     if (row >= nrows) continue;
     const float ps = (FIRST && pair_scale) ? pair_scale[sorted_pair[row0 + row]] : 1.f;       // a factor on the pair's input row
 #pragma unroll
@@ -905,18 +929,18 @@ __global__ __launch_bounds__(kStageThreads) void moe_expert_stage_kernel(const b
   }
 }
 
-template <int FORM, int NB>
-static int launch_moe_stage(int max_tiles, const bf16* rows_in, int ld_in, const bf16* w, const int* tiles, const int* sorted_pair, int top, int n_out,
+template <int FORM, int NB, int MT>
+static int launch_moe_stage(int max_tiles, bool weights_once, const bf16* rows_in, int ld_in, const bf16* w, const int* tiles, const int* sorted_pair, int top, int n_out,
                             int K, void* out, int ld_out, int act, const float* pair_scale, hipStream_t stream) {
-  constexpr int kOutputs = FORM == kFormGated ? NB * 8 : NB * 16, R = NB > 8 ? 3 : 4;
-  constexpr size_t lds = (size_t)R * (NB * 2 + kBigRows / 8) * 1024;
+  constexpr int kOutputs = FORM == kFormGated ? NB * 8 : NB * 16, kStageThreads = StageShape<FORM, NB, MT>::kThreads;
+  constexpr size_t lds = StageShape<FORM, NB, MT>::kLds;
   static_assert(lds <= 160 * 1024, "LDS of one compute unit");
-  auto kernel = moe_expert_stage_kernel<FORM, NB>;
+  auto kernel = moe_expert_stage_kernel<FORM, NB, MT>;
   hipError_t e = hipFuncSetAttribute(reinterpret_cast<const void*>(kernel), hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds);
   if (e != hipSuccess) return (int)e;
   const long n_blocks = (n_out + kOutputs - 1) / kOutputs;
   if (n_blocks * max_tiles > 0x7fffffffL / kStageThreads) return -2;
-  hipLaunchKernelGGL(kernel, dim3((unsigned)(n_blocks * max_tiles)), dim3(kStageThreads), lds, stream, rows_in, ld_in, w, tiles, max_tiles, sorted_pair, top, n_out, K, out,
+  hipLaunchKernelGGL(kernel, dim3((unsigned)(n_blocks * max_tiles)), dim3(kStageThreads), lds, stream, rows_in, ld_in, w, tiles, max_tiles, (int)weights_once, sorted_pair, top, n_out, K, out,
                      ld_out, act, pair_scale);
   return (int)hipGetLastError();
 }
@@ -936,8 +960,8 @@ static int launch_moe_mfma(int tile_rows, int max_tiles, int pairs, const bf16* 
     const long tiles_used = pairs / kBigRows + max(1, (max_tiles - pairs / kBigRows) / 2), rows_of_w = (long)(GATED ? 2 : 1) * n_out;
     const long rounds8 = (tiles_used * ((rows_of_w + 127) / 128) + 255) / 256, rounds16 = (tiles_used * ((rows_of_w + 255) / 256) + 255) / 256;
     if (rounds16 * 48 < rounds8 * 32)
-      return launch_moe_stage<FORM, 16>(max_tiles, rows_in, ld_in, w, tiles, sorted_pair, top, n_out, K, out, ld_out, act, pair_scale, stream);
-    return launch_moe_stage<FORM, 8>(max_tiles, rows_in, ld_in, w, tiles, sorted_pair, top, n_out, K, out, ld_out, act, pair_scale, stream);
+      return launch_moe_stage<FORM, 16, 8>(max_tiles, false, rows_in, ld_in, w, tiles, sorted_pair, top, n_out, K, out, ld_out, act, pair_scale, stream);
+    return launch_moe_stage<FORM, 8, 8>(max_tiles, false, rows_in, ld_in, w, tiles, sorted_pair, top, n_out, K, out, ld_out, act, pair_scale, stream);
   }
   if (tile_rows >= kBigRows) {
     dim3 grid(max_tiles, GATED ? (n_out + 63) / 64 : (n_out + 127) / 128);
@@ -950,6 +974,14 @@ static int launch_moe_mfma(int tile_rows, int max_tiles, int pairs, const bf16* 
     // at most `pairs` tiles hold a row: too few workgroups of the kernel below to reach every compute unit
     dim3 grid(max_tiles, blocks);
     hipLaunchKernelGGL((moe_expert_splitk_kernel<FORM>), grid, dim3(256), 0, stream, rows_in, ld_in, w, tiles, sorted_pair, top, n_out, K, out, ld_out, act, pair_scale);
+  } else if ((K & 63) == 0) {
+    // Tiles of 64 weight rows, two workgroups to a compute unit (tiles of 128 in four stages: 33 tokens' products of 2,048 with 2 of 8
+    // gated experts 38 + 19 us against 30 + 18, 8 tokens' of 1,408 with 4 of 30 49 + 23 against 44 + 21).  Weights are let go by the caches once
+    // read where the experts hold 32 MB or more (a model of such layers does not fit the Infinity Cache; 44 us against 50 in the
+    // last case above); smaller ones may stay there from step to step.
+    const long experts = max_tiles - (pairs + kMoeTileRows - 1) / kMoeTileRows;      // (as many more tiles than whole ones are made room for)
+    const bool once = experts * (GATED ? 2 : 1) * n_out * K >= (16L << 20);
+    return launch_moe_stage<FORM, 4, 1>(max_tiles, once, rows_in, ld_in, w, tiles, sorted_pair, top, n_out, K, out, ld_out, act, pair_scale, stream);
   } else {
     dim3 grid(max_tiles, (blocks + 3) / 4);
     hipLaunchKernelGGL((moe_expert_mfma_kernel<FORM, 1, 1>), grid, dim3(256), 0, stream, rows_in, ld_in, w, tiles, sorted_pair, top, n_out, K, out, ld_out, act, pair_scale);
