@@ -5,8 +5,8 @@
   residual sum + norm in front and an activation or the rotary/cache write behind.
 * bfloat16, 17 to 128 rows (decoding with many requests, short prompt portions): the streaming kernel over the
   weights' tiled copy (``Weight``), with the same epilogues, or with float partial sums of ranges of K that the
-  consuming norm adds; where it was measured slower than the library (the gated product beyond 64 rows, the
-  output head) the library stays.
+  consuming norm adds; where it was measured slower than the library (the gated product and products with float
+  results beyond 64 rows, the output head) the library stays.
 * bfloat16, more rows (prompt portions): the vendor's matrix-product library, with bfloat16 or (logits)
   float results.
 
@@ -54,6 +54,7 @@ TILE_MAX_ROWS = 640                             # rows up to which the tiled ker
 TILE_PARTIAL_FROM_ROWS, TILE_PARTIAL_MIN_ELEMENTS, TILE_PARTIAL_MOST_RANGES = 65, 1 << 24, 12
 STREAM_GATED_MAX_ROWS = 64                      # the gated product: beyond, its rows' traffic costs more than the library's kernel
                                                 # (asked only where the tiled kernel does not take the product: _tiles_gated)
+STREAM_FLOAT_MAX_ROWS = 64                       # a product with float results: beyond, the library's kernel is as fast
 STREAM_LONG_K, STREAM_LONG_K_MAX_ROWS = 8192, 64 # from this K on a product in one range takes the streaming kernel up to so many rows
 
 
@@ -108,7 +109,10 @@ def _streams(x, weight, epi: int, partial_ok: bool = False) -> bool:
     if epi == ops.SL_GATED:
         return rows <= STREAM_GATED_MAX_ROWS
     if epi == ops.SL_F32:
-        return False                                            # (the head: 32000 x 2048 was not faster than the library's kernel)
+        # Branches with float results: up to 64 rows and K below 8192 (33 rows: 2048 x 2048 / 4096 / 5632 5.8 / 10.2 / 13.3 us against the
+        # library's 8.2 / 12.1 / 15.3, 4096 x 2048 7.5 and 11.7, 2048 x 8192 18.5 and 14.1; 64 rows of 2048 x 2048 5.8 and 8.6, 100 rows 8.6
+        # and 8.4).  The head has too many weight rows: 32000 x 2048 was not faster.
+        return weight.pairing == "plain" and rows <= STREAM_FLOAT_MAX_ROWS and k < STREAM_LONG_K and _few_weight_rows(weight)
     # (cut into ranges of K the long products stay ahead of the library up to 128 rows: 4096 x 14336 at 96 / 128 rows 45.7 / 55.4 us
     #  against 62.6 / 74.8, 2048 x 8192 16.1 / 18.4 against 20.8)
     return _few_weight_rows(weight) and (k < STREAM_LONG_K or rows <= STREAM_LONG_K_MAX_ROWS or (partial_ok and epi == ops.SL_BF16))

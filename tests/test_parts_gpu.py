@@ -533,3 +533,23 @@ def test_embedding_and_head_parts(dtype, tol):
     for many in (33, 100):                                   # other row counts take other kernels
         xm = rows(many, 17, dtype)
         assert rel(own.forward(xm.cuda()), xm.float() @ hw.T) <= tol
+
+
+@pytest.mark.parametrize("rows,n,k,streams", [(17, 2048, 2048, True), (64, 96, 5632, True), (64, 4096, 64, True), (65, 2048, 2048, False), (33, 2048, 8192, False),
+                                              (33, 9000, 64, False), (16, 2048, 2048, False)])
+def test_products_with_float_results_choose_their_kernel_by_size(rows, n, k, streams):
+    """17 to 64 rows, K below 8192 and few weight rows take the streaming kernel, the rest the library or the kernel for fewer rows; matrices
+    whose tiles pair rows for another epilogue never do."""
+    from paged_llm_amd.csrc import ops
+    from paged_llm_amd.parts import linear
+    gen = torch.Generator().manual_seed(rows + k)
+    x = torch.randn((rows, k), generator=gen).to(torch.bfloat16).cuda()
+    w = (torch.randn((n, k), generator=gen) * k ** -0.5).to(torch.bfloat16).cuda()
+    plain, gated = linear.Weight(w), linear.Weight(w, "gated")
+    assert linear._streams(x, plain, ops.SL_F32) is streams and not linear._streams(x, gated, ops.SL_F32)
+    want = x.cpu().double() @ w.cpu().double().T
+    for weight in (plain, gated):
+        got = linear.linear(x, weight, torch.float32)
+        # every sum of k products in float, in any order: within k roundings of half a unit of the sum of magnitudes
+        bound = (x.cpu().double().abs() @ w.cpu().double().abs().T) * (k * 2.0 ** -24) + 1e-30
+        assert got.dtype == torch.float32 and bool(((got.cpu().double() - want).abs() <= bound).all())
