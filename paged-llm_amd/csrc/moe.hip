@@ -366,8 +366,9 @@ __global__ __launch_bounds__(256) void moe_expert_gemm_kernel(const T* __restric
 // A workgroup is one tile of MT * 16 rows of one expert times 4 wavefronts * U blocks of 16 outputs (gated: the
 // gate's and the up product's 16 rows each); a wavefront keeps U * MT (gated: 2 U MT) accumulators.  In steps of few
 // tokens (MT = 1) every wavefront streams weight rows that no other one reads, which is all there is to do: such a step
-// is bound by the chosen experts' bytes.  In prompt steps (tiles of 64 rows) the four wavefronts read the same rows
+// is bound by the chosen experts' bytes.  In steps with tiles of 64 rows the four wavefronts read the same rows
 // (the first one's misses are the others' cache hits) and each of its own weight rows once per 64 rows.
+// (Inner sizes that are multiples of 64 take the staged kernel below, unless the step has too few pairs for it.)
 // An output element is one accumulator over ascending k-steps whatever MT and U are, so its value does not depend on
 // the tile it is in, the kernel's shape or the other rows.  K % 8 == 0, ld_in % 8 == 0; a last k-step beyond K reads zeros.
 typedef __attribute__((ext_vector_type(8))) __bf16 moe_bf16x8;
@@ -771,6 +772,8 @@ __global__ __launch_bounds__(256) void moe_expert_tile_kernel(const bf16* __rest
 // stages deep, two workgroups to a compute unit; the kernel for 16 rows above reads its weights a quarter of a line at a time
 // (first and down product, us, above / here: 8 tokens with 4 of 30 gated experts of 1,408 at width 2,048 63 + 30 / 44 + 21, 33 with 2
 // of 8 gated ones of 2,048 46 + 26 / 30 + 18, 64 with 2 of 8 plain ones of 4,096 62 + 59 / 33 + 40; 4.0 to 5.8 TB/s).
+// Steps between (MT 4: tiles of 64 rows x 128 weight rows) drew whole matrices through the kernel above at 1.3 to 2 TB/s (256 tokens with 2 of 16 gated
+// experts of 1,024 at width 1,024 41 + 22 / 16 + 10, 300 with 2 of 8 of 512 27 + 14 / 11 + 7).
 // What bounds large tiles is the drawing of the operands, as in the tiled products of whole steps: the compute unit's rate is the same
 // whatever the tile, so a tile of 256 weight rows (48 KB a stage) takes the place of two of 128 (64 KB) where that needs no more
 // rounds.  The sums run over ascending k in one accumulator per output, as in the kernels above, and give the same bits.
@@ -966,6 +969,8 @@ static int launch_moe_mfma(int tile_rows, int max_tiles, int pairs, const bf16* 
   if (tile_rows >= kBigRows) {
     dim3 grid(max_tiles, GATED ? (n_out + 63) / 64 : (n_out + 127) / 128);
     hipLaunchKernelGGL((moe_expert_tile_kernel<FORM>), grid, dim3(256), 0, stream, rows_in, ld_in, w, tiles, sorted_pair, top, n_out, K, out, ld_out, act, pair_scale);
+  } else if (tile_rows >= 64 && (K & 63) == 0) {
+    return launch_moe_stage<FORM, 8, 4>(max_tiles, false, rows_in, ld_in, w, tiles, sorted_pair, top, n_out, K, out, ld_out, act, pair_scale, stream);
   } else if (tile_rows >= 64) {
     constexpr int U = GATED ? 1 : 2;
     dim3 grid(max_tiles, (blocks + 4 * U - 1) / (4 * U));

@@ -1,6 +1,6 @@
 """y = x W^T for the parts, with the kernel chosen by element type and number of rows.
 
-* float32: the plain kernel with float operands (the true 32-bit path), always.
+* float32: the float matrix-core kernel (the true 32-bit path), always.
 * bfloat16, at most 16 rows (decoding): the fused decode kernel, which also takes in a pending
   residual sum + norm in front and an activation or the rotary/cache write behind.
 * bfloat16, 17 to 128 rows (decoding with many requests, short prompt portions): the streaming kernel over the

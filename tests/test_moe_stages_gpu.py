@@ -1,6 +1,5 @@
-"""The experts' products for inner sizes that are multiples of 64 (tiles of 128 rows x 128 or 256 weight rows, or of 16 rows x 64,
-both operands through LDS in stages): bit for bit what the kernel for tiles of 64 rows gives, which sums in the same order and is tested
-against float64 elsewhere."""
+"""The experts' products for inner sizes that are multiples of 64 (tiles of 128 rows x 128 or 256 weight rows, of 64 rows x 128 or of
+16 rows x 64, both operands through LDS in stages): against float64 sums of the same bfloat16 operands, and the same bits whatever the tile."""
 import pytest
 import torch
 
@@ -14,7 +13,7 @@ pytestmark = pytest.mark.gpu
 @pytest.mark.parametrize("tokens,top,experts,inner,outputs", [(300, 2, 8, 128, 192), (517, 2, 3, 192, 328), (260, 4, 5, 64, 72), (131, 1, 1, 448, 40),
                                                               (64, 3, 3, 320, 1100), (777, 2, 8, 192, 2040), (1178, 2, 8, 64, 2048),
                                                               (40, 2, 8, 1024, 1400)])
-def test_staged_products_give_the_smaller_tiles_bits(tokens, top, experts, inner, outputs):
+def test_staged_products(tokens, top, experts, inner, outputs):
     from paged_llm_amd.csrc import ops
     gen = torch.Generator().manual_seed(tokens)
     h = torch.randn((tokens, inner), generator=gen).to(torch.bfloat16).cuda()
@@ -23,7 +22,7 @@ def test_staged_products_give_the_smaller_tiles_bits(tokens, top, experts, inner
     scale = torch.rand((tokens * top,), generator=gen).cuda()
     count = int((ids < experts).sum())
     for form in ("gated", "plain", "down"):
-        got = {}
+        got, want, spread = {}, None, None
         for rows in (ops.MOE_TILE_ROWS, ops.MOE_MID_TILE_ROWS, ops.MOE_MAX_TILE_ROWS):
             sorted_pair, row_of_pair, tiles = ops.moe_align(ids, experts, rows)
             place = row_of_pair.long()
@@ -36,5 +35,20 @@ def test_staged_products_give_the_smaller_tiles_bits(tokens, top, experts, inner
                 out = ops.moe_expert_gemm(h, weights, tiles, sorted_pair, top, form == "gated", "silu" if form == "gated" else "relu2", tile_rows=rows,
                                           pair_scale=scale if form == "gated" else None, plain=form == "plain")
             got[rows] = out[place[place >= 0]]
+            if want is None:            # pair by pair in float64, with the sums of magnitudes that bound a float sum's error
+                pair = torch.nonzero(place >= 0)[:, 0]
+                rows_of_pairs = (x[place[pair]] if form == "down" else h[pair // top]).double()
+                expert, n = ids.flatten()[pair].long(), outputs if form == "plain" else 2 * outputs
+                sums, spread = torch.empty((count, n), dtype=torch.float64, device="cuda"), torch.empty((count, n), dtype=torch.float64, device="cuda")
+                for e in range(experts):
+                    m, we = expert == e, w[e, :n].double()
+                    sums[m], spread[m] = rows_of_pairs[m] @ we.T, rows_of_pairs[m].abs() @ we.T.abs()
+                factor = scale[pair].double()[:, None]
+                want = (torch.nn.functional.silu(factor * sums[:, :outputs]) * (factor * sums[:, outputs:]) if form == "gated"
+                        else sums.clamp(min=0) ** 2 if form == "plain" else sums)
+        if form == "down":              # inner roundings of half a unit each at most
+            assert bool(((got[64].double() - want).abs() <= inner * 2.0 ** -24 * spread).all())
+        else:                           # the result's rounding to bfloat16 (2^-8, and as much again for the float steps in front of it)
+            assert bool(((got[64].double() - want).abs() <= 2.0 ** -7 * want.abs() + 1e-5).all()), form
         assert got[128].shape[0] == count and torch.isfinite(got[128].float()).all() and torch.equal(got[64], got[128]), form
         assert torch.equal(got[16], got[64]) or (tokens == 131 and torch.allclose(got[16].float(), got[64].float(), rtol=2 ** -7, atol=1e-5)), form
