@@ -2274,8 +2274,8 @@ def moe_tile_rows(pairs: int, experts: int, dtype: torch.dtype, *inner_sizes: in
     """Rows of a tile of the experts' products for a step of ``pairs`` (token, choice) pairs: where the matrix-core
     kernels run (bfloat16, every product's inner size a multiple of 8) 128 if an expert gets 32 pairs or more on average, 64
     where tiles of 128 would leave compute units idle (small experts) unless an expert gets 128; else 16.  (Both products at width
-    2,048, 30 gated experts of 1,408, 512 tokens with 4 choices: 240 us with tiles of 128, 408 with 64, 465 with 16; 16 experts of
-    1,024 at width 1,024, 256 tokens: 73, 66 and 83.)  It depends on the step's number of tokens only, so a replayed step keeps its choice."""
+    2,048, 30 gated experts of 1,408, 256 tokens with 4 choices: 126 us with tiles of 128, 119 with 64, 170 with 16; 16 experts of
+    1,024 at width 1,024, 256 tokens with 2: 27, 25 and 38; 8 of 512, 300 tokens with 2: 22, 18 and 20.)  It depends on the step's number of tokens only, so a replayed step keeps its choice."""
     if dtype == torch.bfloat16 and all(k % 8 == 0 for k in inner_sizes):
         if pairs >= 128 * experts:
             return MOE_MAX_TILE_ROWS

@@ -208,12 +208,13 @@ def _tiles_in_one_round(rows: int, weight) -> bool:
 
 def _tiles_gated(x, weight, rows: int) -> bool:
     """Whether the gated product goes to the tiled kernel.  With two blocks of input rows it takes as long as the library's
-    product (11264 x 2048 at 264 rows: 28 us both) and saves the activation kernel and its pass over the intermediate rows
+    product (11264 x 2048 at 264 rows: 25 us against 28) and saves the activation kernel and its pass over the intermediate rows
     (5 us).  A matrix whose tiles of 128 weight rows fill three quarters of the compute units by themselves takes it with
     one block of rows as well, from a few rows on: there every workgroup draws its own weights and the step's few rows,
     where the streaming kernel's workgroups of 32 to 64 weight rows draw the rows four times as often (28672 x 4096 at
-    32 / 64 / 128 rows: 46 / 46 / 52 us against 50 / 57 us streaming and 53 / 53 / 59 us in the library with the activation
-    kernel; 24576 x 2048 at 64 rows 27 against 33 and 30).  A matrix whose tiles of 128 fill at most half of the compute
+    24 / 64 / 128 rows: 43 / 45 / 54 us against 50 / 57 us streaming at 32 and 64 and 53 / 53 / 59 us in the library with the activation
+    kernel; 24576 x 2048 at 64 rows 27 against 33 and 30).  With two blocks of rows such matrices go in tiles of 256 weight rows
+    (264 rows: 81 us against 78 and 6 for the activation in the library).  A matrix whose tiles of 128 fill at most half of the compute
     units is cut into tiles of 64 weight rows by the kernel when there is one block of rows, twice the workgroups (11264 x
     2048 at 64 / 96 / 128 / 160 rows: 14.0 / 16.1 / 19.0 / 21.7 us against 18.8 / 20.3 / 21.8 / 27.6 in the library with the
     activation kernel and 14.8 streaming at 64; 16384 x 2048 at 32 / 64 rows: 15.7 / 16.8 against 19.0 / 21.0 streaming; inside
