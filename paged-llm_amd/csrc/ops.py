@@ -1491,7 +1491,9 @@ def step_sizes(raw: torch.Tensor, bias: torch.Tensor, a_log: torch.Tensor) -> tu
     return dt, decay
 
 
-RECURRENCE_CHUNKS_FROM = 128      # tokens of the longest sequence of a step from which its recurrences run in chunks
+# Tokens of the longest sequence of a step from which its recurrences may run in pieces or chunks, which round differently than token by
+# token.  Below, every token of the step has the bits that it has alone, and a short portion may be cut anywhere.
+RECURRENCE_CHUNKS_FROM = 128
 
 
 def recurrence_chunk(max_q_len: int, num_tokens: int) -> int:
@@ -1514,12 +1516,12 @@ def recurrence_form(max_q_len: int, num_tokens: int, num_seqs: int, heads: int, 
     """How a step's recurrences run: 0, every sequence token by token in one workgroup per head and block of columns; -1, every
     sequence in one workgroup likewise, in pieces of 32 tokens; else the tokens per chunk of the three passes over chunks, which
     spread a long portion over the GPU at the price of a workspace of one state per chunk and two passes over every sequence."""
-    if max_q_len <= 1:
+    if max_q_len < RECURRENCE_CHUNKS_FROM:
         return 0
     if rows <= (128 if by_row else 256):
-        # What each takes, in us, from 1 to 2,048 tokens of 64 heads of 128 x 64 rows and columns, of 8 of 128 x 257 and 256 x 512, of
-        # 16 of 128 x 128 with a decay per row, alone and beside 32 single tokens.  Single tokens stay token by token (64 heads: 17
-        # us), portions beside many of them in pieces (64 tokens and 32 single ones: token by token 110, pieces 74, chunks 330),
+        # What each takes, in us, up to 2,048 tokens of 64 heads of 128 x 64 rows and columns, of 8 of 128 x 257 and 256 x 512, of
+        # 16 of 128 x 128 with a decay per row, alone and beside 32 single tokens.  Portions beside many single tokens run in
+        # pieces (130 tokens and 32 single ones: token by token 242, pieces 79, chunks 338),
         # long portions in chunks (2,048: pieces 460, chunks 142) of so many pieces that their workgroups fill the GPU once:
         # chunks of 1 / 2 / 4 / 8 pieces take 200 / 159 / 152 / 142, and at 512 tokens 62 / 53 / 64 / 101.
         wide = by_row or rows > 128                     # workgroups of eight wavefronts, one to a compute unit; else of four, two
@@ -1551,9 +1553,10 @@ def linear_recurrence(q: torch.Tensor, k: torch.Tensor, v: torch.Tensor, decay: 
     the state then takes heads * N * (P + 1) floats and y is [T, heads * (P + 1)] with n_t . q_t in every head's last column.
     ``row_decay`` float32 [T, heads, N] (a view, heads side by side, unit inner stride) in place of ``decay`` (None): a decay per
     row of S, S_t = diag(row_decay_t) S_(t-1) + k_t (vscale_t v_t)^T (every head then has its own keys).
-    ``max_q_len``: a bound on the tokens of one sequence in this step (0: unknown); from ``RECURRENCE_CHUNKS_FROM`` on the
-    sequences are cut into chunks that run side by side (a chunk's own contribution from a zero state, the states carried
-    from chunk to chunk, the outputs from each chunk's true starting state), which rounds differently than token by token."""
+    ``max_q_len``: a bound on the tokens of one sequence in this step (0: unknown); from ``RECURRENCE_CHUNKS_FROM`` on
+    ``recurrence_form`` may take the sequences in pieces as matrix products, or cut them into chunks that run side by side (a
+    chunk's own contribution from a zero state, the states carried from chunk to chunk, the outputs from each chunk's true starting
+    state), which rounds differently than token by token.  Below it every token has the bits that it has alone."""
     _on_gpu(q, k, v, decay, state, state_slots, seq_starts, cu_seqlens, vscale, skip)
     _need(q.dim() == 3 and q.shape == k.shape and q.dtype == k.dtype and q.stride() == k.stride() and q.stride(2) == 1
           and q.stride(1) == q.shape[2], "recurrence q, k: [T, key_heads, N] views of one layout with the heads side by side")

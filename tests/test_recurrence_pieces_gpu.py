@@ -109,13 +109,43 @@ def test_a_value_that_is_no_number_reaches_later_tokens_only(by_row, chunk, monk
     assert torch.equal(odd[:, 1][:, keep], plain[:, 1][:, keep])
 
 
+@pytest.mark.parametrize("H,KH,N,P,by_row", [(4, 2, 128, 64, False), (2, 2, 50, 30, True), (2, 1, 256, 20, False)])
+def test_tokens_beside_a_short_portion_have_the_bits_they_have_alone(H, KH, N, P, by_row):
+    """Below the bound that ``linear_recurrence`` states for chunks every token is the same whoever stands beside it: a portion of
+    127 tokens, one of 20 and single tokens in one step, and each of the four token by token in steps of its own."""
+    o = ops()
+    lens, starts = [1, o.RECURRENCE_CHUNKS_FROM - 1, 1, 20], [3, 0, 1, 5]
+    T, g = sum(lens), torch.Generator().manual_seed(N)
+    q, k, v = (torch.randn(T, h, n, generator=g).cuda() for h, n in ((KH, N), (KH, N), (H, P)))
+    decay, row = torch.rand(T, H, generator=g).cuda(), torch.rand(T, H, N, generator=g).cuda()
+    state = torch.randn(4, H * N * P, generator=g).cuda()
+    ints = lambda *x: torch.tensor(x, dtype=torch.int32, device="cuda")
+
+    def step(st, slots, begun, lo, hi, cu):
+        return o.linear_recurrence(q[lo:hi], k[lo:hi], v[lo:hi], None if by_row else decay[lo:hi], st, 0, slots, begun, ints(*cu), len(cu) - 1,
+                                   max_q_len=max(b - a for a, b in zip(cu, cu[1:])), row_decay=row[lo:hi] if by_row else None)
+    cu = [0, *torch.tensor(lens).cumsum(0).tolist()]
+    together, alone = state.clone(), state.clone()
+    y = step(together, ints(0, 1, 2, 3), ints(*starts), 0, T, cu)
+    for s, n in enumerate(lens):
+        for t in range(n):
+            at = cu[s] + t
+            assert torch.equal(step(alone, ints(s), ints(starts[s] + t), at, at + 1, [0, 1])[0], y[at]), (s, t)
+    assert torch.equal(together, alone)
+
+
 def test_which_form_a_step_takes():
-    """Decode steps token by token, long prompts in chunks of whole pieces, portions beside many single tokens in pieces."""
+    """Decode steps and portions of fewer than 128 tokens token by token, long prompts in chunks of whole pieces, longer portions beside
+    many single tokens in pieces."""
     plan = ops().recurrence_form
     for n in (1, 64, 1024):
         assert plan(1, n, n, 64, 128, 64, False, 256) == 0
+    for longest in (2, 16, 64, 127):
+        for beside in (0, 1, 32):
+            for heads, rows, columns, by_row in ((64, 128, 64, False), (8, 256, 512, False), (1, 16, 16, False), (16, 128, 128, True)):
+                assert plan(longest, longest + beside, 1 + beside, heads, rows, columns, by_row, 256) == 0
     for tokens in (200, 2048, 8192):
         chunk = plan(tokens, tokens, 1, 8, 256, 512, False, 256)
         assert chunk > 0 and chunk % 32 == 0
-    assert plan(64, 96, 33, 64, 128, 64, False, 256) == -1
+    assert plan(128, 160, 33, 64, 128, 64, False, 256) == -1
     assert plan(4096, 4096, 1, 4, 512, 64, False, 256) in (64, 128) and plan(0, 5, 5, 4, 128, 64, False, 256) == 0
