@@ -21,6 +21,9 @@
 //     and compute unit from the L2.  Eight wavefronts take two slices each, one after the other, with 216 registers a
 //     lane: 2048 rows x 2048 x 5632 in 445 us (106 TFLOP/s), 301 rows x 2048 x 5632 in 86 us (tiles of 48 x 64 fill the GPU in
 //     one round; 1027 us before).
+//   * Short K (the matrices of heads): bound by memory and by what a workgroup takes to start and end.  Only the wavefronts that
+//     have columns are launched, one for every slice or two of 32 (64 heads of 64 x 64 at 300 / 1500 rows: 6.9 / 20 us, 2.5 TB/s at
+//     the latter; the kernel with all of K in one workgroup's LDS tiles took 13.5 / 29).
 // Which tile a product takes is the host's choice by the rounds of workgroups (ops.float_gemm_plan).
 #include "common.h"
 
@@ -54,20 +57,22 @@ __device__ __forceinline__ f32x4 load_quad(const float* p) {
   return f32x4{p[0], p[1], p[2], p[3]};
 }
 
-template <int MT, int NT, int SPW, int HALVES, int DEPTH, int PER_SIMD, bool VEC>
+// ALL: every slice has columns, and the workgroup all its wavefronts.
+template <int MT, int NT, int SPW, int HALVES, int DEPTH, int PER_SIMD, bool VEC, bool ALL>
 __global__ __launch_bounds__(64 * (kSlices / SPW), PER_SIMD) void gemm_float_kernel(FloatGemm g) {
-  constexpr int kWaves = kSlices / SPW, kStep = 16 * HALVES;
+  constexpr int kStep = 16 * HALVES;
   extern __shared__ __attribute__((aligned(16))) unsigned char gf_lds[];
-  f32x4* parts = reinterpret_cast<f32x4*>(gf_lds);                     // [kWaves][MT * NT][64]
+  f32x4* parts = reinterpret_cast<f32x4*>(gf_lds);                     // [wavefronts][MT * NT][64]
   const int tid = threadIdx.x, lane = tid & 63;
   const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
   const int r16 = lane & 15, quad = lane >> 4;
 
   // The row tiles of one tile of weight rows follow each other on one XCD (workgroup b runs on XCD b % 8), so that its L2
-  // hands the weights from one to the next.
-  const int b = blockIdx.x, group = g.row_tiles * 8;
-  const int col_tile = (b / group) * 8 + (b & 7), row_tile = (b % group) >> 3;
-  if (col_tile >= g.col_tiles) return;
+  // hands the weights from one to the next.  The last group has fewer than eight tiles of weight rows where their number is no
+  // multiple of 8: its workgroups go round the XCDs all the same (64 heads of 64 x 64 at 1500 rows: 20 us; 278 with the
+  // group filled up by workgroups without work, which left the others on one XCD, and with sixteen wavefronts for two slices).
+  const int b = blockIdx.x, group = b / (g.row_tiles * 8), in_group = b - group * g.row_tiles * 8, across = min(8, g.col_tiles - group * 8);
+  const int row_tile = across == 8 ? in_group >> 3 : in_group / across, col_tile = group * 8 + in_group - row_tile * across;
   const int m0 = row_tile * (16 * MT), n0 = col_tile * (16 * NT);
   const float* A = g.A + (size_t)blockIdx.y * g.a_batch;
   const float* W = g.W + (size_t)blockIdx.y * g.w_batch;
@@ -148,12 +153,15 @@ __global__ __launch_bounds__(64 * (kSlices / SPW), PER_SIMD) void gemm_float_ker
   for (int i = 0; i < MT * NT; ++i) parts[(wave * MT * NT + i) * 64 + lane] = total[i];
   __syncthreads();
   const bool wide = (g.ldc & 3) == 0 && (reinterpret_cast<uintptr_t>(C) & 15) == 0;
-  for (int at = tid; at < MT * NT * 64; at += 64 * kWaves) {
+  const int threads = ALL ? 64 * (kSlices / SPW) : (int)blockDim.x;
+  for (int at = tid; at < MT * NT * 64; at += threads) {
     f32x4 sum;
 #pragma unroll
     for (int p = 0; p < kSlices / 2; ++p) {
       constexpr int kEach = MT * NT * 64;
-      const f32x4 pair = SPW == 2 ? parts[p * kEach + at] : parts[2 * p * kEach + at] + parts[(2 * p + 1) * kEach + at];
+      if (!ALL && p > 0 && 2 * p * g.slice >= g.K) break;              // (slices past K are zeros that change no sum: nobody makes them)
+      f32x4 pair = parts[(SPW == 2 ? p : 2 * p) * kEach + at];
+      if (SPW == 1 && (ALL || (2 * p + 1) * g.slice < g.K)) pair += parts[(2 * p + 1) * kEach + at];
       sum = p == 0 ? pair : sum + pair;
     }
     const int tile = at >> 6, m = m0 + 16 * (tile / NT) + (at & 15), n = n0 + 16 * (tile % NT) + 4 * ((at & 63) >> 4);
@@ -174,13 +182,15 @@ static int launch_float_gemm(const FloatGemm& g, int batch, bool vec, hipStream_
   FloatGemm p = g;
   p.row_tiles = (g.M + 16 * MT - 1) / (16 * MT);
   p.col_tiles = (g.N + 16 * NT - 1) / (16 * NT);
-  const size_t lds = (size_t)(kSlices / SPW) * MT * NT * 64 * sizeof(f32x4);
-  auto kernel = vec ? gemm_float_kernel<MT, NT, SPW, HALVES, DEPTH, PER_SIMD, true> : gemm_float_kernel<MT, NT, SPW, HALVES, DEPTH, PER_SIMD, false>;
+  const int used = (g.K + g.slice - 1) / g.slice, waves = (used + SPW - 1) / SPW;     // wavefronts that have columns: 1 to kSlices / SPW
+  const size_t lds = (size_t)waves * MT * NT * 64 * sizeof(f32x4);
+  auto kernel = used == kSlices ? (vec ? gemm_float_kernel<MT, NT, SPW, HALVES, DEPTH, PER_SIMD, true, true> : gemm_float_kernel<MT, NT, SPW, HALVES, DEPTH, PER_SIMD, false, true>)
+                                : (vec ? gemm_float_kernel<MT, NT, SPW, HALVES, DEPTH, PER_SIMD, true, false> : gemm_float_kernel<MT, NT, SPW, HALVES, DEPTH, PER_SIMD, false, false>);
   if (lds > 64 * 1024) {
     hipError_t e = hipFuncSetAttribute(reinterpret_cast<const void*>(kernel), hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds);
     if (e != hipSuccess) return (int)e;
   }
-  const dim3 grid((p.col_tiles + 7) / 8 * 8 * p.row_tiles, batch), block(64 * (kSlices / SPW));
+  const dim3 grid((unsigned)(p.col_tiles * p.row_tiles), batch), block(64 * waves);
   hipLaunchKernelGGL(kernel, grid, block, lds, stream, p);
   PLLM_RETURN_LAST_ERROR();
 }

@@ -281,13 +281,14 @@ def copy_pages(pages: torch.Tensor, src: torch.Tensor, dst: torch.Tensor) -> Non
 
 
 # ------------------------------------------------------------------------------------------- products
-# The float product's tiles (in sixteens of rows and of weight rows): the time of one round of workgroups, one on every
-# compute unit, at K = 2048, and what a launch takes beside its rounds (microseconds, fitted to 1 to 2048 rows of matrices of
-# 1024 to 32000 weight rows; a round is in proportion to K).  Small tiles give a step of few rows enough workgroups, large
-# ones use the matrix cores better; the products of one round or two are decided by how full the rounds are (301 rows x
-# 2048 x 2048: tiles of 48 x 64 in one round 36 us, 64 x 64 47 us, 32 x 32 47 us; 301 x 2560 x 2048: 48 x 64 in two rounds 65 us,
-# 64 x 64 in one 48 us).
-FLOAT_GEMM_TILES = {(1, 1): (7.0, 4.0), (1, 2): (10.4, 4.0), (2, 2): (16.0, 4.0), (3, 4): (33.2, 3.0), (4, 4): (43.0, 3.0)}
+# The float product's tiles (in sixteens of rows and of weight rows): what one round of workgroups, one on every compute unit,
+# takes beside its columns, what the columns of K = 2048 add to it, and what a launch takes beside its rounds (microseconds, fitted to
+# 1 to 4096 rows of single matrices of 64 to 32000 weight rows and of 5 to 64 heads' matrices, K from 32 to 5632).  Small tiles give a
+# step of few rows enough workgroups, large ones use the matrix cores better; the products of one round or two are decided by how
+# full the rounds are (301 rows x 2048 x 2048: tiles of 48 x 64 in one round 36 us, 64 x 64 47 us, 32 x 32 47 us; 301 x 2560 x 2048:
+# 48 x 64 in two rounds 66 us, 64 x 64 in one 48 us), those of short K by what a workgroup takes whatever its columns (8 rows of 64
+# heads of 64 x 64: 16 x 16 3.5 us, 48 x 64 7.1 us, which a cost in proportion to K alone had preferred).
+FLOAT_GEMM_TILES = {(1, 1): (0.3, 7.0, 3.1), (1, 2): (0.1, 10.4, 3.3), (2, 2): (0.3, 14.3, 3.4), (3, 4): (0.9, 31.0, 5.0), (4, 4): (1.1, 41.0, 5.5)}
 
 
 @functools.lru_cache(maxsize=4096)
@@ -295,9 +296,9 @@ def float_gemm_plan(M: int, N: int, K: int, batch: int, compute_units: int) -> t
     """The tile of a float product: the one whose rounds of workgroups take the least time.  The result of the product does
     not depend on it."""
     def cost(tile):
-        per_round, fixed = FLOAT_GEMM_TILES[tile]
+        per_round, per_columns, fixed = FLOAT_GEMM_TILES[tile]
         workgroups = -(-M // (16 * tile[0])) * -(-N // (16 * tile[1])) * batch
-        return fixed + -(-workgroups // compute_units) * per_round * K / 2048
+        return fixed + -(-workgroups // compute_units) * (per_round + per_columns * K / 2048)
     return min(FLOAT_GEMM_TILES, key=cost)
 
 

@@ -39,6 +39,24 @@ def test_float_product_in_every_form(m, n, k):
     assert bool(((outs[0].double() - want).abs() <= chain * 2.0 ** -24 * size + 1e-30).all())
 
 
+@pytest.mark.parametrize("m,n,k", [(300, 16, 32), (70, 130, 64), (33, 260, 96), (40, 9, 480), (129, 600, 7)])
+def test_float_product_of_short_rows_in_every_form(m, n, k):
+    """One, two, three and fifteen slices with columns, each with as many wavefronts; one tile of weight rows, groups of eight tiles that
+    are not full, and the bound above."""
+    test_float_product_in_every_form(m, n, k)
+
+
+@pytest.mark.parametrize("t,heads,n,k", [(700, 9, 64, 64), (130, 3, 128, 40), (5, 16, 512, 128)])
+def test_float_products_of_heads_at_several_tiles(t, heads, n, k):
+    """Rows and weight rows of several tiles in every head's product.  Bound: as for one product."""
+    o = ops()
+    a, w = rnd(t, heads, k, seed=5), rnd(heads, n, k, seed=6)
+    got = o.gemm_heads(a.cuda(), o.HeadMatrices(w.cuda())).cpu().double()
+    for h in range(heads):
+        want, size = a[:, h].double() @ w[h].double().T, a[:, h].double().abs() @ w[h].double().abs().T
+        assert bool(((got[:, h] - want).abs() <= 40 * 2.0 ** -24 * size + 1e-30).all()), h
+
+
 def test_float_product_batches():
     """Heads side by side in the rows, one matrix each, written into wider rows."""
     o = ops()

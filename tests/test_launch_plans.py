@@ -85,3 +85,14 @@ def test_decode_attention_of_large_heads_keeps_to_four_wavefronts():
     for d in (144, 160, 256):
         assert ops.attention_plan(64, 1, 1, 2048, 16, d, 160 * 1024) == (4, 512, 4)
     assert ops.attention_plan(64, 1, 1, 2048, 16, 128, 160 * 1024) == (8, 512, 4)
+
+
+def test_float_products_of_short_rows_take_small_tiles_until_the_gpu_is_full():
+    """What a workgroup takes whatever its columns counts: few rows of heads with short rows go in the smallest tiles, large steps in large
+    ones, and products of long rows as the rounds say."""
+    plan = ops.float_gemm_plan
+    for rows in (1, 8, 16):
+        for heads in (1, 16, 64):
+            assert plan(rows, 64, 64, heads, 256) == (1, 1)
+    assert plan(130, 128, 64, 16, 256) in ((1, 2), (2, 2)) and plan(4096, 64, 64, 64, 256) == (4, 4)
+    assert plan(301, 2048, 2048, 1, 256) == (3, 4) and plan(301, 2560, 2048, 1, 256) == (4, 4) and plan(8, 2048, 2048, 1, 256) == (1, 1)
