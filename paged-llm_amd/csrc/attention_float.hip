@@ -7,10 +7,12 @@
 // is the operand layout of O^T = V^T P^T as it stands: a lane's 16-byte load of V (four consecutive positions of a channel)
 // meets its four weights in four instructions, and nothing is moved between lanes.
 //
-// The keys are cut into blocks of 64 at absolute positions 0, 64, 128, ...; wavefront w of the workgroup's eight (four for
-// heads above 128) takes the blocks whose number is w modulo their count, each with a running maximum of its own, and the
-// wavefronts' results are joined in their order.  A block that a column does not see changes none of its bits, so a
-// column's result is the same however the tokens were cut into steps or batched.
+// The keys are cut into blocks of 64 at absolute positions 0, 64, 128, ...; wavefront w of the workgroup's eight (fewer for
+// heads above 128 and short windows) takes the blocks whose number is w modulo their count, each with a running maximum of its own,
+// and the wavefronts' results are joined in their order.  A block that a column does not see changes none of its bits, so a
+// column's result is the same however the tokens were cut into steps or batched.  Of a block that is seen in part, the tiles of 16
+// keys that no column sees are left out (a prompt of 17 tokens, 32 heads of 64 on 4: 12.5 us, 13.5 with the whole block; 24 heads of
+// 256 on 8: 19 and 27).
 //
 // What bounds it: a wavefront's chain of load, scores, exponentials and values per block for few columns (decoding: 8
 // requests, contexts to 700, 32 heads of 64 on 4: 186 us with one wavefront per token and head), and the matrix cores
@@ -45,7 +47,7 @@ __device__ __forceinline__ float column_sum(float v) {
 
 // DT: head size / 16.
 template <int DT, int WAVES>
-__global__ __launch_bounds__(64 * WAVES) void paged_attention_float_kernel(FloatAttention p) {
+__global__ __launch_bounds__(64 * WAVES, DT <= 8 ? 2 : 1) void paged_attention_float_kernel(FloatAttention p) {
   constexpr int D = 16 * DT, kChunk = DT < 8 ? DT : 8;
   constexpr bool kEarly = DT <= 4;                                     // registers for a whole block's keys and values at once
   __shared__ float lds_m[WAVES][kColumns], lds_l[WAVES][kColumns];
@@ -102,12 +104,14 @@ __global__ __launch_bounds__(64 * WAVES) void paged_attention_float_kernel(Float
     }
     const bool whole = n0 + kBlock - 1 <= pos_min && n0 >= all_from;   // every column sees every key of the block
     f32x4 s[kTiles];
+    bool live[kTiles], all_live = true;                                // (the same for all lanes: a tile that no column sees is left out)
     const float *k_at[kTiles], *v_at[kTiles];                          // (a tile lies inside one page)
 #pragma unroll
     for (int i = 0; i < kTiles; ++i) {
       const int n = n0 + i * kTile;
-      const bool live = n <= pos_max && (n + kTile > any_from || n < p.keep_first);
-      const int from = live ? n : pos_max / kTile * kTile;             // (a tile that no column sees: any valid one, for loads without conditions)
+      live[i] = n <= pos_max && (n + kTile > any_from || n < p.keep_first);
+      all_live = all_live && live[i];
+      const int from = live[i] ? n : pos_max / kTile * kTile;          // (a tile that no column sees: any valid one, for loads without conditions)
       const size_t page = (size_t)bt[from / p.block_size] * p.num_kv_heads + kvh;
       k_at[i] = p.k_pages + (page * p.block_size + from % p.block_size + column) * D + 4 * quad;
       v_at[i] = p.v_pages + (page * D + column) * p.block_size + from % p.block_size + 4 * quad;
@@ -125,16 +129,28 @@ __global__ __launch_bounds__(64 * WAVES) void paged_attention_float_kernel(Float
         for (int t = 0; t < DT; ++t) v_early[i][t] = *reinterpret_cast<const f32x4*>(v_at[i] + (size_t)16 * t * p.block_size);
 #pragma unroll
       for (int i = 0; i < kTiles; ++i) s[i] = f32x4{0.f, 0.f, 0.f, 0.f};
+      if (all_live) {
 #pragma unroll
-      for (int t = 0; t < DT; ++t)
+        for (int t = 0; t < DT; ++t)
 #pragma unroll
-        for (int j = 0; j < 4; ++j)
+          for (int j = 0; j < 4; ++j)
 #pragma unroll
-          for (int i = 0; i < kTiles; ++i) s[i] = __builtin_amdgcn_mfma_f32_16x16x4f32(k[i][t][j], q[t][j], s[i], 0, 0, 0);
+            for (int i = 0; i < kTiles; ++i) s[i] = __builtin_amdgcn_mfma_f32_16x16x4f32(k[i][t][j], q[t][j], s[i], 0, 0, 0);
+      } else {
+#pragma unroll
+        for (int i = 0; i < kTiles; ++i)
+          if (live[i]) {
+#pragma unroll
+            for (int t = 0; t < DT; ++t)
+#pragma unroll
+              for (int j = 0; j < 4; ++j) s[i] = __builtin_amdgcn_mfma_f32_16x16x4f32(k[i][t][j], q[t][j], s[i], 0, 0, 0);
+          }
+      }
     } else {
 #pragma unroll
       for (int i = 0; i < kTiles; ++i) {
         s[i] = f32x4{0.f, 0.f, 0.f, 0.f};
+        if (!live[i]) continue;
 #pragma unroll
         for (int t0 = 0; t0 < DT; t0 += kChunk) {
           f32x4 k[kChunk];
@@ -182,7 +198,8 @@ __global__ __launch_bounds__(64 * WAVES) void paged_attention_float_kernel(Float
       for (int t = 0; t < DT; ++t) o[t] *= alpha;
     }
 #pragma unroll
-    for (int i = 0; i < kTiles; ++i)
+    for (int i = 0; i < kTiles; ++i) {
+      if (!live[i]) continue;
 #pragma unroll
       for (int t0 = 0; t0 < DT; t0 += kChunk) {
         const int n = n0 + i * kTile;
@@ -230,6 +247,7 @@ __global__ __launch_bounds__(64 * WAVES) void paged_attention_float_kernel(Float
           for (int t = 0; t < kChunk; ++t)
             if (t0 + t < DT) o[t0 + t] = __builtin_amdgcn_mfma_f32_16x16x4f32(v[t][j], s[i][j], o[t0 + t], 0, 0, 0);
       }
+    }
   }
 
   l = column_sum(l);
@@ -264,9 +282,15 @@ __global__ __launch_bounds__(64 * WAVES) void paged_attention_float_kernel(Float
   }
 }
 
-template <int DT>
+// Wavefronts of a workgroup: eight (heads above 128: four), or one or two for layers whose window is so short that a tile of columns sees
+// keys of two to four blocks only.  Further wavefronts would find no block, and keep other workgroups off the compute unit (200
+// requests at context 300, 16 heads of 64: a window of 30 31 us with one wavefront and 69 with four, a window of 100 51 us with two,
+// 78 with four and 135 with eight, where the plain kernel takes 28 and 66; one request 12 to 16 us in any form).  The window is the
+// layer's, so a layer's columns keep their order of additions in every step.
+constexpr int kOneWaveWindow = 64, kTwoWaveWindow = 128;
+
+template <int DT, int kWaves>
 static int launch_float_attention(const FloatAttention& p, int total_q, hipStream_t stream) {
-  constexpr int kWaves = DT <= 8 ? 8 : 4;
   const int group = p.num_heads / p.num_kv_heads;
   const dim3 grid((unsigned)((long)total_q * group / kColumns + p.num_seqs), p.num_kv_heads), block(64 * kWaves);
   const size_t lds = (size_t)kWaves * DT * 64 * sizeof(f32x4);
@@ -293,7 +317,12 @@ PLLM_API int pllm_paged_attention_float(const float* q, int q_stride, const floa
   if (!sixteen(q) || !sixteen(k_pages) || !sixteen(v_pages) || !sixteen(out) || q_stride % 4 || out_stride % 4) return -3;
   const FloatAttention p{q, k_pages, v_pages, out, block_tables, cu_seqlens_q, seq_lens_k, head_bias, ScoreTerms{score_cap, slopes, sinks},
                          q_stride, out_stride, bt_stride, num_seqs, num_heads, num_kv_heads, block_size, window, keep_first, weighting, scale};
-#define CASE(n) case n: return launch_float_attention<n>(p, total_q, stream);
+  const int reach = window < 0 ? -window : window;
+#define CASE(n)                                                                                             \
+  case n:                                                                                                   \
+    if (reach > 0 && reach <= kOneWaveWindow) return launch_float_attention<n, 1>(p, total_q, stream);      \
+    if (reach > 0 && reach <= kTwoWaveWindow) return launch_float_attention<n, 2>(p, total_q, stream);      \
+    return launch_float_attention<n, n <= 8 ? 8 : 4>(p, total_q, stream);
   switch (head_dim / 16) {
     CASE(1) CASE(2) CASE(3) CASE(4) CASE(5) CASE(6) CASE(7) CASE(8) CASE(9) CASE(10) CASE(11) CASE(12) CASE(13) CASE(14) CASE(15) CASE(16)
   }

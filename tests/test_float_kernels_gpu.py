@@ -109,6 +109,25 @@ def test_float_attention_does_not_depend_on_the_cut():
             assert torch.equal(part[:hi - lo], whole[lo:hi]) and torch.equal(part[hi - lo:], whole[hi - 1:hi]), (window, lo, hi)
 
 
+@pytest.mark.parametrize("window", [1, 64, 128, 129, -64, -128, -129])
+@pytest.mark.parametrize("heads,kv_heads,d", [(3, 3, 64), (8, 2, 128), (4, 4, 16)])
+def test_float_attention_of_short_windows(heads, kv_heads, d, window):
+    """Windows on both sides of the length from which a workgroup has more wavefronts: a portion and single tokens against the plain kernel
+    (bound as above), and the same bits for a position however it was cut."""
+    o = ops()
+    bs, n = 16, 391
+    q, kp, vp, tables, cu, sl = paged_case([n], [n], heads, kv_heads, d, bs, torch.float32, seed=6)
+    rest, tail = (kp.cuda(), vp.cuda()), (heads, kv_heads, d, d ** -0.5, window)
+    for weights in (None, o.KeyWeights(sigmoid=True)) + ((o.KeyWeights(keep_first=70),) if window > 0 else ()):
+        args = (q.cuda(), *rest, tables.cuda(), cu.cuda(), sl.cuda(), *tail)
+        whole, want = o.paged_attention_float(*args, weights=weights), o.paged_attention_generic(*args, weights=weights)
+        assert float((whole - want).abs().max() / want.abs().max()) <= 4e-5
+        for lo, hi in ((0, 1), (127, 130), (255, 256), (n - 1, n), (60, 200)):
+            part = o.paged_attention_float(q[lo:hi].cuda(), *rest, tables.cuda(), torch.tensor([0, hi - lo], dtype=torch.int32, device="cuda"),
+                                           torch.tensor([hi], dtype=torch.int32, device="cuda"), *tail, weights=weights)
+            assert torch.equal(part, whole[lo:hi]), (lo, hi)
+
+
 def test_float_attention_leaves_unseen_slots_alone():
     """Garbage past the context, in table entries past it and in front of a window changes nothing; an infinite value reaches
     the queries that see its key and no other."""
