@@ -1525,15 +1525,21 @@ def recurrence_form(max_q_len: int, num_tokens: int, num_seqs: int, heads: int, 
         # pieces (130 tokens and 32 single ones: token by token 242, pieces 79, chunks 338),
         # long portions in chunks (2,048: pieces 460, chunks 142) of so many pieces that their workgroups fill the GPU once:
         # chunks of 1 / 2 / 4 / 8 pieces take 200 / 159 / 152 / 142, and at 512 tokens 62 / 53 / 64 / 101.
-        wide = by_row or rows > 128                     # workgroups of eight wavefronts, one to a compute unit; else of four, two
-        slots = compute_units * (1 if wide else 2)
+        # A decay per row costs a piece twice the work of one per head (2,048 tokens and 32 single ones, 64 heads of 64 x 64: pieces 947,
+        # chunks 392; 130 and 8 single ones, 16 heads of 128 x 128: pieces 100, chunks 59).
+        small = rows <= 64 and columns <= 64            # (whose LDS with a decay per row leaves room for two workgroups as well)
+        wide = rows > 128 or (by_row and not small)     # workgroups of eight wavefronts, one to a compute unit; else of four, two
+        slots = compute_units * (1 if wide else 4 if by_row and rows <= 32 and columns <= 32 else 2)     # (the smallest: of two, four)
         groups = heads * -(-columns // (128 if wide else 64))
         pieces, fill = -(-max_q_len // RECURRENCE_PIECE), max(1.0, num_seqs * groups / slots)
         chunk = -(-(-(-num_tokens // RECURRENCE_PIECE) * groups) // slots)
         by_token = 6.0 + 1.25 * max_q_len + 5.0 * fill
-        in_pieces = 25.0 * fill + 12.5 * (pieces - 1) if wide else 16.0 * fill + 7.0 * (pieces - 1)
+        in_pieces = 30.0 * fill + 14.5 * (pieces - 1) if by_row else 25.0 * fill + 12.5 * (pieces - 1) if wide else 16.0 * fill + 7.0 * (pieces - 1)
         beside = (num_seqs - 1) * groups / slots
-        in_chunks = 36.0 + 25.0 * (chunk - 1) + 100.0 * beside if wide else 30.0 + 14.0 * (chunk - 1) + 75.0 * beside
+        if by_row and rows <= 64:                       # (states of few bytes: 32 / 200 single tokens cost 53 / 182 a filled GPU)
+            in_chunks = 36.0 + 25.0 * (chunk - 1) + (25.0 + 0.8 * num_seqs) * beside
+        else:
+            in_chunks = 36.0 + 25.0 * (chunk - 1) + 100.0 * beside if wide or by_row else 30.0 + 14.0 * (chunk - 1) + 75.0 * beside
         return min((by_token, 0), (in_pieces, -1), (in_chunks, RECURRENCE_PIECE * chunk))[1]
     return recurrence_chunk(max_q_len, num_tokens)
 

@@ -887,11 +887,14 @@ static int launch_pieces(RecurrenceArgs a, const ChunkArgs& ca, int max_chunks, 
 
 // Wavefronts (tiles of 16 columns) of a workgroup: eight for tall states and for a decay per row, whose work per piece that
 // all columns share is large and whose LDS leaves room for one workgroup; else four, two workgroups to a compute unit (257
-// columns, a normaliser's: 55 us as four and one tile over, 75 us in workgroups of five, which do not pair up; 777 tokens).
+// columns, a normaliser's: 55 us as four and one tile over, 75 us in workgroups of five, which do not pair up; 777 tokens).  Small
+// states with a decay per row fill their tiles: 100 heads of 32 x 32, 2,048 tokens, 190 us in workgroups of two wavefronts and 286 us
+// padded to 64 x 64 (248 us token by token in chunks).
 template <int MODE>
 static int launch_piece_pass(const RecurrenceArgs& a, const ChunkArgs& ca, int max_chunks, int vec, hipStream_t stream) {
   const int tiles = (a.ld + 15) / 16;
   if (a.row_decay) {
+    if (a.N <= 32 && tiles <= 2) return launch_pieces<2, 2, MODE, true>(a, ca, max_chunks, vec, stream);
     if (a.N <= 64) return tiles <= 4 ? launch_pieces<4, 4, MODE, true>(a, ca, max_chunks, vec, stream) : launch_pieces<4, 8, MODE, true>(a, ca, max_chunks, vec, stream);
     return tiles <= 4 ? launch_pieces<8, 4, MODE, true>(a, ca, max_chunks, vec, stream) : launch_pieces<8, 8, MODE, true>(a, ca, max_chunks, vec, stream);
   }

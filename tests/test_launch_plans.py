@@ -96,3 +96,12 @@ def test_float_products_of_short_rows_take_small_tiles_until_the_gpu_is_full():
             assert plan(rows, 64, 64, heads, 256) == (1, 1)
     assert plan(130, 128, 64, 16, 256) in ((1, 2), (2, 2)) and plan(4096, 64, 64, 64, 256) == (4, 4)
     assert plan(301, 2048, 2048, 1, 256) == (3, 4) and plan(301, 2560, 2048, 1, 256) == (4, 4) and plan(8, 2048, 2048, 1, 256) == (1, 1)
+
+
+def test_recurrences_with_a_decay_per_row_run_in_chunks_beside_few_single_tokens():
+    """Pieces, one workgroup a sequence and head, are for portions beside so many single tokens that a workspace of all their states costs more."""
+    plan = ops.recurrence_form
+    assert plan(2048, 2080, 33, 64, 64, 64, True, 256) > 0 and plan(130, 138, 9, 16, 128, 128, True, 256) > 0
+    assert plan(130, 162, 33, 4, 32, 32, True, 256) == 32 and plan(700, 1164, 6, 64, 64, 64, True, 256) > 0
+    assert plan(8192, 8192, 1, 64, 64, 64, True, 256) <= 1024
+    assert plan(500, 564, 65, 16, 128, 128, True, 256) == -1 and plan(500, 564, 65, 100, 32, 32, True, 256) == -1

@@ -25,7 +25,8 @@ def token_by_token(q, k, v, decay, S):
 CASES = [  # heads, key heads, N, P, kind, type of rows, normaliser, columns of padding in the rows
     (2, 2, 16, 16, "head", torch.float32, False, 0), (4, 1, 128, 64, "steps", torch.bfloat16, False, 8), (2, 2, 256, 130, "constant", torch.float32, False, 0),
     (3, 3, 70, 66, "head", torch.float32, True, 3), (2, 2, 128, 256, "head", torch.float32, True, 0), (2, 2, 128, 128, "row", torch.float32, False, 0),
-    (2, 2, 50, 30, "row", torch.float32, True, 1), (1, 1, 64, 200, "row", torch.float32, False, 4), (2, 1, 33, 17, "constant", torch.bfloat16, False, 5)]
+    (2, 2, 50, 30, "row", torch.float32, True, 1), (1, 1, 64, 200, "row", torch.float32, False, 4), (2, 1, 33, 17, "constant", torch.bfloat16, False, 5),
+    (3, 3, 32, 32, "row", torch.bfloat16, False, 0), (2, 2, 20, 17, "row", torch.float32, True, 3), (2, 2, 32, 33, "row", torch.float32, False, 0)]
 
 
 @pytest.mark.parametrize("chunk", [-1, 32, 96])
