@@ -55,6 +55,7 @@ TILE_PARTIAL_FROM_ROWS, TILE_PARTIAL_MIN_ELEMENTS, TILE_PARTIAL_MOST_RANGES = 65
 STREAM_GATED_MAX_ROWS = 64                      # the gated product: beyond, its rows' traffic costs more than the library's kernel
                                                 # (asked only where the tiled kernel does not take the product: _tiles_gated)
 STREAM_FLOAT_MAX_ROWS = 64                       # a product with float results: beyond, the library's kernel is as fast
+STREAM_FLOAT_LONG_K, STREAM_FLOAT_LONG_MIN_WEIGHT_ROWS = 4608, 2048   # ... and from this K on for matrices of fewer weight rows
 STREAM_LONG_K, STREAM_LONG_K_MAX_ROWS = 8192, 64 # from this K on a product in one range takes the streaming kernel up to so many rows
 
 
@@ -111,8 +112,10 @@ def _streams(x, weight, epi: int, partial_ok: bool = False) -> bool:
     if epi == ops.SL_F32:
         # Branches with float results: up to 64 rows and K below 8192 (33 rows: 2048 x 2048 / 4096 / 5632 5.8 / 10.2 / 13.3 us against the
         # library's 8.2 / 12.1 / 15.3, 4096 x 2048 7.5 and 11.7, 2048 x 8192 18.5 and 14.1; 64 rows of 2048 x 2048 5.8 and 8.6, 100 rows 8.6
-        # and 8.4).  The head has too many weight rows: 32000 x 2048 was not faster.
-        return weight.pairing == "plain" and rows <= STREAM_FLOAT_MAX_ROWS and k < STREAM_LONG_K and _few_weight_rows(weight)
+        # and 8.4).  The head has too many weight rows: 32000 x 2048 was not faster.  Few weight rows of long K are too few workgroups in
+        # one range, where the library cuts K (33 rows: 1024 x 4608 11.2 and 12.2, 1024 x 5632 12.9 and 10.0, 512 x 6144 13.0 and 8.6).
+        return (weight.pairing == "plain" and rows <= STREAM_FLOAT_MAX_ROWS and k < STREAM_LONG_K and _few_weight_rows(weight)
+                and (n >= STREAM_FLOAT_LONG_MIN_WEIGHT_ROWS or k <= STREAM_FLOAT_LONG_K))
     # (cut into ranges of K the long products stay ahead of the library up to 128 rows: 4096 x 14336 at 96 / 128 rows 45.7 / 55.4 us
     #  against 62.6 / 74.8, 2048 x 8192 16.1 / 18.4 against 20.8)
     return _few_weight_rows(weight) and (k < STREAM_LONG_K or rows <= STREAM_LONG_K_MAX_ROWS or (partial_ok and epi == ops.SL_BF16))

@@ -535,8 +535,9 @@ def test_embedding_and_head_parts(dtype, tol):
         assert rel(own.forward(xm.cuda()), xm.float() @ hw.T) <= tol
 
 
-@pytest.mark.parametrize("rows,n,k,streams", [(17, 2048, 2048, True), (64, 96, 5632, True), (64, 4096, 64, True), (65, 2048, 2048, False), (33, 2048, 8192, False),
-                                              (33, 9000, 64, False), (16, 2048, 2048, False)])
+@pytest.mark.parametrize("rows,n,k,streams", [(17, 2048, 2048, True), (64, 96, 4608, True), (64, 4096, 64, True), (65, 2048, 2048, False), (33, 2048, 8192, False),
+                                              (33, 9000, 64, False), (16, 2048, 2048, False), (33, 1024, 4608, True), (33, 1024, 5632, False),
+                                              (20, 512, 6144, False), (64, 2048, 7168, True)])
 def test_products_with_float_results_choose_their_kernel_by_size(rows, n, k, streams):
     """17 to 64 rows, K below 8192 and few weight rows take the streaming kernel, the rest the library or the kernel for fewer rows; matrices
     whose tiles pair rows for another epilogue never do."""
