@@ -457,7 +457,7 @@ __global__ __launch_bounds__(kStreamThreads) void tile_linear_kernel(const Strea
         }
         return;
       }
-if (p.weights_once) issue_blocks(s, slot, true);
+      if (p.weights_once) issue_blocks(s, slot, true);
       else issue_blocks(s, slot, false);
     };
 #pragma unroll
