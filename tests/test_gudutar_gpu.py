@@ -213,21 +213,28 @@ def test_float32_logits_do_not_depend_on_the_cut(folders, name, dtype):
 
 
 @pytest.mark.parametrize("dtype", ["float32", "bfloat16"])
-@pytest.mark.parametrize("name", ["A", "B", "C"])
+@pytest.mark.parametrize("name", ["A", "B", "C", "mamba2_many_state_rows"])
 def test_long_portions_run_in_chunks(folders, name, dtype):
     """Portions of 128 tokens and more take the recurrences' chunked form (a chunk's own state from zero, the states
     carried from chunk to chunk, outputs from each chunk's starting state): lengths at, just past and between the
     chunks' borders, a second long portion that starts from a carried state, and short and single-token sequences beside
-    a long one in the same step."""
+    a long one in the same step.  Chunks of 32 as matrix products, or, for 272 state rows, of 16 token by token."""
     from paged_llm_amd.csrc import ops
-    assert ops.recurrence_chunk(128, 300) == 16 and ops.recurrence_chunk(127, 300) == 0 and ops.recurrence_chunk(2048, 2048) == 64
+    for layer in CONFIGS[name]["layers"]:
+        m, cus = layer["mixer"], torch.cuda.get_device_properties(0).multi_processor_count
+        rows = {"mamba2": "state", "retention": "dim"}.get(layer["type"])
+        if rows:
+            for longest, tokens, seqs in ((129, 130, 2), (191, 197, 3), (128, 256, 2)):
+                form = ops.recurrence_form(longest, tokens, seqs, m["heads"], m[rows], m["vdim"], False, cus)
+                assert form == (32 if m[rows] <= 256 else 16)
+            assert ops.recurrence_form(127, 256, 3, m["heads"], m[rows], m["vdim"], False, cus) == 0
     folder = folders(name, stored_as(dtype))
     vocab = CONFIGS[name]["vocab"]
     reqs = {"long": helpers.random_tokens(449, vocab, 20), "side": helpers.random_tokens(150, vocab, 21),
             "short": helpers.random_tokens(30, vocab, 22)}
     trace = TraceBuilder()
     trace.step([("short", reqs["short"][:9], "all")])
-    trace.step([("short", reqs["short"][9:10], "all"), ("long", reqs["long"][:129], "all")])           # 129 = two chunks and one token
+    trace.step([("short", reqs["short"][9:10], "all"), ("long", reqs["long"][:129], "all")])           # 129 = whole chunks and one token
     trace.step([("short", reqs["short"][10:11], "all"), ("side", reqs["side"][:5], "all"), ("long", reqs["long"][129:320], "all")])
     trace.step([("side", reqs["side"][5:133], "all"), ("long", reqs["long"][320:448], "all")])         # two portions of 128
     trace.step([("long", reqs["long"][448:], "all"), ("side", reqs["side"][133:], "all"), ("short", reqs["short"][11:], "all")],

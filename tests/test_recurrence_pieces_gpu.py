@@ -88,6 +88,19 @@ def test_pieces_against_token_by_token(H, KH, N, P, kind, dtype, normaliser, pad
     assert torch.equal(st[:, :2].cpu(), state[:, :2]) and torch.equal(st[:, 2 + H * N * ld:].cpu(), state[:, 2 + H * N * ld:]) and torch.equal(st[4].cpu(), state[4])
 
 
+TALL = [(2, 1, 272, 20, "head", torch.float32, False, 0), (2, 2, 600, 70, "steps", torch.bfloat16, False, 8), (1, 1, 1024, 16, "constant", torch.float32, True, 3),
+        (2, 2, 144, 40, "row", torch.float32, False, 4), (1, 1, 300, 66, "row", torch.bfloat16, True, 1)]
+
+
+@pytest.mark.parametrize("chunk", [0, 16, 64])
+@pytest.mark.parametrize("H,KH,N,P,kind,dtype,normaliser,pad", TALL)
+def test_states_too_tall_for_pieces(H, KH, N, P, kind, dtype, normaliser, pad, chunk, monkeypatch):
+    """More rows than the matrix form takes: token by token in one workgroup and in chunks, whose borders the lengths meet, pass and
+    miss; the bound above (sums over up to 1,024 rows are cut into as many as there are wavefronts)."""
+    assert ops().recurrence_form(131, 294, 6, H, N, P + normaliser, kind == "row", 256) == 16
+    test_pieces_against_token_by_token(H, KH, N, P, kind, dtype, normaliser, pad, chunk, monkeypatch)
+
+
 @pytest.mark.parametrize("by_row", [False, True])
 @pytest.mark.parametrize("chunk", [-1, 64])
 def test_a_value_that_is_no_number_reaches_later_tokens_only(by_row, chunk, monkeypatch):
