@@ -31,6 +31,24 @@ def test_attention_plan_always_returns_a_launch_the_kernels_take():
             assert ops._merge_lds_bytes(ncb, waves, d) <= lds, what
 
 
+def test_attention_plan_of_up_to_512_keys_in_one_piece():
+    """Eight wavefronts take 257 to 512 keys of up to 16 columns without a merge, for heads up to 128 and work items that fit the compute
+    units; every edge of that has another plan beyond it."""
+    plan, lds = ops.attention_plan, 160 * 1024
+    for keys in (257, 300, 512):
+        assert plan(1, 4, 1, keys, 8, 64, lds) == plan(8, 4, 1, keys, 16, 128, lds) == plan(64, 4, 1, keys, 1, 64, lds) == (8, 0, 1)
+    assert plan(1, 4, 1, 256, 8, 64, lds) == (4, 0, 1) and plan(1, 4, 1, 513, 8, 64, lds) == (4, 256, 3)
+    assert plan(1, 4, 1, 512, 17, 64, lds) == (4, 256, 2) and plan(1, 4, 2, 512, 8, 64, lds) == (8, 0, 1) and plan(1, 4, 3, 512, 8, 64, lds) == (4, 256, 2)
+    assert plan(1, 4, 1, 512, 8, 144, lds) == (4, 256, 2) and plan(257, 1, 1, 512, 8, 64, lds) == (4, 0, 1)
+    rng = np.random.default_rng(8)
+    for _ in range(300):
+        seqs, kv_heads, group = int(rng.integers(1, 300)), int(rng.choice([1, 2, 4, 8, 16])), int(rng.choice([1, 3, 8, 16]))
+        keys, d = int(rng.choice([257, 300, 511, 512])), int(rng.choice([16, 48, 64, 96, 128, 160]))
+        waves, size, parts = plan(seqs, kv_heads, 1, keys, group, d, lds)
+        assert waves in (4, 8) and ((size, parts) == (0, 1) or (parts > 1 and (parts - 1) * size < keys <= parts * size))
+        assert ops._merge_lds_bytes(1, waves, d) <= lds
+
+
 def test_attention_plan_depends_on_sizes_only():
     a = ops.attention_plan(8, 4, 1, 2048, 8, 64, 160 * 1024)
     assert a == ops.attention_plan(8, 4, 1, 2048, 8, 64, 160 * 1024) == (4, 256, 8)
