@@ -455,14 +455,29 @@ __global__ __launch_bounds__(256) void recurrence_carry_kernel(RecurrenceArgs a,
   *slot = S;
 }
 
+// (Chunks come here only for states that the matrix form below does not take: more than 42 rows a wavefront.)
 template <int MODE>
 static void launch_recurrence(const RecurrenceArgs& a, const ChunkArgs& ca, dim3 grid, int waves, int need, hipStream_t stream) {
   dim3 block(64 * waves);
-  if (waves > 4) hipLaunchKernelGGL((linear_recurrence_kernel<64, 1024, MODE>), grid, block, 0, stream, a, ca);
-  else if (need <= 8) hipLaunchKernelGGL((linear_recurrence_kernel<8, 256, MODE>), grid, block, 0, stream, a, ca);
-  else if (need <= 16) hipLaunchKernelGGL((linear_recurrence_kernel<16, 256, MODE>), grid, block, 0, stream, a, ca);
-  else if (need <= 32) hipLaunchKernelGGL((linear_recurrence_kernel<32, 256, MODE>), grid, block, 0, stream, a, ca);
-  else hipLaunchKernelGGL((linear_recurrence_kernel<64, 256, MODE>), grid, block, 0, stream, a, ca);
+  if (waves > 4) {
+    hipLaunchKernelGGL((linear_recurrence_kernel<64, 1024, MODE>), grid, block, 0, stream, a, ca);
+    return;
+  }
+  if constexpr (MODE == kWhole) {
+    if (need <= 8) {
+      hipLaunchKernelGGL((linear_recurrence_kernel<8, 256, MODE>), grid, block, 0, stream, a, ca);
+      return;
+    }
+    if (need <= 16) {
+      hipLaunchKernelGGL((linear_recurrence_kernel<16, 256, MODE>), grid, block, 0, stream, a, ca);
+      return;
+    }
+    if (need <= 32) {
+      hipLaunchKernelGGL((linear_recurrence_kernel<32, 256, MODE>), grid, block, 0, stream, a, ca);
+      return;
+    }
+  }
+  hipLaunchKernelGGL((linear_recurrence_kernel<64, 256, MODE>), grid, block, 0, stream, a, ca);
 }
 
 // ---------------------------------------------------------------------------------------------
