@@ -1,5 +1,6 @@
-// C[M, N] = A[M, K] * W[N, K]^T for bfloat16 operands with float accumulation, for any M, N and K: the fallback for
-// shapes that the matrix-core kernels and the library are not given.
+// C[M, N] = A[M, K] * W[N, K]^T for bfloat16 operands with float accumulation, for any M, N and K: one plain kernel behind
+// ops.gemm_generic for callers of that operation.  The parts do not come here: parts/linear.py gives every bfloat16 product to the
+// matrix-core kernels or to the library.
 //
 // 64 x 64 output tile per workgroup of 256 threads, 4 x 4 outputs per thread, K walked in
 // slabs of 16 through LDS.  Every output element is summed over k in ascending order by one

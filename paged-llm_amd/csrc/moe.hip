@@ -776,7 +776,8 @@ __global__ __launch_bounds__(256) void moe_expert_tile_kernel(const bf16* __rest
 // experts of 1,024 at width 1,024 41 + 22 / 16 + 10, 300 with 2 of 8 of 512 27 + 14 / 11 + 7).
 // What bounds large tiles is the drawing of the operands, as in the tiled products of whole steps: the compute unit's rate is the same
 // whatever the tile, so a tile of 256 weight rows (48 KB a stage) takes the place of two of 128 (64 KB) where that needs no more
-// rounds.  The sums run over ascending k in one accumulator per output, as in the kernels above, and give the same bits.
+// rounds.  The sums run over ascending k in one accumulator per output, in steps of 32: the same bits for tiles of 16, 64 and 128
+// rows, and those of the kernels above for 64 and 128 (the kernel above for 16 rows pairs the elements of two k-steps another way).
 
 constexpr int kReadOnce = 2;                                 // a load's cache policy: nt, the line is the first to leave the caches
 

@@ -310,7 +310,7 @@ def _gemm_float(a_ptr, lda, a_batch, w_ptr, ldw, w_batch, out_ptr, ldc, c_batch,
 
 def gemm_generic(a: torch.Tensor, w: torch.Tensor, out_dtype: torch.dtype | None = None) -> torch.Tensor:
     """a [M, K] times w [N, K] transposed with float accumulation, any sizes: float32 on the float matrix cores (the order of
-    the additions depends on K alone), bfloat16 on the plain kernel (ascending k)."""
+    the additions depends on K alone), bfloat16 on the plain kernel (ascending k; the parts give such products to other kernels)."""
     _on_gpu(a, w)
     _need(a.dim() == 2 and w.dim() == 2 and a.shape[1] == w.shape[1], f"gemm shapes {tuple(a.shape)} x {tuple(w.shape)}^T")
     _need(a.stride(1) == 1 and w.stride(1) == 1, "gemm operands need unit inner stride")
@@ -1381,8 +1381,8 @@ def round_rows(x: torch.Tensor) -> torch.Tensor:
 
 # ------------------------------------------------------------------------------------------- per-head products
 class HeadMatrices:
-    """One matrix per head, [heads, N, K] as a checkpoint stores them, in the order ``gemm_heads`` reads: float32 as they are (the plain
-    kernel takes rows of K), bfloat16 with N innermost, [heads, K, N] contiguous.  (The vendor's batched bfloat16 product has
+    """One matrix per head, [heads, N, K] as a checkpoint stores them, in the order ``gemm_heads`` reads: float32 as they are (the float
+    product takes rows of K), bfloat16 with N innermost, [heads, K, N] contiguous.  (The vendor's batched bfloat16 product has
     faulted on this hardware with a transposed view as its right operand: it is only ever given a contiguous one.)"""
 
     __slots__ = ("data", "heads", "out_features", "in_features")
@@ -2284,8 +2284,10 @@ def moe_tile_rows(pairs: int, experts: int, dtype: torch.dtype, *inner_sizes: in
     """Rows of a tile of the experts' products for a step of ``pairs`` (token, choice) pairs: where the matrix-core
     kernels run (bfloat16, every product's inner size a multiple of 8) 128 if an expert gets 32 pairs or more on average, 64
     where tiles of 128 would leave compute units idle (small experts) unless an expert gets 128; else 16.  (Both products at width
-    2,048, 30 gated experts of 1,408, 256 tokens with 4 choices: 126 us with tiles of 128, 119 with 64, 170 with 16; 16 experts of
-    1,024 at width 1,024, 256 tokens with 2: 27, 25 and 38; 8 of 512, 300 tokens with 2: 22, 18 and 20.)  It depends on the step's number of tokens only, so a replayed step keeps its choice."""
+    2,048, 30 gated experts of 1,408, 256 tokens with 4 choices, 34 pairs an expert: 126 us with tiles of 128, 119 with 64, 170
+    with 16; 16 experts of 1,024 at width 1,024, 256 tokens with 2: 27, 25 and 38; 8 of 512, 300 tokens with 2: 22, 18 and 20.  The
+    lines were drawn with the kernels that inner sizes of no multiple of 64 still take; on the staged ones the first case stands
+    6 % on the wrong side of its line.)  It depends on the step's number of tokens only, so a replayed step keeps its choice."""
     if dtype == torch.bfloat16 and all(k % 8 == 0 for k in inner_sizes):
         if pairs >= 128 * experts:
             return MOE_MAX_TILE_ROWS

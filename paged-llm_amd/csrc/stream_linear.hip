@@ -368,7 +368,8 @@ PLLM_API int pllm_stream_linear(int epi, const void* x, int ldx, const void* wt,
 
 // ---------------------------------------------------------------------------------------------
 // The same products for a few hundred rows (steps that hold a prompt portion, short prompts): tiles of up to 160 input
-// rows x 128 weight rows per workgroup, along x the blocks of weight rows and of input rows, along z ranges of K.  With this many rows every workgroup of the kernel above would read all of them for its 32 weight rows;
+// rows x 128 weight rows per workgroup, along x the blocks of weight rows and of input rows, along z ranges of K.  With this
+// many rows every workgroup of the kernel above would read all of them for its 32 weight rows;
 // here both operands of a stage (64 columns of K) come into LDS once per workgroup, brought by the four loader
 // wavefronts (the weights' tiles are 1 KB of contiguous memory each and land in operand order; the rows as above), and
 // the eight compute wavefronts, as 2 x 4 over the tile (MTW tiles of 16 input rows x 2 blocks of 16 weight rows each),
@@ -690,7 +691,8 @@ static bool wide_takes(int m_blocks, int mt, int weight_blocks16, int cus) {
   return mt >= 8 && tiles > cus && wide_tiles <= cus;
 }
 
-// What `tile_shape` chooses, before `wide_takes` doubles a gated product's tiles, for M input rows and a matrix of `weight_rows` rows on `compute_units` compute units: rows per
+// What `tile_shape` chooses, before `wide_takes` doubles a gated product's tiles, for M input rows and a matrix of `weight_rows`
+// rows on `compute_units` compute units: rows per
 // block of input rows (a multiple of 16) and weight rows per tile (128 or 64); returns the number of workgroups.
 PLLM_API int pllm_tile_linear_shape(int M, int weight_rows, int compute_units, int* block_rows, int* tile_weight_rows) {
   if (M <= 0 || weight_rows <= 0 || compute_units <= 0) return -2;
