@@ -1493,8 +1493,12 @@ def step_sizes(raw: torch.Tensor, bias: torch.Tensor, a_log: torch.Tensor) -> tu
 
 
 # Tokens of the longest sequence of a step from which its recurrences may run in pieces or chunks, which round differently than token by
-# token.  Below, every token of the step has the bits that it has alone, and a short portion may be cut anywhere.
-RECURRENCE_CHUNKS_FROM = 128
+# token.  Below, every token of the step has the bits that it has alone, and a short portion may be cut anywhere.  Where nothing of
+# that is kept by the layers around the recurrence, a caller may let them begin earlier: with operands in bfloat16 a step of more
+# than 16 rows goes through other products, which add in another order, than a step of fewer (parts/linear.py), and a portion of 17
+# tokens is such a step (a prompt of 100 tokens, a layer of 64 heads of 128 x 64 / 16 of 128 x 128 with a decay per row: 36 / 42 us
+# in chunks, 150 / 158 token by token).
+RECURRENCE_CHUNKS_FROM, RECURRENCE_CHUNKS_FROM_IN_BF16 = 128, 17
 
 
 def recurrence_chunk(max_q_len: int, num_tokens: int) -> int:
@@ -1513,14 +1517,15 @@ def recurrence_chunk(max_q_len: int, num_tokens: int) -> int:
 RECURRENCE_PIECE = 32             # tokens that the matrix form of a long portion works off at a time
 
 
-def recurrence_form(max_q_len: int, num_tokens: int, num_seqs: int, heads: int, rows: int, columns: int, by_row: bool, compute_units: int) -> int:
+def recurrence_form(max_q_len: int, num_tokens: int, num_seqs: int, heads: int, rows: int, columns: int, by_row: bool, compute_units: int,
+                    chunks_from: int = RECURRENCE_CHUNKS_FROM) -> int:
     """How a step's recurrences run: 0, every sequence token by token in one workgroup per head and block of columns; -1, every
     sequence in one workgroup likewise, in pieces of 32 tokens; else the tokens per chunk of the three passes over chunks, which
     spread a long portion over the GPU at the price of a workspace of one state per chunk and two passes over every sequence."""
-    if max_q_len < RECURRENCE_CHUNKS_FROM:
+    if max_q_len < chunks_from:
         return 0
     if rows <= (128 if by_row else 256):
-        # What each takes, in us, up to 2,048 tokens of 64 heads of 128 x 64 rows and columns, of 8 of 128 x 257 and 256 x 512, of
+        # What each takes, in us, from 1 to 2,048 tokens of 64 heads of 128 x 64 rows and columns, of 8 of 128 x 257 and 256 x 512, of
         # 16 of 128 x 128 with a decay per row, alone and beside 32 single tokens.  Portions beside many single tokens run in
         # pieces (130 tokens and 32 single ones: token by token 242, pieces 79, chunks 338),
         # long portions in chunks (2,048: pieces 460, chunks 142) of so many pieces that their workgroups fill the GPU once:
@@ -1547,7 +1552,8 @@ def recurrence_form(max_q_len: int, num_tokens: int, num_seqs: int, heads: int, 
 def linear_recurrence(q: torch.Tensor, k: torch.Tensor, v: torch.Tensor, decay: torch.Tensor, state: torch.Tensor, state_offset: int,
                       state_slots: torch.Tensor, seq_starts: torch.Tensor, cu_seqlens: torch.Tensor, num_seqs: int,
                       vscale: torch.Tensor | None = None, skip: torch.Tensor | None = None, max_q_len: int = 0,
-                      step_sizes: tuple | None = None, normaliser: bool = False, row_decay: torch.Tensor | None = None) -> torch.Tensor:
+                      step_sizes: tuple | None = None, normaliser: bool = False, row_decay: torch.Tensor | None = None,
+                      chunks_from: int = RECURRENCE_CHUNKS_FROM) -> torch.Tensor:
     """Per head:  S_t = decay_t S_(t-1) + k_t (vscale_t v_t)^T,   y_t = S_t^T q_t + skip v_t,   S [N, P] float32 at
     ``state[slot, state_offset + head * N * P :]``; a sequence with seq_starts == 0 starts from S = 0.
 
@@ -1560,7 +1566,7 @@ def linear_recurrence(q: torch.Tensor, k: torch.Tensor, v: torch.Tensor, decay: 
     the state then takes heads * N * (P + 1) floats and y is [T, heads * (P + 1)] with n_t . q_t in every head's last column.
     ``row_decay`` float32 [T, heads, N] (a view, heads side by side, unit inner stride) in place of ``decay`` (None): a decay per
     row of S, S_t = diag(row_decay_t) S_(t-1) + k_t (vscale_t v_t)^T (every head then has its own keys).
-    ``max_q_len``: a bound on the tokens of one sequence in this step (0: unknown); from ``RECURRENCE_CHUNKS_FROM`` on
+    ``max_q_len``: a bound on the tokens of one sequence in this step (0: unknown); from ``chunks_from`` on
     ``recurrence_form`` may take the sequences in pieces as matrix products, or cut them into chunks that run side by side (a
     chunk's own contribution from a zero state, the states carried from chunk to chunk, the outputs from each chunk's true starting
     state), which rounds differently than token by token.  Below it every token has the bits that it has alone."""
@@ -1592,7 +1598,7 @@ def linear_recurrence(q: torch.Tensor, k: torch.Tensor, v: torch.Tensor, decay: 
     _check_sequences(state, state_slots, seq_starts, cu_seqlens, num_seqs)
     _need(0 <= state_offset and state_offset + H * N * P <= state.shape[1], "the recurrence's state does not fit the state slot")
     out = torch.empty((T, H * P), dtype=torch.float32, device=v.device)
-    chunk = recurrence_form(max_q_len, T, num_seqs, H, N, P, row_decay is not None, _num_compute_units(v.device))
+    chunk = recurrence_form(max_q_len, T, num_seqs, H, N, P, row_decay is not None, _num_compute_units(v.device), chunks_from)
     max_chunks = T // chunk + num_seqs if chunk > 0 else 0
     ws_state = torch.empty((max_chunks, H * N * P), dtype=torch.float32, device=v.device) if chunk > 0 else None
     ws_decay = torch.empty((max_chunks, H * (N if row_decay is not None else 1)), dtype=torch.float32, device=v.device) if chunk > 0 else None

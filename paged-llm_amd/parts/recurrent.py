@@ -53,6 +53,12 @@ def _out_dtype(ctx):
     return torch.float32 if getattr(ctx, "float_branch", False) else None
 
 
+def _chunks_from(ctx) -> int:
+    """The tokens of a portion from which a step's recurrences may round differently than token by token: in float32, where no sum
+    of a row depends on the batch or the cut, as late as the operation itself has it."""
+    return ops.RECURRENCE_CHUNKS_FROM if ctx.dtype == torch.float32 else ops.RECURRENCE_CHUNKS_FROM_IN_BF16
+
+
 class _StatefulMixer(Mixer):
     graph_capturable = True
     graph_capturable_prompts = True
@@ -115,10 +121,10 @@ class Mamba2Mixer(_StatefulMixer):
             # long portions: step sizes and decays by a kernel of their own, all tokens side by side (inside the recurrence
             # their exponentials would stand in every token's way, twice: once per pass over the chunks)
             dt, decay = ops.step_sizes(dt_raw, w["dt_bias"], w["A_log"])
-            y = ops.linear_recurrence(C, B, x, decay, state, 0, *seqs, vscale=dt, skip=w["D"], max_q_len=ctx.max_q_len)
+            y = ops.linear_recurrence(C, B, x, decay, state, 0, *seqs, vscale=dt, skip=w["D"], max_q_len=ctx.max_q_len, chunks_from=_chunks_from(ctx))
         else:
             y = ops.linear_recurrence(C, B, x, None, state, 0, *seqs, skip=w["D"], max_q_len=ctx.max_q_len,
-                                      step_sizes=(dt_raw, w["dt_bias"], w["A_log"]))
+                                      step_sizes=(dt_raw, w["dt_bias"], w["A_log"]), chunks_from=_chunks_from(ctx))
         u = ops.gated_group_norm(y, z, w["norm"], inner // self.norm_groups, True, self.eps)
         return linear(u, self.w_o, out_dtype=_out_dtype(ctx))
 
@@ -164,7 +170,7 @@ class RetentionMixer(_StatefulMixer):
         v = rows[:, 2 * H * N:2 * H * N + H * P].unflatten(1, (H, P))
         gate = rows[:, 2 * H * N + H * P:]
         y = ops.linear_recurrence(q, k, v, self.decay, state, 0, ctx.state_slots, ctx.seq_starts, ctx.cu_seqlens_q, ctx.num_seqs,
-                                  max_q_len=ctx.max_q_len)
+                                  max_q_len=ctx.max_q_len, chunks_from=_chunks_from(ctx))
         u = ops.gated_group_norm(y, gate, None, P, False, self.eps)
         return linear(u, self.w_o, out_dtype=_out_dtype(ctx))
 
@@ -221,7 +227,8 @@ class MLstmMixer(_StatefulMixer):
         raw_i, raw_f = rows[:, 2 * qk + 2 * vg:2 * qk + 2 * vg + H], rows[:, 2 * qk + 2 * vg + H:]
         seqs = (ctx.state_slots, ctx.seq_starts, ctx.cu_seqlens_q, ctx.num_seqs)
         decay, take, m = ops.mlstm_gates(raw_i, raw_f, w["i.b"], w["f.b"], self.cap, state, self.m_at, *seqs)
-        y = ops.linear_recurrence(q, k, v, decay, state, 0, *seqs, vscale=take, max_q_len=ctx.max_q_len, normaliser=True)
+        y = ops.linear_recurrence(q, k, v, decay, state, 0, *seqs, vscale=take, max_q_len=ctx.max_q_len, normaliser=True,
+                                  chunks_from=_chunks_from(ctx))
         u = ops.mlstm_output(y, m, gate, w["norm"], H, P, N ** -0.5, self.eps, self.dtype)
         return linear(u, self.w_o, out_dtype=_out_dtype(ctx))
 
@@ -267,7 +274,7 @@ class LightningMixer(_StatefulMixer):
         q, k = acts[:, :qk].unflatten(1, (H, N)), acts[:, qk:2 * qk].unflatten(1, (H, N))
         v = acts[:, 2 * qk:].unflatten(1, (H, P))
         y = ops.linear_recurrence(q, k, v, self.decay, state, 0, ctx.state_slots, ctx.seq_starts, ctx.cu_seqlens_q, ctx.num_seqs,
-                                  max_q_len=ctx.max_q_len)
+                                  max_q_len=ctx.max_q_len, chunks_from=_chunks_from(ctx))
         u = ops.gated_group_norm(y, rows[:, 2 * qk + vg:], self._w["norm"], vg, False, self.eps, gate_activation="sigmoid")
         return linear(u, self.w_o, out_dtype=_out_dtype(ctx))
 
@@ -311,7 +318,7 @@ class Hgrn2Mixer(_StatefulMixer):
         q, k, f = (qkf[i].unflatten(1, (H, N)) for i in range(3))
         v = rows[:, 2 * H * N:].unflatten(1, (H, P))
         y = ops.linear_recurrence(q, k, v, None, state, 0, ctx.state_slots, ctx.seq_starts, ctx.cu_seqlens_q, ctx.num_seqs,
-                                  max_q_len=ctx.max_q_len, row_decay=f)
+                                  max_q_len=ctx.max_q_len, row_decay=f, chunks_from=_chunks_from(ctx))
         u = ops.gated_group_norm(y, None, self.norm_w, P, False, self.eps, gate_activation=None, out_dtype=self.dtype)
         return linear(u, self.w_o, out_dtype=_out_dtype(ctx))
 

@@ -123,3 +123,13 @@ def test_recurrences_with_a_decay_per_row_run_in_chunks_beside_few_single_tokens
     assert plan(130, 162, 33, 4, 32, 32, True, 256) == 32 and plan(700, 1164, 6, 64, 64, 64, True, 256) > 0
     assert plan(8192, 8192, 1, 64, 64, 64, True, 256) <= 1024
     assert plan(500, 564, 65, 16, 128, 128, True, 256) == -1 and plan(500, 564, 65, 100, 32, 32, True, 256) == -1
+
+
+def test_float32_steps_keep_the_order_of_their_recurrences_below_the_stated_bound():
+    from types import SimpleNamespace
+
+    import torch
+
+    from paged_llm_amd.parts.recurrent import _chunks_from
+    assert _chunks_from(SimpleNamespace(dtype=torch.float32)) == ops.RECURRENCE_CHUNKS_FROM == 128
+    assert _chunks_from(SimpleNamespace(dtype=torch.bfloat16)) == 17           # (steps of up to 16 rows keep their products' order as well)

@@ -158,6 +158,8 @@ def test_which_form_a_step_takes():
         for beside in (0, 1, 32):
             for heads, rows, columns, by_row in ((64, 128, 64, False), (8, 256, 512, False), (1, 16, 16, False), (16, 128, 128, True)):
                 assert plan(longest, longest + beside, 1 + beside, heads, rows, columns, by_row, 256) == 0
+    assert plan(100, 100, 1, 64, 128, 64, False, 256, chunks_from=17) == 32 and plan(64, 96, 33, 64, 128, 64, False, 256, chunks_from=17) == -1
+    assert plan(16, 16, 1, 64, 128, 64, False, 256, chunks_from=17) == 0
     for tokens in (200, 2048, 8192):
         chunk = plan(tokens, tokens, 1, 8, 256, 512, False, 256)
         assert chunk > 0 and chunk % 32 == 0
