@@ -1539,7 +1539,8 @@ def recurrence_form(max_q_len: int, num_tokens: int, num_seqs: int, heads: int, 
         pieces, fill = -(-max_q_len // RECURRENCE_PIECE), max(1.0, num_seqs * groups / slots)
         chunk = -(-(-(-num_tokens // RECURRENCE_PIECE) * groups) // slots)
         by_token = 6.0 + 1.25 * max_q_len + 5.0 * fill
-        in_pieces = 30.0 * fill + 14.5 * (pieces - 1) if by_row else 25.0 * fill + 12.5 * (pieces - 1) if wide else 16.0 * fill + 7.0 * (pieces - 1)
+        whole = -(-num_seqs * groups // slots)          # (workgroups of eight wavefronts come in whole rounds)
+        in_pieces = 30.0 * fill + 14.5 * (pieces - 1) if by_row else 25.0 * whole + 12.5 * (pieces - 1) if wide else 16.0 * fill + 7.0 * (pieces - 1)
         beside = (num_seqs - 1) * groups / slots
         if by_row and rows <= 64:                       # (states of few bytes: 32 / 200 single tokens cost 53 / 182 a filled GPU)
             in_chunks = 36.0 + 25.0 * (chunk - 1) + (25.0 + 0.8 * num_seqs) * beside

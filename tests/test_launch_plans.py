@@ -125,6 +125,13 @@ def test_recurrences_with_a_decay_per_row_run_in_chunks_beside_few_single_tokens
     assert plan(500, 564, 65, 16, 128, 128, True, 256) == -1 and plan(500, 564, 65, 100, 32, 32, True, 256) == -1
 
 
+def test_pieces_of_tall_states_come_in_whole_rounds():
+    """Nine sequences of 8 heads of 256 x 512 are 288 workgroups of eight wavefronts: two rounds of pieces, longer than 17 tokens one by one."""
+    plan = ops.recurrence_form
+    assert plan(17, 25, 9, 8, 256, 512, False, 256, chunks_from=17) == 0 and plan(17, 24, 8, 8, 256, 512, False, 256, chunks_from=17) == -1
+    assert plan(100, 108, 9, 8, 256, 512, False, 256, chunks_from=17) == -1
+
+
 def test_float32_steps_keep_the_order_of_their_recurrences_below_the_stated_bound():
     from types import SimpleNamespace
 
