@@ -109,10 +109,10 @@ def test_float_attention_does_not_depend_on_the_cut():
             assert torch.equal(part[:hi - lo], whole[lo:hi]) and torch.equal(part[hi - lo:], whole[hi - 1:hi]), (window, lo, hi)
 
 
-@pytest.mark.parametrize("window", [1, 64, 128, 129, -64, -128, -129])
+@pytest.mark.parametrize("window", [1, 32, 33, 64, 128, 129, -32, -64, -128, -129])
 @pytest.mark.parametrize("heads,kv_heads,d", [(3, 3, 64), (8, 2, 128), (4, 4, 16)])
 def test_float_attention_of_short_windows(heads, kv_heads, d, window):
-    """Windows on both sides of the length from which a workgroup has more wavefronts: a portion and single tokens against the plain kernel
+    """Windows on both sides of the lengths from which a workgroup has more wavefronts: a portion and single tokens against the plain kernel
     (bound as above), and the same bits for a position however it was cut."""
     o = ops()
     bs, n = 16, 391
