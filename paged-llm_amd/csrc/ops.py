@@ -79,6 +79,8 @@ _SIGNATURES = {
     "pllm_gemm_nt": [c_int, c_void_p, c_int, c_void_p, c_int, c_void_p, c_int, c_int, c_int, c_int, c_void_p],
     "pllm_gemm_float": [c_void_p, c_int, c_long, c_void_p, c_int, c_long, c_void_p, c_int, c_long, c_int, c_int, c_int, c_int,
                         c_int, c_int, c_void_p],
+    "pllm_gemm_float_fused": [c_int, c_void_p, c_int, c_void_p, c_int, c_void_p, c_int, c_int, c_int, c_int, c_int, c_int, c_int, c_void_p, c_void_p,
+                              c_void_p, c_void_p, c_void_p, c_void_p, c_int, c_int, c_int, c_int, c_void_p],
     "pllm_paged_attention_generic": [c_int, c_void_p, c_int, c_void_p, c_void_p, c_void_p, c_int, c_void_p, c_int,
                                      c_void_p, c_void_p, c_int, c_int, c_int, c_int, c_int, c_int, c_float, c_int,
                                      c_float, c_void_p, c_void_p, c_int, c_int, c_void_p, c_void_p],
@@ -283,12 +285,12 @@ def copy_pages(pages: torch.Tensor, src: torch.Tensor, dst: torch.Tensor) -> Non
 # ------------------------------------------------------------------------------------------- products
 # The float product's tiles (in sixteens of rows and of weight rows): what one round of workgroups, one on every compute unit,
 # takes beside its columns, what the columns of K = 2048 add to it, and what a launch takes beside its rounds (microseconds, fitted to
-# 1 to 4096 rows of single matrices of 64 to 32000 weight rows and of 5 to 64 heads' matrices, K from 32 to 5632).  Small tiles give a
+# 1 to 1024 rows of single matrices of 2048 to 32000 weight rows and of 16 to 64 heads' matrices, K from 64 to 5632).  Small tiles give a
 # step of few rows enough workgroups, large ones use the matrix cores better; the products of one round or two are decided by how
-# full the rounds are (301 rows x 2048 x 2048: tiles of 48 x 64 in one round 36 us, 64 x 64 47 us, 32 x 32 47 us; 301 x 2560 x 2048:
-# 48 x 64 in two rounds 66 us, 64 x 64 in one 48 us), those of short K by what a workgroup takes whatever its columns (8 rows of 64
-# heads of 64 x 64: 16 x 16 3.5 us, 48 x 64 7.1 us, which a cost in proportion to K alone had preferred).
-FLOAT_GEMM_TILES = {(1, 1): (0.3, 7.0, 3.1), (1, 2): (0.1, 10.4, 3.3), (2, 2): (0.3, 14.3, 3.4), (3, 4): (0.9, 31.0, 5.0), (4, 4): (1.1, 41.0, 5.5)}
+# full the rounds are (301 rows x 2048 x 2048: tiles of 48 x 64 in one round 25 us, 64 x 64 29, 32 x 32 35; 301 x 2560 x 2048:
+# 48 x 64 in two rounds 45 us, 64 x 64 in one 30; 64 rows x 2048 x 2048: 16 x 32 in one round 10.3 us, 16 x 16 in two 11.8), those of
+# short K by what a workgroup takes whatever its columns.
+FLOAT_GEMM_TILES = {(1, 1): (0.3, 5.2, 2.4), (1, 2): (0.3, 10.0, 2.6), (2, 2): (0.4, 10.6, 2.6), (3, 4): (1.5, 21.0, 2.7), (4, 4): (1.1, 25.4, 2.9)}
 
 
 @functools.lru_cache(maxsize=4096)
@@ -306,6 +308,57 @@ def _gemm_float(a_ptr, lda, a_batch, w_ptr, ldw, w_batch, out_ptr, ldc, c_batch,
     tile = float_gemm_plan(M, N, K, batch, _num_compute_units(device))
     _check(_fn("gemm_float.hip", "pllm_gemm_float")(a_ptr, lda, a_batch, w_ptr, ldw, w_batch, out_ptr, ldc, c_batch, M, N, K, batch,
                                                     *tile, _stream()), what)
+
+
+FG_GATED, FG_ROPE_KV = 1, 2          # what stands behind a float product (gemm_float.hip)
+
+
+def gemm_float_fused_takes(a: torch.Tensor, w: torch.Tensor) -> bool:
+    """Whether the float product with something behind it takes these rows: 16-byte loads (others go through two kernels)."""
+    return (a.dtype == torch.float32 and w.dtype == torch.float32 and a.is_cuda and a.dim() == 2 and a.shape[0] > 0 and a.stride(1) == 1
+            and w.stride(1) == 1 and a.shape[1] % 4 == 0 and a.stride(0) % 4 == 0 and w.stride(0) % 4 == 0 and a.data_ptr() % 16 == 0 and w.data_ptr() % 16 == 0)
+
+
+def _gemm_float_fused(epi, a, w, out, activation=0, rope=None, what="gemm_float_fused") -> None:
+    M, K = a.shape
+    N, r = w.shape[0], rope or {}
+    tile = float_gemm_plan(M, N, K, 1, _num_compute_units(a.device))
+    _check(_fn("gemm_float.hip", "pllm_gemm_float_fused")(
+        epi, _ptr(a), a.stride(0), _ptr(w), w.stride(0), _ptr(out), out.stride(0), M, N, K, *tile, activation, _ptr(r.get("positions")), _ptr(r.get("cos")),
+        _ptr(r.get("sin")), _ptr(r.get("slots")), _ptr(r.get("k_pages")), _ptr(r.get("v_pages")), int(r.get("num_heads", 0)), int(r.get("num_kv_heads", 0)),
+        int(r.get("head_dim", 0)), int(r.get("block_size", 0)), _stream()), what)
+
+
+def gemm_float_gated(a: torch.Tensor, w: torch.Tensor, activation: str = "silu") -> torch.Tensor:
+    """act(gate) * up [M, N / 2] of float32 rows and w = [gate rows; up rows] [N, K], in the product's kernel: the same bits as
+    ``gate_mul`` of the product (a kernel less, and its pass over [M, N])."""
+    _on_gpu(a, w)
+    _need(gemm_float_fused_takes(a, w) and a.shape[1] == w.shape[1] and w.shape[0] % 2 == 0, f"gemm_float_gated: {tuple(a.shape)} x {tuple(w.shape)}^T")
+    out = torch.empty((a.shape[0], w.shape[0] // 2), dtype=torch.float32, device=a.device)
+    _gemm_float_fused(FG_GATED, a, w, out, activation=activation_code(activation), what="gemm_float_gated")
+    return out
+
+
+def gemm_float_rotary(a: torch.Tensor, w: torch.Tensor, rope: dict) -> torch.Tensor:
+    """q rotated [M, heads * d] of float32 rows and w = [q; k; v] rows; k (rotated) and v written to their pages (``rope`` as for
+    ``decode_linear``), in the product's kernel: the same bits as ``rope_scatter`` of the product."""
+    _on_gpu(a, w)
+    M, nh, nkv, d, bs = a.shape[0], rope["num_heads"], rope["num_kv_heads"], rope["head_dim"], rope["block_size"]
+    _need(gemm_float_fused_takes(a, w) and a.shape[1] == w.shape[1] and w.shape[0] == (nh + 2 * nkv) * d and d % 16 == 0,
+          f"gemm_float_rotary: {tuple(a.shape)} x {tuple(w.shape)}^T")
+    kp, vp = rope["k_pages"], rope["v_pages"]
+    P = kp.shape[0]
+    _need(tuple(kp.shape) == (P, nkv, bs, d) and tuple(vp.shape) == (P, nkv, d, bs) and kp.is_contiguous() and vp.is_contiguous()
+          and kp.dtype == torch.float32 and vp.dtype == torch.float32 and kp.data_ptr() % 16 == 0, "bad cache pages")
+    for name in ("positions", "slots"):
+        t = rope[name]
+        _need(t.dtype == torch.int32 and t.shape == (M,) and t.is_contiguous(), f"{name}: int32 [{M}]")
+    if rope.get("cos") is not None:
+        for t in (rope["cos"], rope["sin"]):
+            _need(t.dtype == torch.float32 and t.dim() == 2 and t.shape[1] == d // 2 and t.is_contiguous(), "rotary tables")
+    out = torch.empty((M, nh * d), dtype=torch.float32, device=a.device)
+    _gemm_float_fused(FG_ROPE_KV, a, w, out, rope=rope, what="gemm_float_rotary")
+    return out
 
 
 def gemm_generic(a: torch.Tensor, w: torch.Tensor, out_dtype: torch.dtype | None = None) -> torch.Tensor:

@@ -1,6 +1,6 @@
 """y = x W^T for the parts, with the kernel chosen by element type and number of rows.
 
-* float32: the float matrix-core kernel (the true 32-bit path), always.
+* float32: the float product kernel (the true 32-bit path), always, with the gate's activation or the rotary/cache write behind.
 * bfloat16, at most 16 rows (decoding): the fused decode kernel, which also takes in a pending
   residual sum + norm in front and an activation or the rotary/cache write behind.
 * bfloat16, 17 to 128 rows (decoding with many requests, short prompt portions): the streaming kernel over the
@@ -252,6 +252,10 @@ def gated_linear(x, w_gate_up, activation: str = "silu") -> torch.Tensor:
         if out is not None:
             return out
     w_gate_up = _plain(w_gate_up)
+    if w_gate_up.dtype == torch.float32:
+        x = rows_of(x)
+        if ops.gemm_float_fused_takes(x, w_gate_up):
+            return ops.gemm_float_gated(x, w_gate_up, activation)
     return ops.gate_mul(linear(x, w_gate_up), activation)
 
 
@@ -285,7 +289,7 @@ def qkv_rotary_cache(x, w_qkv, positions: torch.Tensor, position_encoding, num_h
         rotary_dim = position_encoding.rotary_dim or head_dim
         interleaved = bool(position_encoding.interleaved)
     whole_head_halves = position_encoding is None or (rotary_dim == head_dim and not interleaved)
-    if write and w_qkv.dtype == torch.bfloat16 and head_dim % 16 == 0 and whole_head_halves and bias is None:
+    if write and head_dim % 16 == 0 and whole_head_halves and bias is None:
         rope = dict(positions=positions, cos=cos, sin=sin, slots=slot_mapping, k_pages=k_pages, v_pages=v_pages,
                     num_heads=num_heads, num_kv_heads=num_kv_heads, head_dim=head_dim, block_size=block_size)
         tiled_ok = (isinstance(w_qkv, Weight) and w_qkv.pairing == "rotary" and w_qkv.tiled is not None and x.dtype == torch.bfloat16
@@ -308,9 +312,14 @@ def qkv_rotary_cache(x, w_qkv, positions: torch.Tensor, position_encoding, num_h
         if (isinstance(w_qkv, Weight) and w_qkv.pairing == "rotary" and _streams(x, w_qkv, ops.SL_ROPE_KV)
                 and (cos is None or cos.data_ptr() % 16 == 0)):
             return _stream(x, w_qkv, ops.SL_ROPE_KV, rope=rope)
-        q = _fused(x, w_qkv, ops.EPI_ROPE_KV, rope)
-        if q is not None:
-            return q
+        if w_qkv.dtype == torch.bfloat16:
+            q = _fused(x, w_qkv, ops.EPI_ROPE_KV, rope)
+            if q is not None:
+                return q
+        elif k_pages.dtype == torch.float32:
+            x = rows_of(x)
+            if ops.gemm_float_fused_takes(x, _plain(w_qkv)):
+                return ops.gemm_float_rotary(x, _plain(w_qkv), rope)
     w_qkv = _plain(w_qkv)
     qkv = linear(x, w_qkv, bias=bias)
     ops.rope_scatter(qkv, positions, cos, sin, num_heads, num_kv_heads, head_dim, slot_mapping if write else None,
