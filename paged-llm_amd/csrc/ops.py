@@ -838,20 +838,7 @@ def stream_linear(x: torch.Tensor, w: TiledWeight, epi: int = SL_BF16, nt: int |
     if epi == SL_PARTIAL:
         out = torch.empty((splits, M, N), dtype=torch.float32, device=x.device)
     elif epi == SL_ROPE_KV:
-        nh, nkv, d, bs = r["num_heads"], r["num_kv_heads"], r["head_dim"], r["block_size"]
-        _need(d == w.head_dim and N == (nh + 2 * nkv) * d, "the weights were tiled for other heads")
-        kp, vp = r["k_pages"], r["v_pages"]
-        P = kp.shape[0]
-        _need(tuple(kp.shape) == (P, nkv, bs, d) and tuple(vp.shape) == (P, nkv, d, bs) and kp.is_contiguous() and vp.is_contiguous()
-              and kp.dtype == torch.bfloat16 and vp.dtype == torch.bfloat16, "bad cache pages")
-        for name in ("positions", "slots"):
-            t = r[name]
-            _need(t.dtype == torch.int32 and t.shape == (M,) and t.is_contiguous(), f"{name}: int32 [{M}]")
-        if r.get("cos") is not None:
-            for t in (r["cos"], r["sin"]):
-                _need(t.dtype == torch.float32 and t.dim() == 2 and t.shape[1] == d // 2 and t.is_contiguous() and t.data_ptr() % 16 == 0,
-                      "rotary tables")
-        out = torch.empty((M, nh * d), dtype=torch.bfloat16, device=x.device)
+        out = _rotary_output(x, w, r)
     else:
         out = torch.empty((M, N), dtype=torch.float32 if epi == SL_F32 else torch.bfloat16, device=x.device)
     f = _fn("stream_linear.hip", "pllm_stream_linear", signature=_STREAM_SIG)
@@ -908,20 +895,7 @@ def tile_linear(x: torch.Tensor, w: TiledWeight, epi: int = SL_BF16, splits: int
     if epi == SL_PARTIAL:
         out = torch.empty((splits, M, N), dtype=torch.float32, device=x.device)
     elif epi == SL_ROPE_KV:
-        nh, nkv, d, bs = r["num_heads"], r["num_kv_heads"], r["head_dim"], r["block_size"]
-        _need(d == w.head_dim and N == (nh + 2 * nkv) * d, "the weights were tiled for other heads")
-        kp, vp = r["k_pages"], r["v_pages"]
-        P = kp.shape[0]
-        _need(tuple(kp.shape) == (P, nkv, bs, d) and tuple(vp.shape) == (P, nkv, d, bs) and kp.is_contiguous() and vp.is_contiguous()
-              and kp.dtype == torch.bfloat16 and vp.dtype == torch.bfloat16, "bad cache pages")
-        for name in ("positions", "slots"):
-            t = r[name]
-            _need(t.dtype == torch.int32 and t.shape == (M,) and t.is_contiguous(), f"{name}: int32 [{M}]")
-        if r.get("cos") is not None:
-            for t in (r["cos"], r["sin"]):
-                _need(t.dtype == torch.float32 and t.dim() == 2 and t.shape[1] == d // 2 and t.is_contiguous() and t.data_ptr() % 16 == 0,
-                      "rotary tables")
-        out = torch.empty((M, nh * d), dtype=torch.bfloat16, device=x.device)
+        out = _rotary_output(x, w, r)
     else:
         out = torch.empty((M, N), dtype=torch.float32 if epi == SL_F32 else torch.bfloat16, device=x.device)
     f = _fn("stream_linear.hip", "pllm_tile_linear", signature=_TILE_SIG)
@@ -930,6 +904,79 @@ def tile_linear(x: torch.Tensor, w: TiledWeight, epi: int = SL_BF16, splits: int
              _ptr(r.get("v_pages")), int(r.get("num_heads", 0)), int(r.get("num_kv_heads", 0)), int(r.get("head_dim", 0)),
              int(r.get("block_size", 0)), activation_code(activation), _stream()), "tile_linear")
     return out
+
+
+# Tiles of the wide kernel (rows x weight rows), the smallest first; those above 128 x 160 for gated products.
+WIDE_TILES = ((64, 64), (64, 128), (96, 96), (80, 128), (96, 128), (128, 128), (128, 160))
+WIDE_GATED_TILES = ((192, 192), (160, 256), (224, 192), (256, 192))
+WIDE_LONG_K = 4608                   # from this K on the library's large tiles and its cuts of K pay
+_WIDE_SIG = [c_int, c_void_p, c_int, c_void_p, c_void_p, c_int, c_int, c_int, c_int, c_int, c_int, c_int, c_void_p, c_void_p, c_void_p, c_void_p,
+             c_void_p, c_void_p, c_int, c_int, c_int, c_int, c_int, c_void_p]
+
+
+@functools.lru_cache(maxsize=4096)
+def wide_linear_plan(rows: int, weight_rows: int, K: int, epi: int, compute_units: int) -> tuple[int, int] | None:
+    """The wide kernel's tile for a product of ``rows`` rows with ``weight_rows`` weight rows, or None where other kernels are as fast: the
+    smallest tile whose workgroups fit the compute units in one round (its time is a chain of K / 64 stages in proportion to the tile: 777 rows
+    x 2048 x 2048 in tiles of 64 x 128 13.2 us, 128 x 128 17.6, 15.6 in the library), as long as half of the compute units have one.  Where K is
+    long the library cuts it for few outputs (200 x 2048 x 5632 18.2 us there, 19.4 as 128 tiles of 64 x 64) and has the better large tiles
+    (2048 x 2048 x 5632 53.6 us there, 55.9 as 128 x 128; 1024 x 3072 x 8192 63.5 and 70.7, but K = 4096 37.3 and 34.4).  Plain products of more outputs stay
+    with it (2048 x 8192 x 2048 in tiles of 256 x 256 58 us and 51); gated ones, which need no kernel behind them here, take large tiles in one
+    round (777 rows of 11264 x 2048 41 us and 45) or in two that are nine tenths full (2048 rows: 99 us inside a step of 5.95 ms, 85 + 13 and a
+    kernel more in one of 6.04; two rounds of other fills lose, 1024 rows of 16384 x 3072 115 and 98)."""
+    if K % 64 or weight_rows % (8 if epi == SL_GATED else 4):
+        return None
+    def workgroups(tile):
+        return -(-rows // tile[0]) * -(-weight_rows // tile[1])
+    least = compute_units * 5 // 8 if K >= WIDE_LONG_K else compute_units // 2
+    for tile in WIDE_TILES + (WIDE_GATED_TILES if epi == SL_GATED else ()):
+        if workgroups(tile) <= compute_units:
+            large = tile[0] * tile[1] >= 128 * 128 and epi != SL_GATED
+            return tile if workgroups(tile) >= least and not (large and K >= WIDE_LONG_K) else None
+    if epi == SL_GATED and 18 * compute_units <= 10 * workgroups(tile) <= 20 * compute_units:      # (the largest)
+        return tile
+    return None
+
+
+def wide_linear(x: torch.Tensor, w: TiledWeight, tile: tuple[int, int], epi: int = SL_BF16, rope: dict | None = None, activation: str = "silu") -> torch.Tensor:
+    """x [M, K] bfloat16 times the tiled weights, for prompt steps (``wide_linear_plan``): results as ``stream_linear`` gives them."""
+    _on_gpu(x, w.tiles)
+    M, K = x.shape
+    _need(x.dtype == torch.bfloat16 and x.dim() == 2 and x.stride(1) == 1 and x.stride(0) % 8 == 0 and x.data_ptr() % 16 == 0,
+          "wide_linear: bfloat16 rows that start on 16-byte boundaries")
+    _need(K == w.in_features and K % 64 == 0 and w.tiles.is_contiguous() and tuple(w.tiles.shape[1:]) == (K // 32, 4, 16, 8),
+          f"wide_linear: rows of {K} values against tiled weights of {w.in_features}")
+    _need({SL_GATED: "gated", SL_ROPE_KV: "rotary"}.get(epi, "plain") == w.pairing,
+          f"epilogue {epi} against weights tiled with the {w.pairing} pairing")
+    N, r = w.out_features, rope or {}
+    if epi == SL_ROPE_KV:
+        out = _rotary_output(x, w, r)
+    else:
+        _need(epi in (SL_BF16, SL_F32, SL_GATED), f"wide_linear: epilogue {epi}")
+        out = torch.empty((M, N), dtype=torch.float32 if epi == SL_F32 else torch.bfloat16, device=x.device)
+    f = _fn("wide_linear.hip", "pllm_wide_linear", signature=_WIDE_SIG)
+    _check(f(epi, _ptr(x), x.stride(0), _ptr(w.tiles), _ptr(out), out.stride(0), M, N, K, w.blocks, *tile, _ptr(r.get("positions")), _ptr(r.get("cos")),
+             _ptr(r.get("sin")), _ptr(r.get("slots")), _ptr(r.get("k_pages")), _ptr(r.get("v_pages")), int(r.get("num_heads", 0)), int(r.get("num_kv_heads", 0)),
+             int(r.get("head_dim", 0)), int(r.get("block_size", 0)), activation_code(activation), _stream()), "wide_linear")
+    return out
+
+
+def _rotary_output(x: torch.Tensor, w: TiledWeight, r: dict) -> torch.Tensor:
+    """The queries' rows [M, heads * d], with the operands of a rotary epilogue checked against the weights."""
+    M, nh, nkv, d, bs = x.shape[0], r["num_heads"], r["num_kv_heads"], r["head_dim"], r["block_size"]
+    _need(d == w.head_dim and w.out_features == (nh + 2 * nkv) * d, "the weights were tiled for other heads")
+    kp, vp = r["k_pages"], r["v_pages"]
+    P = kp.shape[0]
+    _need(tuple(kp.shape) == (P, nkv, bs, d) and tuple(vp.shape) == (P, nkv, d, bs) and kp.is_contiguous() and vp.is_contiguous()
+          and kp.dtype == torch.bfloat16 and vp.dtype == torch.bfloat16, "bad cache pages")
+    for name in ("positions", "slots"):
+        t = r[name]
+        _need(t.dtype == torch.int32 and t.shape == (M,) and t.is_contiguous(), f"{name}: int32 [{M}]")
+    if r.get("cos") is not None:
+        for t in (r["cos"], r["sin"]):
+            _need(t.dtype == torch.float32 and t.dim() == 2 and t.shape[1] == d // 2 and t.is_contiguous() and t.data_ptr() % 16 == 0,
+                  "rotary tables")
+    return torch.empty((M, nh * d), dtype=torch.bfloat16, device=x.device)
 
 
 # ------------------------------------------------------------------------------------------- choices

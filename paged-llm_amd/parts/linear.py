@@ -7,8 +7,8 @@
   weights' tiled copy (``Weight``), with the same epilogues, or with float partial sums of ranges of K that the
   consuming norm adds; where it was measured slower than the library (the gated product and products with float
   results beyond 64 rows, the output head) the library stays.
-* bfloat16, more rows (prompt portions): the vendor's matrix-product library, with bfloat16 or (logits)
-  float results.
+* bfloat16, more rows (prompt portions): the wide kernel where its tiles fit the compute units in one round, and for gated products
+  a little beyond; else the vendor's matrix-product library, with bfloat16 or (logits) float results.
 
 The choice depends on the number of rows and the sizes only, never on the rows' content.  ``x`` may
 be a tensor or a ``PendingNorm``; a weight may be a tensor [N, K] or a ``Weight``.
@@ -135,6 +135,29 @@ def _stream(x, weight: Weight, epi: int, rope: dict | None = None, partial_ok: b
     return ops.stream_linear(x, weight.tiled, epi, rope=rope, activation=activation, act_params=act_params)
 
 
+WIDE_MIN_ROWS = 129                              # rows from which the wide kernel is chosen (below, the streaming and tiled kernels are)
+WIDE_GATED_FROM_ROWS_WHEN_LARGE = 321            # ... for gated products in its large tiles, where the tiled kernel has them below
+
+
+def _wide(x, weight, epi: int):
+    """The wide kernel's tile for this product, or None: by sizes and row count only."""
+    if not (isinstance(weight, Weight) and weight.tiled is not None and x.dtype == torch.bfloat16
+            and weight.pairing == {ops.SL_GATED: "gated", ops.SL_ROPE_KV: "rotary"}.get(epi, "plain")):
+        return None
+    rows = x.num_rows if isinstance(x, PendingNorm) else x.shape[0]
+    if rows < WIDE_MIN_ROWS:
+        return None
+    tile = ops.wide_linear_plan(rows, weight.shape[0], weight.shape[1], epi, ops._num_compute_units(weight.plain.device))
+    if tile in ops.WIDE_GATED_TILES and rows < WIDE_GATED_FROM_ROWS_WHEN_LARGE:
+        return None
+    return tile
+
+
+def _aligned_rows(x) -> torch.Tensor:
+    x = rows_of(x)
+    return x if x.stride(1) == 1 and x.stride(0) % 8 == 0 and x.data_ptr() % 16 == 0 else x.contiguous()
+
+
 _PAIRING_OF = {ops.EPI_GATED: "gated", ops.EPI_ROPE_KV: "rotary"}
 
 
@@ -176,6 +199,10 @@ def linear(x, weight, out_dtype: torch.dtype | None = None, partial_ok: bool = F
         if x.stride(1) != 1 or x.stride(0) % 8 or x.data_ptr() % 16:
             x = x.contiguous()
         return ops.tile_linear(x, weight.tiled, ops.SL_PARTIAL)
+    epi = ops.SL_F32 if out_dtype == torch.float32 else ops.SL_BF16
+    tile = _wide(x, weight, epi)
+    if tile is not None:
+        return ops.wide_linear(_aligned_rows(x), weight.tiled, tile, epi)
     if _streams(x, weight, ops.SL_F32 if out_dtype == torch.float32 else ops.SL_BF16, partial_ok):
         return _stream(x, weight, ops.SL_F32 if out_dtype == torch.float32 else ops.SL_BF16, partial_ok=partial_ok)
     if weight.dtype == torch.bfloat16:
@@ -239,6 +266,9 @@ def gated_linear(x, w_gate_up, activation: str = "silu") -> torch.Tensor:
     ``activation``: one of ``ops.ACTIVATIONS``."""
     x = _operand(x)
     rows = x.num_rows if isinstance(x, PendingNorm) else x.shape[0]
+    tile = _wide(x, w_gate_up, ops.SL_GATED)
+    if tile is not None:
+        return ops.wide_linear(_aligned_rows(x), w_gate_up.tiled, tile, ops.SL_GATED, activation=activation)
     tiles = _tiles_gated(x, w_gate_up, rows)
     if not tiles and _streams(x, w_gate_up, ops.SL_GATED) and w_gate_up.pairing == "gated":
         return _stream(x, w_gate_up, ops.SL_GATED, activation=activation)
@@ -295,6 +325,10 @@ def qkv_rotary_cache(x, w_qkv, positions: torch.Tensor, position_encoding, num_h
         tiled_ok = (isinstance(w_qkv, Weight) and w_qkv.pairing == "rotary" and w_qkv.tiled is not None and x.dtype == torch.bfloat16
                     and _few_weight_rows(w_qkv) and (cos is None or cos.data_ptr() % 16 == 0))
         rows = x.num_rows if isinstance(x, PendingNorm) else x.shape[0]
+        tile = _wide(x, w_qkv, ops.SL_ROPE_KV) if tiled_ok else None
+        if tile is not None:
+            # (777 rows of 2560 x 2048: 14.9 us, 20.1 in the tiled kernel; 2048 rows 31, 27.3 in the library and 8.6 for the rotary kernel)
+            return ops.wide_linear(_aligned_rows(x), w_qkv.tiled, tile, ops.SL_ROPE_KV, rope=rope)
         large = tiled_ok and w_qkv.shape[0] * w_qkv.shape[1] >= TILE_ROTARY_LARGE_ELEMENTS
         if (tiled_ok and (TILE_ROTARY_FROM_WHEN_LARGE if large else TILE_ROTARY_ROWS[0]) <= rows <= TILE_ROTARY_ROWS[1]
                 and _tiles_in_one_round(rows, w_qkv)):

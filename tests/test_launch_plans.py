@@ -140,3 +140,20 @@ def test_float32_steps_keep_the_order_of_their_recurrences_below_the_stated_boun
     from paged_llm_amd.parts.recurrent import _chunks_from
     assert _chunks_from(SimpleNamespace(dtype=torch.float32)) == ops.RECURRENCE_CHUNKS_FROM == 128
     assert _chunks_from(SimpleNamespace(dtype=torch.bfloat16)) == 17           # (steps of up to 16 rows keep their products' order as well)
+
+
+def test_wide_products_fill_one_round():
+    """The smallest tile in one round, half of the compute units busy at least; gated products also in two rounds that are nearly full."""
+    plan = ops.wide_linear_plan
+    assert plan(777, 2048, 2048, ops.SL_F32, 256) == (64, 128) and plan(2048, 2048, 4096, ops.SL_BF16, 256) == (128, 128)
+    assert plan(264, 2048, 2048, ops.SL_BF16, 256) == (64, 64) and plan(200, 1024, 2048, ops.SL_BF16, 256) is None
+    assert plan(200, 2048, 5632, ops.SL_F32, 256) is None and plan(640, 2048, 5632, ops.SL_F32, 256) == (64, 128) and plan(2048, 2048, 5632, ops.SL_F32, 256) is None
+    assert plan(2048, 8192, 2048, ops.SL_BF16, 256) is None and plan(2048, 2560, 2048, ops.SL_ROPE_KV, 256) == (128, 160)
+    assert plan(777, 11264, 2048, ops.SL_GATED, 256) == (160, 256) and plan(896, 11264, 2048, ops.SL_GATED, 256) == (224, 192)
+    assert plan(2048, 11264, 2048, ops.SL_GATED, 256) == (256, 192) and plan(4096, 11264, 2048, ops.SL_GATED, 256) is None and plan(777, 2048, 2080, ops.SL_BF16, 256) is None and plan(777, 2046, 2048, ops.SL_BF16, 256) is None
+    for rows in (129, 500, 2000, 8192):
+        for weight_rows in (64, 1000, 2560, 11264, 28672):
+            for epi in (ops.SL_BF16, ops.SL_F32, ops.SL_ROPE_KV, ops.SL_GATED):
+                tile = plan(rows, weight_rows, 2048, epi, 256)
+                if tile is not None:
+                    assert 128 <= -(-rows // tile[0]) * -(-weight_rows // tile[1]) <= (512 if epi == ops.SL_GATED else 256)
