@@ -1615,38 +1615,48 @@ def recurrence_chunk(max_q_len: int, num_tokens: int) -> int:
 
 
 RECURRENCE_PIECE = 32             # tokens that the matrix form of a long portion works off at a time
+RECURRENCE_LONG_PIECE = 64        # ... where queries, keys and values are bfloat16 and one decay holds per head
 
 
 def recurrence_form(max_q_len: int, num_tokens: int, num_seqs: int, heads: int, rows: int, columns: int, by_row: bool, compute_units: int,
-                    chunks_from: int = RECURRENCE_CHUNKS_FROM) -> int:
+                    chunks_from: int = RECURRENCE_CHUNKS_FROM, piece: int = RECURRENCE_PIECE) -> int:
     """How a step's recurrences run: 0, every sequence token by token in one workgroup per head and block of columns; -1, every
-    sequence in one workgroup likewise, in pieces of 32 tokens; else the tokens per chunk of the three passes over chunks, which
+    sequence in one workgroup likewise, in pieces of ``piece`` tokens; else the tokens per chunk of the three passes over chunks, which
     spread a long portion over the GPU at the price of a workspace of one state per chunk and two passes over every sequence."""
     if max_q_len < chunks_from:
         return 0
     if rows <= (128 if by_row else 256):
-        # What each takes, in us, from 1 to 2,048 tokens of 64 heads of 128 x 64 rows and columns, of 8 of 128 x 257 and 256 x 512, of
-        # 16 of 128 x 128 with a decay per row, alone and beside 32 single tokens.  Portions beside many single tokens run in
-        # pieces (130 tokens and 32 single ones: token by token 242, pieces 79, chunks 338),
-        # long portions in chunks (2,048: pieces 460, chunks 142) of so many pieces that their workgroups fill the GPU once:
-        # chunks of 1 / 2 / 4 / 8 pieces take 200 / 159 / 152 / 142, and at 512 tokens 62 / 53 / 64 / 101.
+        # What each takes, in us, from 17 to 2,048 tokens, alone, four at once and beside 32 single tokens: 64 heads of 128 x 64 rows and
+        # columns and 8 of 128 x 257 in bfloat16 (pieces of 64), 8 of 256 x 512 and 16 of 128 x 128 with float keys, 16 of 128 x 128
+        # with a decay per row.  Short portions and portions beside many single tokens run in pieces (64 heads of 128 x 64: 100 tokens 21
+        # and 25 in chunks, 130 tokens and 32 single ones 62 and 331, 2,048 and 32 single ones 244 and 377),
+        # long portions in chunks (2,048: pieces 244, chunks 73) of so many pieces that their workgroups fill the GPU once:
+        # chunks of 1 / 2 / 4 pieces take 101 / 83 / 73, and at 512 tokens 37 / 40 / 56.
         # A decay per row costs a piece twice the work of one per head (2,048 tokens and 32 single ones, 64 heads of 64 x 64: pieces 947,
         # chunks 392; 130 and 8 single ones, 16 heads of 128 x 128: pieces 100, chunks 59).
         small = rows <= 64 and columns <= 64            # (whose LDS with a decay per row leaves room for two workgroups as well)
         wide = rows > 128 or (by_row and not small)     # workgroups of eight wavefronts, one to a compute unit; else of four, two
+        piece = RECURRENCE_PIECE if wide or by_row else piece
         slots = compute_units * (1 if wide else 4 if by_row and rows <= 32 and columns <= 32 else 2)     # (the smallest: of two, four)
         groups = heads * -(-columns // (128 if wide else 64))
-        pieces, fill = -(-max_q_len // RECURRENCE_PIECE), max(1.0, num_seqs * groups / slots)
-        chunk = -(-(-(-num_tokens // RECURRENCE_PIECE) * groups) // slots)
+        pieces, fill = -(-max_q_len // piece), max(1.0, num_seqs * groups / slots)
+        chunk = -(-(-(-num_tokens // piece) * groups) // slots)
         by_token = 6.0 + 1.25 * max_q_len + 5.0 * fill
         whole = -(-num_seqs * groups // slots)          # (workgroups of eight wavefronts come in whole rounds)
-        in_pieces = 30.0 * fill + 14.5 * (pieces - 1) if by_row else 25.0 * whole + 12.5 * (pieces - 1) if wide else 16.0 * fill + 7.0 * (pieces - 1)
         beside = (num_seqs - 1) * groups / slots
-        if by_row and rows <= 64:                       # (states of few bytes: 32 / 200 single tokens cost 53 / 182 a filled GPU)
-            in_chunks = 36.0 + 25.0 * (chunk - 1) + (25.0 + 0.8 * num_seqs) * beside
+        if by_row:
+            in_pieces = 30.0 * fill + 14.5 * (pieces - 1)
+            if rows <= 64:                              # (states of few bytes: 32 / 200 single tokens cost 53 / 182 a filled GPU)
+                in_chunks = 36.0 + 25.0 * (chunk - 1) + (25.0 + 0.8 * num_seqs) * beside
+            else:
+                in_chunks = 36.0 + 25.0 * (chunk - 1) + 100.0 * beside
+        elif wide:                                      # (8 heads of 256 x 512: 33 / 100 / 2,048 tokens in pieces 28 / 46 / 584, in chunks 35 / 40 / 148)
+            in_pieces = 19.0 * whole + 9.0 * (pieces - 1)
+            in_chunks = 31.0 + 17.0 * (chunk - 1) + 140.0 * beside
         else:
-            in_chunks = 36.0 + 25.0 * (chunk - 1) + 100.0 * beside if wide or by_row else 30.0 + 14.0 * (chunk - 1) + 75.0 * beside
-        return min((by_token, 0), (in_pieces, -1), (in_chunks, RECURRENCE_PIECE * chunk))[1]
+            in_pieces = 12.5 * fill + (7.6 if piece == RECURRENCE_LONG_PIECE else 6.4) * (pieces - 1)
+            in_chunks = 22.0 + (9.0 if piece == RECURRENCE_LONG_PIECE else 14.0) * (chunk - 1) + 75.0 * beside
+        return min((by_token, 0), (in_pieces, -1), (in_chunks, piece * chunk))[1]
     return recurrence_chunk(max_q_len, num_tokens)
 
 
@@ -1699,7 +1709,9 @@ def linear_recurrence(q: torch.Tensor, k: torch.Tensor, v: torch.Tensor, decay: 
     _check_sequences(state, state_slots, seq_starts, cu_seqlens, num_seqs)
     _need(0 <= state_offset and state_offset + H * N * P <= state.shape[1], "the recurrence's state does not fit the state slot")
     out = torch.empty((T, H * P), dtype=torch.float32, device=v.device)
-    chunk = recurrence_form(max_q_len, T, num_seqs, H, N, P, row_decay is not None, _num_compute_units(v.device), chunks_from)
+    short = q.dtype == torch.bfloat16 and v.dtype == torch.bfloat16
+    chunk = recurrence_form(max_q_len, T, num_seqs, H, N, P, row_decay is not None, _num_compute_units(v.device), chunks_from,
+                            RECURRENCE_LONG_PIECE if short else RECURRENCE_PIECE)
     max_chunks = T // chunk + num_seqs if chunk > 0 else 0
     ws_state = torch.empty((max_chunks, H * N * P), dtype=torch.float32, device=v.device) if chunk > 0 else None
     ws_decay = torch.empty((max_chunks, H * (N if row_decay is not None else 1)), dtype=torch.float32, device=v.device) if chunk > 0 else None

@@ -16,7 +16,9 @@
 // A batch is token-major without padding: sequence s owns rows cu_seqlens[s] .. cu_seqlens[s + 1] - 1, its state
 // sits in slot state_slots[s], and seq_starts[s] == 0 says that it starts now, from a zero state, whatever the slot
 // held.  Sequences may have no rows at all.  All arithmetic is float; T is the storage type of rows.
-#include "common.h"
+#include "float_split.h"
+
+#include <type_traits>
 
 using namespace pllm;
 
@@ -481,13 +483,13 @@ static void launch_recurrence(const RecurrenceArgs& a, const ChunkArgs& ca, dim3
 }
 
 // ---------------------------------------------------------------------------------------------
-// The first and the third pass as matrix products in float (v_mfma_f32_16x16x4_f32), for heads of up to 256 rows (128 with a
-// decay per row): a workgroup walks its chunk in pieces of 32 tokens.  With D[t, j] the product of the decays of tokens
-// j + 1 .. t of a piece, G_t that of its tokens up to t and S the state in front of it,
-//   Y = (G Q) S + M V + skip V,   M[t, j] = D[t, j] g_j (q_t . k_j) for j <= t,
-//   S <- G_32 S + K^T (g_j D[32, j] V)
+// The first and the third pass with a decay per row as matrix products in float (v_mfma_f32_16x16x4_f32), for heads of up to 128 rows: a
+// workgroup walks its chunk in pieces of 32 tokens.  With D[t, j] the products (one per row) of the decays of tokens j + 1 .. t of a
+// piece, G_t those of its tokens up to t and S the state in front of it,
+//   Y = (G Q) S + M V + skip V,   M[t, j] = g_j (q_t . D[t, j] k_j) for j <= t,
+//   S <- G_32 S + (D[32, j] K)^T (g_j V)
 // (every product of decays is built by multiplication, none from a difference of logarithms: as many roundings as token by
-// token).  A decay per row stands inside the sums over the rows: there (G Q) and K^T carry it element by element; M's tile of
+// token).  The decays stand inside the sums over the rows: there G Q and K^T carry them element by element; M's tile of
 // late queries and early keys takes both from the tiles' border (no factor is above 1), and its two tiles on the diagonal are
 // summed by vector instructions, a thread walking the queries behind one key with the key's rows times their decays at hand.
 //
@@ -497,8 +499,7 @@ static void launch_recurrence(const RecurrenceArgs& a, const ChunkArgs& ca, dim3
 // travel while this one is worked off.
 //
 // What bounds it: the float matrix cores (a third to half busy) beside a piece's barriers and its way through LDS.  A prompt
-// of 2,048 tokens, one layer, states + carry + outputs: 64 heads of 128 x 64 452 us token by token in chunks of 64 -> 142 us (58 + 9 +
-// 102 under the profiler); 8 heads of 256 x 512 758 -> 210 us; 16 heads of 128 x 128 with a decay per row 232 -> 131 us.  Errors
+// of 2,048 tokens, one layer, states + carry + outputs, 16 heads of 128 x 128: 232 us token by token in chunks of 64 -> 131 us.  Errors
 // against 64 bits over 1 to 2,048 tokens: outputs 2.6e-8 to 1.5e-6 as before or below, the last states below (1.1e-7 against
 // 2.0e-7, 2.1e-6 against 6.3e-6).
 constexpr int kPiece = 32, kPieceLd = kPiece + 4;
@@ -546,31 +547,29 @@ __device__ __forceinline__ f32x4 row_quad(const void* base, int dtype, size_t at
 constexpr int kVecRows = 1, kVecValues = 2, kVecOut = 4, kVecDecay = 8;
 
 // Floats of LDS, in the order the kernel lays them out.
-template <int NT, int WAVES, int MODE, bool ROW> constexpr int piece_lds_floats() {
+template <int NT, int WAVES, int MODE> constexpr int piece_lds_floats() {
   constexpr int NP = 16 * NT, rows = kPiece * (NP + 4), half = (kPiece / 2) * (NP + 4);
   int n = NP * kPiece + 16 * WAVES * kPiece;                                     // K^T, V^T
   if (MODE != kChunkState) n += 2 * rows + kPiece * kPieceLd;                      // Q, K, M
-  if (ROW) n += rows + NP + kPiece + (MODE != kChunkState ? 2 * half : rows);      // decays, G_32, g; late queries, early keys (first pass: K)
-  else n += 2 * (kPiece * kPieceLd + kPiece);                                    // D with G behind it and g, of this piece and of the next
+  n += rows + NP + kPiece + (MODE != kChunkState ? 2 * half : rows);              // decays, G_32, g; late queries, early keys (first pass: K)
   return n;
 }
 
-template <int NT, int WAVES, int MODE, bool ROW>
+template <int NT, int WAVES, int MODE>
 __global__ __launch_bounds__(64 * WAVES, 2) void recurrence_piece_kernel(RecurrenceArgs a, ChunkArgs ca, int vec) {
   constexpr int NP = 16 * NT, LD = NP + 4, kThreads = 64 * WAVES, kQuads = (kPiece * NP / 4 + kThreads - 1) / kThreads;
   constexpr bool kOut = MODE != kChunkState;                           // (kWhole: a sequence from the slot's state to the slot's state)
   extern __shared__ __attribute__((aligned(16))) unsigned char piece_lds[];
   float* KT = reinterpret_cast<float*>(piece_lds);                     // [NP][32]
   float* VT = KT + NP * kPiece;                                        // [16 WAVES][32]
-  float* Q = VT + 16 * WAVES * kPiece;                                 // [32][LD]  (ROW: q, then G q)
+  float* Q = VT + 16 * WAVES * kPiece;                                 // [32][LD]  q, then G q
   float* K = kOut ? Q + kPiece * LD : Q;                               // [32][LD]
   float* M = K + kPiece * LD;                                          // [32][kPieceLd]
-  float* rest = kOut ? M + kPiece * kPieceLd : ROW ? M : Q;
-  float* DR = rest;                                                    // ROW: [32][LD] decays
-  float* gC = DR + kPiece * LD;                                        // ROW: [NP]
-  float* gs = gC + NP;                                                 // ROW: [32] g
-  float* Q2 = gs + kPiece;                                             // ROW: [16][LD] late queries, decayed from token 16 on
-  float* K2 = Q2 + (kPiece / 2) * LD;                                  // ROW: [16][LD] early keys, decayed up to token 15
+  float* DR = kOut ? M + kPiece * kPieceLd : M;                        // [32][LD] decays
+  float* gC = DR + kPiece * LD;                                        // [NP]
+  float* gs = gC + NP;                                                 // [32] g
+  float* Q2 = gs + kPiece;                                             // [16][LD] late queries, decayed from token 16 on
+  float* K2 = Q2 + (kPiece / 2) * LD;                                  // [16][LD] early keys, decayed up to token 15
   const int tid = threadIdx.x, lane = tid & 63, c16 = lane & 15, quad = lane >> 4;
   const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
   const int head = blockIdx.x / a.pblocks, pb = blockIdx.x % a.pblocks;
@@ -595,42 +594,9 @@ __global__ __launch_bounds__(64 * WAVES, 2) void recurrence_piece_kernel(Recurre
       S[i][r] = from_state && p < ld && n < a.N ? st[(size_t)n * ld + p] : 0.f;
     }
   const float skip = a.skip ? a.skip[head] : 0.f;
-  const float rate = a.raw ? expf(a.a_log[head]) : 0.f, raw_bias = a.raw ? a.raw_bias[head] : 0.f;
 
-  // D, G and g of a piece, by the last wavefront: lane j < 32 walks the tokens behind token j, lane 32 all of them.  What the
-  // walk reads is asked for a piece ahead.
-  float raw_a = 1.f, raw_g = 0.f;
-  auto ask_decays = [&](int t0) {
-    const bool in = lane < min(kPiece, t_last - t0);
-    const size_t row = (size_t)(q_begin + t0 + (in ? lane : 0));
-    if (a.raw) {
-      raw_a = in ? load_as_f32(a.raw, a.raw_dtype, row * a.raw_stride + head) : 0.f;
-      raw_g = in ? 1.f : 0.f;
-    } else {
-      raw_a = in ? a.decay[row * a.decay_stride + head] : 1.f;
-      raw_g = !in ? 0.f : a.vscale ? a.vscale[row * a.heads + head] : 1.f;
-    }
-  };
-  auto walk_decays = [&](float* D) {
-    float at = raw_a, gt = raw_g;
-    if (a.raw) {
-      const float z = raw_a + raw_bias, step = z > 20.f ? z : log1pf(expf(z));
-      at = raw_g == 0.f ? 1.f : expf(-rate * step);
-      gt *= step;
-    }
-    float d = lane == kPiece ? 1.f : 0.f;
-#pragma unroll 8
-    for (int t = 0; t < kPiece; ++t) {
-      d = lane == t ? 1.f : d * row_lane(at, t);
-      if (lane <= kPiece) D[t * kPieceLd + lane] = d;
-    }
-    if (lane < kPiece) D[kPiece * kPieceLd + lane] = gt;
-  };
-  float* D = rest;                                                     // !ROW
-  if (!ROW && wave == WAVES - 1) ask_decays(t_first);
-
-  f32x4 rq[kOut ? kQuads : 1], rk[kQuads], rd[ROW ? kQuads : 1], rv[2];
-  float rg = 1.f;                                                      // ROW: g of token tid
+  f32x4 rq[kOut ? kQuads : 1], rk[kQuads], rd[kQuads], rv[2];
+  float rg = 1.f;                                                      // g of token tid
   auto fetch = [&](int t0) {
 #pragma unroll
     for (int e = 0; e < kQuads; ++e) {
@@ -640,10 +606,8 @@ __global__ __launch_bounds__(64 * WAVES, 2) void recurrence_piece_kernel(Recurre
       const int most = in ? a.N : 0;
       rk[e] = row_quad(a.k, a.qk_dtype, row * a.qk_stride + (size_t)kh * a.N + n, n, most, vec & kVecRows);
       if (kOut) rq[e] = row_quad(a.q, a.qk_dtype, row * a.qk_stride + (size_t)kh * a.N + n, n, most, vec & kVecRows);
-      if (ROW) {
-        rd[e] = row_quad(a.row_decay, PLLM_F32, row * a.row_decay_stride + (size_t)head * a.N + n, n, most, vec & kVecDecay);
-        if (!in) rd[e] = f32x4{1.f, 1.f, 1.f, 1.f};
-      }
+      rd[e] = row_quad(a.row_decay, PLLM_F32, row * a.row_decay_stride + (size_t)head * a.N + n, n, most, vec & kVecDecay);
+      if (!in) rd[e] = f32x4{1.f, 1.f, 1.f, 1.f};
     }
 #pragma unroll
     for (int e = 0; e < 2; ++e) {
@@ -655,10 +619,9 @@ __global__ __launch_bounds__(64 * WAVES, 2) void recurrence_piece_kernel(Recurre
       for (int i = 0; i < 4; ++i)
         if (in && ld > a.P && col + i == a.P) rv[e][i] = 1.f;          // the normaliser's column
     }
-    if (ROW && tid < kPiece) rg = a.vscale && t0 + tid < t_last ? a.vscale[(size_t)(q_begin + t0 + tid) * a.heads + head] : 1.f;
+    if (tid < kPiece) rg = a.vscale && t0 + tid < t_last ? a.vscale[(size_t)(q_begin + t0 + tid) * a.heads + head] : 1.f;
   };
   fetch(t_first);
-  if (!ROW && wave == WAVES - 1) walk_decays(D);
   float total = 1.f;                                                   // first pass: the product of the chunk's decays
 
   for (int t0 = t_first; t0 < t_last; t0 += kPiece) {
@@ -670,12 +633,8 @@ __global__ __launch_bounds__(64 * WAVES, 2) void recurrence_piece_kernel(Recurre
       const int at = tid + e * kThreads, t = at / (NP / 4), n = at % (NP / 4) * 4;
       if (kPiece * NP / 4 % kThreads && t >= kPiece) break;
       if (kOut) *reinterpret_cast<f32x4*>(Q + t * LD + n) = rq[e];
-      if (kOut || ROW) *reinterpret_cast<f32x4*>(K + t * LD + n) = rk[e];
-      if (ROW) *reinterpret_cast<f32x4*>(DR + t * LD + n) = rd[e];
-      if (!ROW) {
-#pragma unroll
-        for (int i = 0; i < 4; ++i) KT[token_quad(n + i, t >> 2) + (t & 3)] = rk[e][i];
-      }
+      *reinterpret_cast<f32x4*>(K + t * LD + n) = rk[e];
+      *reinterpret_cast<f32x4*>(DR + t * LD + n) = rd[e];
     }
 #pragma unroll
     for (int e = 0; e < 2; ++e) {
@@ -687,98 +646,82 @@ __global__ __launch_bounds__(64 * WAVES, 2) void recurrence_piece_kernel(Recurre
         odd = odd || !(fabsf(x) < INFINITY);
       }
     }
-    if (ROW && tid < kPiece) gs[tid] = rg;
+    if (tid < kPiece) gs[tid] = rg;
     odd = kOut && __syncthreads_or(odd);
     if (!kOut) __syncthreads();
     if (!last) fetch(t0 + kPiece);
-    if (!ROW && wave == WAVES - 1 && !last) ask_decays(t0 + kPiece);
 
-    if constexpr (ROW) {
-      // Thread n < NP walks the tokens forward (queries), thread NP + n backward (keys).
-      for (int who = tid; who < 2 * NP; who += kThreads) {
-        const int n = who % NP;
-        if (who < NP) {
-          if (kOut) {
-            float from16 = 1.f;
+    // Thread n < NP walks the tokens forward (queries), thread NP + n backward (keys).
+    for (int who = tid; who < 2 * NP; who += kThreads) {
+      const int n = who % NP;
+      if (who < NP) {
+        if (kOut) {
+          float from16 = 1.f;
 #pragma unroll 4
-            for (int t = kPiece / 2; t < kPiece; ++t) {
-              from16 *= DR[t * LD + n];
-              Q2[(t - kPiece / 2) * LD + n] = Q[t * LD + n] * from16;
-            }
+          for (int t = kPiece / 2; t < kPiece; ++t) {
+            from16 *= DR[t * LD + n];
+            Q2[(t - kPiece / 2) * LD + n] = Q[t * LD + n] * from16;
           }
-          float all = 1.f;
+        }
+        float all = 1.f;
 #pragma unroll 4
-          for (int t = 0; t < kPiece; ++t) all *= DR[t * LD + n];
-          gC[n] = all;
-        } else {
-          float behind = 1.f;
+        for (int t = 0; t < kPiece; ++t) all *= DR[t * LD + n];
+        gC[n] = all;
+      } else {
+        float behind = 1.f;
 #pragma unroll 4
-          for (int t = kPiece - 1; t >= 0; --t) {
-            KT[token_quad(n, t >> 2) + (t & 3)] = K[t * LD + n] * behind * gs[t];
-            behind *= DR[t * LD + n];
-          }
-          if (kOut) {
-            float to15 = 1.f;
+        for (int t = kPiece - 1; t >= 0; --t) {
+          KT[token_quad(n, t >> 2) + (t & 3)] = K[t * LD + n] * behind * gs[t];
+          behind *= DR[t * LD + n];
+        }
+        if (kOut) {
+          float to15 = 1.f;
 #pragma unroll 4
-            for (int t = kPiece / 2 - 1; t >= 0; --t) {
-              K2[t * LD + n] = K[t * LD + n] * to15;
-              to15 *= DR[t * LD + n];
-            }
+          for (int t = kPiece / 2 - 1; t >= 0; --t) {
+            K2[t * LD + n] = K[t * LD + n] * to15;
+            to15 *= DR[t * LD + n];
           }
         }
       }
-      if constexpr (kOut) {
-        // The tiles of M on the diagonal: sixteen lanes share a key, NT of its rows each.
-        for (int who = tid; who < 512; who += kThreads) {
-          const int j = who >> 4, n = (who & 15) * NT, stop = (j & 16) + 16;
-          float w[NT];
+    }
+    if constexpr (kOut) {
+      // The tiles of M on the diagonal: sixteen lanes share a key, NT of its rows each.
+      for (int who = tid; who < 512; who += kThreads) {
+        const int j = who >> 4, n = (who & 15) * NT, stop = (j & 16) + 16;
+        float w[NT];
 #pragma unroll
-          for (int i = 0; i < NT; ++i) w[i] = K[j * LD + n + i];
-          for (int t = j & 16; t < stop; ++t) {
-            float dot = 0.f;
-            if (t >= j) {
+        for (int i = 0; i < NT; ++i) w[i] = K[j * LD + n + i];
+        for (int t = j & 16; t < stop; ++t) {
+          float dot = 0.f;
+          if (t >= j) {
 #pragma unroll
-              for (int i = 0; i < NT; ++i) {
-                if (t > j) w[i] *= DR[t * LD + n + i];
-                dot = fmaf(w[i], Q[t * LD + n + i], dot);
-              }
+            for (int i = 0; i < NT; ++i) {
+              if (t > j) w[i] *= DR[t * LD + n + i];
+              dot = fmaf(w[i], Q[t * LD + n + i], dot);
             }
-            dot += dpp_move<kDppSwap1>(dot);
-            dot += dpp_move<kDppSwap2>(dot);
-            dot += dpp_move<kDppHalfMirror>(dot);
-            dot += dpp_move<kDppMirror>(dot);
-            if ((who & 15) == 0) M[t * kPieceLd + j] = dot * gs[j];
           }
-        }
-        __syncthreads();
-        for (int n = tid; n < NP; n += kThreads) {                     // (the diagonal is done with the plain queries)
-          float all = 1.f;
-#pragma unroll 4
-          for (int t = 0; t < kPiece; ++t) {
-            all *= DR[t * LD + n];
-            Q[t * LD + n] *= all;
-          }
-        }
-        if (wave == WAVES - 1) {                                       // late queries, early keys
-          const f32x4 m = dot_rows<NT>(K2 + c16 * LD + 4 * quad, Q2 + c16 * LD + 4 * quad);
-          *reinterpret_cast<f32x4*>(M + (16 + c16) * kPieceLd + 4 * quad) = m * lds_quad(gs + 4 * quad);
+          dot += dpp_move<kDppSwap1>(dot);
+          dot += dpp_move<kDppSwap2>(dot);
+          dot += dpp_move<kDppHalfMirror>(dot);
+          dot += dpp_move<kDppMirror>(dot);
+          if ((who & 15) == 0) M[t * kPieceLd + j] = dot * gs[j];
         }
       }
       __syncthreads();
-    } else if constexpr (kOut) {
-      if (wave < 3) {
-        const int tt = wave > 0, jt = wave > 1;                        // tiles of M: (0, 0), (1, 0), (1, 1)
-        f32x4 m = dot_rows<NT>(K + (16 * jt + c16) * LD + 4 * quad, Q + (16 * tt + c16) * LD + 4 * quad);
-        const int t = 16 * tt + c16, j = 16 * jt + 4 * quad;
-        const f32x4 d = lds_quad(D + t * kPieceLd + j), g = lds_quad(D + kPiece * kPieceLd + j);
-#pragma unroll
-        for (int r = 0; r < 4; ++r) {
-          m[r] = j + r <= t ? m[r] * d[r] * g[r] : 0.f;
+      for (int n = tid; n < NP; n += kThreads) {                     // (the diagonal is done with the plain queries)
+        float all = 1.f;
+#pragma unroll 4
+        for (int t = 0; t < kPiece; ++t) {
+          all *= DR[t * LD + n];
+          Q[t * LD + n] *= all;
         }
-        *reinterpret_cast<f32x4*>(M + t * kPieceLd + j) = m;
+      }
+      if (wave == WAVES - 1) {                                       // late queries, early keys
+        const f32x4 m = dot_rows<NT>(K2 + c16 * LD + 4 * quad, Q2 + c16 * LD + 4 * quad);
+        *reinterpret_cast<f32x4*>(M + (16 + c16) * kPieceLd + 4 * quad) = m * lds_quad(gs + 4 * quad);
       }
     }
-    float* D_next = D == rest ? rest + kPiece * kPieceLd + kPiece : rest;
+    __syncthreads();
     f32x4 v[2], y[2], carried[2];
 #pragma unroll
     for (int f = 0; f < 2; ++f) {
@@ -796,39 +739,23 @@ __global__ __launch_bounds__(64 * WAVES, 2) void recurrence_piece_kernel(Recurre
 #pragma unroll
       for (int f = 0; f < 2; ++f) {
         carried[f] = (part[0][f] + part[1][f]) + (part[2][f] + part[3][f]);
-        if (!ROW) carried[f] *= D[(16 * f + c16) * kPieceLd + kPiece];
       }
     }
     if ((MODE != kChunkOut || !last) && live) {
-      f32x4 vs[2];
-#pragma unroll
-      for (int f = 0; f < 2; ++f) {
-        vs[f] = v[f];
-        if (!ROW) vs[f] *= lds_quad(D + (kPiece - 1) * kPieceLd + 16 * f + 4 * quad) * lds_quad(D + kPiece * kPieceLd + 16 * f + 4 * quad);
-      }
-      const float g_all = ROW ? 1.f : D[(kPiece - 1) * kPieceLd + kPiece];
 #pragma unroll
       for (int i = 0; i < NT; ++i) {
-        if (ROW) S[i] *= lds_quad(gC + 16 * i + 4 * quad);
-        else S[i] *= g_all;
+        S[i] *= lds_quad(gC + 16 * i + 4 * quad);
 #pragma unroll
-        for (int f = 0; f < 2; ++f) S[i] = mfma16(lds_quad(KT + token_quad(16 * i + c16, 4 * f + quad)), vs[f], S[i]);
+        for (int f = 0; f < 2; ++f) S[i] = mfma16(lds_quad(KT + token_quad(16 * i + c16, 4 * f + quad)), v[f], S[i]);
       }
     }
-    if (!ROW && wave == WAVES - 1 && !last) walk_decays(D_next);
     if (!kOut) {
-      if (ROW) {
-        if (pb == 0 && tid < a.N) {
-          total *= gC[tid];
-          if (last) ca.ws_decay[((size_t)blockIdx.y * a.heads + head) * a.N + tid] = total;
-        }
-      } else if (pb == 0 && tid == 0) {
-        total *= D[(kPiece - 1) * kPieceLd + kPiece];
-        if (last) ca.ws_decay[(size_t)blockIdx.y * a.heads + head] = total;
+      if (pb == 0 && tid < a.N) {
+        total *= gC[tid];
+        if (last) ca.ws_decay[((size_t)blockIdx.y * a.heads + head) * a.N + tid] = total;
       }
     }
     if constexpr (kOut) {
-      if (!ROW) __syncthreads();                                       // M is whole
       if (live) {
         // (A weight of zero must not meet a value that is no number: such a value reaches its own token and later ones only.)
         f32x4 fine[2] = {v[0], v[1]};
@@ -874,7 +801,6 @@ __global__ __launch_bounds__(64 * WAVES, 2) void recurrence_piece_kernel(Recurre
         }
       }
     }
-    D = D_next;
   }
   if (MODE != kChunkOut && p < ld) {
 #pragma unroll
@@ -887,10 +813,10 @@ __global__ __launch_bounds__(64 * WAVES, 2) void recurrence_piece_kernel(Recurre
   }
 }
 
-template <int NT, int WAVES, int MODE, bool ROW>
+template <int NT, int WAVES, int MODE>
 static int launch_pieces(RecurrenceArgs a, const ChunkArgs& ca, int max_chunks, int vec, hipStream_t stream) {
-  constexpr size_t lds = (size_t)piece_lds_floats<NT, WAVES, MODE, ROW>() * sizeof(float);
-  auto kernel = recurrence_piece_kernel<NT, WAVES, MODE, ROW>;
+  constexpr size_t lds = (size_t)piece_lds_floats<NT, WAVES, MODE>() * sizeof(float);
+  auto kernel = recurrence_piece_kernel<NT, WAVES, MODE>;
   if (lds > 64 * 1024) {
     hipError_t e = hipFuncSetAttribute(reinterpret_cast<const void*>(kernel), hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds);
     if (e != hipSuccess) return (int)e;
@@ -898,6 +824,600 @@ static int launch_pieces(RecurrenceArgs a, const ChunkArgs& ca, int max_chunks, 
   a.pblocks = (a.ld + 16 * WAVES - 1) / (16 * WAVES);
   hipLaunchKernelGGL(kernel, dim3(a.heads * a.pblocks, max_chunks), dim3(64 * WAVES), lds, stream, a, ca, vec);
   return (int)hipGetLastError();
+}
+
+// ---------------------------------------------------------------------------------------------
+// The same with one decay per head, for heads of up to 256 rows, on the bfloat16 matrix cores: a workgroup walks its chunk in pieces of
+// 16 TP tokens.  With D[t, j] the product of the decays of tokens j + 1 .. t of a piece, G_t that of its tokens up to t and S the
+// state in front of it,
+//   Y = G (Q S) + M V + skip V,   M[t, j] = D[t, j] g_j (q_t . k_j) for j <= t,
+//   S <- G_last S + K^T (g_j D[last, j] V).
+// A float goes into a product as three bfloat16 numbers that hold all of its 24 bits (float_split.h), a bfloat16 row as itself: QP and VP
+// say which q, k and v are.  The products of parts that reach 2^-24 are added in float, the small ones first: one to six
+// instructions of 16 x 16 x 32 where the float instruction takes eight of twice the time.
+//
+// Every product of decays is built by multiplication, none from a difference of logarithms.  Inside a tile of 16 tokens D stands in a
+// table; from tile to tile it is E_t (from the tile's first token up to t) times the tiles between times F_j (behind j to the end
+// of its tile), all factors at most 1.
+//
+// A wavefront owns 16 columns of S and all of its rows in registers.  A result's lane (g, c) = (lane >> 4, lane & 15) holds rows 4 g ..
+// 4 g + 3 of column c: two such tiles of S are the operand of Y^T = S^T Q^T as they stand, when q's rows of 32 lie in the order
+// (rows 0-3, 16-19, 4-7, ...).  K lies in LDS by tokens for Q K^T, then, in the same place, by rows for the update.
+// All arrays are blocks of four (8 bytes) in an order that spreads the banks.
+//
+// Values that are no numbers, or round to none in bfloat16, have parts that cancel: columns that meet one are walked token by token.
+//
+// What bounds it: a piece's chain of barriers, splits and products (the matrix cores a quarter busy) with two wavefronts on a
+// SIMD, and beside long chunks the carried states' way through memory.  A prompt of 2,048 tokens, one layer, states + carry + outputs, against
+// the same passes with float matrix instructions in pieces of 32 tokens: 64 heads of 128 x 64 in bfloat16 158 -> 73 us (22 + 9 +
+// 44), 8 heads of 256 x 512 with float keys 223 -> 147 us (51 + 15 + 95), 8 of 128 x 257 in bfloat16 133 -> 64 us, 16 of 128 x 128 in
+// floats 89 -> 78 us; 100 tokens of the first in one workgroup a head 36 -> 21 us.  Errors against 64 bits from 40 to 2,048 tokens:
+// outputs 6.3e-8 to 2.7e-7 (7.7e-8 to 2.6e-7 before), last states 3.5e-8 to 2.5e-7 (4.3e-8 to 3.6e-7).
+typedef unsigned short u16x2 __attribute__((ext_vector_type(2)));
+
+__device__ __forceinline__ void note_largest(u16x2& largest, unsigned pair) {          // of two bfloat16 numbers, without their signs
+  largest = __builtin_elementwise_max(largest, __builtin_bit_cast(u16x2, pair & 0x7fff7fffu));
+}
+__device__ __forceinline__ bool no_number(u16x2 largest) { return largest[0] >= 0x7f80 || largest[1] >= 0x7f80; }
+// Four floats as three pairs of words of bfloat16 parts, each the rest rounded to nearest.
+__device__ __forceinline__ void split4(const f32x4 x, uint2* part, int stride) {
+#pragma unroll
+  for (int i = 0; i < 2; ++i) {
+    f32x2 rest{x[2 * i], x[2 * i + 1]};
+#pragma unroll
+    for (int p = 0; p < 3; ++p) {
+      const unsigned w = __builtin_bit_cast(unsigned, __builtin_convertvector(rest, bf16x2));
+      if (i == 0) part[p * stride].x = w; else part[p * stride].y = w;
+      if (p < 2) rest = f32x2{rest[0] - __uint_as_float(w << 16), rest[1] - __uint_as_float(w & 0xffff0000u)};
+    }
+  }
+}
+__device__ __forceinline__ bf16x8 octet(uint2 a, uint2 b) { return __builtin_bit_cast(bf16x8, u32x4{a.x, a.y, b.x, b.y}); }
+
+// acc += a b over 32 columns, a in PA parts and b in PB.
+template <int PA, int PB>
+__device__ __forceinline__ f32x4 multiply_parts(const bf16x8* a, const bf16x8* b, f32x4 acc) {
+#pragma unroll
+  for (int sum = 2; sum >= 0; --sum)                                   // the small products first
+#pragma unroll
+    for (int i = PA - 1; i >= 0; --i) {
+      const int j = sum - i;
+      if (j >= 0 && j < PB) acc = __builtin_amdgcn_mfma_f32_16x16x32_bf16(a[i], b[j], acc, 0, 0, 0);
+    }
+  return acc;
+}
+
+// Byte offsets of four tokens 4 f .. 4 f + 3 of a row in an array of rows over a piece's T tokens, and of rows n .. n + 3 of a token in an
+// array of tokens over NP rows.  Both orders spread a wavefront's reads of sixteen rows and its writes over all banks.
+template <int T> __device__ __forceinline__ int by_row_at(int row, int f) {
+  if (T == 64) return row * 128 + (((f >> 1) ^ row ^ (row >> 3)) & 7) * 16 + (f & 1) * 8;
+  return (row ^ ((row >> 2) & 1)) * 64 + (((f >> 1) ^ (row >> 1) ^ (row >> 3)) & 3) * 16 + (f & 1) * 8;
+}
+template <int NP> __device__ __forceinline__ int by_token_at(int t, int n) {
+  const int piece = (n >> 5) * 4 + ((n >> 2) & 3);
+  return t * NP * 2 + ((piece & ~7) | ((piece ^ t) & 7)) * 16 + ((n >> 4) & 1) * 8;
+}
+
+template <int TP> struct alignas(16) PieceDecays {
+  float D[TP][16][20];                                                 // inside the tiles; a tile's row t, its columns j
+  float E[16 * TP], F[16 * TP];                                        // (F times g)
+  float G[16 * TP], H[16 * TP];                                        // products up to t of the piece; behind j, times g
+  float a[16 * TP], g[16 * TP];
+  float tiles[TP], all;                                                // of whole tiles, of the whole piece
+};
+
+template <int NT, int WAVES, int MODE, int TP, int QP, int VP> struct PieceLds {
+  static constexpr int kPart = 16 * NT * 16 * TP * 2;                  // bytes of one part of Q or K
+  static constexpr int kV = 16 * WAVES * 16 * TP * 2, kM = 16 * TP * 16 * TP * 2;
+  static constexpr int kK = 0, kVt = kK + QP * kPart, kQ = kVt + VP * kV, kMt = kQ + (MODE != kChunkState ? QP * kPart : 0),
+                       kDecays = kMt + (MODE != kChunkState ? 3 * kM : 0), kOdd = kDecays + 2 * (int)sizeof(PieceDecays<TP>), kBytes = kOdd + 16;
+};
+
+template <int NT, int WAVES, int MODE, int TP, int QP, int VP>
+__global__ __launch_bounds__(64 * WAVES, 2) void recurrence_split_kernel(RecurrenceArgs a, ChunkArgs ca, int vec) {
+  using Lds = PieceLds<NT, WAVES, MODE, TP, QP, VP>;
+  constexpr int NP = 16 * NT, T = 16 * TP, kThreads = 64 * WAVES;
+  constexpr int kBlocks = (NP / 4 * (T / 4) + kThreads - 1) / kThreads, kVBlocks = (4 * WAVES * (T / 4) + kThreads - 1) / kThreads;   // of 4 x 4, a thread's
+  constexpr bool kOut = MODE != kChunkState;                           // (kWhole: a sequence from the slot's state to the slot's state)
+  extern __shared__ __attribute__((aligned(16))) unsigned char piece_lds[];
+  unsigned char *K = piece_lds + Lds::kK, *VT = piece_lds + Lds::kVt, *Q = piece_lds + Lds::kQ, *M = piece_lds + Lds::kMt;
+  PieceDecays<TP>* decays = reinterpret_cast<PieceDecays<TP>*>(piece_lds + Lds::kDecays);
+  int* odd = reinterpret_cast<int*>(piece_lds + Lds::kOdd);            // a piece with values that are no numbers; of this piece and the next
+  const int tid = threadIdx.x, lane = tid & 63, c16 = lane & 15, quad = lane >> 4;
+  const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+  const int head = blockIdx.x / a.pblocks, pb = blockIdx.x % a.pblocks;
+  int seq = blockIdx.y, local = 0;
+  if (MODE != kWhole && !find_chunk(a.cu_seqlens, ca.num_seqs, ca.chunk, blockIdx.y, seq, local)) return;
+  const int q_begin = a.cu_seqlens[seq], q_len = a.cu_seqlens[seq + 1] - q_begin;
+  if (q_len <= 0) return;
+  const int t_first = MODE == kWhole ? 0 : local * ca.chunk, t_last = MODE == kWhole ? q_len : min(t_first + ca.chunk, q_len);
+  const int kh = head / (a.heads / a.key_heads), ld = a.ld, p0 = pb * 16 * WAVES;
+  const int p = p0 + 16 * wave + c16;                                  // this lane's column of S
+  float* st = MODE == kWhole ? a.state + (size_t)a.state_slots[seq] * a.slot_stride + (size_t)head * a.N * ld
+                             : ca.ws_state + ((size_t)blockIdx.y * a.heads + head) * a.N * ld;
+  const bool from_state = MODE == kChunkOut || (MODE == kWhole && a.seq_starts[seq] > 0);
+  const bool live = p0 + 16 * wave < ld;                               // (the wavefront has columns)
+
+  // Memory is read and written through buffers that begin at a place all lanes share: offsets of 32 bits, and where there is nothing to
+  // read the offset -1, which gives zeros, so that no load stands behind a branch.
+  auto buffer = [](const void* base, size_t bytes) {
+    return __builtin_amdgcn_make_buffer_rsrc(const_cast<char*>(reinterpret_cast<const char*>(base)) + bytes, 0, 0x7fffffff, 0x00027000);
+  };
+  f32x4 S[NT];
+  const __amdgpu_buffer_rsrc_t state = buffer(st, 0);
+  const int state_at = p < ld ? (4 * quad * ld + p) * 4 : -1;
+#pragma unroll
+  for (int i = 0; i < NT; ++i)
+#pragma unroll
+    for (int r = 0; r < 4; ++r)
+      S[i][r] = __uint_as_float(__builtin_amdgcn_raw_buffer_load_b32(state, from_state && 16 * i + 4 * quad + r < a.N && state_at >= 0 ? state_at + (16 * i + r) * ld * 4 : -1, 0, 0));
+  const float skip = a.skip ? a.skip[head] : 0.f;
+  const bool skip_in_m = ld == a.P;                                    // (a normaliser's column has no skip)
+  const float rate = a.raw ? expf(a.a_log[head]) : 0.f, raw_bias = a.raw ? a.raw_bias[head] : 0.f;
+
+  // The decays of a piece, by the last wavefront: lane 16 i + j has token j of tile i.  What it reads is asked for a piece ahead.
+  float raw_a = 1.f, raw_g = 0.f;
+  auto ask_decays = [&](int t0) {
+    const bool in = lane < min(T, t_last - t0);
+    const size_t row = (size_t)(q_begin + t0 + (in ? lane : 0));
+    if (a.raw) {
+      raw_a = in ? load_as_f32(a.raw, a.raw_dtype, row * a.raw_stride + head) : 0.f;
+      raw_g = in ? 1.f : 0.f;
+    } else {
+      raw_a = in ? a.decay[row * a.decay_stride + head] : 1.f;
+      raw_g = !in ? 0.f : a.vscale ? a.vscale[row * a.heads + head] : 1.f;
+    }
+  };
+  auto walk_decays = [&](PieceDecays<TP>& o) {
+    float at = raw_a, gt = raw_g;
+    if (a.raw) {
+      const float z = raw_a + raw_bias, step = z > 20.f ? z : log1pf(expf(z));
+      at = raw_g == 0.f ? 1.f : expf(-rate * step);
+      gt *= step;
+    }
+    float d = 0.f;
+#pragma unroll
+    for (int t = 0; t < 16; ++t) {
+      const float now = __shfl(at, (lane & 48) + t);                   // (by all lanes: the one it comes from among them)
+      d = c16 == t ? 1.f : d * now;
+      if (lane < T) o.D[quad][t][c16] = d;
+    }
+    float e = at;                                                      // the products from the tile's first token on
+    auto before = [&](auto shift) {
+      e *= __int_as_float(__builtin_amdgcn_update_dpp(0x3f800000, __float_as_int(e), 0x110 + decltype(shift)::value, 0xf, 0xf, false));
+    };
+    before(std::integral_constant<int, 1>{}); before(std::integral_constant<int, 2>{});
+    before(std::integral_constant<int, 4>{}); before(std::integral_constant<int, 8>{});
+    float up_to = 1.f, behind = 1.f, all = 1.f;                        // whole tiles in front of and behind this lane's
+#pragma unroll
+    for (int i = 0; i < TP; ++i) {
+      const float w = row_lane(e, 16 * i + 15);
+      if (i < quad) up_to *= w;
+      if (i > quad) behind *= w;
+      all *= w;
+      if (lane == 0) o.tiles[i] = w;
+    }
+    if (lane == 0) o.all = all;
+    if (lane < T) {
+      o.E[lane] = e;
+      o.F[lane] = d * gt;
+      o.G[lane] = e * up_to;
+      o.H[lane] = d * behind * gt;
+      o.a[lane] = at;
+      o.g[lane] = gt;
+    }
+  };
+
+  using Quad = std::conditional_t<QP == 1, uint2, f32x4>;              // four elements of a row as they are fetched
+  using VQuad = std::conditional_t<VP == 1, uint2, f32x4>;
+  // Elements n .. n + 3 of a row, zeros past its end.
+  auto ask = [](auto& to, const __amdgpu_buffer_rsrc_t& from, int dtype, int at, int count, bool wide) {    // `at`: in elements; count: elements there are, from `at` on
+    if (dtype == PLLM_F32) {
+      f32x4 x;
+      if (wide) {
+        x = __builtin_bit_cast(f32x4, __builtin_amdgcn_raw_buffer_load_b128(from, count > 0 ? 4 * at : -1, 0, 0));
+      } else {
+#pragma unroll
+        for (int u = 0; u < 4; ++u) x[u] = __uint_as_float(__builtin_amdgcn_raw_buffer_load_b32(from, count > u ? 4 * (at + u) : -1, 0, 0));
+      }
+      if constexpr (std::is_same_v<std::remove_reference_t<decltype(to)>, f32x4>) to = x;
+    } else {
+      uint2 x;
+      if (wide) {
+        x = __builtin_bit_cast(uint2, __builtin_amdgcn_raw_buffer_load_b64(from, count > 0 ? 2 * at : -1, 0, 0));
+      } else {
+        unsigned h[4];
+#pragma unroll
+        for (int u = 0; u < 4; ++u) h[u] = (unsigned)(unsigned short)__builtin_amdgcn_raw_buffer_load_b16(from, count > u ? 2 * (at + u) : -1, 0, 0);
+        x = uint2{h[0] | h[1] << 16, h[2] | h[3] << 16};
+      }
+      if constexpr (std::is_same_v<std::remove_reference_t<decltype(to)>, f32x4>)
+        to = f32x4{__uint_as_float(x.x << 16), __uint_as_float(x.x & 0xffff0000u), __uint_as_float(x.y << 16), __uint_as_float(x.y & 0xffff0000u)};
+      else to = x;
+    }
+  };
+  Quad rq[kOut ? kBlocks : 1][4], rk[kBlocks][4];
+  VQuad rv[kVBlocks][4];
+  const int qk_type = QP == 1 ? PLLM_BF16 : a.qk_dtype, v_type = VP == 1 ? PLLM_BF16 : a.v_dtype;
+  auto fetch = [&](int t0) {
+    const size_t first = (size_t)(q_begin + t0), qk_bytes = qk_type == PLLM_F32 ? 4 : 2, v_bytes = v_type == PLLM_F32 ? 4 : 2;
+    const __amdgpu_buffer_rsrc_t ks = buffer(a.k, (first * a.qk_stride + (size_t)kh * a.N) * qk_bytes), qs = buffer(a.q, (first * a.qk_stride + (size_t)kh * a.N) * qk_bytes),
+                                 vs = buffer(a.v, (first * a.v_stride + (size_t)head * a.P) * v_bytes);
+    const int there = min(T, t_last - t0);
+#pragma unroll
+    for (int e = 0; e < kBlocks; ++e) {
+      const int at = tid + e * kThreads, t = at / (NP / 4) * 4, n = at % (NP / 4) * 4;
+#pragma unroll
+      for (int i = 0; i < 4; ++i) {
+        const int count = t + i < there ? a.N - n : 0, from = (t + i) * a.qk_stride + n;
+        ask(rk[e][i], ks, qk_type, from, count, vec & kVecRows);
+        if constexpr (kOut) ask(rq[e][i], qs, qk_type, from, count, vec & kVecRows);
+      }
+    }
+#pragma unroll
+    for (int e = 0; e < kVBlocks; ++e) {
+      const int at = tid + e * kThreads, t = at / (4 * WAVES) * 4, col = p0 + at % (4 * WAVES) * 4;
+#pragma unroll
+      for (int i = 0; i < 4; ++i) ask(rv[e][i], vs, v_type, (t + i) * a.v_stride + col, t + i < there ? a.P - col : 0, vec & kVecValues);
+    }
+  };
+  // A block's parts by tokens (to[part][token]) and the same transposed (parts of the four tokens of a row).
+  auto parts_of = [&](const auto* raw, uint2 (*to)[4]) {
+    if constexpr (std::is_same_v<std::remove_const_t<std::remove_reference_t<decltype(raw[0])>>, uint2>) {
+#pragma unroll
+      for (int i = 0; i < 4; ++i) to[0][i] = raw[i];
+    } else {
+#pragma unroll
+      for (int i = 0; i < 4; ++i) split4(raw[i], &to[0][i], 4);
+    }
+  };
+  auto check = [&](const uint2* x, int t, int* odd) {                   // a block's tokens with elements that are no numbers
+    u16x2 largest{0, 0};
+#pragma unroll
+    for (int i = 0; i < 4; ++i) {
+      note_largest(largest, x[i].x);
+      note_largest(largest, x[i].y);
+    }
+    if (no_number(largest)) {
+#pragma unroll
+      for (int i = 3; i >= 0; --i) {
+        u16x2 one{0, 0};
+        note_largest(one, x[i].x);
+        note_largest(one, x[i].y);
+        if (no_number(one)) atomicMin(odd, t + i);
+      }
+    }
+  };
+  auto transposed = [&](const uint2* x, int i) {                       // row i of a block of four tokens
+    const unsigned pick = i & 1 ? 0x07060302u : 0x05040100u;
+    return i < 2 ? uint2{__builtin_amdgcn_perm(x[1].x, x[0].x, pick), __builtin_amdgcn_perm(x[3].x, x[2].x, pick)}
+                 : uint2{__builtin_amdgcn_perm(x[1].y, x[0].y, pick), __builtin_amdgcn_perm(x[3].y, x[2].y, pick)};
+  };
+  auto put = [](unsigned char* at, uint2 v) { *reinterpret_cast<uint2*>(at) = v; };
+  auto get = [](const unsigned char* at) { return *reinterpret_cast<const uint2*>(at); };
+  auto get8 = [](const unsigned char* at) { return *reinterpret_cast<const bf16x8*>(at); };
+
+  if (kOut)
+    for (int i = tid; i < 3 * Lds::kM / 16; i += kThreads) reinterpret_cast<u32x4*>(M)[i] = u32x4{0u, 0u, 0u, 0u};   // (late keys' tiles stay zero)
+  if (tid < 2) odd[tid] = T;
+  if (wave == WAVES - 1) ask_decays(t_first);
+  fetch(t_first);
+  if (wave == WAVES - 1) walk_decays(decays[0]);
+  float total = 1.f;                                                   // first pass: the product of the chunk's decays
+
+  for (int t0 = t_first, turn = 0; t0 < t_last; t0 += T, turn ^= 1) {
+    const bool last = t0 + T >= t_last;
+    const PieceDecays<TP>& dec = decays[turn];
+    uint2 kt[kBlocks][QP][4];
+    __syncthreads();                                                   // the piece before is done with LDS
+#pragma unroll
+    for (int e = 0; e < kBlocks; ++e) {
+      const int at = tid + e * kThreads, t = at / (NP / 4) * 4, n = at % (NP / 4) * 4;
+      parts_of(rk[e], kt[e]);
+      check(kt[e][0], t, odd + turn);
+      if (NP * T / 16 % kThreads && t >= T) break;
+      if constexpr (kOut) {
+        uint2 qt[QP][4];
+        parts_of(rq[e], qt);
+        check(qt[0], t, odd + turn);
+#pragma unroll
+        for (int part = 0; part < QP; ++part)
+#pragma unroll
+          for (int i = 0; i < 4; ++i) {
+            put(K + part * Lds::kPart + by_token_at<NP>(t + i, n), kt[e][part][i]);
+            put(Q + part * Lds::kPart + by_token_at<NP>(t + i, n), qt[part][i]);
+          }
+      } else {
+#pragma unroll
+        for (int part = 0; part < QP; ++part)
+#pragma unroll
+          for (int i = 0; i < 4; ++i) put(K + part * Lds::kPart + by_row_at<T>(n + i, t >> 2), transposed(kt[e][part], i));
+      }
+    }
+#pragma unroll
+    for (int e = 0; e < kVBlocks; ++e) {
+      const int at = tid + e * kThreads, t = at / (4 * WAVES) * 4, col = at % (4 * WAVES) * 4;
+      uint2 vt[VP][4];
+      parts_of(rv[e], vt);
+      if (ld > a.P && ((p0 + col) ^ a.P) < 4) {                        // the normaliser's column
+        const unsigned one = 0x3f80u << ((a.P & 1) * 16);
+#pragma unroll
+        for (int i = 0; i < 4; ++i)
+          if (t0 + t + i < t_last) {
+            if (a.P & 2) vt[0][i].y |= one; else vt[0][i].x |= one;
+          }
+      }
+      if (WAVES * T % kThreads && t >= T) break;
+#pragma unroll
+      for (int part = 0; part < VP; ++part)
+#pragma unroll
+        for (int i = 0; i < 4; ++i) put(VT + part * Lds::kV + by_row_at<T>(col + i, t >> 2), transposed(vt[part], i));
+    }
+    __syncthreads();
+    constexpr bool kAskLate = kOut && NT > 8;                           // (beside what the transposed keys take there are no registers)
+    if (!kAskLate && !last) fetch(t0 + T);
+    if (wave == WAVES - 1 && !last) ask_decays(t0 + T);
+
+    f32x4 y[TP];
+    bool odd_state = false;                                            // this lane's rows of S
+    if constexpr (kOut) {
+      for (int id = wave; id < TP * (TP + 1) / 2; id += WAVES) {       // tiles of M on and below the diagonal
+        const int tt = id < 1 ? 0 : id < 3 ? 1 : id < 6 ? 2 : 3, jt = id - tt * (tt + 1) / 2;
+        f32x4 m[2] = {{0.f, 0.f, 0.f, 0.f}, {0.f, 0.f, 0.f, 0.f}};
+        const int j = 16 * jt + 4 * quad, t = 16 * tt + c16;
+#pragma unroll
+        for (int s = 0; s < NT / 2; ++s) {
+          if (NT > 8 && s % 2 == 0) __builtin_amdgcn_sched_barrier(0);             // (reads too far ahead cost registers)
+          bf16x8 kf[QP], qf[QP];
+#pragma unroll
+          for (int part = 0; part < QP; ++part) {
+            kf[part] = get8(K + part * Lds::kPart + by_token_at<NP>(16 * jt + c16, 32 * s + 4 * quad));
+            qf[part] = get8(Q + part * Lds::kPart + by_token_at<NP>(t, 32 * s + 4 * quad));
+          }
+          m[s & 1] = multiply_parts<QP, QP>(kf, qf, m[s & 1]);
+        }
+        m[0] += m[1];
+        if (jt == tt) {
+          const f32x4 d = lds_quad(&dec.D[tt][c16][4 * quad]), g = lds_quad(&dec.g[j]);
+#pragma unroll
+          for (int r = 0; r < 4; ++r) {
+            m[0][r] = j + r <= t ? m[0][r] * d[r] * g[r] : 0.f;
+            if (skip_in_m && j + r == t) m[0][r] += skip;
+          }
+        } else {
+          float from = dec.E[t];
+          for (int i = jt + 1; i < tt; ++i) from *= dec.tiles[i];
+          m[0] *= lds_quad(&dec.F[j]) * from;
+        }
+        uint2 part[3];
+        u16x2 largest{0, 0};
+        split4(m[0], part, 1);
+        note_largest(largest, part[0].x);
+        note_largest(largest, part[0].y);
+        if (no_number(largest)) atomicMin(odd + turn, t);
+#pragma unroll
+        for (int i = 0; i < 3; ++i) put(M + i * Lds::kM + by_row_at<T>(t, 4 * jt + quad), part[i]);
+      }
+      constexpr int kSums = TP == 2 ? 2 : 1;
+      f32x4 sums[kSums][TP];
+#pragma unroll
+      for (int i = 0; i < kSums; ++i)
+#pragma unroll
+        for (int f = 0; f < TP; ++f) sums[i][f] = f32x4{0.f, 0.f, 0.f, 0.f};
+      if (live) {
+        u16x2 largest{0, 0};
+#pragma unroll
+        for (int s = 0; s < NT / 2; ++s) {
+          if (NT > 8) __builtin_amdgcn_sched_barrier(0);
+          uint2 lo[3], hi[3];
+          split4(S[2 * s], lo, 1);
+          split4(S[2 * s + 1], hi, 1);
+          note_largest(largest, lo[0].x); note_largest(largest, lo[0].y);
+          note_largest(largest, hi[0].x); note_largest(largest, hi[0].y);
+          const bf16x8 sf[3] = {octet(lo[0], hi[0]), octet(lo[1], hi[1]), octet(lo[2], hi[2])};
+#pragma unroll
+          for (int f = 0; f < TP; ++f) {
+            bf16x8 qf[QP];
+#pragma unroll
+            for (int part = 0; part < QP; ++part) qf[part] = get8(Q + part * Lds::kPart + by_token_at<NP>(16 * f + c16, 32 * s + 4 * quad));
+            sums[s % kSums][f] = multiply_parts<3, QP>(sf, qf, sums[s % kSums][f]);
+          }
+        }
+        odd_state = no_number(largest);
+      }
+#pragma unroll
+      for (int f = 0; f < TP; ++f) y[f] = (kSums == 2 ? sums[0][f] + sums[kSums - 1][f] : sums[0][f]) * dec.G[16 * f + c16];
+      __syncthreads();                                                 // M is whole; K has been read by tokens
+#pragma unroll
+      for (int e = 0; e < kBlocks; ++e) {
+        const int at = tid + e * kThreads, t = at / (NP / 4) * 4, n = at % (NP / 4) * 4;
+        if (NP * T / 16 % kThreads && t >= T) break;
+#pragma unroll
+        for (int part = 0; part < QP; ++part)
+#pragma unroll
+          for (int i = 0; i < 4; ++i) put(K + part * Lds::kPart + by_row_at<T>(n + i, t >> 2), transposed(kt[e][part], i));
+      }
+      __syncthreads();
+      if (kAskLate && !last) fetch(t0 + T);
+    }
+    // Columns with a value that is no number, and all of them from a token on whose key or query has one, are walked token by token
+    // behind the products, and keep what the products gave for the tokens before.  S waits where it came from or goes to, in
+    // memory that no other workgroup uses meanwhile.
+    int first_odd = odd_state ? 0 : odd[turn];
+    if (tid == 0) odd[turn ^ 1] = T;                                   // (this piece's word is written again two pieces on)
+    {
+      u16x2 largest{0, 0};
+      u32x4 w[TP / 2];
+#pragma unroll
+      for (int f = 0; f < TP / 2; ++f) {
+        w[f] = *reinterpret_cast<const u32x4*>(VT + by_row_at<T>(16 * wave + c16, 8 * f + 2 * quad));
+#pragma unroll
+        for (int i = 0; i < 4; ++i) note_largest(largest, w[f][i]);
+      }
+      if (no_number(largest)) {
+#pragma unroll
+        for (int f = 0; f < TP / 2; ++f)
+#pragma unroll
+          for (int i = 0; i < 8; ++i)
+            if (((w[f][i >> 1] >> (16 * (i & 1))) & 0x7f80u) == 0x7f80u) first_odd = min(first_odd, 32 * f + 8 * quad + i);
+      }
+    }
+    const bool any_odd = __ballot(first_odd < T) != 0;
+    auto keep_state = [&](auto to_memory) {
+      int first_at = state_at, row = 4 * quad;
+      asm volatile("" : "+v"(first_at), "+v"(row));                    // (its offsets are not worth registers outside)
+#pragma unroll
+      for (int i = 0; i < NT; ++i)
+#pragma unroll
+        for (int r = 0; r < 4; ++r) {
+          const int at = 16 * i + row + r < a.N && first_at >= 0 ? first_at + (16 * i + r) * ld * 4 : -1;
+          if constexpr (decltype(to_memory)::value) __builtin_amdgcn_raw_buffer_store_b32(__float_as_uint(S[i][r]), state, at, 0, 0);
+          else S[i][r] = __uint_as_float(__builtin_amdgcn_raw_buffer_load_b32(state, at, 0, 0));
+        }
+    };
+    if (any_odd) {
+      first_odd = min(first_odd, __shfl_xor(first_odd, 16));
+      first_odd = min(first_odd, __shfl_xor(first_odd, 32));
+      keep_state(std::true_type{});
+    }
+    if (live && (MODE != kChunkOut || !last)) {
+      bf16x8 vs[TP / 2][3];
+#pragma unroll
+      for (int f = 0; f < TP / 2; ++f) {
+        f32x4 lo{0.f, 0.f, 0.f, 0.f}, hi = lo;
+#pragma unroll
+        for (int part = VP - 1; part >= 0; --part) {
+          const unsigned char* at = VT + part * Lds::kV + by_row_at<T>(16 * wave + c16, 8 * f + 2 * quad);
+          const u32x4 w = *reinterpret_cast<const u32x4*>(at);
+#pragma unroll
+          for (int i = 0; i < 2; ++i) {
+            lo[2 * i] += __uint_as_float(w[i] << 16); lo[2 * i + 1] += __uint_as_float(w[i] & 0xffff0000u);
+            hi[2 * i] += __uint_as_float(w[2 + i] << 16); hi[2 * i + 1] += __uint_as_float(w[2 + i] & 0xffff0000u);
+          }
+        }
+        uint2 lp[3], hp[3];
+        split4(lo * lds_quad(&dec.H[32 * f + 8 * quad]), lp, 1);
+        split4(hi * lds_quad(&dec.H[32 * f + 8 * quad + 4]), hp, 1);
+#pragma unroll
+        for (int part = 0; part < 3; ++part) vs[f][part] = octet(lp[part], hp[part]);
+      }
+      const float all = dec.all;
+#pragma unroll
+      for (int i = 0; i < NT; ++i) {
+        if (NT > 8 && i % 2 == 0) __builtin_amdgcn_sched_barrier(0);
+        S[i] *= all;
+#pragma unroll
+        for (int f = 0; f < TP / 2; ++f) {
+          bf16x8 kf[QP];
+#pragma unroll
+          for (int part = 0; part < QP; ++part) kf[part] = get8(K + part * Lds::kPart + by_row_at<T>(16 * i + c16, 8 * f + 2 * quad));
+          S[i] = multiply_parts<QP, 3>(kf, vs[f], S[i]);
+        }
+      }
+    }
+    if (kOut && live) {
+#pragma unroll
+      for (int s = 0; s < TP / 2; ++s) {
+        bf16x8 vf[VP];
+#pragma unroll
+        for (int part = 0; part < VP; ++part) {
+          vf[part] = get8(VT + part * Lds::kV + by_row_at<T>(16 * wave + c16, 8 * s + 2 * quad));
+          if (any_odd) {                                               // (a weight of zero must not meet a later value that is no number)
+            u32x4 w = __builtin_bit_cast(u32x4, vf[part]);
+#pragma unroll
+            for (int i = 0; i < 4; ++i) {
+              if ((w[i] & 0x7f80u) == 0x7f80u) w[i] &= 0xffff0000u;
+              if ((w[i] & 0x7f800000u) == 0x7f800000u) w[i] &= 0xffffu;
+            }
+            vf[part] = __builtin_bit_cast(bf16x8, w);
+          }
+        }
+#pragma unroll
+        for (int f = 2 * s; f < TP; ++f) {
+          bf16x8 mf[3];
+#pragma unroll
+          for (int part = 0; part < 3; ++part) mf[part] = get8(M + part * Lds::kM + by_row_at<T>(16 * f + c16, 8 * s + 2 * quad));
+          y[f] = multiply_parts<VP, 3>(vf, mf, y[f]);
+        }
+      }
+      const int col = p0 + 16 * wave + 4 * quad;
+      const __amdgpu_buffer_rsrc_t out = buffer(a.out, ((size_t)(q_begin + t0) * a.heads + head) * ld * 4);
+#pragma unroll
+      for (int f = 0; f < TP; ++f) {
+        const int t = 16 * f + c16, at = t < t_last - t0 ? (t * a.heads * ld + col) * 4 : -1;
+        if (a.skip && !skip_in_m && at >= 0) {
+#pragma unroll
+          for (int r = 0; r < 4; ++r)
+            if (col + r < a.P) y[f][r] = fmaf(skip, load_as_f32(a.v, a.v_dtype, (size_t)(q_begin + t0 + t) * a.v_stride + (size_t)head * a.P + col + r), y[f][r]);
+        }
+        if (vec & kVecOut && !any_odd) {
+          __builtin_amdgcn_raw_buffer_store_b128(__builtin_bit_cast(u32x4, y[f]), out, col < ld ? at : -1, 0, 0);
+        } else {
+#pragma unroll
+          for (int r = 0; r < 4; ++r) {
+            const int before = any_odd ? __shfl(first_odd, 4 * quad + r) : T;
+            __builtin_amdgcn_raw_buffer_store_b32(__float_as_uint(y[f][r]), out, col + r < ld && at >= 0 && t < before ? at + 4 * r : -1, 0, 0);
+          }
+        }
+      }
+    }
+    if (any_odd && first_odd < T && p < ld) {                          // (the lanes of one column together)
+#pragma unroll 1
+      for (int t = 0; t < min(T, t_last - t0); ++t) {                  // (rows as they stand in memory)
+        const size_t row = (size_t)(q_begin + t0 + t), qk_at = row * a.qk_stride + (size_t)kh * a.N;
+        const float x = p < a.P ? load_as_f32(a.v, a.v_dtype, row * a.v_stride + (size_t)head * a.P + p) : 1.f, xg = x * dec.g[t], at = dec.a[t];
+        float dot = 0.f;
+#pragma unroll 1
+        for (int n = 4 * quad; n < a.N; n += (n & 3) == 3 ? 13 : 1) {
+          float* s = st + (size_t)n * ld + p;
+          const float next = fmaf(load_as_f32(a.k, a.qk_dtype, qk_at + n), xg, at * *s);
+          *s = next;
+          if constexpr (kOut) dot = fmaf(next, load_as_f32(a.q, a.qk_dtype, qk_at + n), dot);
+        }
+        if constexpr (kOut) {
+          dot += __shfl_xor(dot, 16);
+          dot += __shfl_xor(dot, 32);
+          if (quad == 0 && t >= first_odd) a.out[(size_t)(q_begin + t0 + t) * ((size_t)a.heads * ld) + (size_t)head * ld + p] = p < a.P && a.skip ? fmaf(skip, x, dot) : dot;
+        }
+      }
+      keep_state(std::false_type{});
+    }
+    if (wave == WAVES - 1 && !last) walk_decays(decays[turn ^ 1]);
+    if (!kOut && pb == 0 && tid == 0) {
+      total *= dec.all;
+      if (last) ca.ws_decay[(size_t)blockIdx.y * a.heads + head] = total;
+    }
+  }
+  if (MODE != kChunkOut) {
+#pragma unroll
+    for (int i = 0; i < NT; ++i)
+#pragma unroll
+      for (int r = 0; r < 4; ++r)
+        __builtin_amdgcn_raw_buffer_store_b32(__float_as_uint(S[i][r]), state, 16 * i + 4 * quad + r < a.N && state_at >= 0 ? state_at + (16 * i + r) * ld * 4 : -1, 0, 0);
+  }
+}
+
+template <int NT, int WAVES, int MODE, int TP, int QP, int VP>
+static int launch_split(RecurrenceArgs a, const ChunkArgs& ca, int max_chunks, int vec, hipStream_t stream) {
+  constexpr int lds = PieceLds<NT, WAVES, MODE, TP, QP, VP>::kBytes;
+  static_assert(lds <= (WAVES == 8 ? 160 : 80) * 1024, "LDS of a compute unit, or half of it");
+  auto kernel = recurrence_split_kernel<NT, WAVES, MODE, TP, QP, VP>;
+  if (lds > 64 * 1024) {
+    hipError_t e = hipFuncSetAttribute(reinterpret_cast<const void*>(kernel), hipFuncAttributeMaxDynamicSharedMemorySize, lds);
+    if (e != hipSuccess) return (int)e;
+  }
+  a.pblocks = (a.ld + 16 * WAVES - 1) / (16 * WAVES);
+  hipLaunchKernelGGL(kernel, dim3(a.heads * a.pblocks, max_chunks), dim3(64 * WAVES), lds, stream, a, ca, vec);
+  return (int)hipGetLastError();
+}
+
+// Pieces of 64 tokens where q and k are bfloat16, of 32 where they come as three parts and LDS holds no more.
+template <int NT, int WAVES, int MODE>
+static int launch_split_types(const RecurrenceArgs& a, const ChunkArgs& ca, int max_chunks, int vec, hipStream_t stream) {
+  const bool v16 = a.v_dtype != PLLM_F32, q16 = a.qk_dtype != PLLM_F32;
+  if (q16 && v16) return launch_split<NT, WAVES, MODE, NT <= 8 ? 4 : 2, 1, 1>(a, ca, max_chunks, vec, stream);
+  if (v16) return launch_split<NT, WAVES, MODE, 2, 3, 1>(a, ca, max_chunks, vec, stream);
+  return launch_split<NT, WAVES, MODE, 2, 3, 3>(a, ca, max_chunks, vec, stream);
 }
 
 // Wavefronts (tiles of 16 columns) of a workgroup: eight for tall states and for a decay per row, whose work per piece that
@@ -909,12 +1429,12 @@ template <int MODE>
 static int launch_piece_pass(const RecurrenceArgs& a, const ChunkArgs& ca, int max_chunks, int vec, hipStream_t stream) {
   const int tiles = (a.ld + 15) / 16;
   if (a.row_decay) {
-    if (a.N <= 32 && tiles <= 2) return launch_pieces<2, 2, MODE, true>(a, ca, max_chunks, vec, stream);
-    if (a.N <= 64) return tiles <= 4 ? launch_pieces<4, 4, MODE, true>(a, ca, max_chunks, vec, stream) : launch_pieces<4, 8, MODE, true>(a, ca, max_chunks, vec, stream);
-    return tiles <= 4 ? launch_pieces<8, 4, MODE, true>(a, ca, max_chunks, vec, stream) : launch_pieces<8, 8, MODE, true>(a, ca, max_chunks, vec, stream);
+    if (a.N <= 32 && tiles <= 2) return launch_pieces<2, 2, MODE>(a, ca, max_chunks, vec, stream);
+    if (a.N <= 64) return tiles <= 4 ? launch_pieces<4, 4, MODE>(a, ca, max_chunks, vec, stream) : launch_pieces<4, 8, MODE>(a, ca, max_chunks, vec, stream);
+    return tiles <= 4 ? launch_pieces<8, 4, MODE>(a, ca, max_chunks, vec, stream) : launch_pieces<8, 8, MODE>(a, ca, max_chunks, vec, stream);
   }
-  if (a.N > 128) return launch_pieces<16, 8, MODE, false>(a, ca, max_chunks, vec, stream);
-  return a.N > 64 ? launch_pieces<8, 4, MODE, false>(a, ca, max_chunks, vec, stream) : launch_pieces<4, 4, MODE, false>(a, ca, max_chunks, vec, stream);
+  if (a.N > 128) return launch_split_types<16, 8, MODE>(a, ca, max_chunks, vec, stream);
+  return a.N > 64 ? launch_split_types<8, 4, MODE>(a, ca, max_chunks, vec, stream) : launch_split_types<4, 4, MODE>(a, ca, max_chunks, vec, stream);
 }
 
 // v_cols: P, or P - 1 for a recurrence with a normaliser (v holds P - 1 columns per head; column P - 1 of S holds
@@ -942,16 +1462,17 @@ PLLM_API int pllm_linear_recurrence(const void* q, const void* k, int qk_dtype, 
   a.decay_stride = decay_stride; a.heads = heads; a.key_heads = key_heads; a.N = N; a.P = v_cols; a.ld = P; a.pblocks = (v_cols + 63) / 64;
   ChunkArgs ca{ws_state, ws_decay, chunk, num_seqs};
   const int waves = (N + 63) / 64, need = (N + waves - 1) / waves;   // rows of S per wave
-  const bool pieces = N <= (row_decay ? 128 : 256);
+  // (the pieces' kernels count with 32 bits inside a piece)
+  const bool near = qk_stride < (1 << 22) && v_stride < (1 << 22) && (long)heads * P < (1 << 22), pieces = near && N <= (row_decay ? 128 : 256);
   auto wide = [](const void* p, int dtype, long stride) { return (reinterpret_cast<uintptr_t>(p) & (dtype == PLLM_F32 ? 15 : 7)) == 0 && stride % 4 == 0; };
   const int vec = (N % 4 == 0 && wide(q, qk_dtype, qk_stride) && wide(k, qk_dtype, qk_stride) ? kVecRows : 0) |
                   (v_cols % 4 == 0 && wide(v, v_dtype, v_stride) ? kVecValues : 0) | (P % 4 == 0 && wide(out, PLLM_F32, 0) ? kVecOut : 0) |
                   (row_decay && N % 4 == 0 && wide(row_decay, PLLM_F32, row_decay_stride) ? kVecDecay : 0);
-  if (chunk < 0) {
+  if (chunk < 0 && (pieces || near)) {
     if (!pieces) return -2;
     return launch_piece_pass<kWhole>(a, ca, num_seqs, vec, stream);
   }
-  if (chunk == 0) {
+  if (chunk <= 0) {
     launch_recurrence<kWhole>(a, ca, dim3(heads * a.pblocks, num_seqs), waves, need, stream);
   } else {
     if (pieces) {
