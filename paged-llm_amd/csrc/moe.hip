@@ -247,40 +247,80 @@ PLLM_API int pllm_moe_route(int dtype, const void* h, int ld, const float* route
 //   row_of_pair [pairs]   the sorted row of each pair, -1 for a pass-through expert
 //   tiles [max_tiles][3]  (expert, first row, rows) of every tile of at most tile_rows rows; tiles[.][2] = 0 past the last
 // One workgroup; the order of the pairs of one expert is whatever the atomics give (the products do not depend on it).
-constexpr int kMoeMaxExperts = 1024;
+//
+// What bounds it: one workgroup's chain of LDS round trips.  A thread has an expert for its rows and tiles (a prefix sum over the wavefronts
+// in place of one thread that walks the experts), and in steps of up to kHeldPairs pairs a thread the place among an expert's rows is
+// kept from the count.  8 tokens x 4 of 64 experts 7.6 -> 2.5 us, 33 x 6 of 64 8.6 -> 2.8, 300 x 8 of 256 33 -> 5.0, 4,096 x 4 of 64
+// 23 -> 13.
+constexpr int kMoeMaxExperts = 1024, kHeldPairs = 4;
 
 __global__ __launch_bounds__(1024) void moe_align_kernel(const int* __restrict__ ids, int pairs, int experts, int* __restrict__ sorted_pair,
                                                          int* __restrict__ row_of_pair, int* __restrict__ tiles, int max_tiles, int tile_rows) {
-  __shared__ int count[kMoeMaxExperts], first[kMoeMaxExperts], cursor[kMoeMaxExperts];
-  for (int e = threadIdx.x; e < experts; e += blockDim.x) { count[e] = 0; cursor[e] = 0; }
-  __syncthreads();
-  for (int p = threadIdx.x; p < pairs; p += blockDim.x) {
-    const int e = ids[p];
-    if (e >= 0 && e < experts) atomicAdd(&count[e], 1);
+  __shared__ int count[kMoeMaxExperts], first[kMoeMaxExperts], wave_rows[16], wave_tiles[16];
+  const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6, threads = blockDim.x, waves = threads >> 6;   // (a thread for every expert)
+  const bool held = pairs <= kHeldPairs * threads;
+  int expert[kHeldPairs], place[kHeldPairs];
+  if (held) {
+#pragma unroll
+    for (int i = 0; i < kHeldPairs; ++i) expert[i] = tid + i * threads < pairs ? ids[tid + i * threads] : -1;
   }
+  if (tid < experts) count[tid] = 0;
   __syncthreads();
-  if (threadIdx.x == 0) {
-    int at = 0, nt = 0;
-    for (int e = 0; e < experts; ++e) {
-      first[e] = at;
-      for (int r = 0; r < count[e] && nt < max_tiles; r += tile_rows, ++nt) {
-        tiles[3 * nt] = e;
-        tiles[3 * nt + 1] = at + r;
-        tiles[3 * nt + 2] = min(tile_rows, count[e] - r);
-      }
-      at += count[e];
+  if (held) {
+#pragma unroll
+    for (int i = 0; i < kHeldPairs; ++i)
+      if (expert[i] >= 0 && expert[i] < experts) place[i] = atomicAdd(&count[expert[i]], 1);
+  } else {
+    for (int p = tid; p < pairs; p += threads) {
+      const int e = ids[p];
+      if (e >= 0 && e < experts) atomicAdd(&count[e], 1);
     }
-    for (; nt < max_tiles; ++nt) { tiles[3 * nt] = 0; tiles[3 * nt + 1] = 0; tiles[3 * nt + 2] = 0; }
   }
   __syncthreads();
-  for (int p = threadIdx.x; p < pairs; p += blockDim.x) {
-    const int e = ids[p];
-    if (e >= 0 && e < experts) {
-      const int row = first[e] + atomicAdd(&cursor[e], 1);
-      sorted_pair[row] = p;
-      row_of_pair[p] = row;
-    } else {
-      row_of_pair[p] = -1;
+  const int rows = tid < experts ? count[tid] : 0, own_tiles = (rows + tile_rows - 1) / tile_rows;
+  int rows_to = rows, tiles_to = own_tiles;                            // up to and with this expert's
+#pragma unroll
+  for (int d = 1; d < 64; d <<= 1) {
+    const int r = __shfl_up(rows_to, d), t = __shfl_up(tiles_to, d);
+    if (lane >= d) { rows_to += r; tiles_to += t; }
+  }
+  if (lane == 63) { wave_rows[wave] = rows_to; wave_tiles[wave] = tiles_to; }
+  __syncthreads();
+  int rows_before = 0, tiles_before = 0, all_tiles = 0;                // of the wavefronts in front
+  for (int w = 0; w < waves; ++w) {
+    if (w < wave) { rows_before += wave_rows[w]; tiles_before += wave_tiles[w]; }
+    all_tiles += wave_tiles[w];
+  }
+  const int row0 = rows_before + rows_to - rows, tile0 = tiles_before + tiles_to - own_tiles;
+  if (tid < experts) {
+    first[tid] = row0;
+    if (!held) count[tid] = 0;                                         // (the rows given out so far, from here on)
+    for (int i = 0; i < own_tiles && tile0 + i < max_tiles; ++i) {
+      int* tile = tiles + 3 * (tile0 + i);
+      tile[0] = tid;
+      tile[1] = row0 + i * tile_rows;
+      tile[2] = min(tile_rows, rows - i * tile_rows);
+    }
+  }
+  for (int i = 3 * all_tiles + tid; i < 3 * max_tiles; i += threads) tiles[i] = 0;
+  __syncthreads();
+  auto give = [&](int p, int row) {
+    sorted_pair[row] = p;
+    row_of_pair[p] = row;
+  };
+  if (held) {
+#pragma unroll
+    for (int i = 0; i < kHeldPairs; ++i) {
+      const int p = tid + i * threads;
+      if (p >= pairs) break;
+      if (expert[i] >= 0 && expert[i] < experts) give(p, first[expert[i]] + place[i]);
+      else row_of_pair[p] = -1;
+    }
+  } else {
+    for (int p = tid; p < pairs; p += threads) {
+      const int e = ids[p];
+      if (e >= 0 && e < experts) give(p, first[e] + atomicAdd(&count[e], 1));
+      else row_of_pair[p] = -1;
     }
   }
 }
@@ -290,7 +330,9 @@ PLLM_API int pllm_moe_align(const int* ids, int pairs, int experts, int* sorted_
   if (pairs <= 0) return 0;
   if (tile_rows < kMoeTileRows || tile_rows % kMoeTileRows || tile_rows > kMoeMaxTileRows) return -2;
   if (experts <= 0 || experts > kMoeMaxExperts || max_tiles < (pairs + tile_rows - 1) / tile_rows + experts) return -2;
-  hipLaunchKernelGGL(moe_align_kernel, dim3(1), dim3(1024), 0, stream, ids, pairs, experts, sorted_pair, row_of_pair, tiles, max_tiles, tile_rows);
+  // (a thread for every expert, and for every pair of a small step: fewer wavefronts meet sooner at the barriers)
+  const int threads = min(1024, (max(pairs, experts) + 63) / 64 * 64);
+  hipLaunchKernelGGL(moe_align_kernel, dim3(1), dim3(threads), 0, stream, ids, pairs, experts, sorted_pair, row_of_pair, tiles, max_tiles, tile_rows);
   PLLM_RETURN_LAST_ERROR();
 }
 
