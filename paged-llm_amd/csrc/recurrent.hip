@@ -100,6 +100,83 @@ __global__ __launch_bounds__(256) void causal_conv_kernel(
   }
 }
 
+constexpr int kConvFours = 8;      // tokens of a workgroup of the kernel below
+
+// The same with four taps and four neighbouring channels a thread, for portions in chunks.  The workgroups of a sequence's first chunk,
+// which alone read the state, leave the new one.
+// What bounds it: memory, and the exact SiLU's vector instructions (8 us of them at 2,048 tokens x 4,352 channels).  A thread's loads are
+// 8 bytes (float rows 16) instead of 2, all of its tokens' under way at once, no tap is asked whether it is there, and no second kernel
+// leaves the state.  us with what leaves the state: 2,048 tokens x 4,352 channels 28 -> 17.4 (16 tokens a workgroup 20.8), 8 x 512 tokens
+// 44 -> 26, 1,178 x 2,048 13.1 -> 8.8, 777 x 1,024 10.9 -> 7.6.  From 256 tokens on (100 tokens 11.0 and 11.2), and not beside more than
+// a sixteenth as many sequences, where most workgroups have no tokens (65 tokens and 100 single ones 11.3 and 12.5).
+template <typename T>
+__global__ __launch_bounds__(256) void causal_conv4_kernel(
+    const T* __restrict__ in, int in_stride, const float* __restrict__ w, const float* __restrict__ bias,
+    float* state, size_t slot_stride, const int* __restrict__ state_slots,
+    const int* __restrict__ seq_starts, const int* __restrict__ cu_seqlens, T* __restrict__ out, int out_stride, int channels, int act) {
+  constexpr int kTaps = 4, V = 4;
+  struct alignas(V * sizeof(T)) Four { T v[V]; };
+  const int c = (blockIdx.x * blockDim.x + threadIdx.x) * V;
+  const int seq = blockIdx.y, t0 = blockIdx.z * kConvFours;
+  const int q_begin = cu_seqlens[seq], q_len = cu_seqlens[seq + 1] - q_begin;
+  if (c >= channels || (t0 >= q_len && t0 > 0)) return;
+  const int count = min(kConvFours, q_len - t0);
+  const T* rows = in + (size_t)(q_begin + t0) * in_stride + c;
+  Four fetched[kConvFours];
+#pragma unroll
+  for (int u = 0; u < kConvFours; ++u)
+    if (u < count) fetched[u] = *reinterpret_cast<const Four*>(rows + (size_t)u * in_stride);
+  float wj[V][kTaps], win[V][kTaps - 1], b[V];
+  float* st = state + (size_t)state_slots[seq] * slot_stride + (size_t)c * (kTaps - 1);
+  const bool carried = seq_starts[seq] > 0;
+#pragma unroll
+  for (int j = 0; j < kTaps - 1; ++j) {
+    const int rel = t0 - (kTaps - 1) + j;                              // token of this step (>= 0) or an input of earlier steps (< 0)
+    Four before;
+    if (rel >= 0) before = *reinterpret_cast<const Four*>(rows + (j - (kTaps - 1)) * (ptrdiff_t)in_stride);
+#pragma unroll
+    for (int v = 0; v < V; ++v) win[v][j] = rel >= 0 ? to_f32(before.v[v]) : carried ? st[v * (kTaps - 1) + (kTaps - 1) + rel] : 0.f;
+  }
+  if (t0 == 0) {
+#pragma unroll
+    for (int j = 0; j < kTaps - 1; ++j) {
+      const int rel = q_len - (kTaps - 1) + j;                         // (below 0: the carried input that many places on)
+      Four late;
+      if (rel >= 0) late = *reinterpret_cast<const Four*>(rows + (size_t)rel * in_stride);
+#pragma unroll
+      for (int v = 0; v < V; ++v) {
+        float x = q_len <= 0 ? win[v][j] : 0.f;
+        if (rel >= 0) x = to_f32(late.v[v]);
+        else if (q_len > 0 && j + q_len < kTaps - 1) x = q_len == 1 ? win[v][j + 1 < kTaps - 1 ? j + 1 : 0] : win[v][j + 2 < kTaps - 1 ? j + 2 : 0];
+        st[v * (kTaps - 1) + j] = x;
+      }
+    }
+  }
+#pragma unroll
+  for (int v = 0; v < V; ++v) {
+    b[v] = bias ? bias[c + v] : 0.f;
+#pragma unroll
+    for (int j = 0; j < kTaps; ++j) wj[v][j] = w[(size_t)(c + v) * kTaps + j];
+  }
+#pragma unroll
+  for (int u = 0; u < kConvFours; ++u) {
+    Four o;
+#pragma unroll
+    for (int v = 0; v < V; ++v) {
+      const float cur = to_f32(fetched[u].v[v]);
+      float acc = b[v];
+#pragma unroll
+      for (int j = 0; j < kTaps - 1; ++j) acc = fmaf(wj[v][j], win[v][j], acc);
+      acc = fmaf(wj[v][kTaps - 1], cur, acc);
+      win[v][0] = win[v][1];
+      win[v][1] = win[v][2];
+      win[v][2] = cur;
+      o.v[v] = from_f32<T>(act ? silu_f32(acc) : acc);
+    }
+    if (u < count) *reinterpret_cast<Four*>(out + (size_t)(q_begin + t0 + u) * out_stride + c) = o;
+  }
+}
+
 // state[k] <- the input at token q_len - (taps - 1) + k of this step, or what the state held for it.
 template <typename T, int MAXT>
 __global__ __launch_bounds__(256) void conv_state_update_kernel(
@@ -134,11 +211,18 @@ static void launch_causal_conv(const void* in, int in_stride, const float* w, co
   dim3 block(256), grid((channels + 255) / 256, num_seqs, (max_q_len + chunk - 1) / chunk);
   dim3 grid_state((channels + 255) / 256, num_seqs);
   const int fused = grid.z == 1 && taps > 1;
-  hipLaunchKernelGGL((causal_conv_kernel<T, MAXT>), grid, block, 0, stream, (const T*)in, in_stride, w, bias, state,
-                     (size_t)slot_stride, state_slots, seq_starts, cu_seqlens, (T*)out, out_stride, channels, taps, act, fused, chunk);
-  if (taps > 1 && !fused)
-    hipLaunchKernelGGL((conv_state_update_kernel<T, MAXT>), grid_state, block, 0, stream, (const T*)in, in_stride, state,
-                       (size_t)slot_stride, state_slots, seq_starts, cu_seqlens, channels, taps);
+  const auto fours = [](const void* p, int stride) { return reinterpret_cast<uintptr_t>(p) % (4 * sizeof(T)) == 0 && stride % 4 == 0; };
+  // (where each is ahead: above causal_conv4_kernel)
+  if (max_q_len >= 256 && num_seqs * 16 <= max_q_len && taps == 4 && channels % 4 == 0 && fours(in, in_stride) && fours(out, out_stride)) {
+    hipLaunchKernelGGL(causal_conv4_kernel<T>, dim3((channels / 4 + 255) / 256, num_seqs, (max_q_len + kConvFours - 1) / kConvFours), block, 0, stream, (const T*)in, in_stride, w, bias, state,
+                       (size_t)slot_stride, state_slots, seq_starts, cu_seqlens, (T*)out, out_stride, channels, act);
+  } else {
+    hipLaunchKernelGGL((causal_conv_kernel<T, MAXT>), grid, block, 0, stream, (const T*)in, in_stride, w, bias, state,
+                       (size_t)slot_stride, state_slots, seq_starts, cu_seqlens, (T*)out, out_stride, channels, taps, act, fused, chunk);
+    if (taps > 1 && !fused)
+      hipLaunchKernelGGL((conv_state_update_kernel<T, MAXT>), grid_state, block, 0, stream, (const T*)in, in_stride, state,
+                         (size_t)slot_stride, state_slots, seq_starts, cu_seqlens, channels, taps);
+  }
 }
 
 PLLM_API int pllm_causal_conv(int dtype, const void* in, int in_stride, const float* w, const float* bias, float* state,
