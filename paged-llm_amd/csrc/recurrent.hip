@@ -541,7 +541,7 @@ __global__ __launch_bounds__(256) void recurrence_carry_kernel(RecurrenceArgs a,
   *slot = S;
 }
 
-// (Chunks come here only for states that the matrix form below does not take: more than 42 rows a wavefront.)
+// (Chunks come here only for what the matrix forms below do not take: more than 256 rows, 128 with a decay per row, and rows 2^22 elements apart.)
 template <int MODE>
 static void launch_recurrence(const RecurrenceArgs& a, const ChunkArgs& ca, dim3 grid, int waves, int need, hipStream_t stream) {
   dim3 block(64 * waves);
