@@ -23,7 +23,12 @@
 // 7.7 / 30.6 / 73 us; 8.9 / 39 / 96 with the float instruction, 10.2 / 36 / 84 element by element).
 // Results that are not finite are made again by the whole workgroup, each wavefront its slices of K, in tiles of 16 x 16 (a row of NaN: 8 rows x 2048 x
 // 2048 9.7 -> 13.5 us, 301 rows 26 -> 55, 8 rows x 32000 x 2048 51 -> 102).
-// Which tile a product takes is the host's choice by the rounds of workgroups (ops.float_gemm_plan).
+// Which tile a product takes is the host's choice by the rounds of workgroups (ops.float_gemm_plan, ops.float_split_plan).
+//
+// SPLIT: with many rows the split was most of a wavefront's vector instructions, and each tile of weights was split again by every workgroup
+// of its rows.  A second copy of the weights holds their parts, made once, in operand order: whole kilobytes that go straight to
+// the matrix cores.  Of the steady state's 2.3 us a step of two wavefronts (64 x 64, 32 columns each) the products are 1.6 now.  301 rows x 2048 x
+// 2048 27.4 -> 24.1 us, x 5632 62.8 -> 52.7, 11264 x 2048 gated 125.6 -> 107.8, 32000 x 2048 313 -> 287; 512 rows x 2048 x 5632 82 -> 70.
 #include "float_split.h"
 
 #include <type_traits>
@@ -33,6 +38,7 @@ using namespace pllm;
 struct FloatGemm {
   const float* A;
   const float* W;
+  const bf16x8* W_split;                                               // (SPLIT) the weights' parts, or null
   float* C;
   long a_batch, w_batch, c_batch;
   int lda, ldw, ldc, M, N, K, slice, row_tiles, col_tiles;             // N: weight rows
@@ -60,7 +66,8 @@ __device__ __forceinline__ int weight_row(const FloatGemm& g, int at) {
 
 // ALL: every slice has columns, and the workgroup all its wavefronts.  SPW: slices of a wavefront.
 // FAR: rows so far apart that an offset inside a tile takes 64 bits.
-template <int MT, int NT, int SPW, int PER_SIMD, int EPI, bool FAR, bool ALL>
+// SPLIT: the weights' parts come from W_split, as pllm_float_split_weights lays them out.
+template <int MT, int NT, int SPW, int PER_SIMD, int EPI, bool FAR, bool ALL, bool SPLIT>
 __global__ __launch_bounds__(64 * (kSlices / SPW), PER_SIMD) void gemm_float_kernel(FloatGemm g) {
   constexpr int kPad = 272;                                            // bytes: a chunk of 16 bytes of 16 rows, and 16 against bank conflicts
   extern __shared__ __attribute__((aligned(16))) unsigned char gf_lds[];
@@ -94,7 +101,7 @@ __global__ __launch_bounds__(64 * (kSlices / SPW), PER_SIMD) void gemm_float_ker
 #pragma unroll
     for (int i = 0; i < MT; ++i) a_at[i][j] = (Offset)min(16 * i + r, g.M - 1 - m0) * g.lda + c8;
 #pragma unroll
-    for (int i = 0; i < NT; ++i) w_at[i][j] = (Offset)(weight_row<EPI>(g, n0 + 16 * i + r) - w_first) * g.ldw + c8;
+    for (int i = 0; i < NT; ++i) w_at[i][j] = SPLIT ? 0 : (Offset)(weight_row<EPI>(g, n0 + 16 * i + r) - w_first) * g.ldw + c8;
   }
   const float *a_rows = A + (size_t)m0 * g.lda, *w_rows = W + (size_t)w_first * g.ldw;
   auto load = [&](const float* rows, const Offset* at, int k, bool tail) {   // `tail`: zeros from column K on
@@ -123,45 +130,94 @@ __global__ __launch_bounds__(64 * (kSlices / SPW), PER_SIMD) void gemm_float_ker
   const int steps = (end - begin) / kStep, per_slice = g.slice / kStep;  // whole steps; the last slice may have a tail
 #pragma unroll
   for (int i = 0; i < MT * NT; ++i) acc[i] = f32x4{0.f, 0.f, 0.f, 0.f};
-  if (steps > 0) {
-    Tile a[MT], w[NT];
+  auto second_slice = [&](int step) {                                  // which starts from zero
+    if (SPW != 2 || step + 1 != per_slice) return;
 #pragma unroll
-    for (int n = 0; n < NT; ++n) w[n] = load(w_rows, w_at[n], begin, false);
+    for (int i = 0; i < MT * NT; ++i) {
+      own_part[i * 64] = acc[i];
+      acc[i] = f32x4{0.f, 0.f, 0.f, 0.f};
+    }
+  };
+  if constexpr (SPLIT) {
+    // The parts of a tile of 16 weight rows are 3 KB for every 32 columns, in operand order; a step's are asked for a step ahead.
+    const int all_steps = (g.K + kStep - 1) / kStep, last_tile = (g.N + 15) / 16 - 1;
+    const bf16x8* parts_of[NT];
 #pragma unroll
-    for (int i = 0; i < MT; ++i) a[i] = load(a_rows, a_at[i], begin, false);
-    __builtin_amdgcn_sched_barrier(0);
-#pragma unroll 1
-    for (int step = 0; step < steps; ++step) {
-      const int k = begin + min(step + 1, steps - 1) * kStep;          // (past the last step: that one again, not used)
-      Triple wt[NT];
+    for (int n = 0; n < NT; ++n) parts_of[n] = g.W_split + (size_t)min(col_tile * NT + n, last_tile) * all_steps * (3 * 64) + lane;
+    auto load_parts = [&](Triple* w, int k) {
 #pragma unroll
-      for (int n = 0; n < NT; ++n) {
-        wt[n] = split(operand(w[n]));
-        w[n] = load(w_rows, w_at[n], k, false);
-      }
+      for (int n = 0; n < NT; ++n)
 #pragma unroll
-      for (int i = 0; i < MT; ++i) {
-        const Triple at = split(operand(a[i]));
-        a[i] = load(a_rows, a_at[i], k, false);
-        __builtin_amdgcn_sched_barrier(0);                             // (a load that a loop hands on would be moved to its use in the next round)
-        multiply(wt, at, i);
-      }
-      if (SPW == 2 && step + 1 == per_slice) {                         // the second slice starts from zero
+        for (int p = 0; p < 3; ++p) w[n].part[p] = parts_of[n][(size_t)(k / kStep) * (3 * 64) + p * 64];
+    };
+    if (steps > 0) {
+      Tile a[MT];
+      Triple w0[NT], w1[NT];
+      load_parts(w0, begin);
 #pragma unroll
-        for (int i = 0; i < MT * NT; ++i) {
-          own_part[i * 64] = acc[i];
-          acc[i] = f32x4{0.f, 0.f, 0.f, 0.f};
+      for (int i = 0; i < MT; ++i) a[i] = load(a_rows, a_at[i], begin, false);
+      __builtin_amdgcn_sched_barrier(0);
+      auto one_step = [&](const Triple* now, Triple* next, int step) {
+        const int k = begin + min(step + 1, steps - 1) * kStep;        // (past the last step: that one again, not used)
+        load_parts(next, k);
+#pragma unroll
+        for (int i = 0; i < MT; ++i) {
+          const Triple at = split(operand(a[i]));
+          a[i] = load(a_rows, a_at[i], k, false);
+          __builtin_amdgcn_sched_barrier(0);
+          multiply(now, at, i);
         }
+        second_slice(step);
+      };
+#pragma unroll 1
+      for (int step = 0; step + 1 < steps; step += 2) {
+        one_step(w0, w1, step);
+        one_step(w1, w0, step + 1);
+      }
+      if (steps & 1) one_step(w0, w1, steps - 1);
+    }
+    if (begin + steps * kStep < end) {                                 // less than a step is left (the parts past K are zeros)
+      const int k = begin + steps * kStep;
+      Triple w0[NT];
+      load_parts(w0, k);
+#pragma unroll
+      for (int i = 0; i < MT; ++i) multiply(w0, split(operand(load(a_rows, a_at[i], k, true))), i);
+    }
+  } else {
+    if (steps > 0) {
+      Tile a[MT], w[NT];
+#pragma unroll
+      for (int n = 0; n < NT; ++n) w[n] = load(w_rows, w_at[n], begin, false);
+#pragma unroll
+      for (int i = 0; i < MT; ++i) a[i] = load(a_rows, a_at[i], begin, false);
+      __builtin_amdgcn_sched_barrier(0);
+#pragma unroll 1
+      for (int step = 0; step < steps; ++step) {
+        const int k = begin + min(step + 1, steps - 1) * kStep;          // (past the last step: that one again, not used)
+        Triple wt[NT];
+#pragma unroll
+        for (int n = 0; n < NT; ++n) {
+          wt[n] = split(operand(w[n]));
+          w[n] = load(w_rows, w_at[n], k, false);
+        }
+#pragma unroll
+        for (int i = 0; i < MT; ++i) {
+          const Triple at = split(operand(a[i]));
+          a[i] = load(a_rows, a_at[i], k, false);
+          __builtin_amdgcn_sched_barrier(0);                             // (a load that a loop hands on would be moved to its use in the next round)
+          multiply(wt, at, i);
+        }
+        second_slice(step);
       }
     }
-  }
-  if (begin + steps * kStep < end) {                                   // less than a step is left
-    const int k = begin + steps * kStep;
-    Triple wt[NT];
+    if (begin + steps * kStep < end) {                                   // less than a step is left
+      const int k = begin + steps * kStep;
+      Triple wt[NT];
 #pragma unroll
-    for (int n = 0; n < NT; ++n) wt[n] = split(operand(load(w_rows, w_at[n], k, true)));
+      for (int n = 0; n < NT; ++n) wt[n] = split(operand(load(w_rows, w_at[n], k, true)));
 #pragma unroll
-    for (int i = 0; i < MT; ++i) multiply(wt, split(operand(load(a_rows, a_at[i], k, true))), i);
+      for (int i = 0; i < MT; ++i) multiply(wt, split(operand(load(a_rows, a_at[i], k, true))), i);
+    }
   }
   if (SPW == 1) __syncthreads();                                       // (the sums take the place of the tiles on their way)
 #pragma unroll
@@ -273,7 +329,7 @@ __global__ __launch_bounds__(64 * (kSlices / SPW), PER_SIMD) void gemm_float_ker
   }
 }
 
-template <int MT, int NT, int SPW, int PER_SIMD, int EPI>
+template <int MT, int NT, int SPW, int PER_SIMD, int EPI, bool SPLIT = false>
 static int launch_float_gemm(const FloatGemm& g, int batch, bool far, hipStream_t stream) {
   FloatGemm p = g;
   p.row_tiles = (g.M + 16 * MT - 1) / (16 * MT);
@@ -284,9 +340,9 @@ static int launch_float_gemm(const FloatGemm& g, int batch, bool far, hipStream_
   const size_t lds = SPW == 2 ? (size_t)kSlices / SPW * 8 * 272 + sums : (sums + kept > turns ? sums + kept : turns);
   static_assert(SPW == 1 || MT * NT * 64 * sizeof(f32x4) <= kSlices / SPW * 8 * 272, "the tiles that wait fit there");
   constexpr int kFewer = SPW == 1 ? 4 : PER_SIMD;                      // (workgroups of fewer wavefronts)
-  auto kernel = used == kSlices ? gemm_float_kernel<MT, NT, SPW, PER_SIMD, EPI, false, true> : gemm_float_kernel<MT, NT, SPW, kFewer, EPI, false, false>;
-  if constexpr (EPI == FG_PLAIN) {
-    if (far) kernel = used == kSlices ? gemm_float_kernel<MT, NT, SPW, PER_SIMD, EPI, true, true> : gemm_float_kernel<MT, NT, SPW, kFewer, EPI, true, false>;
+  auto kernel = used == kSlices ? gemm_float_kernel<MT, NT, SPW, PER_SIMD, EPI, false, true, SPLIT> : gemm_float_kernel<MT, NT, SPW, kFewer, EPI, false, false, SPLIT>;
+  if constexpr (EPI == FG_PLAIN && !SPLIT) {
+    if (far) kernel = used == kSlices ? gemm_float_kernel<MT, NT, SPW, PER_SIMD, EPI, true, true, false> : gemm_float_kernel<MT, NT, SPW, kFewer, EPI, true, false, false>;
   }
   if (lds > 64 * 1024) {
     hipError_t e = hipFuncSetAttribute(reinterpret_cast<const void*>(kernel), hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds);
@@ -318,20 +374,58 @@ PLLM_API int pllm_gemm_float(const float* A, int lda, long a_batch, const float*
                              int M, int N, int K, int batch, int rows_tile, int cols_tile, hipStream_t stream) {
   if (M <= 0 || N <= 0 || batch <= 0) return 0;
   if (K <= 0 || batch > 65535) return -2;
-  const FloatGemm g{A, W, C, a_batch, w_batch, c_batch, lda, ldw, ldc, M, N, K, slice_columns(K), 0, 0, 0, 0, 0, 0, 0, nullptr, nullptr, nullptr, nullptr, nullptr, nullptr};
+  const FloatGemm g{A, W, nullptr, C, a_batch, w_batch, c_batch, lda, ldw, ldc, M, N, K, slice_columns(K), 0, 0, 0, 0, 0, 0, 0, nullptr, nullptr, nullptr, nullptr, nullptr, nullptr};
   return launch_tile<FG_PLAIN>(g, batch, far(lda, ldw), rows_tile, cols_tile, stream);
 }
 
-// One product with something behind it (FG_GATED, FG_ROPE_KV above); all weight rows within 2^32 elements.  N: the weight rows.
-PLLM_API int pllm_gemm_float_fused(int epi, const float* A, int lda, const float* W, int ldw, float* C, int ldc, int M, int N, int K, int rows_tile,
-                                   int cols_tile, int activation, const int* positions, const float* cos_table, const float* sin_table, const int* slots,
-                                   float* k_pages, float* v_pages, int num_heads, int num_kv_heads, int head_dim, int block_size, hipStream_t stream) {
+template <int EPI>
+static int launch_split_tile(const FloatGemm& g, int rows_tile, int cols_tile, hipStream_t stream) {
+  switch (rows_tile * 10 + cols_tile) {
+    case 24: return launch_float_gemm<2, 4, 2, 2, EPI, true>(g, 1, false, stream);
+    case 34: return launch_float_gemm<3, 4, 2, 2, EPI, true>(g, 1, false, stream);
+    case 44: return launch_float_gemm<4, 4, 2, 2, EPI, true>(g, 1, false, stream);
+    default: return -3;
+  }
+}
+
+// One product (FG_PLAIN), or one with something behind it (FG_GATED, FG_ROPE_KV above); all weight rows within 2^32 elements.  N: the
+// weight rows.  W_split: the weights' parts in the order that this product takes them, or null; with them the tile is one of those above.
+PLLM_API int pllm_gemm_float_fused(int epi, const float* A, int lda, const float* W, int ldw, const void* W_split, float* C, int ldc, int M, int N, int K,
+                                   int rows_tile, int cols_tile, int activation, const int* positions, const float* cos_table, const float* sin_table,
+                                   const int* slots, float* k_pages, float* v_pages, int num_heads, int num_kv_heads, int head_dim, int block_size,
+                                   hipStream_t stream) {
   if (M <= 0 || N <= 0) return 0;
-  if (K <= 0 || N % 2 || far(lda, 0) || (long)N * ldw > 1l << 32) return -2;
-  const FloatGemm g{A, W, C, 0, 0, 0, lda, ldw, ldc, M, N, K, slice_columns(K), 0, 0, activation, num_heads, num_kv_heads, head_dim, block_size,
-                    positions, slots, cos_table, sin_table, k_pages, v_pages};
-  if (epi == FG_GATED) return activation >= 0 && activation < PLLM_ACT_COUNT ? launch_tile<FG_GATED>(g, 1, false, rows_tile, cols_tile, stream) : -2;
+  if (K <= 0 || far(lda, 0) || (long)N * ldw > 1l << 32 || reinterpret_cast<uintptr_t>(W_split) % 16) return -2;
+  const FloatGemm g{A, W, (const bf16x8*)W_split, C, 0, 0, 0, lda, ldw, ldc, M, N, K, slice_columns(K), 0, 0, activation, num_heads, num_kv_heads, head_dim,
+                    block_size, positions, slots, cos_table, sin_table, k_pages, v_pages};
+  if (epi == FG_PLAIN) return W_split ? launch_split_tile<FG_PLAIN>(g, rows_tile, cols_tile, stream) : -3;
+  if (N % 2) return -2;
+  if (epi == FG_GATED) {
+    if (activation < 0 || activation >= PLLM_ACT_COUNT) return -2;
+    return W_split ? launch_split_tile<FG_GATED>(g, rows_tile, cols_tile, stream) : launch_tile<FG_GATED>(g, 1, false, rows_tile, cols_tile, stream);
+  }
   if (epi != FG_ROPE_KV) return -3;
   if (head_dim <= 0 || head_dim % 16 || block_size <= 0 || N != (num_heads + 2 * num_kv_heads) * head_dim || !sixteen_bytes(C, ldc, 0) || !sixteen_bytes(k_pages, 0, 0)) return -2;
-  return launch_tile<FG_ROPE_KV>(g, 1, false, rows_tile, cols_tile, stream);
+  return W_split ? launch_split_tile<FG_ROPE_KV>(g, rows_tile, cols_tile, stream) : launch_tile<FG_ROPE_KV>(g, 1, false, rows_tile, cols_tile, stream);
+}
+
+// The parts of a matrix's floats in the order in which a product with this epilogue takes them:
+// [tiles of 16 weight rows][steps of 32 columns][3 parts][64 lanes][8], zeros past column K.
+template <int EPI>
+__global__ __launch_bounds__(64) void float_split_weights_kernel(FloatGemm g, bf16x8* out) {
+  const int lane = threadIdx.x, k = blockIdx.x * kStep + 4 * (lane >> 4);
+  const float* row = g.W + (size_t)weight_row<EPI>(g, 16 * blockIdx.y + (lane & 15)) * g.ldw + k;
+  const Triple t = split(Octet{four_of(row, g.K - k), four_of(row + 16, g.K - k - 16)});
+#pragma unroll
+  for (int p = 0; p < 3; ++p) out[(((size_t)blockIdx.y * gridDim.x + blockIdx.x) * 3 + p) * 64 + lane] = t.part[p];
+}
+
+PLLM_API int pllm_float_split_weights(int epi, const float* W, int ldw, int N, int K, int head_dim, void* out, hipStream_t stream) {
+  if (N <= 0 || K <= 0 || (N + 15) / 16 > 65535 || reinterpret_cast<uintptr_t>(out) % 16) return -2;
+  if ((epi == FG_GATED && N % 2) || (epi == FG_ROPE_KV && (head_dim <= 0 || head_dim % 16 || N % head_dim))) return -2;
+  FloatGemm g{};
+  g.W = W; g.ldw = ldw; g.N = N; g.K = K; g.head_dim = head_dim;
+  auto kernel = epi == FG_PLAIN ? float_split_weights_kernel<FG_PLAIN> : epi == FG_GATED ? float_split_weights_kernel<FG_GATED> : float_split_weights_kernel<FG_ROPE_KV>;
+  hipLaunchKernelGGL(kernel, dim3((K + kStep - 1) / kStep, (N + 15) / 16), dim3(64), 0, stream, g, (bf16x8*)out);
+  PLLM_RETURN_LAST_ERROR();
 }

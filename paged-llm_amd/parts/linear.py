@@ -28,13 +28,16 @@ class Weight:
     order that the streaming kernel reads (1 KB tiles in the matrix instruction's operand order; see
     ``ops.tile_weight``).  ``pairing``: which rows share a tile, by what the epilogue behind the product needs:
     "plain", "gated" ([gate; up] rows) or "rotary" ([q; k; v] rows of heads of ``head_dim``).  The plain copy serves
-    the other kernels and the library; a step reads one of the two."""
+    the other kernels and the library; a step reads one of the two.  A float32 matrix has its elements' bfloat16 parts as the second
+    copy instead (``split``, 6 bytes an element), which float products of many rows take (``ops.float_split_plan``)."""
 
     def __init__(self, plain: torch.Tensor, pairing: str = "plain", head_dim: int = 0):
         self.plain = plain
         self.pairing = pairing
         ok = ops.stream_linear_takes(plain) and (pairing != "rotary" or (head_dim > 0 and head_dim % 16 == 0))
         self.tiled = ops.tile_weight(plain, pairing, head_dim) if ok else None
+        ok = ops.float_split_takes(plain) and (pairing != "rotary" or (head_dim > 0 and head_dim % 16 == 0))
+        self.split = ops.float_split_weights(plain, pairing, head_dim) if ok else None
 
     @property
     def shape(self):
@@ -212,10 +215,15 @@ def linear(x, weight, out_dtype: torch.dtype | None = None, partial_ok: bool = F
         out = _fused(x, weight, ops.EPI_F32 if out_dtype == torch.float32 else ops.EPI_BF16)
         if out is not None:
             return out
+    split = weight.split if isinstance(weight, Weight) and weight.pairing == "plain" else None
     weight = _plain(weight)
     x = rows_of(x)
     if x.dtype == torch.bfloat16 and weight.dtype == torch.bfloat16:
         return ops.gemm_bf16(x, weight, out_dtype)
+    if split is not None and x.dtype == torch.float32:
+        out = ops.gemm_float_split(x, weight, split)
+        if out is not None:
+            return out
     return ops.gemm_generic(x, weight, out_dtype)
 
 
@@ -284,11 +292,12 @@ def gated_linear(x, w_gate_up, activation: str = "silu") -> torch.Tensor:
         out = _fused(x, w_gate_up, ops.EPI_GATED, activation=activation)
         if out is not None:
             return out
+    split = w_gate_up.split if isinstance(w_gate_up, Weight) and w_gate_up.pairing == "gated" else None
     w_gate_up = _plain(w_gate_up)
     if w_gate_up.dtype == torch.float32:
         x = rows_of(x)
         if ops.gemm_float_fused_takes(x, w_gate_up):
-            return ops.gemm_float_gated(x, w_gate_up, activation)
+            return ops.gemm_float_gated(x, w_gate_up, activation, split)
     return ops.gate_mul(linear(x, w_gate_up), activation)
 
 
@@ -358,7 +367,8 @@ def qkv_rotary_cache(x, w_qkv, positions: torch.Tensor, position_encoding, num_h
         elif k_pages.dtype == torch.float32:
             x = rows_of(x)
             if ops.gemm_float_fused_takes(x, _plain(w_qkv)):
-                return ops.gemm_float_rotary(x, _plain(w_qkv), rope)
+                split = w_qkv.split if isinstance(w_qkv, Weight) and w_qkv.pairing == "rotary" else None
+                return ops.gemm_float_rotary(x, _plain(w_qkv), rope, split)
     w_qkv = _plain(w_qkv)
     qkv = linear(x, w_qkv, bias=bias)
     ops.rope_scatter(qkv, positions, cos, sin, num_heads, num_kv_heads, head_dim, slot_mapping if write else None,

@@ -1,0 +1,81 @@
+"""Float products whose weights come as their bfloat16 parts, laid out once: the bits of the products that split the floats themselves."""
+
+import pytest
+import torch
+
+from tests.test_kernels_gpu import rnd
+
+pytestmark = pytest.mark.gpu
+
+
+def ops():
+    from paged_llm_amd.csrc import ops as o
+    return o
+
+
+def each_tile(monkeypatch):
+    for tile in ops().FLOAT_SPLIT_TILES:
+        monkeypatch.setattr(ops(), "float_split_plan", lambda *a, tile=tile: tile)
+        yield tile
+
+
+# rows and weight rows past the last tile, one step of columns, slices without columns (K = 520, 1408), an odd number of steps a slice, a tail
+@pytest.mark.parametrize("m,n,k", [(1, 16, 32), (33, 70, 520), (96, 130, 1408), (65, 2048, 2052), (150, 48, 3000), (70, 2049, 512)])
+def test_plain_product_from_parts(m, n, k, monkeypatch):
+    o = ops()
+    a, w = rnd(m, k, seed=1).cuda(), rnd(n, k, seed=2).cuda()
+    want, split = o.gemm_generic(a, w), o.float_split_weights(w)
+    for tile in each_tile(monkeypatch):
+        assert torch.equal(o.gemm_float_split(a, w, split), want), tile
+
+
+@pytest.mark.parametrize("m,ff,k", [(40, 129, 512), (97, 12, 100), (130, 40, 2048)])
+def test_gated_product_from_parts(m, ff, k, monkeypatch):
+    o = ops()
+    a, w = rnd(m, k, seed=3).cuda(), rnd(2 * ff, k, seed=4).cuda()
+    want, split = o.gemm_float_gated(a, w), o.float_split_weights(w, "gated")
+    for tile in each_tile(monkeypatch):
+        assert torch.equal(o.gemm_float_gated(a, w, split=split), want), tile
+
+
+@pytest.mark.parametrize("heads,kv_heads,d,bs", [(4, 2, 64, 16), (3, 1, 48, 32)])
+def test_rotary_product_from_parts(heads, kv_heads, d, bs, monkeypatch):
+    o = ops()
+    m, k = 100, 512
+    a, w = rnd(m, k, seed=5).cuda(), rnd((heads + 2 * kv_heads) * d, k, seed=6).cuda()
+    slots = torch.randperm(2 * m, generator=torch.Generator().manual_seed(7))[:m].to(torch.int32).cuda()
+    cos, sin = (rnd(m, d // 2, seed=s).cuda() for s in (8, 9))
+    split = o.float_split_weights(w, "rotary", d)
+
+    def product(split):
+        k_pages, v_pages = torch.zeros((2 * m // bs + 1, kv_heads, bs, d), device="cuda"), torch.zeros((2 * m // bs + 1, kv_heads, d, bs), device="cuda")
+        q = o.gemm_float_rotary(a, w, dict(positions=torch.arange(m, dtype=torch.int32, device="cuda"), cos=cos, sin=sin, slots=slots, k_pages=k_pages,
+                                           v_pages=v_pages, num_heads=heads, num_kv_heads=kv_heads, head_dim=d, block_size=bs), split)
+        return q, k_pages, v_pages
+    want = product(None)
+    for tile in each_tile(monkeypatch):
+        assert all(torch.equal(x, y) for x, y in zip(product(split), want)), tile
+
+
+def test_results_that_are_not_finite_from_parts(monkeypatch):
+    """Infinities, NaN and numbers past the largest bfloat16 among rows and weights: made again from the floats, as without the parts."""
+    o = ops()
+    a, w = rnd(70, 1030, seed=10), rnd(50, 1030, seed=11)
+    a[1, 3], w[2, 1029], w[3, 0], a[4] = float("inf"), float("-inf"), float("nan"), a[4] * 2.0 ** -120
+    a[2, :], w[4, :] = 0.0, 0.0
+    a[2, 5], w[4, 5] = 3.4e38, 0.5
+    a, w = a.cuda(), w.cuda()
+    a, w = a[:, :1028], w[:, :1028]                       # (rows with a stride of their own: not on 16-byte boundaries, and so from the floats)
+    split = o.float_split_weights(w)
+    for tile in each_tile(monkeypatch):
+        assert o.gemm_float_split(a, w, split) is None
+        x, y = a.contiguous(), w.contiguous()
+        got, want = o.gemm_float_split(x, y, split), o.gemm_generic(x, y)
+        assert torch.equal(got.isnan(), want.isnan()) and torch.equal(got.nan_to_num(nan=0.0), want.nan_to_num(nan=0.0)), tile
+
+
+def test_which_products_take_the_parts():
+    o = ops()
+    assert o.float_split_plan(95, 2048, 2048, 256) is None and o.float_split_plan(301, 2048, 480, 256) is None
+    assert o.float_split_plan(301, 2048, 2048, 256) == (3, 4) and o.float_split_plan(301, 11264, 2048, 256) == (4, 4)
+    assert o.float_split_plan(128, 2048, 2048, 256) is None               # (tiles of 32 x 32 from the floats are ahead)
