@@ -13,6 +13,10 @@
 //     32 (2048 weight rows are 128 workgroups) and few enough registers for two workgroups on a compute unit: 8 rows x 2048 x 2048 in 7.0
 //     us (8.5 with the float instruction, which takes the weights' loads in operand order as well), 11264 x 2048 in 18.4 (23.4), 2048 x
 //     5632 in 14.4 (18.6); 64 rows x 2048 x 2048 in 10.1 (13.4).
+//     There the split is what bounds the smaller ones (half of a wavefront's vector instructions are the rows', half the weights'; more
+//     loads under way, two to four steps, made every one of them slower), and 128 workgroups leave half of the compute units idle: where the reader adds
+//     two sums, two workgroups take eight slices each (pllm_gemm_float_halves: 8 rows x 2048 x 2048 8.1 -> 6.4 us, x 5632 19.0 -> 13.5 with weights
+//     from memory).
 //   * Many rows: bound by the same way (a tile of 64 x 64 draws 42 bytes a clock at the matrix cores' rate, of 45 that the L2 gives) and
 //     by a wavefront's chain of load, turn, split and product.  Eight wavefronts take two slices each, one after the other, with up to 256
 //     registers a lane; the first slice's sums wait in LDS.  301 rows x 2048 x 2048 / 5632 in 27 / 64 us (37 / 86 with the float
@@ -40,7 +44,7 @@ struct FloatGemm {
   const float* W;
   const bf16x8* W_split;                                               // (SPLIT) the weights' parts, or null
   float* C;
-  long a_batch, w_batch, c_batch;
+  long a_batch, w_batch, c_batch, c_range;                             // (c_range: from the first range's sums to the second's)
   int lda, ldw, ldc, M, N, K, slice, row_tiles, col_tiles;             // N: weight rows
   // Behind the product:
   int activation, num_heads, num_kv_heads, head_dim, block_size;
@@ -67,8 +71,12 @@ __device__ __forceinline__ int weight_row(const FloatGemm& g, int at) {
 // ALL: every slice has columns, and the workgroup all its wavefronts.  SPW: slices of a wavefront.
 // FAR: rows so far apart that an offset inside a tile takes 64 bits.
 // SPLIT: the weights' parts come from W_split, as pllm_float_split_weights lays them out.
-template <int MT, int NT, int SPW, int PER_SIMD, int EPI, bool FAR, bool ALL, bool SPLIT>
-__global__ __launch_bounds__(64 * (kSlices / SPW), PER_SIMD) void gemm_float_kernel(FloatGemm g) {
+// RANGES: workgroups of a tile (blockIdx.z), each with as many of the slices, whose sums are results of their own.
+template <int MT, int NT, int SPW, int PER_SIMD, int EPI, bool FAR, bool ALL, bool SPLIT, int RANGES>
+__global__ __launch_bounds__(64 * (kSlices / SPW / RANGES), PER_SIMD) void gemm_float_kernel(FloatGemm g) {
+  static_assert(RANGES == 1 || (RANGES == 2 && SPW == 1 && EPI == FG_PLAIN && ALL), "halves of the tree");
+  constexpr int kOwn = kSlices / RANGES;
+  const int first_slice = RANGES == 1 ? 0 : (int)blockIdx.z * kOwn;
   constexpr int kPad = 272;                                            // bytes: a chunk of 16 bytes of 16 rows, and 16 against bank conflicts
   extern __shared__ __attribute__((aligned(16))) unsigned char gf_lds[];
   __shared__ unsigned waiting;                                         // the tiles of 16 x 16 with a sum that is not finite
@@ -88,7 +96,7 @@ __global__ __launch_bounds__(64 * (kSlices / SPW), PER_SIMD) void gemm_float_ker
   const int m0 = row_tile * (16 * MT), n0 = col_tile * (16 * NT);
   const float* A = g.A + (size_t)blockIdx.y * g.a_batch;
   const float* W = g.W + (size_t)blockIdx.y * g.w_batch;
-  float* C = g.C + (size_t)blockIdx.y * g.c_batch;
+  float* C = g.C + (size_t)blockIdx.y * g.c_batch + (RANGES == 1 ? 0 : (size_t)blockIdx.z * g.c_range);
 
   // A tile of 16 rows x 32 columns under way: two loads of 8 rows x 128 bytes.
   struct Tile { f32x4 x[2]; };
@@ -126,7 +134,7 @@ __global__ __launch_bounds__(64 * (kSlices / SPW), PER_SIMD) void gemm_float_ker
         acc[i * NT + n] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(w[n].part[kProducts[p][0]], a.part[kProducts[p][1]], acc[i * NT + n], 0, 0, 0);
   };
 
-  const int begin = min(wave * SPW * g.slice, g.K), end = min(begin + SPW * g.slice, g.K);
+  const int begin = min((first_slice + wave * SPW) * g.slice, g.K), end = min(begin + SPW * g.slice, g.K);
   const int steps = (end - begin) / kStep, per_slice = g.slice / kStep;  // whole steps; the last slice may have a tail
 #pragma unroll
   for (int i = 0; i < MT * NT; ++i) acc[i] = f32x4{0.f, 0.f, 0.f, 0.f};
@@ -226,17 +234,19 @@ __global__ __launch_bounds__(64 * (kSlices / SPW), PER_SIMD) void gemm_float_ker
 
   const bool wide = (g.ldc & 3) == 0 && (reinterpret_cast<uintptr_t>(C) & 15) == 0;
   constexpr int kEach = MT * NT * 64;
-  const int threads = ALL ? 64 * (kSlices / SPW) : (int)blockDim.x;
+  const int threads = ALL ? 64 * (kOwn / SPW) : (int)blockDim.x;
   auto sum_at = [&](int at) {                                          // of a lane's four weight rows and row
-    f32x4 pair[kSlices / 2];
+    f32x4 pair[kOwn / 2];
 #pragma unroll
-    for (int i = 0; i < kSlices / 2; ++i) {
+    for (int i = 0; i < kOwn / 2; ++i) {
       pair[i] = f32x4{0.f, 0.f, 0.f, 0.f};                             // (slices past K are zeros that nobody makes)
       if (!ALL && 2 * i * g.slice >= g.K) continue;
       pair[i] = parts[(SPW == 2 ? i : 2 * i) * kEach + at];
       if (SPW == 1 && (ALL || (2 * i + 1) * g.slice < g.K)) pair[i] += parts[(2 * i + 1) * kEach + at];
     }
-    return ((pair[0] + pair[1]) + (pair[2] + pair[3])) + ((pair[4] + pair[5]) + (pair[6] + pair[7]));
+    const f32x4 half = (pair[0] + pair[1]) + (pair[2] + pair[3]);
+    if constexpr (RANGES == 2) return half;
+    else return half + ((pair[4] + pair[5]) + (pair[6] + pair[7]));
   };
   auto write_four = [&](float* c, f32x4 x, int n, int N) {             // columns n .. n + 3 of N
     if (wide && n + 4 <= N) {
@@ -313,7 +323,7 @@ __global__ __launch_bounds__(64 * (kSlices / SPW), PER_SIMD) void gemm_float_ker
     f32x4 sum{0.f, 0.f, 0.f, 0.f};
 #pragma unroll 1
     for (int s = wave * SPW; s < wave * SPW + SPW; ++s) {
-      const f32x4 x = plain_sums(a, w, min(s * g.slice, g.K), min((s + 1) * g.slice, g.K));
+      const f32x4 x = plain_sums(a, w, min((first_slice + s) * g.slice, g.K), min((first_slice + s + 1) * g.slice, g.K));
       sum = s == wave * SPW ? x : sum + x;
     }
     own_part[i * 64] = sum;
@@ -329,26 +339,30 @@ __global__ __launch_bounds__(64 * (kSlices / SPW), PER_SIMD) void gemm_float_ker
   }
 }
 
-template <int MT, int NT, int SPW, int PER_SIMD, int EPI, bool SPLIT = false>
+template <int MT, int NT, int SPW, int PER_SIMD, int EPI, bool SPLIT = false, int RANGES = 1>
 static int launch_float_gemm(const FloatGemm& g, int batch, bool far, hipStream_t stream) {
   FloatGemm p = g;
   p.row_tiles = (g.M + 16 * MT - 1) / (16 * MT);
   p.col_tiles = (g.N + 16 * NT - 1) / (16 * NT);
-  const int used = (g.K + g.slice - 1) / g.slice, waves = (used + SPW - 1) / SPW;     // wavefronts that have columns: 1 to kSlices / SPW
+  const int used = (g.K + g.slice - 1) / g.slice, waves = (used / RANGES + SPW - 1) / SPW;   // wavefronts that have columns: 1 to kSlices / SPW
+  if (RANGES > 1 && used != kSlices) return -2;
   const size_t sums = (size_t)waves * MT * NT * 64 * sizeof(f32x4), turns = (size_t)waves * 8 * 272;
   const size_t kept = (size_t)MT * NT * 64 * sizeof(f32x4);                            // (SPW = 2: in the place of the tiles on their way)
   const size_t lds = SPW == 2 ? (size_t)kSlices / SPW * 8 * 272 + sums : (sums + kept > turns ? sums + kept : turns);
   static_assert(SPW == 1 || MT * NT * 64 * sizeof(f32x4) <= kSlices / SPW * 8 * 272, "the tiles that wait fit there");
   constexpr int kFewer = SPW == 1 ? 4 : PER_SIMD;                      // (workgroups of fewer wavefronts)
-  auto kernel = used == kSlices ? gemm_float_kernel<MT, NT, SPW, PER_SIMD, EPI, false, true, SPLIT> : gemm_float_kernel<MT, NT, SPW, kFewer, EPI, false, false, SPLIT>;
-  if constexpr (EPI == FG_PLAIN && !SPLIT) {
-    if (far) kernel = used == kSlices ? gemm_float_kernel<MT, NT, SPW, PER_SIMD, EPI, true, true, false> : gemm_float_kernel<MT, NT, SPW, kFewer, EPI, true, false, false>;
+  auto kernel = gemm_float_kernel<MT, NT, SPW, PER_SIMD, EPI, false, true, SPLIT, RANGES>;
+  if constexpr (RANGES == 1) {
+    if (used != kSlices) kernel = gemm_float_kernel<MT, NT, SPW, kFewer, EPI, false, false, SPLIT, 1>;
+  }
+  if constexpr (EPI == FG_PLAIN && !SPLIT && RANGES == 1) {
+    if (far) kernel = used == kSlices ? gemm_float_kernel<MT, NT, SPW, PER_SIMD, EPI, true, true, false, 1> : gemm_float_kernel<MT, NT, SPW, kFewer, EPI, true, false, false, 1>;
   }
   if (lds > 64 * 1024) {
     hipError_t e = hipFuncSetAttribute(reinterpret_cast<const void*>(kernel), hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds);
     if (e != hipSuccess) return (int)e;
   }
-  const dim3 grid((unsigned)(p.col_tiles * p.row_tiles), batch), block(64 * waves);
+  const dim3 grid((unsigned)(p.col_tiles * p.row_tiles), batch, RANGES), block(64 * waves);
   hipLaunchKernelGGL(kernel, grid, block, lds, stream, p);
   PLLM_RETURN_LAST_ERROR();
 }
@@ -374,8 +388,17 @@ PLLM_API int pllm_gemm_float(const float* A, int lda, long a_batch, const float*
                              int M, int N, int K, int batch, int rows_tile, int cols_tile, hipStream_t stream) {
   if (M <= 0 || N <= 0 || batch <= 0) return 0;
   if (K <= 0 || batch > 65535) return -2;
-  const FloatGemm g{A, W, nullptr, C, a_batch, w_batch, c_batch, lda, ldw, ldc, M, N, K, slice_columns(K), 0, 0, 0, 0, 0, 0, 0, nullptr, nullptr, nullptr, nullptr, nullptr, nullptr};
+  const FloatGemm g{A, W, nullptr, C, a_batch, w_batch, c_batch, 0, lda, ldw, ldc, M, N, K, slice_columns(K), 0, 0, 0, 0, 0, 0, 0, nullptr, nullptr, nullptr, nullptr, nullptr, nullptr};
   return launch_tile<FG_PLAIN>(g, batch, far(lda, ldw), rows_tile, cols_tile, stream);
+}
+
+// The same product of few rows as two sums, C [2][M][N]: of the first and of the last eight slices, whose sum is the result (K with columns in all
+// sixteen, rows and weight rows within 32-bit offsets of a tile).
+PLLM_API int pllm_gemm_float_halves(const float* A, int lda, const float* W, int ldw, float* C, int M, int N, int K, int cols_tile, hipStream_t stream) {
+  if (M <= 0 || N <= 0) return 0;
+  if (K <= 0 || far(lda, ldw)) return -2;
+  const FloatGemm g{A, W, nullptr, C, 0, 0, 0, (long)M * N, lda, ldw, N, M, N, K, slice_columns(K), 0, 0, 0, 0, 0, 0, 0, nullptr, nullptr, nullptr, nullptr, nullptr, nullptr};
+  return cols_tile == 1 ? launch_float_gemm<1, 1, 1, 4, FG_PLAIN, false, 2>(g, 1, false, stream) : launch_float_gemm<1, 2, 1, 4, FG_PLAIN, false, 2>(g, 1, false, stream);
 }
 
 template <int EPI>
@@ -396,7 +419,7 @@ PLLM_API int pllm_gemm_float_fused(int epi, const float* A, int lda, const float
                                    hipStream_t stream) {
   if (M <= 0 || N <= 0) return 0;
   if (K <= 0 || far(lda, 0) || (long)N * ldw > 1l << 32 || reinterpret_cast<uintptr_t>(W_split) % 16) return -2;
-  const FloatGemm g{A, W, (const bf16x8*)W_split, C, 0, 0, 0, lda, ldw, ldc, M, N, K, slice_columns(K), 0, 0, activation, num_heads, num_kv_heads, head_dim,
+  const FloatGemm g{A, W, (const bf16x8*)W_split, C, 0, 0, 0, 0, lda, ldw, ldc, M, N, K, slice_columns(K), 0, 0, activation, num_heads, num_kv_heads, head_dim,
                     block_size, positions, slots, cos_table, sin_table, k_pages, v_pages};
   if (epi == FG_PLAIN) return W_split ? launch_split_tile<FG_PLAIN>(g, rows_tile, cols_tile, stream) : -3;
   if (N % 2) return -2;

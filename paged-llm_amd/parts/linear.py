@@ -1,6 +1,7 @@
 """y = x W^T for the parts, with the kernel chosen by element type and number of rows.
 
-* float32: the float product kernel (the true 32-bit path), always, with the gate's activation or the rotary/cache write behind.
+* float32: the float product kernel (the true 32-bit path), always, with the gate's activation or the rotary/cache write behind; of few rows
+  as two sums where the consuming norm adds them, of many from the weights' parts (``Weight``).
 * bfloat16, at most 16 rows (decoding): the fused decode kernel, which also takes in a pending
   residual sum + norm in front and an activation or the rotary/cache write behind.
 * bfloat16, 17 to 128 rows (decoding with many requests, short prompt portions): the streaming kernel over the
@@ -220,8 +221,10 @@ def linear(x, weight, out_dtype: torch.dtype | None = None, partial_ok: bool = F
     x = rows_of(x)
     if x.dtype == torch.bfloat16 and weight.dtype == torch.bfloat16:
         return ops.gemm_bf16(x, weight, out_dtype)
-    if split is not None and x.dtype == torch.float32:
-        out = ops.gemm_float_split(x, weight, split)
+    if x.dtype == weight.dtype == torch.float32:
+        out = ops.gemm_float_halves(x, weight) if partial_ok else None
+        if out is None and split is not None:
+            out = ops.gemm_float_split(x, weight, split)
         if out is not None:
             return out
     return ops.gemm_generic(x, weight, out_dtype)

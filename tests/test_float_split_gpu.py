@@ -74,6 +74,25 @@ def test_results_that_are_not_finite_from_parts(monkeypatch):
         assert torch.equal(got.isnan(), want.isnan()) and torch.equal(got.nan_to_num(nan=0.0), want.nan_to_num(nan=0.0)), tile
 
 
+# one row, rows and weight rows past the last tile, tiles of 16 x 16 and 16 x 32, a last slice of one column
+@pytest.mark.parametrize("m,n,k", [(1, 16, 512), (8, 2048, 2048), (17, 1030, 1000), (24, 2048, 993), (16, 4090, 2044)])
+def test_product_as_two_sums(m, n, k):
+    o = ops()
+    a, w = rnd(m, k, seed=12).cuda(), rnd(n, k, seed=13).cuda()
+    a[0, 0], a[0, k - 1] = float("inf"), float("nan")
+    halves, want = o.gemm_float_halves(a, w), o.gemm_generic(a, w)
+    assert halves.shape == (2, m, n) and bool(want[0].isnan().all()) and bool(halves[1, 0].isnan().all()) and not bool(halves[0, 0].isfinite().any())
+    assert torch.equal((halves[0] + halves[1])[1:], want[1:])
+    a[0] = 1.0
+    assert torch.equal(o.gemm_float_halves(a, w).sum(0)[:1], o.gemm_generic(a, w)[:1])
+
+
+def test_which_products_come_as_two_sums():
+    o = ops()
+    assert o.float_halves_plan(8, 2048, 2048, 256) == 1 and o.float_halves_plan(24, 2048, 2048, 256) == o.float_halves_plan(8, 4096, 2048, 256) == 2
+    assert o.float_halves_plan(33, 2048, 2048, 256) is None and o.float_halves_plan(8, 2048, 520, 256) is None       # (too many tiles; slices without columns)
+
+
 def test_which_products_take_the_parts():
     o = ops()
     assert o.float_split_plan(95, 2048, 2048, 256) is None and o.float_split_plan(301, 2048, 480, 256) is None
