@@ -328,7 +328,7 @@ __global__ __launch_bounds__(1024) void moe_align_kernel(const int* __restrict__
 PLLM_API int pllm_moe_align(const int* ids, int pairs, int experts, int* sorted_pair, int* row_of_pair, int* tiles, int max_tiles,
                             int tile_rows, hipStream_t stream) {
   if (pairs <= 0) return 0;
-  if (tile_rows < kMoeTileRows || tile_rows % kMoeTileRows || tile_rows > kMoeMaxTileRows) return -2;
+  if (tile_rows < kMoeTileRows || tile_rows % kMoeTileRows || tile_rows > 256) return -2;
   if (experts <= 0 || experts > kMoeMaxExperts || max_tiles < (pairs + tile_rows - 1) / tile_rows + experts) return -2;
   // (a thread for every expert, and for every pair of a small step: fewer wavefronts meet sooner at the barriers)
   const int threads = min(1024, (max(pairs, experts) + 63) / 64 * 64);
@@ -802,7 +802,7 @@ __global__ __launch_bounds__(256) void moe_expert_tile_kernel(const bf16* __rest
   }
 }
 
-// The products where K is a multiple of 64: a tile of MT blocks of 16 rows of one expert times NB blocks of 16 weight rows (gated: a
+// The products where K is a multiple of 64 (with 70 rows an expert and more those of moe_wide.hip are ahead): a tile of MT blocks of 16 rows of one expert times NB blocks of 16 weight rows (gated: a
 // gate's block and its up block in turn), for prompt steps eight wavefronts that multiply and four that bring the operands: stages of 64 columns
 // go from memory straight into LDS, R stages deep, a load taking the whole 128-byte lines of eight rows, whose eight pieces
 // lie XOR-ed by the row so that operand reads meet no bank twice.  Workgroups that follow each other on a chiplet

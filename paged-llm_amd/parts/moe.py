@@ -118,11 +118,14 @@ class RoutedExperts(FeedForward):
         routed = ops.moe_route(h, self.router, self.correction, self.groups, self.keep, self.top, self.scoring, extra=1 if self.shared_gate else 0,
                                group_mark=self.group_mark)
         ids, weights = routed[0], routed[1]
-        rows = ops.moe_tile_rows(ids.numel(), self.experts, h.dtype, self.hidden, self.inter, h.stride(0))
+        wide = None
+        if h.dtype == torch.bfloat16 and h.stride(0) % 8 == 0 and h.data_ptr() % 16 == 0:
+            wide = ops.moe_wide_plan(ids.numel(), self.experts, self.hidden, self.inter, self.gated, ops._num_compute_units(h.device))
+        rows, first_columns, down_columns = wide or (ops.moe_tile_rows(ids.numel(), self.experts, h.dtype, self.hidden, self.inter, h.stride(0)), 0, 0)
         sorted_pair, row_of_pair, tiles = ops.moe_align(ids, self.experts, rows)
         act = ops.moe_expert_gemm(h, self.w_gate_up, tiles, sorted_pair, self.top, self.gated, self.activation, tile_rows=rows,
-                                  pair_scale=weights if inside else None, plain=not self.gated)
-        out = ops.moe_expert_gemm(act, self.w_down, tiles, sorted_pair, self.top, False, tile_rows=rows)
+                                  pair_scale=weights if inside else None, plain=not self.gated, wide_columns=first_columns)
+        out = ops.moe_expert_gemm(act, self.w_down, tiles, sorted_pair, self.top, False, tile_rows=rows, wide_columns=down_columns)
         shared = gate = None
         if self.shared_inter:
             shared = linear(gated_linear(h, self.w_shared_gate_up, self.activation), self.w_shared_down, out_dtype=torch.float32)
