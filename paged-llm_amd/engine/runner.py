@@ -44,12 +44,14 @@ class GraphCache:
             entries.move_to_end(key)
         return entry
 
-    def put(self, key, entry) -> None:
-        entries = self._of(key)
+    def put(self, key, entry):
+        """Returns the key of the entry that had to go, or None."""
+        entries, gone = self._of(key), None
         while len(entries) >= self.per_kind and key not in entries:
-            entries.popitem(last=False)
+            gone, _ = entries.popitem(last=False)
         entries[key] = entry
         entries.move_to_end(key)
+        return gone
 
     def __iter__(self):
         return (key for entries in self._kinds.values() for key in entries)
@@ -63,7 +65,7 @@ class GraphCache:
 
 class ModelRunner:
     def __init__(self, model, kv_storage: KVCacheStorage, num_state_slots: int = 0, use_graphs: bool = False,
-                 max_graph_batch: int = 1024, max_graph_tokens: int = 1024, graph_after_sightings: int = 2):
+                 max_graph_batch: int = 1024, max_graph_tokens: int = 2048, graph_after_sightings: int = 2):
         self.model = model
         # Graph replay needs every part of the model to do nothing but launch kernels on the
         # current stream; parts say so with ``graph_capturable`` (steps of single tokens) and
@@ -71,7 +73,7 @@ class ModelRunner:
         self.use_graphs = bool(use_graphs) and model.graph_capturable()
         self.prompt_graphs = self.use_graphs and model.graph_capturable(prompts=True)
         self.max_graph_batch = max_graph_batch
-        # Steps with prompt portions are replayed from graphs up to this many portion tokens (eight times as many
+        # Steps with prompt portions are replayed from graphs up to this many portion tokens (four times as many
         # when no padding is needed), and once their shape has been seen this often (a capture costs several
         # steps' time; shapes that never come back are not worth one).
         self.max_graph_tokens = max_graph_tokens
@@ -410,11 +412,14 @@ class ModelRunner:
 
     # ------------------------------------------------------------------ steps with prompt portions as HIP graphs
     MAX_GRAPH_PORTIONS = 4
+    MAX_GRAPH_LOGITS = 64                 # rows of logits that a graph of such a step holds
 
     @staticmethod
     def _token_bucket(n: int) -> int:
-        """Portion tokens a graph is captured for: steps of 32 up to 128, of 64 up to 512, of 128 up to 1024, of 256 beyond."""
-        for limit, step in ((128, 32), (512, 64), (1024, 128)):
+        """Portion tokens a graph is captured for, and wanted rows beyond 64: steps of 32 up to 1024, of 16 up to 2048, of 256 beyond.  The rows
+        between are computed for nothing: 777 tokens in a graph of 896 / 832 / 800 took 2.87 / 2.85 / 2.75 ms (Renadra, width 2,048), and
+        beyond 1,024 a step may bear 1 to 2 % of them before the launches from Python are cheaper."""
+        for limit, step in ((1024, 32), (2048, 16)):
             if n <= limit:
                 return -(-n // step) * step
         return -(-n // 256) * 256
@@ -444,13 +449,13 @@ class ModelRunner:
         bucket = self._token_bucket(portion_tokens)
         bound = ((longest + 511) // 512) * 512 if longest <= 8192 else 1 << (longest - 1).bit_length()
         bound = min(bound, max(self.model.max_positions, longest))
-        # Padded steps up to max_graph_tokens (beyond it the padding's work costs more than the host's launches); steps
-        # that fill their bucket exactly (the portions of a long prompt under a token budget) up to eight times that.
-        limit = self.max_graph_tokens * (8 if bucket == portion_tokens else 1)
-        if bucket > min(limit, bound):                      # (the padding sequence's positions stay below the bound)
+        # Padded steps up to max_graph_tokens; steps that fill their bucket exactly (the portions of a long prompt under a
+        # token budget) up to four times that.
+        limit = self.max_graph_tokens * (4 if bucket == portion_tokens else 1)
+        if bucket > limit or bucket - portion_tokens > bound:   # (the padding sequence's positions stay below the bound)
             return None
         rows = self._bucket(singles) if singles else 0
-        wanted = max(self._bucket(asked), asked) if asked else 0
+        wanted = 0 if not asked else self._bucket(asked) if asked <= self.MAX_GRAPH_LOGITS else self._token_bucket(asked)
         # The portions' own contexts, as far as the attention's launch depends on them: nothing below 1024 (no
         # partitions of keys there), else a power of two.
         portion_context = 0 if longest_portion < 1024 else min(bound, 1 << (longest_portion - 1).bit_length())
@@ -547,9 +552,9 @@ class ModelRunner:
             ctx.launch_cache[akey] = entry["static"][lay["offsets"][base + j]: lay["offsets"][base + j] + lay["sizes"][base + j]]
         return ctx
 
-    def _capture_prompt_graph(self, entry: dict) -> None:
+    def _capture_prompt_graph(self, entry: dict):
         """Warm-up and capture on a batch of the graph's shape that writes nothing: empty single-token rows and
-        portions that are all padding."""
+        portions that are all padding.  Returns the key of the graph that had to go for it, or None."""
         _, rows, portions, bucket, wanted, bound, _ = entry["key"]
         lay = entry["layout"]
         view, offsets, sizes, S, T = entry["view"], lay["offsets"], lay["sizes"], lay["S"], lay["T"]
@@ -571,17 +576,21 @@ class ModelRunner:
         ctx = self._prompt_context(entry)
         stream = torch.cuda.Stream(device=self.device)
         stream.wait_stream(torch.cuda.current_stream(self.device))
+        # Many logits (a text that is scored) are made behind the replay, for the wanted rows alone and into memory of their own: in the graph
+        # they would be copied out of it and padded (603 rows of 128,256: 113 us for the copy).
+        apart = wanted > self.MAX_GRAPH_LOGITS
+        forward = (lambda: self.model.forward(ctx, self.kv, self.states, rows_only=True)) if apart else (lambda: self.model.forward(ctx, self.kv, self.states))
         with torch.cuda.stream(stream):
-            self.model.forward(ctx, self.kv, self.states)
+            forward()
         torch.cuda.current_stream(self.device).wait_stream(stream)
         torch.cuda.synchronize(self.device)
         if self._graph_pool is None:
             self._graph_pool = torch.cuda.graph_pool_handle()
         graph = torch.cuda.CUDAGraph()
         with torch.cuda.graph(graph, stream=stream, pool=self._graph_pool):
-            logits = self.model.forward(ctx, self.kv, self.states)
-        entry.update(graph=graph, logits=logits, ctx=ctx)
-        self._graphs.put(entry["key"], entry)
+            result = forward()
+        entry.update(graph=graph, ctx=ctx, **{"head_rows" if apart else "logits": result})
+        return self._graphs.put(entry["key"], entry)
 
     def _prompt_graph_step(self, key, entries: list, borrow: bool) -> torch.Tensor | None:
         entry = self._graphs.get(key)
@@ -592,13 +601,17 @@ class ModelRunner:
                     self._sightings.clear()
                 return None                                 # run it eagerly this time
             entry = self._new_prompt_graph(key)
-            self._capture_prompt_graph(entry)
+            evicted = self._capture_prompt_graph(entry)
+            if evicted is not None:                         # (more shapes in use than there is room for: a capture costs a dozen steps, so its
+                self._sightings[evicted] = self.graph_after_sightings - 16     #  shape waits for as many before it takes another's place)
         else:
             entry["copied"].synchronize()
         n_want = self._stage_prompt_graph(entry, entries)
         entry["static"].copy_(entry["pinned"], non_blocking=True)
         entry["copied"].record()
         entry["graph"].replay()
+        if "head_rows" in entry:
+            return self.model.logits(entry["head_rows"][:n_want])
         logits = entry["logits"][:n_want]
         return logits if borrow else logits.clone()
 

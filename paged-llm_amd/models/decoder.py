@@ -9,6 +9,7 @@ from ..cache.kv_cache import CacheGroup
 from ..csrc import ops
 from ..parts import registry
 from ..parts.base import name_under, tensor_name
+from ..parts.norm import rows_of
 from ..parts.registry import BuildEnv
 from ..parts.spec import ModelSpec, WeightSpec
 
@@ -129,9 +130,9 @@ class DecoderModel:
         return out
 
     # ------------------------------------------------------------------ compute
-    def forward(self, ctx, kv_storage, states: dict) -> torch.Tensor:
+    def forward(self, ctx, kv_storage, states: dict, rows_only: bool = False) -> torch.Tensor:
         """Float logits [n, vocab] at ctx.logits_index (empty tensor when nothing is wanted;
-        the layers still run to fill the cache)."""
+        the layers still run to fill the cache).  ``rows_only``: the rows that the head takes, for ``logits``."""
         assert self._ready, "weights not loaded"
         stateful_embedding = hasattr(self.embedding, "forward_step")
         schedule = self.spec.schedule
@@ -191,4 +192,8 @@ class DecoderModel:
         if n == 0:
             return torch.empty((0, self.spec.vocab_size), dtype=torch.float32, device=self.device)
         h = self.final_norm.pending(x, delta, ctx.logits_index, write_residual=False)
-        return self.head.forward(h)
+        return rows_of(h) if rows_only else self.head.forward(h)
+
+    def logits(self, rows: torch.Tensor) -> torch.Tensor:
+        """The logits of rows that ``forward`` gave with ``rows_only``."""
+        return self.head.forward(rows)
