@@ -152,24 +152,46 @@ __device__ __forceinline__ float group_sum(float v) {      // the same four term
 // Partials of one (token, head, partition): [m (log2 units), l, acc[D]].
 constexpr int kPartialFloats = D + 2;
 
+// Decode attention: a workgroup per (sequence, kv head, partition of the keys).  What bounds it is how many of a compute unit's loads
+// are under way: a wavefront asks for its next block of 64 keys before it computes one (head sizes up to 64), and nothing may stand
+// between that and the wait for the older block's loads, which counts the younger ones, that would make the compiler wait for all (a
+// branch around a load, or a loop with a second exit; with both of them in, each block was waited for with the next one's loads in
+// flight behind it: 16 sequences x 4 kv heads of 64 x 2,048 keys in one piece 23.0 us against 17.9, 64 x 4 x 1,024 20.9 against 17.9, 16 x 2 kv
+// heads of 256 x 1,000 ragged in four partitions 22.6 against 17.5).
+//
+// Which of at most 64 sequences workgroup row z takes where a compute unit gets several of unequal length (per_round > 0: rows that reach
+// all compute units once): the rounds take them by length, the first one its shortest first, every other one its longest, so
+// that a compute unit with a long one gets a short one with it (the order costs about 1 us: every wavefront reads all lengths and
+// counts the longer ones).
+__device__ __forceinline__ int sequence_in_turn(const int* __restrict__ seq_lens_k, int num_seqs, int z, int per_round) {
+  const int lane = threadIdx.x & 63;
+  const unsigned key = lane < num_seqs ? ((unsigned)seq_lens_k[lane] << 6) + 63 - lane : 0;      // (no two alike)
+  int longer = 0;
+#pragma unroll
+  for (int j = 0; j < 64; ++j) longer += (unsigned)__builtin_amdgcn_readlane(key, j) > key;
+  const int round = z / per_round, first = round * per_round;
+  const int rank = round & 1 ? z : min(first + per_round, num_seqs) - 1 - (z - first);
+  return __builtin_ctzll(__ballot(lane < num_seqs && longer == rank));
+}
+
 template <int NCB, int WAVES>
-__global__ __launch_bounds__(WAVES * 64) void paged_attention_mfma_kernel(
+__global__ __launch_bounds__(WAVES * 64, NCB == 1 && D <= 64 ? 2 : 1) void paged_attention_mfma_kernel(
     const bf16* __restrict__ q, int q_stride, const bf16* __restrict__ k_pages, const bf16* __restrict__ v_pages,
     bf16* __restrict__ out, int out_stride, const int* __restrict__ block_tables, int bt_stride,
     const int* __restrict__ cu_seqlens_q, const int* __restrict__ seq_lens_k, int num_heads, int num_kv_heads,
-    int block_size, float scale, int window, int partition_size, int num_partitions, float* __restrict__ partials PLLM_TERMS_PARAM) {
+    int block_size, float scale, int window, int partition_size, int num_partitions, float* __restrict__ partials, int per_round PLLM_TERMS_PARAM) {
   // Fetch all arguments in one go (left alone, the compiler fetches each where it is first used, and every fetch is
   // a wait of its own in the chain lengths -> page table -> keys).
   constexpr bool kLookupsTogether = D <= 64;
   if constexpr (kLookupsTogether)
     asm volatile("" ::"s"(q), "s"(q_stride), "s"(k_pages), "s"(v_pages), "s"(out), "s"(out_stride), "s"(block_tables), "s"(bt_stride),
                  "s"(cu_seqlens_q), "s"(seq_lens_k), "s"(num_heads), "s"(num_kv_heads), "s"(block_size), "s"(scale), "s"(window),
-                 "s"(partition_size), "s"(num_partitions), "s"(partials));
+                 "s"(partition_size), "s"(num_partitions), "s"(partials), "s"(per_round));
   // The wavefront's index is the same in all its lanes; saying so keeps everything derived from it (key ranges,
   // page-table entries, page addresses) in scalar registers.
   const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), r = lane & 15, g = lane >> 4;
   const int bs_shift = __builtin_ctz(block_size);              // pages hold a power of two of positions
-  const int seq = blockIdx.z;
+  const int seq = WAVES > 1 && per_round > 0 ? sequence_in_turn(seq_lens_k, gridDim.z, blockIdx.z, per_round) : blockIdx.z;
   const int kvh = blockIdx.y / num_partitions, part = blockIdx.y - kvh * num_partitions;
   const int G = num_heads / num_kv_heads;
   const int q_begin = as_constant(cu_seqlens_q)[seq], num_q = as_constant(cu_seqlens_q)[seq + 1] - q_begin;
@@ -254,12 +276,12 @@ __global__ __launch_bounds__(WAVES * 64) void paged_attention_mfma_kernel(
   struct KVBlock {
     bf16x8 k[4][KSTEPS];
     bf16x4 v[4][DBLOCKS];
-    bool on[4];
   };
   const int last_tile = (k_hi - 1) & ~15;
+  // The four tiles' page-table entries first, together (a tile past the range is the range's last tile once more, so no entry past the
+  // context is read, and there is no branch around a load: behind one the compiler can no longer count which loads
+  // are under way and waits for all, the next block's with them).
   auto load_block = [&](KVBlock& blk, int n0) {
-    // The four tiles' page-table entries first, together (a tile past the range looks the range's last tile up
-    // again, so no entry past the context is read): one wait, not one per tile.
     int pages[4];
 #pragma unroll
     for (int kt = 0; kt < 4; ++kt) pages[kt] = bt[min(n0 + kt * 16, last_tile) >> bs_shift];
@@ -269,12 +291,8 @@ __global__ __launch_bounds__(WAVES * 64) void paged_attention_mfma_kernel(
     if constexpr (kLookupsTogether) asm volatile("" ::"s"(pages[0]), "s"(pages[1]), "s"(pages[2]), "s"(pages[3]));
 #pragma unroll
     for (int kt = 0; kt < 4; ++kt) {
-      const int nk = n0 + kt * 16;
-      blk.on[kt] = nk < k_hi;                                   // uniform
-      if (!blk.on[kt]) continue;
-      const int page = pages[kt];
-      const int off = nk & (block_size - 1);
-      const size_t base = (size_t)page * page_stride + (size_t)kvh * page_elems;
+      const int off = min(n0 + kt * 16, last_tile) & (block_size - 1);
+      const size_t base = (size_t)pages[kt] * page_stride + (size_t)kvh * page_elems;
       const bf16* krow = k_pages + base + (size_t)(off + r) * D;
 #pragma unroll
       for (int s = 0; s < KSTEPS; ++s) {
@@ -296,7 +314,6 @@ __global__ __launch_bounds__(WAVES * 64) void paged_attention_mfma_kernel(
     for (int kt = 0; kt < 4; ++kt) {
 #pragma unroll
       for (int cb = 0; cb < NCB; ++cb) s_t[kt][cb] = floatx4{0.f, 0.f, 0.f, 0.f};
-      if (!blk.on[kt]) continue;
 #pragma unroll
       for (int s = 0; s < KSTEPS; ++s)
 #pragma unroll
@@ -309,7 +326,6 @@ __global__ __launch_bounds__(WAVES * 64) void paged_attention_mfma_kernel(
 #pragma unroll
     for (int cb = 0; cb < NCB; ++cb) {
       float sc[4][4];
-      float mx = -INFINITY;
       float mul = sl2;
       if constexpr (kForms) {
         if (form.any()) {
@@ -329,16 +345,22 @@ __global__ __launch_bounds__(WAVES * 64) void paged_attention_mfma_kernel(
 #pragma unroll
       for (int kt = 0; kt < 4; ++kt)
 #pragma unroll
-        for (int i = 0; i < 4; ++i) {
-          float v = s_t[kt][cb][i] * mul;
-          if (!interior) {
+        for (int i = 0; i < 4; ++i) sc[kt][i] = s_t[kt][cb][i] * mul;
+      if (!interior) {
+        const int end = min(k_hi, my_qpos[cb] + 1);
+#pragma unroll
+        for (int kt = 0; kt < 4; ++kt)
+#pragma unroll
+          for (int i = 0; i < 4; ++i) {
             const int n = n0 + kt * 16 + g * 4 + i;
-            const bool vis = blk.on[kt] && n <= my_qpos[cb] && n >= my_first[cb];
-            v = vis ? v : -INFINITY;
+            sc[kt][i] = (n < end) & (n >= my_first[cb]) ? sc[kt][i] : -INFINITY;
           }
-          sc[kt][i] = v;
-          mx = fmaxf(mx, v);
-        }
+      }
+      float mx = -INFINITY;
+#pragma unroll
+      for (int kt = 0; kt < 4; ++kt)
+#pragma unroll
+        for (int i = 0; i < 4; ++i) mx = fmaxf(mx, sc[kt][i]);
       mx = group_max(mx);
       const float m_new = fmaxf(m_run[cb], mx);
       const float m_safe = (m_new == -INFINITY) ? 0.f : m_new;  // a column that has seen nothing yet
@@ -359,32 +381,25 @@ __global__ __launch_bounds__(WAVES * 64) void paged_attention_mfma_kernel(
     }
 
     // ---- O^T += V^T P^T : A operand = 16 channels x 32 keys (k slots 0-3: tile 2a, 4-7: tile 2a+1)
+    if (!interior) {
+#pragma unroll
+      for (int kt = 0; kt < 4; ++kt)
+#pragma unroll
+        for (int i = 0; i < 4; ++i) {
+          const int n = n0 + kt * 16 + g * 4 + i;
+          const bool out_of_range = (n >= k_hi) | (n < vis_lo);
+#pragma unroll
+          for (int db = 0; db < DBLOCKS; ++db)
+            if (out_of_range) blk.v[kt][db][i] = (__bf16)0.0f;
+        }
+    }
 #pragma unroll
     for (int a = 0; a < 2; ++a) {
-      if (!blk.on[2 * a]) continue;
 #pragma unroll
       for (int db = 0; db < DBLOCKS; ++db) {
         bf16x8 vreg;
 #pragma unroll
-        for (int h = 0; h < 2; ++h) {
-          const int kt = 2 * a + h;
-          bf16x4 v4;
-          if (blk.on[kt]) {
-            v4 = blk.v[kt][db];
-            if (!interior) {
-#pragma unroll
-              for (int i = 0; i < 4; ++i) {
-                const int n = n0 + kt * 16 + g * 4 + i;
-                if (n >= vis_hi || n < vis_lo) v4[i] = (__bf16)0.0f;
-              }
-            }
-          } else {
-#pragma unroll
-            for (int i = 0; i < 4; ++i) v4[i] = (__bf16)0.0f;
-          }
-#pragma unroll
-          for (int i = 0; i < 4; ++i) vreg[h * 4 + i] = v4[i];
-        }
+        for (int i = 0; i < 8; ++i) vreg[i] = blk.v[2 * a + (i >> 2)][db][i & 3];
 #pragma unroll
         for (int cb = 0; cb < NCB; ++cb)
           acc[cb][db] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(vreg, p_op[a][cb], acc[cb][db], 0, 0, 0);
@@ -398,25 +413,26 @@ __global__ __launch_bounds__(WAVES * 64) void paged_attention_mfma_kernel(
   // Registers of one block: with small heads two blocks fit and the next one travels while the current
   // one is used; with large heads one block is all there is room for (the caller then sizes partitions
   // so that a wavefront has a single block).
-  constexpr bool kTwoBlocks = 4 * KSTEPS * 4 + 4 * DBLOCKS * 2 <= 64;
+  constexpr bool kTwoBlocks = 4 * KSTEPS * 4 + 4 * DBLOCKS * 2 <= 64 && (NCB < 4 || WAVES < 8);
   if constexpr (WAVES > 1 && kTwoBlocks) {
     KVBlock blk_a, blk_b;
     int n0 = k_lo + wave * 64;
     if (n0 < k_hi) {
       load_block(blk_a, n0);
-      while (true) {
-        const int n1 = n0 + kStride;
-        const bool has1 = n1 < k_hi;
-        if (has1) load_block(blk_b, n1);
+      // (the next block's loads are behind no condition either)
+      for (; n0 + 2 * kStride < k_hi; n0 += 2 * kStride) {
+        load_block(blk_b, n0 + kStride);
         compute_block(blk_a, n0);
-        if (!has1) break;
-        const int n2 = n1 + kStride;
-        const bool has2 = n2 < k_hi;
-        if (has2) load_block(blk_a, n2);
-        compute_block(blk_b, n1);
-        if (!has2) break;
-        n0 = n2;
+        load_block(blk_a, n0 + 2 * kStride);
+        compute_block(blk_b, n0 + kStride);
       }
+      if (n0 + kStride < k_hi) {
+        load_block(blk_b, n0 + kStride);
+        compute_block(blk_a, n0);
+        blk_a = blk_b;
+        n0 += kStride;
+      }
+      compute_block(blk_a, n0);
     }
   } else {
     KVBlock blk;
@@ -1090,7 +1106,7 @@ static int launch_attention(const void* q, int q_stride, const void* k_pages, co
                             const int* seq_lens_k, int num_seqs, int total_q, int max_q_len, int num_heads,
                             int num_kv_heads, int block_size, float scale, int window, int partition_size,
                             int num_partitions, float* partials, int waves, int column_blocks, const int* work_list, int num_work,
-                            int single_prompt, [[maybe_unused]] ScoreTerms terms, hipStream_t stream) {
+                            int single_prompt, int longest, [[maybe_unused]] ScoreTerms terms, hipStream_t stream) {
   if (total_q <= 0 || num_seqs <= 0) return 0;
   if (num_kv_heads <= 0 || num_heads % num_kv_heads) return -2;
   const int G = num_heads / num_kv_heads;
@@ -1156,6 +1172,13 @@ static int launch_attention(const void* q, int q_stride, const void* k_pages, co
     return (int)hipGetLastError();
   }
   dim3 grid(tiles, num_kv_heads * num_partitions, num_seqs), block(64 * waves);
+  // Sequences by length where the workgroups are more than the compute units and the longest may take a while (ragged contexts up to
+  // 2,000, us, as given / by length: 61 sequences x 8 kv heads of 64 38.3 / 31.3, 40 31.4 / 25.4 with eight wavefronts, 61 x 8 of 128 69.1 / 57.3;
+  // 64 up to 600 13.5 / 13.6, all of 2,000 58.8 / 58.7; with a compute unit for every workgroup the order only costs: 33 x 4 up to 1,200 12.7 / 13.8).
+  const int cus = num_compute_units();
+  const bool by_length = waves > 1 && partition_size == 0 && tiles == 1 && longest > 512 && longest < 1 << 24 && num_seqs <= 64 &&
+                         num_kv_heads <= cus && num_seqs * num_kv_heads > cus;
+  const int per_round = by_length ? cus / num_kv_heads : 0;
   const size_t lds = waves > 1 ? merge_lds_bytes(ncb, waves) : 0;
 #define PLLM_LAUNCH(NCB_, WAVES_)                                                                                                    \
   do {                                                                                                                               \
@@ -1166,7 +1189,7 @@ static int launch_attention(const void* q, int q_stride, const void* k_pages, co
     }                                                                                                                                \
     hipLaunchKernelGGL(kern, grid, block, lds, stream, (const bf16*)q, q_stride, (const bf16*)k_pages, (const bf16*)v_pages,         \
                        (bf16*)out, out_stride, block_tables, bt_stride, cu_seqlens_q, seq_lens_k, num_heads, num_kv_heads,           \
-                       block_size, scale, window, partition_size, num_partitions, partials PLLM_TERMS_ARG);                          \
+                       block_size, scale, window, partition_size, num_partitions, partials, per_round PLLM_TERMS_ARG);               \
   } while (0)
 #define PLLM_BY_WAVES(NCB_)                                                                          \
   do {                                                                                               \
@@ -1199,10 +1222,11 @@ PLLM_API int pllm_paged_attention_mfma(const void* q, int q_stride, const void* 
                                        hipStream_t stream) {
   return launch_attention(q, q_stride, k_pages, v_pages, out, out_stride, block_tables, bt_stride, cu_seqlens_q, seq_lens_k, num_seqs,
                           total_q, max_q_len, num_heads, num_kv_heads, block_size, scale, window, partition_size, num_partitions,
-                          partials, waves, column_blocks, work_list, num_work, 0, ScoreTerms{0.f, nullptr, nullptr}, stream);
+                          partials, waves, column_blocks, work_list, num_work, 0, 0, ScoreTerms{0.f, nullptr, nullptr}, stream);
 }
 
-// The same with a hint for the prompt kernel's form (single_prompt: all queries but a few belong to one sequence) and
+// The same with a hint for the prompt kernel's form (single_prompt: all queries but a few belong to one sequence), a bound on any sequence's keys (longest; 0:
+// unknown; the results do not depend on it) and
 // with further terms of the score: score_cap > 0 caps the scaled products (c tanh(x / c)), slopes [heads]
 // adds slope * (key position - query position), sinks [heads] gives every head a logit that takes part in the
 // softmax's sum only (null: none).  A library refuses the terms it was compiled without.
@@ -1213,13 +1237,13 @@ PLLM_API int pllm_paged_attention_mfma_terms(const void* q, int q_stride, const 
                                              const int* seq_lens_k, int num_seqs, int total_q, int max_q_len, int num_heads,
                                              int num_kv_heads, int block_size, float scale, int window, int partition_size,
                                              int num_partitions, float* partials, int waves, int column_blocks, const int* work_list,
-                                             int num_work, int single_prompt, float score_cap, const float* slopes, const float* sinks,
+                                             int num_work, int single_prompt, int longest, float score_cap, const float* slopes, const float* sinks,
                                              hipStream_t stream) {
   const ScoreTerms given{score_cap, slopes, sinks};
   if (!(score_cap >= 0.f) || (given.any() && !kTerms) || ((score_cap > 0.f || slopes) && !kForms)) return -2;
   return launch_attention(q, q_stride, k_pages, v_pages, out, out_stride, block_tables, bt_stride, cu_seqlens_q, seq_lens_k, num_seqs,
                           total_q, max_q_len, num_heads, num_kv_heads, block_size, scale, window, partition_size, num_partitions,
-                          partials, waves, column_blocks, work_list, num_work, single_prompt, given, stream);
+                          partials, waves, column_blocks, work_list, num_work, single_prompt, longest, given, stream);
 }
 
 // What the library that holds the no-allocation entry point needs from this one (see attention_noalloc.h): the head
