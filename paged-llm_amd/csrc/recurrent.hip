@@ -736,10 +736,10 @@ __global__ __launch_bounds__(64 * WAVES, 2) void recurrence_piece_kernel(Recurre
     if (!kOut) __syncthreads();
     if (!last) fetch(t0 + kPiece);
 
-    // Thread n < NP walks the tokens forward (queries), thread NP + n backward (keys).
-    for (int who = tid; who < 2 * NP; who += kThreads) {
-      const int n = who % NP;
-      if (who < NP) {
+    // Four walks along the tokens, a row a thread: late queries and the piece's product forward, all keys and early keys backward.
+    for (int who = tid; who < 4 * NP; who += kThreads) {
+      const int n = who % NP, walk = who / NP;
+      if (walk == 0) {
         if (kOut) {
           float from16 = 1.f;
 #pragma unroll 4
@@ -748,28 +748,28 @@ __global__ __launch_bounds__(64 * WAVES, 2) void recurrence_piece_kernel(Recurre
             Q2[(t - kPiece / 2) * LD + n] = Q[t * LD + n] * from16;
           }
         }
+      } else if (walk == 1) {
         float all = 1.f;
 #pragma unroll 4
         for (int t = 0; t < kPiece; ++t) all *= DR[t * LD + n];
         gC[n] = all;
-      } else {
+      } else if (walk == 2) {
         float behind = 1.f;
 #pragma unroll 4
         for (int t = kPiece - 1; t >= 0; --t) {
           KT[token_quad(n, t >> 2) + (t & 3)] = K[t * LD + n] * behind * gs[t];
           behind *= DR[t * LD + n];
         }
-        if (kOut) {
-          float to15 = 1.f;
+      } else if (kOut) {
+        float to15 = 1.f;
 #pragma unroll 4
-          for (int t = kPiece / 2 - 1; t >= 0; --t) {
-            K2[t * LD + n] = K[t * LD + n] * to15;
-            to15 *= DR[t * LD + n];
-          }
+        for (int t = kPiece / 2 - 1; t >= 0; --t) {
+          K2[t * LD + n] = K[t * LD + n] * to15;
+          to15 *= DR[t * LD + n];
         }
       }
     }
-    if constexpr (kOut) {
+    if constexpr (kOut && NT == 2) {
       // The tiles of M on the diagonal: sixteen lanes share a key, NT of its rows each.
       for (int who = tid; who < 512; who += kThreads) {
         const int j = who >> 4, n = (who & 15) * NT, stop = (j & 16) + 16;
@@ -792,6 +792,53 @@ __global__ __launch_bounds__(64 * WAVES, 2) void recurrence_piece_kernel(Recurre
           if ((who & 15) == 0) M[t * kPieceLd + j] = dot * gs[j];
         }
       }
+    }
+    if constexpr (kOut && NT > 2) {
+      // The same with a wavefront's lanes along the rows and four of a tile's keys at a time, every fourth one: a token's decays and queries are
+      // read once for four keys (with sixteen lanes to a key all wavefronts read them for every key: 18,000 of a piece's 42,000 clocks;
+      // 777 tokens, 16 heads of 128 x 128: 441 us then, 338 so).  Rows up to 32 would leave half the lanes idle and keep the other form.
+      constexpr int kRows = NP / 64;
+      for (int four = wave; four < 8; four += WAVES) {
+        const int first = (four >> 2) * 16, j0 = first + (four & 3), n = lane * kRows;
+        float w[4][kRows];
+#pragma unroll
+        for (int k = 0; k < 4; ++k)
+#pragma unroll
+          for (int i = 0; i < kRows; ++i) w[k][i] = K[(j0 + 4 * k) * LD + n + i];
+        const int mine = j0 + ((quad & 1) * 2 + (quad >> 1)) * 4;      // the key whose sum this lane gets
+        const float g = gs[mine];
+#pragma unroll 4
+        for (int t = first; t < first + 16; ++t) {
+          float d[kRows], q[kRows], dot[4];
+#pragma unroll
+          for (int i = 0; i < kRows; ++i) { d[i] = DR[t * LD + n + i]; q[i] = Q[t * LD + n + i]; }
+#pragma unroll
+          for (int k = 0; k < 4; ++k) {
+            const int j = j0 + 4 * k;                                  // (the same for all lanes)
+            dot[k] = 0.f;
+#pragma unroll
+            for (int i = 0; i < kRows; ++i) {
+              w[k][i] = t > j ? w[k][i] * d[i] : w[k][i];
+              dot[k] = fmaf(w[k][i], q[i], dot[k]);
+            }
+            dot[k] = t >= j ? dot[k] : 0.f;
+          }
+          // (sums of keys 0, 2, 1, 3 in the four rows of lanes)
+          auto halves = [](float x, float y) {
+            const auto r = __builtin_amdgcn_permlane32_swap(__float_as_uint(x), __float_as_uint(y), false, false);
+            return __uint_as_float(r[0]) + __uint_as_float(r[1]);
+          };
+          const auto rows = __builtin_amdgcn_permlane16_swap(__float_as_uint(halves(dot[0], dot[1])), __float_as_uint(halves(dot[2], dot[3])), false, false);
+          float sum = __uint_as_float(rows[0]) + __uint_as_float(rows[1]);
+          sum += dpp_move<kDppSwap1>(sum);
+          sum += dpp_move<kDppSwap2>(sum);
+          sum += dpp_move<kDppHalfMirror>(sum);
+          sum += dpp_move<kDppMirror>(sum);
+          if (c16 == 0) M[t * kPieceLd + mine] = sum * g;
+        }
+      }
+    }
+    if constexpr (kOut) {
       __syncthreads();
       for (int n = tid; n < NP; n += kThreads) {                     // (the diagonal is done with the plain queries)
         float all = 1.f;
