@@ -100,67 +100,82 @@ __global__ __launch_bounds__(256) void causal_conv_kernel(
   }
 }
 
+template <typename T> struct alignas(4 * sizeof(T)) Quad { T v[4]; };
+
 constexpr int kConvFours = 8;      // tokens of a workgroup of the kernel below
 
 // The same with four taps and four neighbouring channels a thread, for portions in chunks.  The workgroups of a sequence's first chunk,
 // which alone read the state, leave the new one.
 // What bounds it: memory, and the exact SiLU's vector instructions (8 us of them at 2,048 tokens x 4,352 channels).  A thread's loads are
 // 8 bytes (float rows 16) instead of 2, all of its tokens' under way at once, no tap is asked whether it is there, and no second kernel
-// leaves the state.  us with what leaves the state: 2,048 tokens x 4,352 channels 28 -> 17.4 (16 tokens a workgroup 20.8), 8 x 512 tokens
-// 44 -> 26, 1,178 x 2,048 13.1 -> 8.8, 777 x 1,024 10.9 -> 7.6.  From 256 tokens on (100 tokens 11.0 and 11.2), and not beside more than
-// a sixteenth as many sequences, where most workgroups have no tokens (65 tokens and 100 single ones 11.3 and 12.5).
+// leaves the state.  us with what leaves the state, by channels and so: 2,048 tokens x 4,352 channels 28 and 15.4, 8 x 512 tokens
+// 44 and 23.5.  Before its loads were asked for at once it took 17.4 there (16 tokens a workgroup 20.8), 1,178 x 2,048 13.1 and 8.8,
+// 777 x 1,024 10.9 and 7.6; and the line was drawn: from 256 tokens on (100 tokens 11.0 and 11.2), and not beside more than a sixteenth as
+// many sequences, where most workgroups have no tokens (65 tokens and 100 single ones 11.3 and 12.5).
 template <typename T>
 __global__ __launch_bounds__(256) void causal_conv4_kernel(
     const T* __restrict__ in, int in_stride, const float* __restrict__ w, const float* __restrict__ bias,
     float* state, size_t slot_stride, const int* __restrict__ state_slots,
     const int* __restrict__ seq_starts, const int* __restrict__ cu_seqlens, T* __restrict__ out, int out_stride, int channels, int act) {
   constexpr int kTaps = 4, V = 4;
-  struct alignas(V * sizeof(T)) Four { T v[V]; };
   const int c = (blockIdx.x * blockDim.x + threadIdx.x) * V;
   const int seq = blockIdx.y, t0 = blockIdx.z * kConvFours;
-  const int q_begin = cu_seqlens[seq], q_len = cu_seqlens[seq + 1] - q_begin;
-  if (c >= channels || (t0 >= q_len && t0 > 0)) return;
+  const int q_begin = cu_seqlens[seq], q_len = cu_seqlens[seq + 1] - q_begin, slot = state_slots[seq];
+  const bool first = t0 == 0, carried = seq_starts[seq] > 0;
+  if (c >= channels || (t0 >= q_len && !first)) return;
+  float* st = state + (size_t)slot * slot_stride + (size_t)c * (kTaps - 1);
+  if (q_len <= 0) {                                                    // no tokens: only an empty state is left
+    if (!carried)
+      for (int i = 0; i < V * (kTaps - 1); ++i) st[i] = 0.f;
+    return;
+  }
   const int count = min(kConvFours, q_len - t0);
   const T* rows = in + (size_t)(q_begin + t0) * in_stride + c;
-  Four fetched[kConvFours];
+  // Everything that memory holds for this thread is asked for before anything is used (rows that are not there as their neighbours): with the
+  // inputs before the first, the weights and the bias each behind a wait of their own, 2,048 x 4,352 took 18.0 us and not 15.4.
+  Quad<T> fetched[kConvFours], before[kTaps - 1];
 #pragma unroll
-  for (int u = 0; u < kConvFours; ++u)
-    if (u < count) fetched[u] = *reinterpret_cast<const Four*>(rows + (size_t)u * in_stride);
-  float wj[V][kTaps], win[V][kTaps - 1], b[V];
-  float* st = state + (size_t)state_slots[seq] * slot_stride + (size_t)c * (kTaps - 1);
-  const bool carried = seq_starts[seq] > 0;
+  for (int u = 0; u < kConvFours; ++u) fetched[u] = *reinterpret_cast<const Quad<T>*>(rows + (size_t)min(u, count - 1) * in_stride);
 #pragma unroll
-  for (int j = 0; j < kTaps - 1; ++j) {
-    const int rel = t0 - (kTaps - 1) + j;                              // token of this step (>= 0) or an input of earlier steps (< 0)
-    Four before;
-    if (rel >= 0) before = *reinterpret_cast<const Four*>(rows + (j - (kTaps - 1)) * (ptrdiff_t)in_stride);
+  for (int j = 0; j < kTaps - 1; ++j) before[j] = *reinterpret_cast<const Quad<T>*>(rows + (first ? 0 : j - (kTaps - 1)) * (ptrdiff_t)in_stride);
+  float wj[V][kTaps], win[V][kTaps - 1], b[V] = {0.f, 0.f, 0.f, 0.f};
 #pragma unroll
-    for (int v = 0; v < V; ++v) win[v][j] = rel >= 0 ? to_f32(before.v[v]) : carried ? st[v * (kTaps - 1) + (kTaps - 1) + rel] : 0.f;
-  }
-  if (t0 == 0) {
-#pragma unroll
-    for (int j = 0; j < kTaps - 1; ++j) {
-      const int rel = q_len - (kTaps - 1) + j;                         // (below 0: the carried input that many places on)
-      Four late;
-      if (rel >= 0) late = *reinterpret_cast<const Four*>(rows + (size_t)rel * in_stride);
-#pragma unroll
-      for (int v = 0; v < V; ++v) {
-        float x = q_len <= 0 ? win[v][j] : 0.f;
-        if (rel >= 0) x = to_f32(late.v[v]);
-        else if (q_len > 0 && j + q_len < kTaps - 1) x = q_len == 1 ? win[v][j + 1 < kTaps - 1 ? j + 1 : 0] : win[v][j + 2 < kTaps - 1 ? j + 2 : 0];
-        st[v * (kTaps - 1) + j] = x;
-      }
-    }
-  }
-#pragma unroll
-  for (int v = 0; v < V; ++v) {
-    b[v] = bias ? bias[c + v] : 0.f;
+  for (int v = 0; v < V; ++v)
 #pragma unroll
     for (int j = 0; j < kTaps; ++j) wj[v][j] = w[(size_t)(c + v) * kTaps + j];
+  if (bias) {
+#pragma unroll
+    for (int v = 0; v < V; ++v) b[v] = bias[c + v];
+  }
+  if (first) {
+    float held[V][kTaps - 1];
+    Quad<T> late[kTaps - 1];
+#pragma unroll
+    for (int v = 0; v < V; ++v)
+#pragma unroll
+      for (int j = 0; j < kTaps - 1; ++j) held[v][j] = st[v * (kTaps - 1) + j];
+#pragma unroll
+    for (int j = 0; j < kTaps - 1; ++j) late[j] = *reinterpret_cast<const Quad<T>*>(rows + (size_t)max(q_len - (kTaps - 1) + j, 0) * in_stride);
+#pragma unroll
+    for (int v = 0; v < V; ++v) {
+#pragma unroll
+      for (int j = 0; j < kTaps - 1; ++j) win[v][j] = carried ? held[v][j] : 0.f;
+#pragma unroll
+      for (int j = 0; j < kTaps - 1; ++j) {
+        // (the last inputs of this step; with fewer than three the carried ones of one or two places on in front of them)
+        const float kept = q_len == 1 ? win[v][j + 1 < kTaps - 1 ? j + 1 : 0] : win[v][j + 2 < kTaps - 1 ? j + 2 : 0];
+        st[v * (kTaps - 1) + j] = q_len - (kTaps - 1) + j >= 0 ? to_f32(late[j].v[v]) : kept;
+      }
+    }
+  } else {
+#pragma unroll
+    for (int v = 0; v < V; ++v)
+#pragma unroll
+      for (int j = 0; j < kTaps - 1; ++j) win[v][j] = to_f32(before[j].v[v]);
   }
 #pragma unroll
   for (int u = 0; u < kConvFours; ++u) {
-    Four o;
+    Quad<T> o;
 #pragma unroll
     for (int v = 0; v < V; ++v) {
       const float cur = to_f32(fetched[u].v[v]);
@@ -173,7 +188,7 @@ __global__ __launch_bounds__(256) void causal_conv4_kernel(
       win[v][2] = cur;
       o.v[v] = from_f32<T>(act ? silu_f32(acc) : acc);
     }
-    if (u < count) *reinterpret_cast<Four*>(out + (size_t)(q_begin + t0 + u) * out_stride + c) = o;
+    if (u < count) *reinterpret_cast<Quad<T>*>(out + (size_t)(q_begin + t0 + u) * out_stride + c) = o;
   }
 }
 
@@ -1765,8 +1780,6 @@ __global__ __launch_bounds__(256) void gated_group_norm_kernel(const float* __re
 // registers: every value is read once, four channels per lane and load.  Needs group % 4 == 0, rows that start on
 // 16-byte (float) and 8-byte (bfloat16) boundaries, and at most kGroupRegs * 256 channels per wave.
 constexpr int kGroupRegs = 8;
-
-template <typename T> struct alignas(4 * sizeof(T)) Quad { T v[4]; };
 
 template <typename T>
 __global__ __launch_bounds__(256) void gated_group_norm_regs_kernel(const float* __restrict__ y, const T* __restrict__ gate,
