@@ -289,6 +289,46 @@ __global__ void rotary_to_float_kernel(const T* __restrict__ in, int in_stride, 
   }
 }
 
+// The same in quads: a thread turns four pairs, or carries four elements behind the rotated ones over.
+// What bounds it: memory (6 bytes an element from bfloat16: 5 TB/s at 2,048 tokens).  A thread of the kernel above asks for an element's
+// partner again, for 4 bytes of a table and for 2 of a row at a time, behind two divisions.  us by elements and so, queries and keys of 8
+// heads of 256: 2,048 tokens 20.3 and 10.0, 777 9.8 and 5.8, 8 or 1 as long as a launch takes; 16 of 64 in pairs of neighbours, 1,500 tokens
+// 8.7 and 6.2; float rows of 8 of 128, half of it turned, 301 tokens 4.1 and 3.7.
+template <typename T>
+__global__ __launch_bounds__(256) void rotary_to_float_quads_kernel(const T* __restrict__ in, int in_stride, const int* __restrict__ positions,
+                                                                    const float* __restrict__ cos_t, const float* __restrict__ sin_t,
+                                                                    float* __restrict__ out, int heads, int head_dim, int rot_dims, int interleaved,
+                                                                    float scale, int second_at, size_t second_out, float scale2) {
+  const int tok = blockIdx.x;
+  if (blockIdx.y == 1) { in += second_at; out += second_out; scale = scale2; }
+  const int half = rot_dims / 2, turns = half / 4, items = turns + (head_dim - rot_dims) / 4;
+  const T* row = in + (size_t)tok * in_stride;
+  float* orow = out + (size_t)tok * heads * head_dim;
+  const size_t table = (size_t)positions[tok] * half;
+  for (int idx = threadIdx.x; idx < heads * items; idx += blockDim.x) {
+    const int h = idx / items, r = idx - h * items, base = h * head_dim;
+    if (r < turns) {
+      const int at0 = base + (interleaved ? 8 * r : 4 * r), at1 = at0 + (interleaved ? 4 : half);
+      const Quad<T> x0 = *reinterpret_cast<const Quad<T>*>(row + at0), x1 = *reinterpret_cast<const Quad<T>*>(row + at1);
+      const Quad<float> c = *reinterpret_cast<const Quad<float>*>(cos_t + table + 4 * r), s = *reinterpret_cast<const Quad<float>*>(sin_t + table + 4 * r);
+      float lo[4], hi[4];
+#pragma unroll
+      for (int i = 0; i < 4; ++i) {
+        const T even = i < 2 ? x0.v[2 * i & 3] : x1.v[2 * i & 3], odd = i < 2 ? x0.v[(2 * i & 3) + 1] : x1.v[(2 * i & 3) + 1];
+        rotate_pair(to_f32(interleaved ? even : x0.v[i]), to_f32(interleaved ? odd : x1.v[i]), c.v[i], s.v[i], lo[i], hi[i]);
+        lo[i] *= scale;
+        hi[i] *= scale;
+      }
+      *reinterpret_cast<Quad<float>*>(orow + at0) = interleaved ? Quad<float>{lo[0], hi[0], lo[1], hi[1]} : Quad<float>{lo[0], lo[1], lo[2], lo[3]};
+      *reinterpret_cast<Quad<float>*>(orow + at1) = interleaved ? Quad<float>{lo[2], hi[2], lo[3], hi[3]} : Quad<float>{hi[0], hi[1], hi[2], hi[3]};
+    } else {
+      const int at = base + rot_dims + 4 * (r - turns);
+      const Quad<T> x = *reinterpret_cast<const Quad<T>*>(row + at);
+      *reinterpret_cast<Quad<float>*>(orow + at) = Quad<float>{to_f32(x.v[0]) * scale, to_f32(x.v[1]) * scale, to_f32(x.v[2]) * scale, to_f32(x.v[3]) * scale};
+    }
+  }
+}
+
 PLLM_API int pllm_rotary_to_float(int dtype, const void* in, int in_stride, const int* positions, const float* cos_t,
                                   const float* sin_t, float* out, int num_tokens, int heads, int head_dim, int rot_dims,
                                   int interleaved, float scale, int sets, int second_at, long second_out, float scale2,
@@ -296,12 +336,15 @@ PLLM_API int pllm_rotary_to_float(int dtype, const void* in, int in_stride, cons
   if (num_tokens <= 0) return 0;
   if (rot_dims < 0 || rot_dims > head_dim || rot_dims % 2 || sets < 1 || sets > 2) return -2;
   dim3 grid(num_tokens, sets), block(256);
-  if (dtype == PLLM_F32)
-    hipLaunchKernelGGL(rotary_to_float_kernel<float>, grid, block, 0, stream, (const float*)in, in_stride, positions, cos_t, sin_t,
-                       out, heads, head_dim, rot_dims, interleaved, scale, second_at, (size_t)second_out, scale2);
-  else
-    hipLaunchKernelGGL(rotary_to_float_kernel<bf16>, grid, block, 0, stream, (const bf16*)in, in_stride, positions, cos_t, sin_t,
-                       out, heads, head_dim, rot_dims, interleaved, scale, second_at, (size_t)second_out, scale2);
+  // Quads where everything that they load and store lies on their boundaries (figures: above the kernel).
+  const uintptr_t size = dtype == PLLM_F32 ? 4 : 2;
+  const bool quads = rot_dims % 8 == 0 && head_dim % 4 == 0 && in_stride % 4 == 0 && second_at % 4 == 0 && second_out % 4 == 0 &&
+                     (uintptr_t)in % (4 * size) == 0 && ((uintptr_t)out | (uintptr_t)cos_t | (uintptr_t)sin_t) % 16 == 0;
+#define PLLM_ROTARY(KERNEL, T) hipLaunchKernelGGL(KERNEL<T>, grid, block, 0, stream, (const T*)in, in_stride, positions, cos_t, sin_t, \
+                                                  out, heads, head_dim, rot_dims, interleaved, scale, second_at, (size_t)second_out, scale2)
+  if (dtype == PLLM_F32) { if (quads) PLLM_ROTARY(rotary_to_float_quads_kernel, float); else PLLM_ROTARY(rotary_to_float_kernel, float); }
+  else { if (quads) PLLM_ROTARY(rotary_to_float_quads_kernel, bf16); else PLLM_ROTARY(rotary_to_float_kernel, bf16); }
+#undef PLLM_ROTARY
   PLLM_RETURN_LAST_ERROR();
 }
 

@@ -6,6 +6,34 @@ pytestmark = pytest.mark.gpu
 
 
 @pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16])
+@pytest.mark.parametrize("interleaved", [False, True])
+@pytest.mark.parametrize("heads,dim,rot", [(1, 4, 0), (3, 8, 8), (5, 12, 8), (8, 256, 256), (7, 64, 24), (9, 132, 128)])
+def test_rotations_by_quads_are_those_by_elements(heads, dim, rot, interleaved, dtype):
+    """The same bits as by single elements, which rows one column on (off every boundary) still take."""
+    from paged_llm_amd.csrc import ops
+    gen = torch.Generator().manual_seed(dim)
+    T, width = 37, heads * dim
+    rows = torch.randn(T, 2 * width, generator=gen).to(dtype).cuda()
+    off = torch.zeros(T, 2 * width + 4, dtype=dtype, device="cuda")
+    off[:, 1:2 * width + 1] = rows
+    positions = torch.randint(0, 50, (T,), generator=gen, dtype=torch.int32).cuda()
+    angles = torch.rand(50, rot // 2, generator=gen) * 6.0
+    tables = angles.cos().cuda(), angles.sin().cuda()
+    args = (positions, *tables, heads, dim, rot, interleaved, 0.7)
+    got = ops.rotary_to_float(rows, *args, second_at=width, scale2=0.3)
+    assert torch.equal(got, ops.rotary_to_float(off[:, 1:], *args, second_at=width, scale2=0.3))
+    x = rows.cpu().double().view(T, 2, heads, dim).transpose(0, 1)
+    c, s = (t.cpu().double()[positions.cpu().long()][:, None] for t in tables)
+    lo, hi = (x[..., 0:rot:2], x[..., 1:rot:2]) if interleaved else (x[..., :rot // 2], x[..., rot // 2:rot])
+    turned = lo * c - hi * s, hi * c + lo * s
+    want = x.clone()
+    want[..., :rot] = torch.stack(turned, -1).flatten(-2) if interleaved else torch.cat(turned, -1)
+    want *= torch.tensor([0.7, 0.3], dtype=torch.float64).view(2, 1, 1, 1)
+    # (two products, their sum and the scale, each rounded to 24 bits)
+    assert float((got.cpu().double() - want).abs().max()) <= 4 * 2.0 ** -24 * 2 * max(1.0, float(x.abs().max()))
+
+
+@pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16])
 @pytest.mark.parametrize("lens", [[256, 0], [257, 1, 2, 3], [0, 300], [2, 263, 0, 0], [1, 1, 1, 1, 1, 255 + 9]])
 def test_convolutions_of_long_portions_beside_short_and_empty_ones(lens, dtype):
     """Carried and fresh states beside every length below the taps: outputs and what is left, against 64 bits."""
