@@ -1822,9 +1822,13 @@ __global__ __launch_bounds__(256) void gated_group_norm_kernel(const float* __re
 // The same for groups whose channels a wave (or, with fewer groups than waves, a few waves side by side) holds in
 // registers: every value is read once, four channels per lane and load.  Needs group % 4 == 0, rows that start on
 // 16-byte (float) and 8-byte (bfloat16) boundaries, and at most kGroupRegs * 256 channels per wave.
+// All of a group's loads are asked for before the first is used (with the gate's conversion beside each load they waited in turn, and the
+// weights' for the sum): QUADS is the fewest of 1, 2, 4 and 8 that hold a wave's channels.  What bounds it: memory (8 bytes a channel with a
+// bfloat16 gate: 4.1 to 4.5 TB/s at 2,048 rows).  us in turn and at once: 2,048 rows of 4,096 channels 21.2 and 16.5, in groups of 512 20.7
+// and 14.9; 777 of 2,048 in groups of 256 6.1 and 5.7; 301 of 8,192 11.7 and 8.7; 8 of 4,096 6.3 and 4.5.
 constexpr int kGroupRegs = 8;
 
-template <typename T>
+template <typename T, int QUADS>
 __global__ __launch_bounds__(256) void gated_group_norm_regs_kernel(const float* __restrict__ y, const T* __restrict__ gate,
                                                                     int gate_stride, const float* __restrict__ w, T* __restrict__ out,
                                                                     int inner, int group, int gate_first, int gate_act, float eps) {
@@ -1839,24 +1843,32 @@ __global__ __launch_bounds__(256) void gated_group_norm_regs_kernel(const float*
   T* orow = out + (size_t)row * inner;
   for (int g = wave / parts; g < groups; g += 4 / parts) {
     const int base = g * group + (wave % parts) * slice;
-    float u[kGroupRegs][4], s[kGroupRegs][4];
+    Quad<float> yv[QUADS], wv[QUADS];
+    Quad<T> gv[QUADS];
+#pragma unroll
+    for (int j = 0; j < QUADS; ++j) yv[j] = *reinterpret_cast<const Quad<float>*>(yr + base + min((j * 64 + lane) * 4, slice - 4));
+    if (gate_act != kGateNone) {
+#pragma unroll
+      for (int j = 0; j < QUADS; ++j) gv[j] = *reinterpret_cast<const Quad<T>*>(gr + base + min((j * 64 + lane) * 4, slice - 4));
+    }
+    if (w) {
+#pragma unroll
+      for (int j = 0; j < QUADS; ++j)
+#pragma unroll
+        for (int e = 0; e < 4; ++e) wv[j].v[e] = w[base + min((j * 64 + lane) * 4, slice - 4) + e];
+    }
+    float u[QUADS][4], s[QUADS][4];
     float ss = 0.f;
 #pragma unroll
-    for (int j = 0; j < kGroupRegs; ++j) {
-      const int at = (j * 64 + lane) * 4;
-      if (at < slice) {
-        const float4 yv = *reinterpret_cast<const float4*>(yr + base + at);
-        Quad<T> gv;
-        if (gate_act != kGateNone) gv = *reinterpret_cast<const Quad<T>*>(gr + base + at);
-        const float yy[4] = {yv.x, yv.y, yv.z, yv.w};
+    for (int j = 0; j < QUADS; ++j)
+      if ((j * 64 + lane) * 4 < slice) {
 #pragma unroll
         for (int e = 0; e < 4; ++e) {
-          s[j][e] = gate_act == kGateNone ? 1.f : gate_f32(to_f32(gv.v[e]), gate_act);
-          u[j][e] = gate_first ? yy[e] * s[j][e] : yy[e];
+          s[j][e] = gate_act == kGateNone ? 1.f : gate_f32(to_f32(gv[j].v[e]), gate_act);
+          u[j][e] = gate_first ? yv[j].v[e] * s[j][e] : yv[j].v[e];
           ss = fmaf(u[j][e], u[j][e], ss);
         }
       }
-    }
     ss = wave_sum(ss);
     if (parts > 1) {                                       // (then every wave runs this loop exactly once)
       scratch[wave] = ss;
@@ -1866,14 +1878,14 @@ __global__ __launch_bounds__(256) void gated_group_norm_regs_kernel(const float*
     }
     const float inv = 1.f / sqrtf(ss / (float)group + eps);
 #pragma unroll
-    for (int j = 0; j < kGroupRegs; ++j) {
+    for (int j = 0; j < QUADS; ++j) {
       const int at = (j * 64 + lane) * 4;
       if (at < slice) {
         Quad<T> o;
 #pragma unroll
         for (int e = 0; e < 4; ++e) {
           float r = gate_first ? u[j][e] * inv : (u[j][e] * inv) * s[j][e];
-          if (w) r *= w[base + at + e];
+          if (w) r *= wv[j].v[e];
           o.v[e] = from_f32<T>(r);
         }
         *reinterpret_cast<Quad<T>*>(orow + base + at) = o;
@@ -1931,6 +1943,16 @@ static bool group_norm_in_registers(const float* y, const void* gate, int gate_s
          (uintptr_t)y % 16 == 0 && (uintptr_t)gate % (4 * sizeof(T)) == 0 && (uintptr_t)out % (4 * sizeof(T)) == 0;
 }
 
+template <typename T>
+static void launch_group_norm_regs(const float* y, const void* gate, int gate_stride, const float* w, void* out, int num_tokens, int inner, int group,
+                                   int gate_first, int gate_act, float eps, hipStream_t stream) {
+  const int groups = inner / group, slice = group / (groups >= 4 ? 1 : 4 / groups);
+#define PLLM_NORM(QUADS) hipLaunchKernelGGL((gated_group_norm_regs_kernel<T, QUADS>), dim3(num_tokens), dim3(256), 0, stream, y, (const T*)gate, gate_stride, w, \
+                                            (T*)out, inner, group, gate_first, gate_act, eps)
+  if (slice <= 256) PLLM_NORM(1); else if (slice <= 512) PLLM_NORM(2); else if (slice <= 1024) PLLM_NORM(4); else PLLM_NORM(kGroupRegs);
+#undef PLLM_NORM
+}
+
 PLLM_API int pllm_gated_group_norm(int dtype, const float* y, const void* gate, int gate_stride, const float* w, void* out,
                                    int num_tokens, int inner, int group, int gate_first, int gate_act, float eps, hipStream_t stream) {
   if (num_tokens <= 0) return 0;
@@ -1943,8 +1965,7 @@ PLLM_API int pllm_gated_group_norm(int dtype, const float* y, const void* gate, 
       hipLaunchKernelGGL(gated_group_norm_lanes_kernel<float>, lanes_grid, lanes_block, 0, stream, y, (const float*)gate, gate_stride, w, (float*)out,
                          inner, group, gate_first, gate_act, eps);
     else if (group_norm_in_registers<float>(y, gate, gate_stride, out, inner, group))
-      hipLaunchKernelGGL(gated_group_norm_regs_kernel<float>, grid, block, 0, stream, y, (const float*)gate, gate_stride, w, (float*)out,
-                         inner, group, gate_first, gate_act, eps);
+      launch_group_norm_regs<float>(y, gate, gate_stride, w, out, num_tokens, inner, group, gate_first, gate_act, eps, stream);
     else
       hipLaunchKernelGGL(gated_group_norm_kernel<float>, grid, block, 0, stream, y, (const float*)gate, gate_stride, w, (float*)out,
                          inner, group, gate_first, gate_act, eps);
@@ -1953,8 +1974,7 @@ PLLM_API int pllm_gated_group_norm(int dtype, const float* y, const void* gate, 
       hipLaunchKernelGGL(gated_group_norm_lanes_kernel<bf16>, lanes_grid, lanes_block, 0, stream, y, (const bf16*)gate, gate_stride, w, (bf16*)out,
                          inner, group, gate_first, gate_act, eps);
     else if (group_norm_in_registers<bf16>(y, gate, gate_stride, out, inner, group))
-      hipLaunchKernelGGL(gated_group_norm_regs_kernel<bf16>, grid, block, 0, stream, y, (const bf16*)gate, gate_stride, w, (bf16*)out,
-                         inner, group, gate_first, gate_act, eps);
+      launch_group_norm_regs<bf16>(y, gate, gate_stride, w, out, num_tokens, inner, group, gate_first, gate_act, eps, stream);
     else
       hipLaunchKernelGGL(gated_group_norm_kernel<bf16>, grid, block, 0, stream, y, (const bf16*)gate, gate_stride, w, (bf16*)out,
                          inner, group, gate_first, gate_act, eps);

@@ -33,6 +33,26 @@ def test_rotations_by_quads_are_those_by_elements(heads, dim, rot, interleaved, 
     assert float((got.cpu().double() - want).abs().max()) <= 4 * 2.0 ** -24 * 2 * max(1.0, float(x.abs().max()))
 
 
+@pytest.mark.parametrize("groups,group", [(4, 132), (5, 252), (4, 256), (6, 260), (4, 512), (7, 516), (4, 1024), (4, 1028), (5, 2048),
+                                          (1, 1024), (1, 1040), (1, 8192), (2, 2056), (3, 300)])
+@pytest.mark.parametrize("gate_first,act,weighted", [(True, "silu", True), (False, "sigmoid", False), (False, None, True)])
+def test_norms_of_groups_at_the_edges_of_what_a_wavefront_holds(groups, group, gate_first, act, weighted):
+    """Float rows against 64 bits: a sum of ``group`` squares in 32 bits is off by less than (64 + log2 group) x 2 ** -24 of itself here (a lane adds
+    up to 32 in a row, half of which the root takes), the gate and the four products behind it by a few roundings more."""
+    from paged_llm_amd.csrc import ops
+    gen = torch.Generator().manual_seed(group)
+    T, inner = 5, groups * group
+    y, gate, w = torch.randn(T, inner, generator=gen) * 3, torch.randn(T, inner + 8, generator=gen), torch.rand(inner, generator=gen) + 0.5
+    got = ops.gated_group_norm(y.cuda(), None if act is None else gate.cuda()[:, 4:4 + inner], w.cuda() if weighted else None, group, gate_first, 1e-5,
+                               gate_activation=act, out_dtype=torch.float32).cpu().double()
+    g = gate[:, 4:4 + inner].double()
+    s = torch.ones_like(g) if act is None else torch.sigmoid(g) * (g if act == "silu" else 1.0)
+    u = y.double() * s if gate_first else y.double()
+    u = (u.view(T, groups, group) / (u.view(T, groups, group).square().mean(-1, keepdim=True) + 1e-5).sqrt()).view(T, inner)
+    want = (u if gate_first else u * s) * (w.double() if weighted else 1.0)
+    assert bool(((got - want).abs() <= 64 * 2.0 ** -24 * want.abs() + 1e-30).all())
+
+
 @pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16])
 @pytest.mark.parametrize("lens", [[256, 0], [257, 1, 2, 3], [0, 300], [2, 263, 0, 0], [1, 1, 1, 1, 1, 255 + 9]])
 def test_convolutions_of_long_portions_beside_short_and_empty_ones(lens, dtype):
