@@ -66,6 +66,11 @@ __device__ __forceinline__ bool scan_chunk_of(const int* __restrict__ cu, int nu
 // contribution from a zero state, walked from its last token to its first (the decays behind a token are then one
 // exponential of A times the step sizes summed so far), and the softplus of its step sizes.  kScanOut: a chunk's tokens
 // from the state the sequence had when the chunk began.
+// What bounds the chunks: the exponentials (16 a channel and token in both passes) with two to three wavefronts a SIMD, so nothing may wait for memory:
+// the next four tokens' rows and the next token's B and C are under way while a token is walked.  us of the three passes, with every
+// token's B and C and every four tokens' rows waited for, and so (16 numbers of state): 602 and 576 tokens x 4,096 channels 80.5 and 77.4,
+// 300 x 2,048 34.1 and 28.3, 129 x 4,096 33.1 and 28.1, 777 x 1,000 with 8 numbers 31.7 and 28.7, 2,048 x 4,096 100.6 and 100.4 (the
+// exponentials); rows ahead alone gave 0 to 4 % of it.
 template <typename T, typename TB, int NR, int MAX_THREADS, int MODE>
 __global__ __launch_bounds__(MAX_THREADS) void selective_scan_kernel(ScanArgs a, const TB* __restrict__ bc, long bc_stride) {
   __shared__ float part[2][MAX_THREADS / 64][64];
@@ -96,38 +101,64 @@ __global__ __launch_bounds__(MAX_THREADS) void selective_scan_kernel(ScanArgs a,
   float* dp = a.dt + (size_t)q_begin * C + cc;
   T* op = reinterpret_cast<T*>(a.out) + (size_t)q_begin * C + cc;
   float behind = 0.f;                                         // kScanState: the step sizes of the tokens behind, summed
-  for (int tb = t_first; tb < t_last; tb += kScanAhead) {
-    T xv[kScanAhead], zv[kScanAhead];
-    float rv[kScanAhead];
+  struct Ahead {
+    T x[kScanAhead], z[kScanAhead];
+    float r[kScanAhead];
+  };
+  auto fetch = [&](Ahead& f, int tb) {
 #pragma unroll
     for (int u = 0; u < kScanAhead; ++u) {
       const int n = min(tb + u, t_last - 1);
       const int t = MODE == kScanState ? t_last - 1 - (n - t_first) : n;
-      xv[u] = xp[(size_t)t * a.x_stride];
-      rv[u] = rp[(size_t)t * C];
-      if (MODE != kScanState) zv[u] = zp[(size_t)t * a.z_stride];
+      f.x[u] = xp[(size_t)t * a.x_stride];
+      f.r[u] = rp[(size_t)t * C];
+      if (MODE != kScanState) f.z[u] = zp[(size_t)t * a.z_stride];
     }
+  };
+  constexpr bool kRowAhead = MODE != kScanWhole && NR <= 16;            // (two rows of up to 32 numbers fit the scalar registers; more do not)
+  float nb[NR], nc[NR];                                                 // the next token's B and C
+  auto row_of = [&](int n) { return bc + (size_t)(q_begin + (MODE == kScanState ? t_last - 1 - (n - t_first) : n)) * bc_stride; };
+  auto fetch_row = [&](int n) {
+    const TB* row = row_of(min(n, t_last - 1));
+#pragma unroll
+    for (int i = 0; i < NR; ++i) {
+      nb[i] = uniform_element(row, n0 + i);
+      if (MODE != kScanState) nc[i] = uniform_element(row, a.N + n0 + i);
+    }
+  };
+  if (kRowAhead) fetch_row(t_first);
+  auto walk = [&](const Ahead& f, int tb) {
 #pragma unroll
     for (int u = 0; u < kScanAhead; ++u) {
-      if (tb + u >= t_last) break;
+      if (tb + u >= t_last) return;
       const int t = MODE == kScanState ? t_last - 1 - (tb + u - t_first) : tb + u;
-      const float x = to_f32(xv[u]);
-      const TB* row = bc + (size_t)(q_begin + t) * bc_stride;           // B, then C
-      float dt = rv[u];
+      const float x = to_f32(f.x[u]);
+      if (!kRowAhead) fetch_row(tb + u);
+      float rb[NR], rc[NR];                                             // B and C
+#pragma unroll
+      for (int i = 0; i < NR; ++i) { rb[i] = nb[i]; if (MODE != kScanState) rc[i] = nc[i]; }
+      if (kRowAhead) {
+        // (this token's row has to be here before the next one's is asked for: scalar loads come in any order)
+#pragma unroll
+        for (int i = 0; i < NR; ++i) { asm volatile("" : "+s"(rb[i])); if (MODE != kScanState) asm volatile("" : "+s"(rc[i])); }
+        fetch_row(tb + u + 1);
+        __builtin_amdgcn_sched_barrier(0);
+      }
+      float dt = f.r[u];
       if (MODE != kScanOut) dt = softplus_f32(dt + bias);     // (kScanOut: the first pass has left it)
       const float dx = dt * x;
       if (MODE == kScanState) {
         if (ok && wv == 0) dp[(size_t)t * C] = dt;
 #pragma unroll
-        for (int i = 0; i < NR; ++i) S[i] = fmaf(__builtin_amdgcn_exp2f(A[i] * behind), dx * uniform_element(row, n0 + i), S[i]);
+        for (int i = 0; i < NR; ++i) S[i] = fmaf(__builtin_amdgcn_exp2f(A[i] * behind), dx * rb[i], S[i]);
         behind += dt;
         continue;
       }
       float y[2] = {0.f, 0.f};
 #pragma unroll
       for (int i = 0; i < NR; ++i) {
-        S[i] = fmaf(__builtin_amdgcn_exp2f(A[i] * dt), S[i], dx * uniform_element(row, n0 + i));
-        y[i & 1] = fmaf(S[i], uniform_element(row, a.N + n0 + i), y[i & 1]);
+        S[i] = fmaf(__builtin_amdgcn_exp2f(A[i] * dt), S[i], dx * rb[i]);
+        y[i & 1] = fmaf(S[i], rc[i], y[i & 1]);
       }
       float total = y[0] + y[1];
       if (waves > 1) {
@@ -137,9 +168,27 @@ __global__ __launch_bounds__(MAX_THREADS) void selective_scan_kernel(ScanArgs a,
         for (int w = 1; w < waves; ++w) total += part[t & 1][w][lane];
       }
       if (ok && wv == 0) {
-        const float z = to_f32(zv[u]);
+        const float z = to_f32(f.z[u]);
         op[(size_t)t * C] = from_f32<T>(fmaf(skip, x, total) * (z / (1.f + expf(-z))));
       }
+    }
+  };
+  Ahead one;
+  if constexpr (MODE == kScanWhole) {                         // (mostly single tokens)
+    for (int tb = t_first; tb < t_last; tb += kScanAhead) {
+      fetch(one, tb);
+      walk(one, tb);
+    }
+  } else {
+    // The next tokens' rows are under way while these are walked (rows past the last are the last one again; behind a condition the compiler
+    // would wait for them too).
+    Ahead two;
+    fetch(one, t_first);
+    for (int tb = t_first; tb < t_last; tb += 2 * kScanAhead) {
+      fetch(two, tb + kScanAhead);
+      walk(one, tb);
+      fetch(one, tb + 2 * kScanAhead);
+      walk(two, tb + kScanAhead);
     }
   }
   if (MODE == kScanOut || !ok) return;
