@@ -402,10 +402,12 @@ __global__ __launch_bounds__(256) void rms_sandwich_kernel(const float* __restri
 // The same for rows of up to 4,096 elements that 256 threads hold in registers (G groups of VEC neighbours each,
 // 16 at most): everything a row needs (branch and bias, the stream's row, both weights) is asked for before the first sum, so the
 // kernel waits for memory once where the one above waits three times (decode steps: the weights have left the caches since the
-// last layer).  Inside a step 8 rows of 2,048 without a branch 6.8 -> 4.8 us.  The branch may be a sum of experts' rows (`sum.expert_out` set), formed here instead of by a kernel of its own.
+// last layer).  Partial sums and their order are the ones of the kernel above.  The branch may be a sum of experts' rows
+// (`sum.expert_out` set), formed here instead of by a kernel of its own.  Replayed from a graph, us of the kernel above's way (a branch: of one
+// element a load) and so: 8 rows of 2,048 with a branch 5.2 and 3.4, without one 3.7 and 2.7; 777 rows with a branch 8.5 and 7.6.
 constexpr int kHeldPerThread = 16, kHeldThreads = 256;
 
-// Element e of group j of a thread's part of a row; a group past the row's end reads the row's first elements and counts nowhere.
+// The first element of group j of a thread's part of a row; a group past the row's end reads the row's first elements and counts nowhere.
 template <int VEC> __device__ __forceinline__ int held_at(int j) { return (kHeldThreads * j + (int)threadIdx.x) * VEC; }
 
 template <int VEC>
@@ -446,12 +448,29 @@ __device__ __forceinline__ void load_held_groups(const T* p, int hidden, float (
   for (int j = 0; j < G; ++j) load_group<VEC>(p + (held_at<VEC>(j) < hidden ? held_at<VEC>(j) : 0), v + j * VEC);
 }
 
+// The same for rows that need not lie on the boundaries of VEC elements (`fours`: they do).
+template <int VEC, int G, typename T>
+__device__ __forceinline__ void load_held_rows(const T* p, int hidden, bool fours, float (&v)[VEC * G]) {
+  if (VEC == 1 || fours) return load_held_groups<VEC, G>(p, hidden, v);
+#pragma unroll
+  for (int j = 0; j < G; ++j)
+#pragma unroll
+    for (int e = 0; e < VEC; ++e) v[j * VEC + e] = to_f32(p[(held_at<VEC>(j) < hidden ? held_at<VEC>(j) : 0) + e]);
+}
+
+template <int VEC, typename T>
+__device__ __forceinline__ void store_held_rows(T* p, const float* v, bool fours) {
+  if (VEC == 1 || fours) return store_group<VEC>(p, v);
+#pragma unroll
+  for (int e = 0; e < VEC; ++e) p[e] = from_f32<T>(v[e]);
+}
+
 // f += the sum of row r's choices, in their order.  What bounds it in a decode step: trips to memory.  A lane asks for one choice's
 // row number and weight, then the rows of four choices are asked for at once (and the token's own row, where some choice hands it
-// back): two trips up to four choices, where a choice after the other waits for its row number and then for its row.  Inside a step, 8 rows
-// of 2,048 elements with both norms and 4 choices 15.0 -> 5.5 us (a plain branch 6.9 -> 4.6), 1,178 rows of 2 choices 13.2 -> 8.9.
+// back): two trips up to four choices, where a choice after the other waits for its row number and then for its row.  Replayed from a graph, us in turn and
+// so: 8 rows of 2,048 elements with both norms and 4 choices 9.6 and 4.5, 1,178 rows of 2 choices 23.2 and 10.8, 64 rows of 4,096 and 4 24.0 and 7.4.
 template <typename TH, int VEC, int G>
-__device__ __forceinline__ void add_choices(const ChoiceSum& sum, int rows_lane, float weights_lane, int r, int hidden, float (&f)[VEC * G]) {
+__device__ __forceinline__ void add_choices(const ChoiceSum& sum, int rows_lane, float weights_lane, int r, int hidden, bool own_fours, float (&f)[VEC * G]) {
   const int lane = threadIdx.x & 63;
   for (int k0 = 0; k0 < sum.top; k0 += 64) {
     const int count = min(64, sum.top - k0);
@@ -462,7 +481,7 @@ __device__ __forceinline__ void add_choices(const ChoiceSum& sum, int rows_lane,
     float own[VEC * G];
 #pragma unroll
     for (int i = 0; i < VEC * G; ++i) own[i] = 0.f;
-    if (__any(rows_lane < 0)) load_held_groups<VEC, G>(reinterpret_cast<const TH*>(sum.h) + (size_t)r * sum.ld_h, hidden, own);
+    if (__any(rows_lane < 0)) load_held_rows<VEC, G>(reinterpret_cast<const TH*>(sum.h) + (size_t)r * sum.ld_h, hidden, own_fours, own);
     for (int k1 = 0; k1 < count; k1 += kSumAhead) {
       float v[kSumAhead][VEC * G];
 #pragma unroll
@@ -482,13 +501,43 @@ __device__ __forceinline__ void add_choices(const ChoiceSum& sum, int rows_lane,
   }
 }
 
+// A thread's sum of its row's squares in the order of the kernel above, elements threadIdx.x, threadIdx.x + 256, ..., whichever elements it
+// holds: four neighbours to a thread go through LDS first (with sums of their own a row's bits would hang on where it lies in memory; that took
+// 0.2 to 0.5 us less for 8 rows, 0.8 of 10 for 1,178, 2 of 14.8 for 2,048).
+// `in_order` may be used again behind a held_sum of the result.
+template <int VEC, int G>
+__device__ __forceinline__ float squares_of_row(const float (&v)[VEC * G], int hidden, float4* in_order) {
+  float x[VEC * G], sq = 0.f;
+  if constexpr (VEC == 4) {
+#pragma unroll
+    for (int j = 0; j < G; ++j) in_order[kHeldThreads * j + threadIdx.x] = make_float4(v[4 * j], v[4 * j + 1], v[4 * j + 2], v[4 * j + 3]);
+    __syncthreads();
+  }
+#pragma unroll
+  for (int j = 0; j < VEC * G; ++j) x[j] = VEC == 4 ? reinterpret_cast<const float*>(in_order)[held_at<1>(j)] : v[j];
+#pragma unroll
+  for (int j = 0; j < VEC * G; ++j) {
+    const float with = fmaf(x[j], x[j], sq);
+    sq = held_at<1>(j) < hidden ? with : sq;
+  }
+  return sq;
+}
+
+// block_sum's sum in its order, of four wavefronts that add with this `sums` once: one barrier, one trip to LDS.
+__device__ __forceinline__ float held_sum(float v, float4& sums) {
+  v = wave_sum(v);
+  if ((threadIdx.x & 63) == 0) reinterpret_cast<float*>(&sums)[threadIdx.x >> 6] = v;
+  __syncthreads();
+  return ((sums.x + sums.y) + sums.z) + sums.w;
+}
+
 template <typename TO, typename TH, int VEC, int G>
 __global__ __launch_bounds__(kHeldThreads) void rms_sandwich_held_kernel(const float* __restrict__ branch, const BranchPair pair, const ChoiceSum sum,
                                                                          const float* __restrict__ bias, const float* __restrict__ w_branch,
                                                                          float mult, float* stream, const int* __restrict__ row_index,
                                                                          const float* __restrict__ w_next, float eps, TO* __restrict__ rows,
-                                                                         long rows_stride, int hidden) {
-  __shared__ float scratch[16];
+                                                                         long rows_stride, int hidden, bool own_fours, bool out_fours) {
+  __shared__ float4 sums[2], in_order[VEC == 4 ? kHeldThreads * G : 1];
   const int r = blockIdx.x, lane = threadIdx.x & 63;
   const bool added = branch || sum.expert_out;
   float* s = stream + (!added && row_index ? (size_t)row_index[r] : (size_t)r) * hidden;
@@ -513,20 +562,12 @@ __global__ __launch_bounds__(kHeldThreads) void rms_sandwich_held_kernel(const f
 #pragma unroll
     for (int i = 0; i < VEC * G; ++i) f[i] = pair.first_scale * f[i] + pair.second_scale * second[i];
   }
-  if (sum.expert_out) add_choices<TH, VEC, G>(sum, rows_lane, weights_lane, r, hidden, f);
-  float bsq = 0.f;
+  if (sum.expert_out) add_choices<TH, VEC, G>(sum, rows_lane, weights_lane, r, hidden, own_fours, f);
+  if (bias) {
 #pragma unroll
-  for (int j = 0; j < G; ++j)
-    if (held_at<VEC>(j) < hidden) {
-#pragma unroll
-      for (int e = 0; e < VEC; ++e) {
-        float& b = f[j * VEC + e];
-        if (bias) b += add[j * VEC + e];
-        bsq = fmaf(b, b, bsq);
-      }
-    }
-  const float inv = added && w_branch ? 1.f / sqrtf(block_sum(bsq, scratch) / (float)hidden + eps) : 1.f;
-  float sq = 0.f;
+    for (int i = 0; i < VEC * G; ++i) f[i] += add[i];
+  }
+  const float inv = added && w_branch ? 1.f / sqrtf(held_sum(squares_of_row<VEC, G>(f, hidden, in_order), sums[0]) / (float)hidden + eps) : 1.f;
 #pragma unroll
   for (int j = 0; j < G; ++j)
     if (held_at<VEC>(j) < hidden) {
@@ -534,20 +575,19 @@ __global__ __launch_bounds__(kHeldThreads) void rms_sandwich_held_kernel(const f
       for (int e = 0; e < VEC; ++e) {
         const int i = j * VEC + e;
         if (added) sv[i] += mult * (w_branch ? f[i] * inv * wb[i] : f[i]);
-        sq = fmaf(sv[i], sv[i], sq);
       }
       if (added) store_group<VEC>(s + held_at<VEC>(j), sv + j * VEC);
     }
   if (!rows) return;
   TO* out = rows + (size_t)r * rows_stride;
-  const float inv_next = w_next ? 1.f / sqrtf(block_sum(sq, scratch) / (float)hidden + eps) : 1.f;
+  const float inv_next = w_next ? 1.f / sqrtf(held_sum(squares_of_row<VEC, G>(sv, hidden, in_order), sums[1]) / (float)hidden + eps) : 1.f;
 #pragma unroll
   for (int j = 0; j < G; ++j)
     if (held_at<VEC>(j) < hidden) {
       float y[VEC];
 #pragma unroll
       for (int e = 0; e < VEC; ++e) y[e] = w_next ? sv[j * VEC + e] * inv_next * wn[j * VEC + e] : sv[j * VEC + e];
-      store_group<VEC>(out + held_at<VEC>(j), y);
+      store_held_rows<VEC>(out + held_at<VEC>(j), y, out_fours);
     }
 }
 
@@ -566,7 +606,7 @@ template <typename TO, typename TH, int VEC, int G>
 __global__ __launch_bounds__(kHeldThreads) void rms_depth_kernel(const float* __restrict__ branch, const ChoiceSum sum, const DepthSum depth,
                                                                  const float* __restrict__ bias, const float* __restrict__ w_branch, float mult,
                                                                  float* __restrict__ stream, const float* __restrict__ w_next, float eps,
-                                                                 TO* __restrict__ rows, long rows_stride, int hidden) {
+                                                                 TO* __restrict__ rows, long rows_stride, int hidden, bool own_fours, bool out_fours) {
   __shared__ float scratch[16];
   const int r = blockIdx.x, lane = threadIdx.x & 63;
   float* s = stream + (size_t)r * hidden;
@@ -601,7 +641,7 @@ __global__ __launch_bounds__(kHeldThreads) void rms_depth_kernel(const float* __
         }
     }
   }
-  if (sum.expert_out) add_choices<TH, VEC, G>(sum, rows_lane, weights_lane, r, hidden, f);
+  if (sum.expert_out) add_choices<TH, VEC, G>(sum, rows_lane, weights_lane, r, hidden, own_fours, f);
   float bsq = 0.f;
 #pragma unroll
   for (int j = 0; j < G; ++j)
@@ -644,17 +684,13 @@ __global__ __launch_bounds__(kHeldThreads) void rms_depth_kernel(const float* __
       if (w_next) load_group<VEC>(w_next + held_at<VEC>(j), wn);
 #pragma unroll
       for (int e = 0; e < VEC; ++e) y[e] = w_next ? acc[j * VEC + e] * inv_next * wn[e] : acc[j * VEC + e];
-      store_group<VEC>(out + held_at<VEC>(j), y);
+      store_held_rows<VEC>(out + held_at<VEC>(j), y, out_fours);
     }
 }
 
-// Whether rows of `hidden` elements at these addresses go four elements a load (`floats`: the addresses of float rows put together
-// by `or`; the tokens' own rows and the output rows have a type and a stride of their own).
-static bool rows_by_fours(int hidden, uintptr_t floats, int h_dtype, const void* h, long ld_h, int out_dtype, const void* rows, long rows_stride) {
-  const uintptr_t h_bytes = h_dtype == PLLM_F32 ? 16 : 8, out_bytes = out_dtype == PLLM_F32 ? 16 : 8;
-  return hidden % 4 == 0 && floats % 16 == 0 && (!h || ((uintptr_t)h % h_bytes == 0 && ld_h % 4 == 0)) &&
-         (!rows || ((uintptr_t)rows % out_bytes == 0 && rows_stride % 4 == 0));
-}
+// Whether rows of this type at this address go four elements a load.
+static bool rows_by_fours(int dtype, const void* rows, long stride) { return (uintptr_t)rows % (dtype == PLLM_F32 ? 16 : 8) == 0 && stride % 4 == 0; }
+
 // Groups of elements a thread: as few as hold the row (one element a load: all 16, whose loads past the row's end repeat its first).
 #define PLLM_HELD_FORM(LAUNCH, TO, TH, FOURS)                                          \
   do {                                                                                 \
@@ -676,10 +712,12 @@ PLLM_API int pllm_rms_depth(int out_dtype, int h_dtype, const float* branch, con
   const ChoiceSum sum{expert_out, h, ld_h, row_of_pair, weights, top};
   const DepthSum depth{history, plane, depth_w, count};
   const uintptr_t all = (uintptr_t)branch | (uintptr_t)expert_out | (uintptr_t)history | (uintptr_t)bias | (uintptr_t)w_branch | (uintptr_t)stream | (uintptr_t)w_next;
-  const bool fours = plane % 4 == 0 && rows_by_fours(hidden, all, h_dtype, expert_out ? h : nullptr, ld_h, out_dtype, rows, rows_stride);
+  // (which elements a thread sums hangs on the float rows alone)
+  const bool fours = hidden % 4 == 0 && plane % 4 == 0 && all % 16 == 0;
+  const bool own_fours = expert_out && rows_by_fours(h_dtype, h, ld_h), out_fours = rows_by_fours(out_dtype, rows, rows_stride);
 #define PLLM_RD_FORM(TO, TH, VEC, G)                                                                                                     \
   hipLaunchKernelGGL((rms_depth_kernel<TO, TH, VEC, G>), dim3(num_rows), dim3(kHeldThreads), 0, stream_, branch, sum, depth, bias, w_branch, \
-                     mult, stream, w_next, eps, (TO*)rows, rows_stride, hidden)
+                     mult, stream, w_next, eps, (TO*)rows, rows_stride, hidden, own_fours, out_fours)
 #define PLLM_RD(TO, TH) PLLM_HELD_FORM(PLLM_RD_FORM, TO, TH, fours)
   if (out_dtype == PLLM_F32) { if (h_dtype == PLLM_F32) PLLM_RD(float, float); else PLLM_RD(float, bf16); }
   else { if (h_dtype == PLLM_F32) PLLM_RD(bf16, float); else PLLM_RD(bf16, bf16); }
@@ -712,10 +750,11 @@ static void launch_sandwich_held(int h_dtype, const float* branch, const BranchP
                                  float* stream, const int* row_index, const float* w_next, float eps, void* rows, long rows_stride, int num_rows, int hidden,
                                  hipStream_t stream_) {
   const uintptr_t all = (uintptr_t)branch | (uintptr_t)pair.second | (uintptr_t)sum.expert_out | (uintptr_t)bias | (uintptr_t)w_branch | (uintptr_t)stream | (uintptr_t)w_next;
-  const bool fours = rows_by_fours(hidden, all, h_dtype, sum.h, sum.ld_h, sizeof(TO) == 4 ? PLLM_F32 : PLLM_BF16, rows, rows_stride);
+  const bool fours = hidden % 4 == 0 && all % 16 == 0;
+  const bool own_fours = sum.expert_out && rows_by_fours(h_dtype, sum.h, sum.ld_h), out_fours = rows_by_fours(sizeof(TO) == 4 ? PLLM_F32 : PLLM_BF16, rows, rows_stride);
 #define PLLM_SH_FORM(T, TH, VEC, G)                                                                                                               \
   hipLaunchKernelGGL((rms_sandwich_held_kernel<T, TH, VEC, G>), dim3(num_rows), dim3(kHeldThreads), 0, stream_, branch, pair, sum, bias, w_branch, \
-                     mult, stream, row_index, w_next, eps, (T*)rows, rows_stride, hidden)
+                     mult, stream, row_index, w_next, eps, (T*)rows, rows_stride, hidden, own_fours, out_fours)
   if (h_dtype == PLLM_F32) PLLM_HELD_FORM(PLLM_SH_FORM, TO, float, fours);
   else PLLM_HELD_FORM(PLLM_SH_FORM, TO, bf16, fours);
 #undef PLLM_SH_FORM

@@ -47,3 +47,48 @@ def test_picked_rows_without_a_branch(width):
         assert torch.equal(ops.rms_sandwich(s, None, None, 0.0, 1e-5, out_dtype=torch.bfloat16, row_index=None if index is None else index.cuda()).cpu(),
                            rows.to(torch.bfloat16))
     assert torch.equal(s.cpu(), x)
+
+
+def shifted(x):
+    """The same numbers one element further on in memory: rows that no 16-byte boundary fits."""
+    return torch.cat([x.new_zeros(1), x.reshape(-1)])[1:].view(x.shape)
+
+
+@pytest.mark.parametrize("width", [1024, 1028, 2048, 4096])
+@pytest.mark.parametrize("kind", ["rows", "choices", "pair", "none"])
+def test_a_rows_bits_do_not_hang_on_where_it_lies(width, kind):
+    """Four elements a load or one: the same partial sums in the same order, whatever stands in front of the norm."""
+    from paged_llm_amd.csrc import ops
+    rows, top = 3, 2
+    stream, a, b = (rnd(rows, width, seed=s).cuda() for s in (1, 2, 3))
+    wb, wn, bias = (rnd(width, seed=s).cuda() for s in (4, 5, 6))
+    e, h, weights = rnd(rows * top, width, seed=7).cuda(), rnd(rows, width, seed=8).cuda(), rnd(rows, top, seed=9).cuda()
+    places = torch.tensor([3, -1, 0, 5, 2, 1], dtype=torch.int32, device="cuda")
+
+    def norm(place):
+        s = place(stream.clone())
+        branch = {"rows": lambda: place(a), "pair": lambda: ops.WeightedPair(place(a), 0.3, place(b), 1.7), "none": lambda: None,
+                  "choices": lambda: ops.ChoiceSum(place(e), place(h), places, weights)}[kind]()
+        out = place(torch.zeros_like(stream))
+        ops.rms_sandwich(s, branch, None if kind == "none" else place(wb), 0.5, 1e-5, w_next=place(wn), out=out, bias=None if kind == "none" else place(bias))
+        return s, out
+    for x, y in zip(norm(lambda t: t), norm(shifted)):
+        assert torch.equal(x, y)
+
+
+@pytest.mark.parametrize("width", [1024, 4096])
+def test_the_depth_norms_bits_do_not_hang_on_where_its_rows_go(width):
+    """The tokens' own rows and the output may lie anywhere: which elements a thread sums follows from the float rows alone."""
+    from paged_llm_amd.csrc import ops
+    rows, top = 3, 2
+    stream, h, wb, wn = rnd(rows, width, seed=1).cuda(), rnd(rows, width, seed=2).to(torch.bfloat16).cuda(), rnd(width, seed=3).cuda(), rnd(width, seed=4).cuda()
+    e, weights = rnd(rows * top, width, seed=5).cuda(), rnd(rows, top, seed=6).cuda()
+    places = torch.tensor([3, -1, 0, 5, 2, 1], dtype=torch.int32, device="cuda")
+
+    def norm(own, out):
+        s, history = stream.clone(), rnd(3, rows, width, seed=7).cuda()
+        ops.rms_sandwich(s, ops.ChoiceSum(e, own, places, weights), wb, 0.5, 1e-5, w_next=wn, out=out, depth=ops.DepthSum(history, rnd(3, seed=8).cuda()))
+        return s, history, out
+    plain = norm(h, torch.zeros(rows, width, device="cuda", dtype=torch.bfloat16))
+    for x, y in zip(plain, norm(shifted(h), torch.zeros(rows, width + 3, device="cuda", dtype=torch.bfloat16)[:, :width])):
+        assert torch.equal(x, y)
