@@ -827,76 +827,42 @@ __global__ __launch_bounds__(64 * WAVES, 2) void recurrence_piece_kernel(Recurre
         }
       }
     }
-    if constexpr (kOut && NT == 2) {
-      // The tiles of M on the diagonal: sixteen lanes share a key, NT of its rows each.
-      for (int who = tid; who < 512; who += kThreads) {
-        const int j = who >> 4, n = (who & 15) * NT, stop = (j & 16) + 16;
-        float w[NT];
+    if constexpr (kOut) {
+      // The tiles of M on the diagonal: sixteen lanes share a key, NT of its rows each, added in their order and then over the lanes.
+      // What bounds it is LDS: so every sixteen lanes take two keys, a token's decays and queries read for both, and nothing stands
+      // behind a condition, so that the reads of the tokens to come are under way (16 heads
+      // of 128 x 128, 777 tokens in pieces 441 -> 298 us with the walks above, in chunks 66.5 -> 56.4; 64 of 64 x 64 333 -> 232 and 94 -> 74).
+      for (int eight = wave; eight < 4; eight += WAVES) {
+        const int first = (eight >> 1) * 16, j0 = first + (eight & 1) * 8 + quad, n = c16 * NT;      // keys j0 and j0 + 4
+        float w[2][NT];
 #pragma unroll
-        for (int i = 0; i < NT; ++i) w[i] = K[j * LD + n + i];
-        for (int t = j & 16; t < stop; ++t) {
-          float dot = 0.f;
-          if (t >= j) {
+        for (int k = 0; k < 2; ++k)
 #pragma unroll
-            for (int i = 0; i < NT; ++i) {
-              if (t > j) w[i] *= DR[t * LD + n + i];
-              dot = fmaf(w[i], Q[t * LD + n + i], dot);
-            }
-          }
-          dot += dpp_move<kDppSwap1>(dot);
-          dot += dpp_move<kDppSwap2>(dot);
-          dot += dpp_move<kDppHalfMirror>(dot);
-          dot += dpp_move<kDppMirror>(dot);
-          if ((who & 15) == 0) M[t * kPieceLd + j] = dot * gs[j];
-        }
-      }
-    }
-    if constexpr (kOut && NT > 2) {
-      // The same with a wavefront's lanes along the rows and four of a tile's keys at a time, every fourth one: a token's decays and queries are
-      // read once for four keys (with sixteen lanes to a key all wavefronts read them for every key: 18,000 of a piece's 42,000 clocks;
-      // 777 tokens, 16 heads of 128 x 128: 441 us then, 338 so).  Rows up to 32 would leave half the lanes idle and keep the other form.
-      constexpr int kRows = NP / 64;
-      for (int four = wave; four < 8; four += WAVES) {
-        const int first = (four >> 2) * 16, j0 = first + (four & 3), n = lane * kRows;
-        float w[4][kRows];
-#pragma unroll
-        for (int k = 0; k < 4; ++k)
-#pragma unroll
-          for (int i = 0; i < kRows; ++i) w[k][i] = K[(j0 + 4 * k) * LD + n + i];
-        const int mine = j0 + ((quad & 1) * 2 + (quad >> 1)) * 4;      // the key whose sum this lane gets
-        const float g = gs[mine];
+          for (int i = 0; i < NT; ++i) w[k][i] = K[(j0 + 4 * k) * LD + n + i];
+        const float g = gs[j0 + 4 * (c16 & 1)];
 #pragma unroll 4
         for (int t = first; t < first + 16; ++t) {
-          float d[kRows], q[kRows], dot[4];
+          float d[NT], q[NT], dot[2];
 #pragma unroll
-          for (int i = 0; i < kRows; ++i) { d[i] = DR[t * LD + n + i]; q[i] = Q[t * LD + n + i]; }
+          for (int i = 0; i < NT; ++i) { d[i] = DR[t * LD + n + i]; q[i] = Q[t * LD + n + i]; }
 #pragma unroll
-          for (int k = 0; k < 4; ++k) {
-            const int j = j0 + 4 * k;                                  // (the same for all lanes)
+          for (int k = 0; k < 2; ++k) {
+            const int j = j0 + 4 * k;
             dot[k] = 0.f;
 #pragma unroll
-            for (int i = 0; i < kRows; ++i) {
+            for (int i = 0; i < NT; ++i) {
               w[k][i] = t > j ? w[k][i] * d[i] : w[k][i];
               dot[k] = fmaf(w[k][i], q[i], dot[k]);
             }
             dot[k] = t >= j ? dot[k] : 0.f;
+            dot[k] += dpp_move<kDppSwap1>(dot[k]);
+            dot[k] += dpp_move<kDppSwap2>(dot[k]);
+            dot[k] += dpp_move<kDppHalfMirror>(dot[k]);
+            dot[k] += dpp_move<kDppMirror>(dot[k]);
           }
-          // (sums of keys 0, 2, 1, 3 in the four rows of lanes)
-          auto halves = [](float x, float y) {
-            const auto r = __builtin_amdgcn_permlane32_swap(__float_as_uint(x), __float_as_uint(y), false, false);
-            return __uint_as_float(r[0]) + __uint_as_float(r[1]);
-          };
-          const auto rows = __builtin_amdgcn_permlane16_swap(__float_as_uint(halves(dot[0], dot[1])), __float_as_uint(halves(dot[2], dot[3])), false, false);
-          float sum = __uint_as_float(rows[0]) + __uint_as_float(rows[1]);
-          sum += dpp_move<kDppSwap1>(sum);
-          sum += dpp_move<kDppSwap2>(sum);
-          sum += dpp_move<kDppHalfMirror>(sum);
-          sum += dpp_move<kDppMirror>(sum);
-          if (c16 == 0) M[t * kPieceLd + mine] = sum * g;
+          if (c16 < 2) M[t * kPieceLd + j0 + 4 * c16] = (c16 ? dot[1] : dot[0]) * g;
         }
       }
-    }
-    if constexpr (kOut) {
       __syncthreads();
       for (int n = tid; n < NP; n += kThreads) {                     // (the diagonal is done with the plain queries)
         float all = 1.f;

@@ -43,3 +43,17 @@ def test_an_infinite_key_reaches_its_own_token_and_later_ones_only(N):
     y = ops.linear_recurrence(q.cuda(), k.cuda(), torch.rand(32, 2, 16).cuda() + 0.1, None, torch.zeros(1, 2 * N * 16, device="cuda"), 0, at(0), at(0),
                               at(0, 32), 1, max_q_len=32, row_decay=f.cuda()).cpu().view(32, 2, 16)
     assert bool(torch.isfinite(y[:, 0]).all() and torch.isfinite(y[:7, 1]).all() and not torch.isfinite(y[7:, 1]).any())
+
+
+@pytest.mark.parametrize("N", [64, 128])
+def test_neighbouring_rows_are_added_in_their_order(N, monkeypatch):
+    """Sixteen lanes share a key, N / 16 neighbouring rows each: 2^24 + 1 + 1 - 2^24 is 0 in that order, and 1 where a lane had fewer rows."""
+    from paged_llm_amd.csrc import ops
+    monkeypatch.setattr(ops, "recurrence_form", lambda *a, **k: -1)             # (in pieces of 32 tokens, two tiles each)
+    q, k, v = torch.zeros(32, 1, N), torch.ones(32, 1, N), torch.zeros(32, 1, 16)
+    q[:, 0, :4] = torch.tensor([2.0 ** 24, 1.0, 1.0, -2.0 ** 24])
+    v[0] = 1.0
+    at = lambda *x: torch.tensor(x, dtype=torch.int32, device="cuda")
+    y = ops.linear_recurrence(q.cuda(), k.cuda(), v.cuda(), None, torch.zeros(1, N * 16, device="cuda"), 0, at(0), at(0), at(0, 32), 1, max_q_len=32,
+                              row_decay=torch.ones(32, 1, N).cuda())
+    assert not bool(y[:16].any())
