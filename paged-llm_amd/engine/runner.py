@@ -552,6 +552,11 @@ class ModelRunner:
             ctx.launch_cache[akey] = entry["static"][lay["offsets"][base + j]: lay["offsets"][base + j] + lay["sizes"][base + j]]
         return ctx
 
+    @staticmethod
+    def _even_portions(tokens: int, count: int) -> list:
+        """``tokens`` as ``count`` lengths that differ by one at most: none is longer than the bound of a shape that holds them."""
+        return [tokens // count + (i < tokens % count) for i in range(count)]
+
     def _capture_prompt_graph(self, entry: dict):
         """Warm-up and capture on a batch of the graph's shape that writes nothing: empty single-token rows and
         portions that are all padding.  Returns the key of the graph that had to go for it, or None."""
@@ -559,8 +564,7 @@ class ModelRunner:
         lay = entry["layout"]
         view, offsets, sizes, S, T = entry["view"], lay["offsets"], lay["sizes"], lay["S"], lay["T"]
         view[:] = 0
-        each = [bucket // (portions + 1)] * (portions + 1)
-        each[-1] += bucket - sum(each)
+        each = self._even_portions(bucket, portions + 1)
         q_lens = [1] * rows + each
         view[offsets[1]: offsets[1] + T] = np.concatenate([np.zeros(rows, dtype=np.int32)] + [np.arange(n, dtype=np.int32) for n in each])
         view[offsets[2]: offsets[2] + S + 1] = np.concatenate([[0], np.cumsum(q_lens)])
