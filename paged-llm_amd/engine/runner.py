@@ -65,15 +65,16 @@ class GraphCache:
 
 class ModelRunner:
     def __init__(self, model, kv_storage: KVCacheStorage, num_state_slots: int = 0, use_graphs: bool = False,
-                 max_graph_batch: int = 1024, max_graph_tokens: int = 2048, graph_after_sightings: int = 2):
+                 max_graph_batch: int = 1024, max_graph_tokens: int = 1024, graph_after_sightings: int = 2):
         self.model = model
         # Graph replay needs every part of the model to do nothing but launch kernels on the
         # current stream; parts say so with ``graph_capturable`` (steps of single tokens) and
         # ``graph_capturable_prompts`` (steps that hold prompt portions as well).
         self.use_graphs = bool(use_graphs) and model.graph_capturable()
         self.prompt_graphs = self.use_graphs and model.graph_capturable(prompts=True)
+        self.padding_is_a_chunk = model.padding_is_a_chunk()
         self.max_graph_batch = max_graph_batch
-        # Steps with prompt portions are replayed from graphs up to this many portion tokens (four times as many
+        # Steps with prompt portions are replayed from graphs up to this many portion tokens (eight times as many
         # when no padding is needed), and once their shape has been seen this often (a capture costs several
         # steps' time; shapes that never come back are not worth one).
         self.max_graph_tokens = max_graph_tokens
@@ -414,23 +415,44 @@ class ModelRunner:
     MAX_GRAPH_PORTIONS = 4
     MAX_GRAPH_LOGITS = 64                 # rows of logits that a graph of such a step holds
 
+    # What a capture costs: 6 to 12 ms, three to five steps' time.  A graph of a step's own shape (``_token_bucket``) saves a step 0.4 of the share of
+    # padding that the shared shape (``_shared_bucket``) has, so it is captured once as much padding has been computed as ten whole steps
+    # hold.  Beyond ``max_graph_tokens`` there is no shared shape: Python's launches take 0 to 2 % of a step at width 2,048 and more of a narrower model's, and a
+    # graph has paid after a hundred sightings or so.  But a padding sequence is one more chunk of a linear recurrence (``padding_is_a_chunk``), which can be one
+    # more round of workgroups: at widths above 1,024 those models' own shapes are the ones that need no padding.  One prompt, ms, eager and from a graph
+    # of its own shape, at width 1,024: Gudutar 1,100 tokens 2.16 and 1.71, 1,500 2.03 and 1.98, 1,900 2.17 and 2.10, Renadra 2.46 and 1.82, 2.16 and 2.03, 2.43
+    # and 2.37; at 2,048: Gudutar 2.71 and 2.67, 3.18 and 3.24, 3.78 and 3.76, Renadra 3.45 and 3.37, 4.06 and 4.13, 4.83 and 4.76, Mekusun 4.33 and 4.26,
+    # 5.00 and 4.96, 6.05 and 6.02 (two texts of 603 and 575 4.58 and 4.42), TinyLlama 4.02 and 3.95, 4.91 and 4.85, 5.95 and 5.95.
+    PADDING_WORTH_A_CAPTURE = 10          # steps
+    OWN_SHAPE_AFTER = 100                 # sightings, beyond max_graph_tokens
+    NARROW = 1024
+
     @staticmethod
     def _token_bucket(n: int) -> int:
-        """Portion tokens a graph is captured for, and wanted rows beyond 64: steps of 32 up to 1024, of 16 up to 2048, of 256 beyond.  The rows
-        between are computed for nothing: 777 tokens in a graph of 896 / 832 / 800 took 2.87 / 2.85 / 2.75 ms (Renadra, width 2,048), and
-        beyond 1,024 a step may bear 1 to 2 % of them before the launches from Python are cheaper."""
+        """Portion tokens of a graph of a step's own shape, and wanted rows beyond 64: steps of 32 up to 1024, of 16 up to 2048, of 256
+        beyond.  The rows between are computed for nothing."""
         for limit, step in ((1024, 32), (2048, 16)):
             if n <= limit:
                 return -(-n // step) * step
         return -(-n // 256) * 256
 
-    def _prompt_graph_key(self, entries: list):
+    @staticmethod
+    def _shared_bucket(n: int) -> int:
+        """Portion tokens of a graph that more lengths share: steps of 32 up to 128, of 64 up to 512, of 128 up to 1024, of 256 beyond (777 tokens
+        in a graph of 800 / 896: TinyLlama 2.99 / 3.09 ms, Renadra at width 1,024 1.47 / 1.51, at 2,048 2.69 / 2.77; eager 2.98, 2.13, 2.67)."""
+        for limit, step in ((128, 32), (512, 64), (1024, 128)):
+            if n <= limit:
+                return -(-n // step) * step
+        return -(-n // 256) * 256
+
+    def _prompt_graph_key(self, entries: list, shared: bool = False):
         """A step that holds prompt portions (entries of two or more tokens), alone or beside single tokens, can be
         replayed from a graph whose launch shapes depend on: the number of single-token rows (rounded up as for
         decode steps), the number of portions (at most four), the portions' tokens together (rounded up to a
         bucket; a sequence of padding tokens that writes nothing fills the rest, none when the portions fill the bucket
         exactly, as the portions of a long prompt under a token budget do step after step), the wanted rows and
-        a bound on the context lengths.  None when the step is not of that kind or too large to be worth it."""
+        a bound on the context lengths.  None when the step is not of that kind or too large to be worth it.  ``shared``: the coarser of the two
+        shapes that a step may be replayed in."""
         if not self.prompt_graphs:
             return None
         singles = portions = portion_tokens = asked = longest = longest_portion = 0
@@ -446,16 +468,21 @@ class ModelRunner:
             longest = max(longest, e.start + n)
         if portions == 0 or portions > self.MAX_GRAPH_PORTIONS or singles > self.max_graph_batch:
             return None
-        bucket = self._token_bucket(portion_tokens)
+        bucket_of = self._shared_bucket if shared else self._token_bucket
+        bucket = bucket_of(portion_tokens)
         bound = ((longest + 511) // 512) * 512 if longest <= 8192 else 1 << (longest - 1).bit_length()
         bound = min(bound, max(self.model.max_positions, longest))
-        # Padded steps up to max_graph_tokens; steps that fill their bucket exactly (the portions of a long prompt under a
-        # token budget) up to four times that.
-        limit = self.max_graph_tokens * (4 if bucket == portion_tokens else 1)
+        # Padded steps up to max_graph_tokens; steps that fill a shared bucket exactly (the portions of a long prompt under a
+        # token budget) up to eight times that.
+        if shared:
+            limit = self.max_graph_tokens * (8 if bucket == portion_tokens else 1)
+        else:
+            worth = bucket == portion_tokens or not self.padding_is_a_chunk or self.model.spec.hidden_size <= self.NARROW
+            limit = self.max_graph_tokens * (2 if bucket > 1024 and worth else 1)
         if bucket > limit or bucket - portion_tokens > bound:   # (the padding sequence's positions stay below the bound)
             return None
         rows = self._bucket(singles) if singles else 0
-        wanted = 0 if not asked else self._bucket(asked) if asked <= self.MAX_GRAPH_LOGITS else self._token_bucket(asked)
+        wanted = 0 if not asked else self._bucket(asked) if asked <= self.MAX_GRAPH_LOGITS else bucket_of(asked)
         # The portions' own contexts, as far as the attention's launch depends on them: nothing below 1024 (no
         # partitions of keys there), else a power of two.
         portion_context = 0 if longest_portion < 1024 else min(bound, 1 << (longest_portion - 1).bit_length())
@@ -596,20 +623,54 @@ class ModelRunner:
         entry.update(graph=graph, ctx=ctx, **{"head_rows" if apart else "logits": result})
         return self._graphs.put(entry["key"], entry)
 
-    def _prompt_graph_step(self, key, entries: list, borrow: bool) -> torch.Tensor | None:
+    def _prompt_graph(self, entries: list) -> dict | None:
+        """The graph that a step with prompt portions is replayed from: that of its own shape, else the one that more lengths share, either
+        captured now if it has been seen often enough; None: run it eagerly this time."""
+        shared, own = self._prompt_graph_key(entries, shared=True), self._prompt_graph_key(entries)
+        if own is not None and own != shared:
+            entry = self._known_prompt_graph(own)
+            if entry is not None:
+                return entry
+            if self._seen(own) >= self._worth_its_own(own, shared):
+                return self._captured_prompt_graph(own)
+        if shared is None:
+            return None
+        entry = self._known_prompt_graph(shared)
+        if entry is None and self._seen(shared) >= self.graph_after_sightings:
+            entry = self._captured_prompt_graph(shared)
+        return entry
+
+    def _worth_its_own(self, own, shared) -> int:
+        """Sightings after which a graph of a step's own shape has paid for its capture."""
+        if shared is None:
+            return self.OWN_SHAPE_AFTER
+        return -(-self.PADDING_WORTH_A_CAPTURE * own[3] // max(1, shared[3] - own[3]))
+
+    def _known_prompt_graph(self, key) -> dict | None:
         entry = self._graphs.get(key)
+        if entry is not None:
+            entry["copied"].synchronize()                   # the last step's copy has left the pinned buffer
+        return entry
+
+    def _seen(self, key) -> int:
+        """How often a shape without a graph has been asked for, this time with it."""
+        if len(self._sightings) > 4096:
+            self._sightings.clear()
+        seen = self._sightings[key] = self._sightings.get(key, 0) + 1
+        return seen
+
+    def _captured_prompt_graph(self, key) -> dict:
+        entry = self._new_prompt_graph(key)
+        evicted = self._capture_prompt_graph(entry)
+        del self._sightings[key]
+        if evicted is not None:                             # (more shapes in use than there is room for: one that has just gone waits for 16 sightings
+            self._sightings[evicted] = -16                  #  more than a new one before it takes another's place)
+        return entry
+
+    def _prompt_graph_step(self, entries: list, borrow: bool) -> torch.Tensor | None:
+        entry = self._prompt_graph(entries)
         if entry is None:
-            seen = self._sightings[key] = self._sightings.get(key, 0) + 1
-            if seen < self.graph_after_sightings:
-                if len(self._sightings) > 4096:
-                    self._sightings.clear()
-                return None                                 # run it eagerly this time
-            entry = self._new_prompt_graph(key)
-            evicted = self._capture_prompt_graph(entry)
-            if evicted is not None:                         # (more shapes in use than there is room for: a capture costs a dozen steps, so its
-                self._sightings[evicted] = self.graph_after_sightings - 16     #  shape waits for as many before it takes another's place)
-        else:
-            entry["copied"].synchronize()
+            return None
         n_want = self._stage_prompt_graph(entry, entries)
         entry["static"].copy_(entry["pinned"], non_blocking=True)
         entry["copied"].record()
@@ -695,10 +756,8 @@ class ModelRunner:
         key = self._graph_key(entries)
         if key is not None:
             return self._graph_step(key, entries, borrow)
-        key = self._prompt_graph_key(entries)
-        if key is not None:
-            logits = self._prompt_graph_step(key, entries, borrow)
-            if logits is not None:
-                return logits
+        logits = self._prompt_graph_step(entries, borrow) if self.prompt_graphs else None
+        if logits is not None:
+            return logits
         ctx = self.build_context(entries)
         return self.model.forward(ctx, self.kv, self.states)

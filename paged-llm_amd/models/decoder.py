@@ -122,6 +122,10 @@ class DecoderModel:
         flag = "graph_capturable_prompts" if prompts else "graph_capturable"
         return all(b.graph_capturable(prompts) for b in self.blocks) and all(getattr(op, flag, False) for op in self.stream_ops)
 
+    def padding_is_a_chunk(self) -> bool:
+        """Whether some layer's part pays for a sequence of padding tokens with more than its tokens (see ``ModelRunner``)."""
+        return any(b.padding_is_a_chunk() for b in self.blocks)
+
     def graph_step_arrays(self, layout) -> dict:
         """Host-made integer arrays the layers' parts need for a replayed step of that layout (equal keys are one array)."""
         out = {}

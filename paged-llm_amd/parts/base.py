@@ -274,6 +274,10 @@ class Block(Part):
         flag = "graph_capturable_prompts" if prompts else "graph_capturable"
         return all(getattr(p, flag, False) for role, p in self.parts.items() if self.ROLES[role] != "norm")
 
+    def padding_is_a_chunk(self) -> bool:
+        """Whether a sequence of padding tokens in a step with prompt portions costs a part more than its tokens (``padding_is_a_chunk`` on it)."""
+        return any(getattr(p, "padding_is_a_chunk", False) for p in self.parts.values())
+
     def graph_step_arrays(self, layout) -> dict:
         out = {}
         for part in self.parts.values():

@@ -62,6 +62,8 @@ def _chunks_from(ctx) -> int:
 class _StatefulMixer(Mixer):
     graph_capturable = True
     graph_capturable_prompts = True
+    # Whether its portions run in chunks whose workgroups fill the GPU just once (``ops.recurrence_form``): a padding sequence is a chunk more.
+    padding_is_a_chunk = False
     MATRICES: tuple = ()
 
     def _keep(self, name, tensor):
@@ -78,6 +80,8 @@ class Mamba2Mixer(_StatefulMixer):
     """params: ``heads``, ``head_dim`` (P), ``state`` (N), ``groups``, ``conv`` (taps), ``norm_groups``, ``eps``.
     Tensors: ``in`` [2 inner + 2 groups N + heads, width] laid out [z | x | B | C | dt], ``conv`` [inner + 2 groups N,
     taps] with ``conv.b``, ``dt_bias``, ``A_log``, ``D`` [heads], ``norm`` [inner], ``o`` [width, inner]."""
+
+    padding_is_a_chunk = True
 
     def __init__(self, params: dict, env: BuildEnv):
         self.hidden = env.hidden_size
@@ -132,6 +136,8 @@ class Mamba2Mixer(_StatefulMixer):
 class RetentionMixer(_StatefulMixer):
     """params: ``heads``, ``key_dim`` (N), ``head_dim`` (P), ``decay`` (one number per head), ``position`` (a position
     encoding spec, or None), ``eps``.  Tensors ``q``, ``k`` [heads N, width], ``v``, ``g`` [heads P, width], ``o``."""
+
+    padding_is_a_chunk = True
 
     def __init__(self, params: dict, env: BuildEnv):
         self.hidden = env.hidden_size
@@ -191,6 +197,8 @@ class MLstmMixer(_StatefulMixer):
     N, width], ``v``, ``g`` [heads P, width], ``i``, ``f`` [heads, width] with ``i.b``, ``f.b`` [heads], ``norm`` [heads P],
     ``o`` [width, heads P]."""
 
+    padding_is_a_chunk = True
+
     def __init__(self, params: dict, env: BuildEnv):
         self.hidden = env.hidden_size
         self.heads, self.N, self.P = int(params["heads"]), int(params["key_dim"]), int(params["head_dim"])
@@ -242,6 +250,8 @@ class LightningMixer(_StatefulMixer):
     params: ``heads``, ``key_dim`` (N), ``head_dim`` (P), ``decay`` (one number per head), ``eps``.  Tensors ``q``, ``k`` [heads N,
     width], ``v``, ``g`` [heads P, width], ``norm`` [heads P], ``o`` [width, heads P]."""
 
+    padding_is_a_chunk = True
+
     def __init__(self, params: dict, env: BuildEnv):
         self.hidden = env.hidden_size
         self.heads, self.N, self.P = int(params["heads"]), int(params["key_dim"]), int(params["head_dim"])
@@ -288,6 +298,8 @@ class Hgrn2Mixer(_StatefulMixer):
 
     params: ``heads``, ``key_dim`` (N), ``head_dim`` (P), ``eps``.  Tensors ``q``, ``f`` [heads N, width], ``f.b``, ``lower`` [heads N],
     ``v`` [heads P, width], ``norm`` [P], ``o`` [width, heads P]."""
+
+    padding_is_a_chunk = True
 
     def __init__(self, params: dict, env: BuildEnv):
         self.hidden = env.hidden_size

@@ -51,6 +51,65 @@ def portions(*lengths, singles=0, want="last"):
             + [StepEntry(f"p{i}", [1] * n, 0, {}, None, list(range(n)) if want == "all" else [n - 1]) for i, n in enumerate(lengths)])
 
 
+def taken(runner, *lengths, **kind):
+    """Portion tokens of the graph that the step is replayed from; None: eagerly."""
+    entry = runner._prompt_graph(portions(*lengths, **kind))
+    return None if entry is None else entry["key"][3]
+
+
+def test_a_step_shares_a_graph_until_its_own_shape_has_paid_for_one():
+    """140 tokens: in the shape of 192 from the second time on, in their own of 160 once 32 rows of padding were computed 50 times (as many as ten
+    steps of 160 hold); 180 tokens fill their own shape and the shared one alike."""
+    runner = runner_for()
+    assert [taken(runner, 140) for _ in range(49)] == [None] + [192] * 48
+    assert [taken(runner, 140) for _ in range(3)] == [160] * 3 and taken(runner, 180) == 192 and taken(runner, 192) == 192
+    assert [k[3] for k in runner.captured] == [192, 160]
+
+
+def test_graphs_beyond_a_thousand_tokens():
+    """Where a shared shape is filled exactly, and own shapes that come back again and again: not those of wide models with linear recurrences, for
+    which a padding sequence is a chunk more."""
+    plain, narrow, wide = runner_for(width=2048), runner_for(width=1024), runner_for(width=1025)
+    narrow.padding_is_a_chunk = wide.padding_is_a_chunk = True
+    for runner in (plain, narrow):
+        assert [taken(runner, 1100) for _ in range(101)] == [None] * 99 + [1104] * 2
+    assert [taken(wide, 1100) for _ in range(200)] == [None] * 200 and [taken(wide, 1104) for _ in range(101)] == [None] * 99 + [1104] * 2
+    for runner in (plain, narrow, wide):
+        assert [taken(runner, 2048) for _ in range(3)] == [None, 2048, 2048] and [taken(runner, 1280) for _ in range(3)] == [None, 1280, 1280]
+        assert [taken(runner, 2050) for _ in range(200)] == [None] * 200
+
+
+def test_which_models_say_that_padding_is_a_chunk():
+    from paged_llm_amd.engine.loading import build_model
+    from tests.gudutar_configs import GUDU_A
+    from tests.mekusun_configs import MEKU_A
+    from tests.tiny_configs import TINY_A
+    assert build_model(GUDU_A, "bfloat16", "cpu").padding_is_a_chunk()
+    assert not build_model(MEKU_A, "bfloat16", "cpu").padding_is_a_chunk() and not build_model(TINY_A, "bfloat16", "cpu").padding_is_a_chunk()
+
+
+def test_a_stream_of_prompts_of_every_length_captures_few_shapes():
+    """500 prompts of 16 to 2,048 tokens: no more captures than there are shared shapes (14 up to 1,024 tokens, four filled exactly beyond), and most steps
+    up to 1,024 tokens are replayed."""
+    import random
+    for width in (1024, 2048):
+        rng, runner = random.Random(5), runner_for(width=width)
+        lengths = [rng.randint(16, 2048) for _ in range(500)]
+        replayed = sum(taken(runner, n) is not None for n in lengths)
+        assert len(runner.captured) <= 18 and len(set(runner.captured)) == len(runner.captured)
+        assert replayed >= sum(n <= 1024 for n in lengths) - 18
+    scored = runner_for()
+    for n in lengths:
+        taken(scored, n, want="all")
+    assert len(scored.captured) <= 18
+
+
+def test_a_shape_that_had_to_go_waits_before_it_takes_anothers_place():
+    runner = runner_for(per_kind=1)
+    assert [taken(runner, 30) for _ in range(3)] == [None, 32, 32] and [taken(runner, 60) for _ in range(2)] == [None, 64]
+    assert [taken(runner, 30) for _ in range(19)] == [None] * 17 + [32] * 2
+
+
 def test_the_warm_up_of_a_shape_stays_within_its_bound():
     """Its portions are as long as one another, so none has positions that the model has no tables for: four portions of 26 tokens, all that a model
     of 26 positions takes, share a shape of 128 tokens with a padding sequence, of 26 each at most."""
@@ -58,7 +117,8 @@ def test_the_warm_up_of_a_shape_stays_within_its_bound():
         runner = runner_for(max_positions=positions)
         for count in (1, 2, 3, 4):
             for n in range(2, positions + 1):
-                key = runner._prompt_graph_key(portions(*[n] * count))
-                if key is not None:
-                    each = runner._even_portions(key[3], count + 1)
-                    assert sum(each) == key[3] and max(each) <= key[5] <= positions, (positions, count, n)
+                for shared in (True, False):
+                    key = runner._prompt_graph_key(portions(*[n] * count), shared=shared)
+                    if key is not None:
+                        each = runner._even_portions(key[3], count + 1)
+                        assert sum(each) == key[3] and max(each) <= key[5] <= positions, (positions, count, n)

@@ -46,3 +46,34 @@ def test_logits_of_a_replay_are_the_callers(folders):  # noqa: F811
     other = step("b", texts[1])
     assert first.shape == (140, TINY_A["vocab_size"]) and other.shape == (155, TINY_A["vocab_size"]) and torch.equal(first, kept)
     assert torch.equal(step("c", texts[0]), kept)
+
+
+@pytest.mark.parametrize("dtype", ["float32", "bfloat16"])
+def test_portions_that_hold_more_tokens_than_the_context_bound(folders, dtype):  # noqa: F811
+    """Four portions together longer than any position of the model, replayed from one graph and, between the replays, run eagerly: the same
+    logits up to the type's rounding (a padded step's products may take other tiles)."""
+    from paged_llm_amd.engine.batch import StepEntry
+    from paged_llm_amd.engine.loading import build_runtime, load_model
+    from tests.test_replay_gpu import TOL
+    model = load_model(folders["A", dtype], dtype, "cuda")
+    manager, _, runner = build_runtime(model, 16, 80, 8, enable_prefix_caching=False, use_graphs=True, graph_after_sightings=1)
+
+    def logits(lengths, graphs):
+        entries = []
+        for i, n in enumerate(lengths):
+            assert manager.allocate(i, 0, n)
+            tables, slot, version = manager.step_fields(i)
+            entries.append(StepEntry(i, helpers.random_tokens(n, TINY_A["vocab_size"], seed=n + i), 0, {g: list(t) for g, t in tables.items()}, slot,
+                                     [0, n - 1], version))
+        runner.prompt_graphs = True
+        key = runner._prompt_graph_key(entries, shared=True)
+        assert key[3] > key[5] == model.max_positions
+        runner.prompt_graphs = graphs
+        out = runner.step(entries)
+        for i in range(len(lengths)):
+            manager.free(i)
+        return out
+    for lengths in [(100, 101, 99, 90), (60, 130, 120, 111), (2, 200, 100, 96), (100, 101, 99, 90)]:
+        got, want = logits(lengths, True), logits(lengths, False)
+        assert (got - want).abs().max() <= TOL[dtype] * want.abs().max()
+    assert [k[0] for k in runner._graphs] == ["prompt"], "one shape holds them all"
