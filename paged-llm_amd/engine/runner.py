@@ -9,6 +9,8 @@ of the new tokens.
 
 from __future__ import annotations
 
+import contextlib
+import gc
 from collections import OrderedDict
 
 import numpy as np
@@ -21,6 +23,19 @@ from .batch import GroupView, StepContext, StepEntry
 
 class StepError(ValueError):
     pass
+
+
+@contextlib.contextmanager
+def _no_collection():
+    """No garbage collection by itself during a capture: the collector may come upon the graphs of a runner that is gone, and a graph
+    cannot be destroyed while a stream is capturing (the process would abort)."""
+    was = gc.isenabled()
+    gc.disable()
+    try:
+        yield
+    finally:
+        if was:
+            gc.enable()
 
 
 class GraphCache:
@@ -319,7 +334,7 @@ class ModelRunner:
         torch.cuda.current_stream(self.device).wait_stream(stream)
         torch.cuda.synchronize(self.device)
         graph = torch.cuda.CUDAGraph()
-        with torch.cuda.graph(graph, stream=stream):
+        with _no_collection(), torch.cuda.graph(graph, stream=stream):
             logits = self.model.forward(ctx, self.kv, self.states)
         entry.update(graph=graph, logits=logits, ctx=ctx)
         self._graphs.put(entry["key"], entry)
@@ -618,7 +633,7 @@ class ModelRunner:
         if self._graph_pool is None:
             self._graph_pool = torch.cuda.graph_pool_handle()
         graph = torch.cuda.CUDAGraph()
-        with torch.cuda.graph(graph, stream=stream, pool=self._graph_pool):
+        with _no_collection(), torch.cuda.graph(graph, stream=stream, pool=self._graph_pool):
             result = forward()
         entry.update(graph=graph, ctx=ctx, **{"head_rows" if apart else "logits": result})
         return self._graphs.put(entry["key"], entry)

@@ -77,3 +77,35 @@ def test_portions_that_hold_more_tokens_than_the_context_bound(folders, dtype): 
         got, want = logits(lengths, True), logits(lengths, False)
         assert (got - want).abs().max() <= TOL[dtype] * want.abs().max()
     assert [k[0] for k in runner._graphs] == ["prompt"], "one shape holds them all"
+
+
+@pytest.mark.parametrize("tokens", [1, 40])
+def test_a_capture_leaves_the_graphs_of_a_runner_that_is_gone_alone(folders, tokens):  # noqa: F811
+    """A runner that only a cycle keeps, dropped while another one captures: its graphs go with a later collection."""
+    import gc
+    from paged_llm_amd.engine.batch import StepEntry
+    from paged_llm_amd.engine.loading import build_runtime, load_model
+    model = load_model(folders["A", "bfloat16"], "bfloat16", "cuda")
+
+    def stepped(n):
+        manager, _, runner = build_runtime(model, 16, 16, 2, enable_prefix_caching=False, use_graphs=True, graph_after_sightings=1)
+        assert manager.allocate(0, 0, n)
+        tables, slot, version = manager.step_fields(0)
+        return runner, runner.step([StepEntry(0, [5] * n, 0, {g: list(t) for g, t in tables.items()}, slot, [n - 1], version)])
+    gone, want = stepped(tokens)
+    gone.itself = gone
+    held, forward = [gone], model.forward
+    del gone
+
+    def dropping(*args, **kwargs):
+        if torch.cuda.is_current_stream_capturing() and held:
+            held.clear()
+            [[i] for i in range(100000)]                    # (so many containers start a collection)
+            assert not gc.isenabled()
+        return forward(*args, **kwargs)
+    model.forward = dropping
+    try:
+        runner, got = stepped(tokens)
+    finally:
+        del model.forward
+    assert not held and len(runner._graphs) == 1 and gc.isenabled() and torch.equal(got, want)
