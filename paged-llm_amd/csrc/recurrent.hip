@@ -831,7 +831,7 @@ __global__ __launch_bounds__(64 * WAVES, 2) void recurrence_piece_kernel(Recurre
       // The tiles of M on the diagonal: sixteen lanes share a key, NT of its rows each, added in their order and then over the lanes.
       // What bounds it is LDS: so every sixteen lanes take two keys, a token's decays and queries read for both, and nothing stands
       // behind a condition, so that the reads of the tokens to come are under way (16 heads
-      // of 128 x 128, 777 tokens in pieces 441 -> 298 us with the walks above, in chunks 66.5 -> 56.4; 64 of 64 x 64 333 -> 232 and 94 -> 74).
+      // of 128 x 128, 777 tokens in pieces 441 -> 289 us with the walks above, in chunks 66.5 -> 55.5; 64 of 64 x 64 333 -> 224 and 94 -> 73).
       for (int eight = wave; eight < 4; eight += WAVES) {
         const int first = (eight >> 1) * 16, j0 = first + (eight & 1) * 8 + quad, n = c16 * NT;      // keys j0 and j0 + 4
         float w[2][NT];
@@ -854,13 +854,13 @@ __global__ __launch_bounds__(64 * WAVES, 2) void recurrence_piece_kernel(Recurre
               w[k][i] = t > j ? w[k][i] * d[i] : w[k][i];
               dot[k] = fmaf(w[k][i], q[i], dot[k]);
             }
-            dot[k] = t >= j ? dot[k] : 0.f;
             dot[k] += dpp_move<kDppSwap1>(dot[k]);
             dot[k] += dpp_move<kDppSwap2>(dot[k]);
             dot[k] += dpp_move<kDppHalfMirror>(dot[k]);
             dot[k] += dpp_move<kDppMirror>(dot[k]);
           }
-          if (c16 < 2) M[t * kPieceLd + j0 + 4 * c16] = (c16 ? dot[1] : dot[0]) * g;
+          // (a key behind the token: zero, whatever its gain is)
+          if (c16 < 2) M[t * kPieceLd + j0 + 4 * c16] = t >= j0 + 4 * c16 ? (c16 ? dot[1] : dot[0]) * g : 0.f;
         }
       }
       __syncthreads();

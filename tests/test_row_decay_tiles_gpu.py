@@ -57,3 +57,18 @@ def test_neighbouring_rows_are_added_in_their_order(N, monkeypatch):
     y = ops.linear_recurrence(q.cuda(), k.cuda(), v.cuda(), None, torch.zeros(1, N * 16, device="cuda"), 0, at(0), at(0), at(0, 32), 1, max_q_len=32,
                               row_decay=torch.ones(32, 1, N).cuda())
     assert not bool(y[:16].any())
+
+
+@pytest.mark.parametrize("N", [32, 64, 128])
+@pytest.mark.parametrize("form", [-1, 64])
+@pytest.mark.parametrize("value", [float("nan"), float("inf")])
+def test_a_gain_that_is_no_number_reaches_its_own_token_and_later_ones_only(N, form, value, monkeypatch):
+    """In pieces and in chunks, with earlier tokens of the same tile, other tiles and another head beside it."""
+    from paged_llm_amd.csrc import ops
+    monkeypatch.setattr(ops, "recurrence_form", lambda *a, **k: form)
+    q, k, v, gain = torch.rand(100, 2, N) + 0.1, torch.rand(100, 2, N), torch.rand(100, 2, 16) + 0.1, torch.rand(100, 2) + 0.1
+    gain[41, 0] = value
+    at = lambda *x: torch.tensor(x, dtype=torch.int32, device="cuda")
+    y = ops.linear_recurrence(q.cuda(), k.cuda(), v.cuda(), None, torch.zeros(1, 2 * N * 16, device="cuda"), 0, at(0), at(0), at(0, 100), 1,
+                              vscale=gain.cuda(), max_q_len=100, row_decay=torch.full((100, 2, N), 0.9).cuda()).cpu().view(100, 2, 16)
+    assert bool(torch.isfinite(y[:, 1]).all() and torch.isfinite(y[:41, 0]).all()) and not bool(torch.isfinite(y[41:, 0]).any())
