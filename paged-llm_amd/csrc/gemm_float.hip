@@ -437,18 +437,20 @@ PLLM_API int pllm_gemm_float_fused(int epi, const float* A, int lda, const float
 template <int EPI>
 __global__ __launch_bounds__(64) void float_split_weights_kernel(FloatGemm g, bf16x8* out) {
   const int lane = threadIdx.x, k = blockIdx.x * kStep + 4 * (lane >> 4);
-  const float* row = g.W + (size_t)weight_row<EPI>(g, 16 * blockIdx.y + (lane & 15)) * g.ldw + k;
-  const Triple t = split(Octet{four_of(row, g.K - k), four_of(row + 16, g.K - k - 16)});
+  for (int tile = blockIdx.y; tile < g.col_tiles; tile += gridDim.y) {   // (a grid has 65,535 of them at most)
+    const float* row = g.W + (size_t)weight_row<EPI>(g, 16 * tile + (lane & 15)) * g.ldw + k;
+    const Triple t = split(Octet{four_of(row, g.K - k), four_of(row + 16, g.K - k - 16)});
 #pragma unroll
-  for (int p = 0; p < 3; ++p) out[(((size_t)blockIdx.y * gridDim.x + blockIdx.x) * 3 + p) * 64 + lane] = t.part[p];
+    for (int p = 0; p < 3; ++p) out[(((size_t)tile * gridDim.x + blockIdx.x) * 3 + p) * 64 + lane] = t.part[p];
+  }
 }
 
 PLLM_API int pllm_float_split_weights(int epi, const float* W, int ldw, int N, int K, int head_dim, void* out, hipStream_t stream) {
-  if (N <= 0 || K <= 0 || (N + 15) / 16 > 65535 || reinterpret_cast<uintptr_t>(out) % 16) return -2;
+  if (N <= 0 || N > 0x7fffffff - 15 || K <= 0 || reinterpret_cast<uintptr_t>(out) % 16) return -2;
   if ((epi == FG_GATED && N % 2) || (epi == FG_ROPE_KV && (head_dim <= 0 || head_dim % 16 || N % head_dim))) return -2;
   FloatGemm g{};
-  g.W = W; g.ldw = ldw; g.N = N; g.K = K; g.head_dim = head_dim;
+  g.W = W; g.ldw = ldw; g.N = N; g.K = K; g.head_dim = head_dim; g.col_tiles = (N + 15) / 16;
   auto kernel = epi == FG_PLAIN ? float_split_weights_kernel<FG_PLAIN> : epi == FG_GATED ? float_split_weights_kernel<FG_GATED> : float_split_weights_kernel<FG_ROPE_KV>;
-  hipLaunchKernelGGL(kernel, dim3((K + kStep - 1) / kStep, (N + 15) / 16), dim3(64), 0, stream, g, (bf16x8*)out);
+  hipLaunchKernelGGL(kernel, dim3((K + kStep - 1) / kStep, min(g.col_tiles, 65535)), dim3(64), 0, stream, g, (bf16x8*)out);
   PLLM_RETURN_LAST_ERROR();
 }

@@ -98,3 +98,22 @@ def test_which_products_take_the_parts():
     assert o.float_split_plan(95, 2048, 2048, 256) is None and o.float_split_plan(301, 2048, 480, 256) is None
     assert o.float_split_plan(301, 2048, 2048, 256) == (3, 4) and o.float_split_plan(301, 11264, 2048, 256) == (4, 4)
     assert o.float_split_plan(128, 2048, 2048, 256) is None               # (tiles of 32 x 32 from the floats are ahead)
+
+
+@pytest.mark.parametrize("pairing,n", [("plain", 1 << 20), ("plain", (1 << 20) - 15), ("gated", 1 << 20)])
+def test_parts_of_as_many_rows_as_a_matrix_may_have(pairing, n):
+    """65,536 tiles of 16 rows, one more than a grid has: the last rows' parts are those of a matrix of these rows alone."""
+    o = ops()
+    w = torch.zeros(n, 32, device="cuda")
+    last = rnd(40, 32, seed=14).cuda()
+    w[-40:] = last
+    assert o.float_split_takes(w)
+    parts = o.float_split_weights(w, pairing)
+    if pairing == "plain":
+        few = o.float_split_weights(w[(n - 40) // 16 * 16:])
+        assert parts.shape[0] == (n + 15) // 16 and torch.equal(parts[-few.shape[0]:].view(torch.int16), few.view(torch.int16))
+    else:
+        gate, up = torch.zeros(48, 32, device="cuda"), w[-48:]
+        assert torch.equal(parts[-6:].view(torch.int16), o.float_split_weights(torch.cat([gate, up]), "gated").view(torch.int16))
+    del parts, w
+    torch.cuda.empty_cache()
