@@ -27,6 +27,8 @@ def pages_that_fit(model, config) -> int:
     stay within ``gpu_memory_utilization`` of the device, but never more than ``max_num_seqs`` requests of
     ``max_model_len`` positions could hold."""
     device, bs = model.device, config.block_size
+    # (what a model lays out with its first steps, as copies of weights in another order, is resting memory: it is there before anything is measured)
+    _probe_step(model, bs, config.max_num_batched_tokens, config.max_num_seqs)
     torch.cuda.empty_cache()
     torch.cuda.reset_peak_memory_stats(device)
     resting = torch.cuda.memory_allocated(device)

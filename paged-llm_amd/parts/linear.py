@@ -18,6 +18,8 @@ be a tensor or a ``PendingNorm``; a weight may be a tensor [N, K] or a ``Weight`
 
 from __future__ import annotations
 
+import threading
+
 import torch
 
 from ..csrc import ops
@@ -29,16 +31,49 @@ class Weight:
     order that the streaming kernel reads (1 KB tiles in the matrix instruction's operand order; see
     ``ops.tile_weight``).  ``pairing``: which rows share a tile, by what the epilogue behind the product needs:
     "plain", "gated" ([gate; up] rows) or "rotary" ([q; k; v] rows of heads of ``head_dim``).  The plain copy serves
-    the other kernels and the library; a step reads one of the two.  A float32 matrix has its elements' bfloat16 parts as the second
-    copy instead (``split``, 6 bytes an element), which float products of many rows take (``ops.float_split_plan``)."""
+    the other kernels and the library; a step reads one of the two.  A float32 matrix gets its elements' bfloat16 parts as the second
+    copy instead (6 bytes an element), which float products of many rows take (``ops.float_split_plan``), with the first of them:
+    a program whose steps have few rows, or whose products go another way, has the floats alone (``parts``)."""
+
+    # The share of the GPU's memory up to which this process may have allocated memory, a copy of parts with it.  A copy saves a product of many
+    # rows 10 to 20 %; the floats of a model that needs more, or of one beside a large cache pool, stay as they are.
+    PARTS_MEMORY_SHARE = 0.25
+    _parts_lock = threading.Lock()
 
     def __init__(self, plain: torch.Tensor, pairing: str = "plain", head_dim: int = 0):
         self.plain = plain
         self.pairing = pairing
         ok = ops.stream_linear_takes(plain) and (pairing != "rotary" or (head_dim > 0 and head_dim % 16 == 0))
         self.tiled = ops.tile_weight(plain, pairing, head_dim) if ok else None
-        ok = ops.float_split_takes(plain) and (pairing != "rotary" or (head_dim > 0 and head_dim % 16 == 0))
-        self.split = ops.float_split_weights(plain, pairing, head_dim) if ok else None
+        self.head_dim = head_dim
+        self._parts = None
+        self._takes_parts = ops.float_split_takes(plain) and (pairing != "rotary" or (head_dim > 0 and head_dim % 16 == 0))
+
+    def parts(self, rows: int, pairing: str) -> torch.Tensor | None:
+        """The parts for a float product of ``rows`` rows with the epilogue of ``pairing``, made when the first product asks for them that is faster from
+        them; None: a product from the floats (the same bits).  The copy is there for every stream before anybody sees it, and none is made
+        inside a capture."""
+        if self._parts is not None or not self._takes_parts or pairing != self.pairing:
+            return self._parts if pairing == self.pairing else None
+        device = self.plain.device
+        if ops.float_split_plan(rows, *self.plain.shape, ops._num_compute_units(device)) is None or torch.cuda.is_current_stream_capturing():
+            return None
+        with self._parts_lock:
+            if self._parts is None and self._takes_parts:
+                self._parts = self._made_parts(device)
+                self._takes_parts = self._parts is not None
+        return self._parts
+
+    def _made_parts(self, device) -> torch.Tensor | None:
+        limit = self.PARTS_MEMORY_SHARE * torch.cuda.get_device_properties(device).total_memory
+        if torch.cuda.memory_allocated(device) + ops.float_split_bytes(*self.plain.shape) > limit:
+            return None
+        try:
+            parts = ops.float_split_weights(self.plain, self.pairing, self.head_dim)
+        except torch.OutOfMemoryError:                      # (somebody else's memory)
+            return None
+        torch.cuda.current_stream(device).synchronize()
+        return parts
 
     @property
     def shape(self):
@@ -51,6 +86,13 @@ class Weight:
     def rows(self, count: int) -> torch.Tensor:
         """The first ``count`` rows as a plain matrix (a view)."""
         return self.plain[:count]
+
+
+def _parts_for(x: torch.Tensor, weight, pairing: str) -> torch.Tensor | None:
+    """The parts of a float32 matrix that the product of these rows takes, or None."""
+    if not isinstance(weight, Weight) or not ops.gemm_float_fused_takes(x, weight.plain):
+        return None
+    return weight.parts(x.shape[0], pairing)
 
 
 STREAM_MIN_ROWS, STREAM_MAX_ROWS = 17, 128      # rows the streaming kernel is chosen for
@@ -216,14 +258,14 @@ def linear(x, weight, out_dtype: torch.dtype | None = None, partial_ok: bool = F
         out = _fused(x, weight, ops.EPI_F32 if out_dtype == torch.float32 else ops.EPI_BF16)
         if out is not None:
             return out
-    split = weight.split if isinstance(weight, Weight) and weight.pairing == "plain" else None
-    weight = _plain(weight)
+    matrix, weight = weight, _plain(weight)
     x = rows_of(x)
     if x.dtype == torch.bfloat16 and weight.dtype == torch.bfloat16:
         return ops.gemm_bf16(x, weight, out_dtype)
     if x.dtype == weight.dtype == torch.float32:
         out = ops.gemm_float_halves(x, weight) if partial_ok else None
-        if out is None and split is not None:
+        split = _parts_for(x, matrix, "plain") if out is None else None
+        if split is not None:
             out = ops.gemm_float_split(x, weight, split)
         if out is not None:
             return out
@@ -295,12 +337,11 @@ def gated_linear(x, w_gate_up, activation: str = "silu") -> torch.Tensor:
         out = _fused(x, w_gate_up, ops.EPI_GATED, activation=activation)
         if out is not None:
             return out
-    split = w_gate_up.split if isinstance(w_gate_up, Weight) and w_gate_up.pairing == "gated" else None
-    w_gate_up = _plain(w_gate_up)
+    matrix, w_gate_up = w_gate_up, _plain(w_gate_up)
     if w_gate_up.dtype == torch.float32:
         x = rows_of(x)
         if ops.gemm_float_fused_takes(x, w_gate_up):
-            return ops.gemm_float_gated(x, w_gate_up, activation, split)
+            return ops.gemm_float_gated(x, w_gate_up, activation, _parts_for(x, matrix, "gated"))
     return ops.gate_mul(linear(x, w_gate_up), activation)
 
 
@@ -370,8 +411,7 @@ def qkv_rotary_cache(x, w_qkv, positions: torch.Tensor, position_encoding, num_h
         elif k_pages.dtype == torch.float32:
             x = rows_of(x)
             if ops.gemm_float_fused_takes(x, _plain(w_qkv)):
-                split = w_qkv.split if isinstance(w_qkv, Weight) and w_qkv.pairing == "rotary" else None
-                return ops.gemm_float_rotary(x, _plain(w_qkv), rope, split)
+                return ops.gemm_float_rotary(x, _plain(w_qkv), rope, _parts_for(x, w_qkv, "rotary"))
     w_qkv = _plain(w_qkv)
     qkv = linear(x, w_qkv, bias=bias)
     ops.rope_scatter(qkv, positions, cos, sin, num_heads, num_kv_heads, head_dim, slot_mapping if write else None,

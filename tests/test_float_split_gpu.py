@@ -117,3 +117,56 @@ def test_parts_of_as_many_rows_as_a_matrix_may_have(pairing, n):
         assert torch.equal(parts[-6:].view(torch.int16), o.float_split_weights(torch.cat([gate, up]), "gated").view(torch.int16))
     del parts, w
     torch.cuda.empty_cache()
+
+
+def test_a_matrix_has_its_parts_from_the_first_product_on_that_is_faster_from_them(monkeypatch):
+    """Not for few rows, short rows or another epilogue, not inside a capture, and not past the share of the memory; the product's bits are the same."""
+    from paged_llm_amd.parts import linear as L
+    o = ops()
+    w, x = rnd(2048, 2048, seed=15).cuda(), rnd(301, 2048, seed=16).cuda()
+    want = o.gemm_generic(x, w)
+    matrix = L.Weight(w)
+    assert torch.equal(L.linear(x[:8], matrix), o.gemm_generic(x[:8], w)) and matrix._parts is None
+    assert matrix.parts(301, "gated") is None and L.Weight(w[:, :480].contiguous()).parts(301, "plain") is None
+    graph, stream = torch.cuda.CUDAGraph(), torch.cuda.Stream()
+    with torch.cuda.graph(graph, stream=stream):
+        captured = L.linear(x, matrix)
+    graph.replay()
+    assert torch.equal(captured, want) and matrix._parts is None
+    with torch.cuda.stream(stream):
+        made = L.linear(x, matrix)
+    assert matrix._parts is not None and torch.equal(L.linear(x, matrix), want)          # (another stream than the one that made them)
+    stream.synchronize()
+    assert torch.equal(made, want)
+    for share in (0.0, 0.25):
+        monkeypatch.setattr(L.Weight, "PARTS_MEMORY_SHARE", share)
+        other = L.Weight(w)
+        assert torch.equal(L.linear(x, other), want) and (other._parts is None) == (share == 0.0)
+
+    def out_of_memory(*a):
+        raise torch.OutOfMemoryError
+    monkeypatch.setattr(o, "float_split_weights", out_of_memory)
+    other = L.Weight(w)
+    assert torch.equal(L.linear(x, other), want) and other._parts is None and other.parts(301, "plain") is None
+
+
+def test_several_threads_ask_for_the_parts_at_once():
+    import threading
+
+    from paged_llm_amd.parts import linear as L
+    o = ops()
+    w, x = rnd(2048, 2048, seed=17).cuda(), rnd(301, 2048, seed=18).cuda()
+    want, matrix, got = o.gemm_generic(x, w), L.Weight(w), [None] * 6
+    torch.cuda.synchronize()
+
+    def product(i):
+        stream = torch.cuda.Stream()
+        with torch.cuda.stream(stream):
+            got[i] = L.linear(x, matrix)
+        stream.synchronize()
+    threads = [threading.Thread(target=product, args=(i,)) for i in range(6)]
+    for t in threads:
+        t.start()
+    for t in threads:
+        t.join()
+    assert all(torch.equal(y, want) for y in got)
