@@ -63,3 +63,12 @@ def test_which_cut():
     plan = lambda q, seqs, keys, heads=32, kv=4, d=64: o.float_attention_plan(q, seqs, heads, kv, d, 0, keys, 256)
     assert plan(8, 8, 700) == plan(1, 1, 180) == plan(61, 61, 2000) == plan(8, 8, 512, 16, 1, 256) == 4
     assert plan(12, 12, 100) == plan(301, 1, 301) == plan(64, 1, 64) == plan(128, 1, 128) == plan(2000, 1, 2000) == 1
+
+
+def test_short_windows_are_one_workgroups():
+    """The kernel has one form for windows that reach up to 128 positions, so no place is set aside for the parts of four workgroups."""
+    o = ops()
+    plan = lambda window, q=8, seqs=8, heads=32, kv=4, d=64: o.float_attention_plan(q, seqs, heads, kv, d, window, 2000, 256)
+    for window in (1, 16, 100, 128):
+        assert plan(window) == plan(-window) == plan(window, 1, 1, 16, 1, 256) == 1
+    assert plan(0) == plan(1024) == 4
