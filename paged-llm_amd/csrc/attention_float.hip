@@ -21,8 +21,10 @@
 // block in front of it and its values behind that block's, blocks are so small that keys, values and a group fit 168 registers (three
 // wavefronts a SIMD; two for heads to 128, one beyond), and few tiles go to four times the compute units.  Against eight wavefronts a tile with
 // blocks of 64 loaded as they come (32 heads of 64 on 4): decoding 8 requests at contexts to 700 18.5 -> 12.1 us, at 2,040 38 -> 18.3, one at 180 10.1 ->
-// 8.0, 61 at contexts to 2,000 57 -> 46; prompts of 301 tokens 29.6 -> 17.5, 2,000 358 -> 266; 16 heads of 256 on one at 512 44 -> 19.3.  A portion of
-// 100 tokens behind 1,000 lies between the forms: 26 -> 28.
+// 8.0, 61 at contexts to 2,000 57 -> 46; prompts of 301 tokens 29.6 -> 17.5, 2,000 358 -> 266; 16 heads of 256 on one at 512 44 -> 19.3.  Over 576 shapes
+// (1 to 61 sequences of 1 to 1,000 tokens at contexts of 60 to 3,000, heads of 64 to 256) 22 % less time with heads of 64, 27 % to 128 and 38 % beyond; what lies
+// between the forms is slower: as many tiles as compute units with heads of 256 (200 tokens 23.7 -> 27.8, 1,000 172 -> 191), one head a kv head
+// (16 requests at 700, 12 heads of 64: 21.9 -> 24.0), portions of 100 tokens behind 1,000 25.8 -> 26.3.
 #include "common.h"
 
 using namespace pllm;

@@ -72,3 +72,10 @@ def test_short_windows_are_one_workgroups():
     for window in (1, 16, 100, 128):
         assert plan(window) == plan(-window) == plan(window, 1, 1, 16, 1, 256) == 1
     assert plan(0) == plan(1024) == 4
+
+
+def test_portions_behind_a_context_take_the_form_that_was_ahead():
+    o = ops()
+    plan = lambda q, keys, heads=32, kv=4, d=64: o.float_attention_plan(q, 1, heads, kv, d, 0, keys, 256)
+    assert plan(100, 600) == plan(301, 301) == plan(200, 1200, 16, 1, 256) == plan(200, 200, 16, 1, 256) == 1
+    assert plan(25, 1025) == plan(50, 1050) == plan(33, 2033) == plan(100, 1100, 16, 1, 256) == plan(100, 1100, 16, 8, 128) == 4
