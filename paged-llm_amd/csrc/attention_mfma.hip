@@ -1175,6 +1175,7 @@ static int launch_attention(const void* q, int q_stride, const void* k_pages, co
   // Sequences by length where the workgroups are more than the compute units and the longest may take a while (ragged contexts up to
   // 2,000, us, as given / by length: 61 sequences x 8 kv heads of 64 38.3 / 31.3, 40 31.4 / 25.4 with eight wavefronts, 61 x 8 of 128 69.1 / 57.3;
   // 64 up to 600 13.5 / 13.6, all of 2,000 58.8 / 58.7; with a compute unit for every workgroup the order only costs: 33 x 4 up to 1,200 12.7 / 13.8).
+  // At most 64 of them, a lane each of the wavefront that counts: more keep the order given.
   const int cus = num_compute_units();
   const bool by_length = waves > 1 && partition_size == 0 && tiles == 1 && longest > 512 && longest < 1 << 24 && num_seqs <= 64 &&
                          num_kv_heads <= cus && num_seqs * num_kv_heads > cus;

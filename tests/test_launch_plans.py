@@ -168,3 +168,11 @@ def test_wide_products_fill_one_round():
                 tile = plan(rows, weight_rows, 2048, epi, 256)
                 if tile is not None:
                     assert 128 <= -(-rows // tile[0]) * -(-weight_rows // tile[1]) <= 256
+
+
+def test_sequences_behind_a_window_are_taken_as_they_come():
+    """The order by length is for layers that see whole sequences: without a window, or with one that no sequence is longer than."""
+    assert ops.longest_in_turn(0, 2000) == ops.longest_in_turn(2000, 2000) == ops.longest_in_turn(-4096, 2000) == 2000
+    for window in (1, 128, 512, 1024, 1999, -512):
+        assert ops.longest_in_turn(window, 2000) == 0
+    assert ops.longest_in_turn(0, 0) == ops.longest_in_turn(512, 0) == 0
