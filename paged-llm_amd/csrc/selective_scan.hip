@@ -49,6 +49,7 @@ __device__ __forceinline__ float uniform_element(const bf16* row, int i) {
   return __uint_as_float((i & 1) ? pair & 0xffff0000u : pair << 16);
 }
 
+constexpr int kAheadWaves = 3 * 1024;     // three a SIMD of 256 compute units
 enum { kScanWhole = 0, kScanState = 1, kScanOut = 2 };
 constexpr int kScanAhead = 4;            // tokens whose rows are asked for at once
 
@@ -71,7 +72,10 @@ __device__ __forceinline__ bool scan_chunk_of(const int* __restrict__ cu, int nu
 // token's B and C and every four tokens' rows waited for, and so (16 numbers of state): 602 and 576 tokens x 4,096 channels 80.5 and 77.4,
 // 300 x 2,048 34.1 and 28.3, 129 x 4,096 33.1 and 28.1, 777 x 1,000 with 8 numbers 31.7 and 28.7, 2,048 x 4,096 100.6 and 100.4 (the
 // exponentials); rows ahead alone gave 0 to 4 % of it.
-template <typename T, typename TB, int NR, int MAX_THREADS, int MODE>
+// AHEAD: so.  The two sets of rows take 8 to 13 registers, and with 32 numbers a lane that is a wavefront less on a SIMD: ahead while there are no more
+// wavefronts than three a SIMD (300 x 2,048 with 64 numbers 63.7 and 58.8, 500 x 1,024 with 128 69.8 and 64.3), not beyond (2,048 x 2,048 with 64 153
+// and 170, 2,048 x 4,096 with 32 149 and 156).
+template <typename T, typename TB, int NR, int MAX_THREADS, int MODE, bool AHEAD>
 __global__ __launch_bounds__(MAX_THREADS) void selective_scan_kernel(ScanArgs a, const TB* __restrict__ bc, long bc_stride) {
   __shared__ float part[2][MAX_THREADS / 64][64];
   const int lane = threadIdx.x & 63, wv = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), waves = blockDim.x >> 6;
@@ -115,7 +119,7 @@ __global__ __launch_bounds__(MAX_THREADS) void selective_scan_kernel(ScanArgs a,
       if (MODE != kScanState) f.z[u] = zp[(size_t)t * a.z_stride];
     }
   };
-  constexpr bool kRowAhead = MODE != kScanWhole && NR <= 16;            // (two rows of up to 32 numbers fit the scalar registers; more do not)
+  constexpr bool kRowAhead = AHEAD && NR <= 16;            // (two rows of up to 32 numbers fit the scalar registers; more do not)
   float nb[NR], nc[NR];                                                 // the next token's B and C
   auto row_of = [&](int n) { return bc + (size_t)(q_begin + (MODE == kScanState ? t_last - 1 - (n - t_first) : n)) * bc_stride; };
   auto fetch_row = [&](int n) {
@@ -174,7 +178,7 @@ __global__ __launch_bounds__(MAX_THREADS) void selective_scan_kernel(ScanArgs a,
     }
   };
   Ahead one;
-  if constexpr (MODE == kScanWhole) {                         // (mostly single tokens)
+  if constexpr (!AHEAD) {
     for (int tb = t_first; tb < t_last; tb += kScanAhead) {
       fetch(one, tb);
       walk(one, tb);
@@ -238,11 +242,15 @@ template <typename T, typename TB, int MODE>
 static void launch_scan(const ScanArgs& a, const void* bc, long bc_stride, int rows, hipStream_t stream) {
   const int waves = (a.N + 31) / 32;
   dim3 grid((a.channels + 63) / 64, rows), block(64 * waves);
-#define PLLM_SCAN(NR, MAX_THREADS) hipLaunchKernelGGL((selective_scan_kernel<T, TB, NR, MAX_THREADS, MODE>), grid, block, 0, stream, a, (const TB*)bc, bc_stride)
-  if (a.N == 8) PLLM_SCAN(8, 256);
-  else if (a.N == 16) PLLM_SCAN(16, 256);
-  else if (waves <= 4) PLLM_SCAN(32, 256);
-  else PLLM_SCAN(32, 1024);
+  constexpr bool kChunks = MODE != kScanWhole;                // (whole sequences are mostly single tokens)
+  const bool ahead = kChunks && (long)grid.x * rows * waves <= kAheadWaves;
+#define PLLM_SCAN(NR, MAX_THREADS, AHEAD) \
+  hipLaunchKernelGGL((selective_scan_kernel<T, TB, NR, MAX_THREADS, MODE, AHEAD>), grid, block, 0, stream, a, (const TB*)bc, bc_stride)
+  if (a.N == 8) PLLM_SCAN(8, 256, kChunks);
+  else if (a.N == 16) PLLM_SCAN(16, 256, kChunks);
+  else if (waves <= 4) { if (ahead) PLLM_SCAN(32, 256, kChunks); else PLLM_SCAN(32, 256, false); }
+  else if (ahead) PLLM_SCAN(32, 1024, kChunks);
+  else PLLM_SCAN(32, 1024, false);
 #undef PLLM_SCAN
 }
 

@@ -36,3 +36,23 @@ def test_portions_around_the_tokens_asked_for_at_once(lens, N):
             assert bool(((held[s].cpu().double().view(N, C) - h).abs() <= bound * size + 1e-12).all())
         else:
             assert torch.equal(held[s].cpu(), state[s])
+
+
+@pytest.mark.parametrize("N", [32, 64, 256])
+def test_launches_of_many_wavefronts_give_the_bits_of_few(N):
+    """Beyond three wavefronts a SIMD states of more than 16 numbers a lane do not ask for rows ahead: the first channels alone, which do, are the same."""
+    from paged_llm_amd.csrc import ops
+    gen = torch.Generator(device="cuda").manual_seed(N)
+    T, C, few = 2048, 4096, 70
+    rand = lambda *shape: torch.randn(*shape, generator=gen, device="cuda")
+    x, z, raw, bias, bc, skip, state = rand(T, C), rand(T, C), rand(T, C), rand(C) - 3.0, rand(T, 2 * N), rand(C), rand(1, N * C)
+    a2 = -torch.rand(N, C, generator=gen, device="cuda") * 4.0
+    at = lambda *v: torch.tensor(v, dtype=torch.int32, device="cuda")
+
+    def scan(c):
+        held = state.view(N, C)[:, :c].reshape(1, -1).clone()
+        part = lambda t: t[..., :c].contiguous()
+        y = ops.selective_scan(part(x), part(raw), part(bias), bc, part(a2), part(skip), part(z), held, at(0), at(1), at(0, T), 1, T)
+        return y, held.view(N, c)
+    for whole, first in zip(scan(C), scan(few)):
+        assert torch.equal(whole[:, :few], first)
