@@ -170,6 +170,15 @@ def test_wide_products_fill_one_round():
                     assert 128 <= -(-rows // tile[0]) * -(-weight_rows // tile[1]) <= 256
 
 
+def test_experts_stay_with_the_staged_kernel_where_wide_tiles_were_behind():
+    """Small experts of few rows (600 tokens with 8 of 64 of 512: 61 us staged, 86 in the wide tiles once chosen; of 1,536 at width 4,096 511 and 632)."""
+    for case in ((4800, 64, 1024, 512, True), (4800, 64, 4096, 1536, True)):
+        assert ops.moe_wide_plan(*case, 256) is None, case
+    for case in ((4096, 16, 2048, 2048, False), (2048, 8, 2048, 4096, False), (4096, 8, 2048, 2048, True), (1600, 16, 2048, 2048, False)):
+        rows, first, down = ops.moe_wide_plan(*case, 256)
+        assert rows in ops.MOE_WIDE_ROWS and first in ops.MOE_WIDE_COLUMNS and down in ops.MOE_WIDE_COLUMNS
+
+
 def test_sequences_behind_a_window_are_taken_as_they_come():
     """The order by length is for layers that see whole sequences: without a window, or with one that no sequence is longer than."""
     assert ops.longest_in_turn(0, 2000) == ops.longest_in_turn(2000, 2000) == ops.longest_in_turn(-4096, 2000) == 2000
