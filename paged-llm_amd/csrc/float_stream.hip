@@ -404,7 +404,7 @@ __global__ __launch_bounds__(256) void rms_sandwich_kernel(const float* __restri
 // kernel waits for memory once where the one above waits three times (decode steps: the weights have left the caches since the
 // last layer).  Partial sums and their order are the ones of the kernel above.  The branch may be a sum of experts' rows
 // (`sum.expert_out` set), formed here instead of by a kernel of its own.  Replayed from a graph, us of the kernel above's way (a branch: of one
-// element a load) and so: 8 rows of 2,048 with a branch 5.2 and 3.4, without one 3.7 and 2.7; 777 rows with a branch 8.5 and 7.6.
+// element a load) and so: 8 rows of 2,048 with a branch 5.2 and 3.5, without one 3.7 and 2.7; 777 rows with a branch 8.5 and 7.5; of 4,096 13.1 and 12.6.
 constexpr int kHeldPerThread = 16, kHeldThreads = 256;
 
 // The first element of group j of a thread's part of a row; a group past the row's end reads the row's first elements and counts nowhere.
@@ -468,7 +468,7 @@ __device__ __forceinline__ void store_held_rows(T* p, const float* v, bool fours
 // f += the sum of row r's choices, in their order.  What bounds it in a decode step: trips to memory.  A lane asks for one choice's
 // row number and weight, then the rows of four choices are asked for at once (and the token's own row, where some choice hands it
 // back): two trips up to four choices, where a choice after the other waits for its row number and then for its row.  Replayed from a graph, us in turn and
-// so: 8 rows of 2,048 elements with both norms and 4 choices 9.6 and 4.5, 1,178 rows of 2 choices 23.2 and 10.8, 64 rows of 4,096 and 4 24.0 and 7.4.
+// so: 8 rows of 2,048 elements with both norms and 4 choices 9.6 and 3.9, 1,178 rows of 2 choices 23.2 and 10.1, 64 rows of 4,096 and 4 24.0 and 6.6.
 template <typename TH, int VEC, int G>
 __device__ __forceinline__ void add_choices(const ChoiceSum& sum, int rows_lane, float weights_lane, int r, int hidden, bool own_fours, float (&f)[VEC * G]) {
   const int lane = threadIdx.x & 63;
@@ -489,6 +489,9 @@ __device__ __forceinline__ void add_choices(const ChoiceSum& sum, int rows_lane,
         const int row = __builtin_amdgcn_readlane(rows_lane, min(k1 + u, count - 1));
         load_held_groups<VEC, G>(sum.expert_out + (size_t)max(row, 0) * hidden, hidden, v[u]);
       }
+      // (Loads that wait for one another spare registers, and cost more than these give: 8 rows of 4,095 elements 10.1 us, 5.4 so.  Many rows of more
+      // than 2,048 in fours want the wavefronts: 1,178 of 4,096 23.0 us so, 20.6.)
+      if constexpr (VEC == 1 || G <= 2) __builtin_amdgcn_sched_barrier(0);
 #pragma unroll
       for (int u = 0; u < kSumAhead; ++u) {
         if (k1 + u >= count) break;
@@ -503,7 +506,7 @@ __device__ __forceinline__ void add_choices(const ChoiceSum& sum, int rows_lane,
 
 // A thread's sum of its row's squares in the order of the kernel above, elements threadIdx.x, threadIdx.x + 256, ..., whichever elements it
 // holds: four neighbours to a thread go through LDS first (with sums of their own a row's bits would hang on where it lies in memory; that took
-// 0.2 to 0.5 us less for 8 rows, 0.8 of 10 for 1,178, 2 of 14.8 for 2,048).
+// 0.2 to 0.4 us less for 8 rows, 1.2 of 13.9 for 2,048 with a plain branch).
 // `in_order` may be used again behind a held_sum of the result.
 template <int VEC, int G>
 __device__ __forceinline__ float squares_of_row(const float (&v)[VEC * G], int hidden, float4* in_order) {
@@ -531,7 +534,9 @@ __device__ __forceinline__ float held_sum(float v, float4& sums) {
   return ((sums.x + sums.y) + sums.z) + sums.w;
 }
 
-template <typename TO, typename TH, int VEC, int G>
+// SUM: the branch is a sum of experts' rows.  (Its rows under way take 64 registers at 4,096 elements, which leave three workgroups to a compute unit;
+// without them four: 777 rows with a plain branch 14.4 -> 12.6 us, 2,048 26.6 -> 24.6.)
+template <typename TO, typename TH, int VEC, int G, bool SUM>
 __global__ __launch_bounds__(kHeldThreads) void rms_sandwich_held_kernel(const float* __restrict__ branch, const BranchPair pair, const ChoiceSum sum,
                                                                          const float* __restrict__ bias, const float* __restrict__ w_branch,
                                                                          float mult, float* stream, const int* __restrict__ row_index,
@@ -539,11 +544,11 @@ __global__ __launch_bounds__(kHeldThreads) void rms_sandwich_held_kernel(const f
                                                                          long rows_stride, int hidden, bool own_fours, bool out_fours) {
   __shared__ float4 sums[2], in_order[VEC == 4 ? kHeldThreads * G : 1];
   const int r = blockIdx.x, lane = threadIdx.x & 63;
-  const bool added = branch || sum.expert_out;
+  const bool added = SUM || branch;
   float* s = stream + (!added && row_index ? (size_t)row_index[r] : (size_t)r) * hidden;
   int rows_lane = 0;
   float weights_lane = 0.f;
-  if (sum.expert_out) {                                     // (asked for first: the choices' rows wait for these alone)
+  if (SUM) {                                                // (asked for first: the choices' rows wait for these alone)
     const size_t at = (size_t)r * sum.top + min(lane, min(64, sum.top) - 1);
     rows_lane = sum.row_of_pair[at];
     weights_lane = sum.weights[at];
@@ -551,18 +556,18 @@ __global__ __launch_bounds__(kHeldThreads) void rms_sandwich_held_kernel(const f
   float f[VEC * G], sv[VEC * G], wb[VEC * G], wn[VEC * G], add[VEC * G];
 #pragma unroll
   for (int i = 0; i < VEC * G; ++i) { f[i] = 0.f; wb[i] = wn[i] = 1.f; add[i] = 0.f; }
-  if (branch) load_held_groups<VEC, G>(branch + (size_t)r * hidden, hidden, f);
+  if (!SUM && branch) load_held_groups<VEC, G>(branch + (size_t)r * hidden, hidden, f);
   load_held_groups<VEC, G>(s, hidden, sv);
   if (w_branch) load_held_groups<VEC, G>(w_branch, hidden, wb);
   if (w_next) load_held_groups<VEC, G>(w_next, hidden, wn);
   if (bias) load_held_groups<VEC, G>(bias, hidden, add);
-  if (pair.second) {
+  if (!SUM && pair.second) {
     float second[VEC * G];
     load_held_groups<VEC, G>(pair.second + (size_t)r * hidden, hidden, second);
 #pragma unroll
     for (int i = 0; i < VEC * G; ++i) f[i] = pair.first_scale * f[i] + pair.second_scale * second[i];
   }
-  if (sum.expert_out) add_choices<TH, VEC, G>(sum, rows_lane, weights_lane, r, hidden, own_fours, f);
+  if (SUM) add_choices<TH, VEC, G>(sum, rows_lane, weights_lane, r, hidden, own_fours, f);
   if (bias) {
 #pragma unroll
     for (int i = 0; i < VEC * G; ++i) f[i] += add[i];
@@ -745,17 +750,17 @@ PLLM_API int pllm_depth_sum(float* stream, float* history, long plane, const flo
   PLLM_RETURN_LAST_ERROR();
 }
 
-template <typename TO>
+template <typename TO, bool SUM>
 static void launch_sandwich_held(int h_dtype, const float* branch, const BranchPair& pair, const ChoiceSum& sum, const float* bias, const float* w_branch, float mult,
                                  float* stream, const int* row_index, const float* w_next, float eps, void* rows, long rows_stride, int num_rows, int hidden,
                                  hipStream_t stream_) {
   const uintptr_t all = (uintptr_t)branch | (uintptr_t)pair.second | (uintptr_t)sum.expert_out | (uintptr_t)bias | (uintptr_t)w_branch | (uintptr_t)stream | (uintptr_t)w_next;
   const bool fours = hidden % 4 == 0 && all % 16 == 0;
-  const bool own_fours = sum.expert_out && rows_by_fours(h_dtype, sum.h, sum.ld_h), out_fours = rows_by_fours(sizeof(TO) == 4 ? PLLM_F32 : PLLM_BF16, rows, rows_stride);
+  const bool own_fours = SUM && rows_by_fours(h_dtype, sum.h, sum.ld_h), out_fours = rows_by_fours(sizeof(TO) == 4 ? PLLM_F32 : PLLM_BF16, rows, rows_stride);
 #define PLLM_SH_FORM(T, TH, VEC, G)                                                                                                               \
-  hipLaunchKernelGGL((rms_sandwich_held_kernel<T, TH, VEC, G>), dim3(num_rows), dim3(kHeldThreads), 0, stream_, branch, pair, sum, bias, w_branch, \
+  hipLaunchKernelGGL((rms_sandwich_held_kernel<T, TH, VEC, G, SUM>), dim3(num_rows), dim3(kHeldThreads), 0, stream_, branch, pair, sum, bias, w_branch, \
                      mult, stream, row_index, w_next, eps, (T*)rows, rows_stride, hidden, own_fours, out_fours)
-  if (h_dtype == PLLM_F32) PLLM_HELD_FORM(PLLM_SH_FORM, TO, float, fours);
+  if (!SUM || h_dtype == PLLM_F32) PLLM_HELD_FORM(PLLM_SH_FORM, TO, float, fours);      // (a plain branch knows no type of the tokens' rows)
   else PLLM_HELD_FORM(PLLM_SH_FORM, TO, bf16, fours);
 #undef PLLM_SH_FORM
 }
@@ -767,8 +772,8 @@ PLLM_API int pllm_rms_sandwich_sum(int out_dtype, int h_dtype, const float* expe
   if (num_rows <= 0) return 0;
   if (hidden <= 0 || hidden > kHeldPerThread * kHeldThreads || !stream || !w_branch || !expert_out || !h || !row_of_pair || !weights || top <= 0) return -2;
   const ChoiceSum sum{expert_out, h, ld_h, row_of_pair, weights, top};
-  if (out_dtype == PLLM_F32) launch_sandwich_held<float>(h_dtype, nullptr, BranchPair{nullptr, 1.f, 1.f}, sum, bias, w_branch, mult, stream, nullptr, w_next, eps, rows, rows_stride, num_rows, hidden, stream_);
-  else launch_sandwich_held<bf16>(h_dtype, nullptr, BranchPair{nullptr, 1.f, 1.f}, sum, bias, w_branch, mult, stream, nullptr, w_next, eps, rows, rows_stride, num_rows, hidden, stream_);
+  if (out_dtype == PLLM_F32) launch_sandwich_held<float, true>(h_dtype, nullptr, BranchPair{nullptr, 1.f, 1.f}, sum, bias, w_branch, mult, stream, nullptr, w_next, eps, rows, rows_stride, num_rows, hidden, stream_);
+  else launch_sandwich_held<bf16, true>(h_dtype, nullptr, BranchPair{nullptr, 1.f, 1.f}, sum, bias, w_branch, mult, stream, nullptr, w_next, eps, rows, rows_stride, num_rows, hidden, stream_);
   PLLM_RETURN_LAST_ERROR();
 }
 
@@ -779,8 +784,8 @@ static int rms_sandwich_launch(int out_dtype, const float* branch, const BranchP
   if (hidden <= 0 || !stream) return -2;
   if (hidden <= kHeldPerThread * kHeldThreads) {
     const ChoiceSum none{nullptr, nullptr, 0, nullptr, nullptr, 0};
-    if (out_dtype == PLLM_F32) launch_sandwich_held<float>(PLLM_F32, branch, pair, none, bias, w_branch, mult, stream, row_index, w_next, eps, rows, rows_stride, num_rows, hidden, stream_);
-    else launch_sandwich_held<bf16>(PLLM_F32, branch, pair, none, bias, w_branch, mult, stream, row_index, w_next, eps, rows, rows_stride, num_rows, hidden, stream_);
+    if (out_dtype == PLLM_F32) launch_sandwich_held<float, false>(PLLM_F32, branch, pair, none, bias, w_branch, mult, stream, row_index, w_next, eps, rows, rows_stride, num_rows, hidden, stream_);
+    else launch_sandwich_held<bf16, false>(PLLM_F32, branch, pair, none, bias, w_branch, mult, stream, row_index, w_next, eps, rows, rows_stride, num_rows, hidden, stream_);
     PLLM_RETURN_LAST_ERROR();
   }
   const size_t lds = (size_t)(hidden + 16) * sizeof(float);
