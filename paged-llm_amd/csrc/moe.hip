@@ -802,7 +802,7 @@ __global__ __launch_bounds__(256) void moe_expert_tile_kernel(const bf16* __rest
   }
 }
 
-// The products where K is a multiple of 64 (with 70 rows an expert and more those of moe_wide.hip are ahead): a tile of MT blocks of 16 rows of one expert times NB blocks of 16 weight rows (gated: a
+// The products where K is a multiple of 64 (with 70 rows an expert and more those of moe_wide.hip are asked first): a tile of MT blocks of 16 rows of one expert times NB blocks of 16 weight rows (gated: a
 // gate's block and its up block in turn), for prompt steps eight wavefronts that multiply and four that bring the operands: stages of 64 columns
 // go from memory straight into LDS, R stages deep, a load taking the whole 128-byte lines of eight rows, whose eight pieces
 // lie XOR-ed by the row so that operand reads meet no bank twice.  Workgroups that follow each other on a chiplet

@@ -1,7 +1,7 @@
 // The experts' products of prompt steps (moe.hip: the forms, the sorted pairs and their tiles) in tiles of 64 to 192 rows of one expert x 128 or 256
 // weight rows, one workgroup of four wavefronts a tile, where K is a multiple of 64.
 //
-// The structure is that of wide_linear.hip, and so are the reasons: one wavefront per SIMD with up to 512 registers, stages of 64 columns in
+// The structure is that of wide_linear.hip (what is mended in one belongs in the other), and so are the reasons: one wavefront per SIMD with up to 512 registers, stages of 64 columns in
 // LDS filled by global_load_lds, R of them, the operands of a step of 32 columns read while the products of the step before it run, loads, reads
 // and products dealt out evenly, the sums held in the accumulation registers.  Rows and weights both come as pieces of 8 rows x 128 bytes
 // whose eight 16-byte parts lie XOR-ed by the row.

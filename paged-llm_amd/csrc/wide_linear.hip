@@ -18,6 +18,7 @@
 // 40.6 / 46.5 (33.0 / 45.4 / 58.6).
 // Which tile a product takes, and whether it comes here, is the host's choice (ops.wide_linear_plan, ops.wide_rotary_plan).
 // An output is one chain in ascending k whatever its tile.
+// moe_wide.hip has the same stages, waits and held sums for the experts' products: what is mended in one belongs in the other.
 #include "common.h"
 
 using namespace pllm;

@@ -1,4 +1,4 @@
-"""Prompts whose tokens all want logits, replayed from graphs (from the third time a shape is seen): more wanted rows than a graph holds logits
+"""Prompts whose tokens all want logits, replayed from graphs (the session captures a shape when it first sees it): more wanted rows than a graph holds logits
 for, lengths that share a graph, and results that a later replay leaves alone."""
 
 import pytest
