@@ -170,3 +170,24 @@ def test_several_threads_ask_for_the_parts_at_once():
     for t in threads:
         t.join()
     assert all(torch.equal(y, want) for y in got)
+
+
+def test_what_a_model_lays_out_with_its_first_step_counts_once_for_the_cache_pool(monkeypatch):
+    """A probing step that leaves 1 GB behind and needs 100 MB for itself: as many pages as when the 1 GB is there already."""
+    from types import SimpleNamespace
+
+    from paged_llm_amd.engine import pool_sizing
+    from paged_llm_amd.engine.loading import random_model
+    from tests.tiny_configs import TINY_A
+    model = random_model(TINY_A, dtype="float32")
+    left = []
+
+    def probe(*args):
+        torch.empty(100 << 20, dtype=torch.uint8, device="cuda")
+        if not left:
+            left.append(torch.empty(1 << 30, dtype=torch.uint8, device="cuda"))
+    monkeypatch.setattr(pool_sizing, "_probe_step", probe)
+    config = SimpleNamespace(block_size=16, max_num_batched_tokens=64, max_num_seqs=1 << 20, max_model_len=1 << 20, gpu_memory_utilization=0.9)
+    page = sum(g.bytes_per_page(16, model.dtype) for g in model.cache_groups().values())
+    pages = [pool_sizing.pages_that_fit(model, config) for _ in range(2)]
+    assert abs(pages[0] - pages[1]) * page < 200 << 20
