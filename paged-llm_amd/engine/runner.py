@@ -9,8 +9,8 @@ of the new tokens.
 
 from __future__ import annotations
 
-import contextlib
 import gc
+import threading
 from collections import OrderedDict
 
 import numpy as np
@@ -25,17 +25,28 @@ class StepError(ValueError):
     pass
 
 
-@contextlib.contextmanager
-def _no_collection():
-    """No garbage collection by itself during a capture: the collector may come upon the graphs of a runner that is gone, and a graph
-    cannot be destroyed while a stream is capturing (the process would abort)."""
-    was = gc.isenabled()
-    gc.disable()
-    try:
-        yield
-    finally:
-        if was:
-            gc.enable()
+class _NoCollection:
+    """No garbage collection by itself while any capture is under way: the collector may come upon the graphs of a runner that is gone, and a graph
+    cannot be destroyed while a stream is capturing (the process would abort).  The last capture to end, of whatever thread, puts things back."""
+
+    def __init__(self):
+        self._lock, self._under_way, self._was = threading.Lock(), 0, False
+
+    def __enter__(self):
+        with self._lock:
+            if self._under_way == 0:
+                self._was = gc.isenabled()
+                gc.disable()
+            self._under_way += 1
+
+    def __exit__(self, *exc):
+        with self._lock:
+            self._under_way -= 1
+            if self._under_way == 0 and self._was:
+                gc.enable()
+
+
+_no_collection = _NoCollection()
 
 
 class GraphCache:
@@ -334,7 +345,7 @@ class ModelRunner:
         torch.cuda.current_stream(self.device).wait_stream(stream)
         torch.cuda.synchronize(self.device)
         graph = torch.cuda.CUDAGraph()
-        with _no_collection(), torch.cuda.graph(graph, stream=stream):
+        with _no_collection, torch.cuda.graph(graph, stream=stream):
             logits = self.model.forward(ctx, self.kv, self.states)
         entry.update(graph=graph, logits=logits, ctx=ctx)
         self._graphs.put(entry["key"], entry)
@@ -633,7 +644,7 @@ class ModelRunner:
         if self._graph_pool is None:
             self._graph_pool = torch.cuda.graph_pool_handle()
         graph = torch.cuda.CUDAGraph()
-        with _no_collection(), torch.cuda.graph(graph, stream=stream, pool=self._graph_pool):
+        with _no_collection, torch.cuda.graph(graph, stream=stream, pool=self._graph_pool):
             result = forward()
         entry.update(graph=graph, ctx=ctx, **{"head_rows" if apart else "logits": result})
         return self._graphs.put(entry["key"], entry)

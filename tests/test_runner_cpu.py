@@ -300,3 +300,23 @@ def test_graphs_of_decode_steps_outlive_a_burst_of_prompt_shapes():
         cache.get(decode_key)
     assert decode_key in cache and (100, 1, 512) not in cache and (169, 1, 512) in cache
     assert sorted(k[0] for k in cache if k[0] != "prompt")[:2] == [8, 107]
+
+
+def test_the_collector_rests_until_the_last_capture_has_ended():
+    import gc
+
+    from paged_llm_amd.engine.runner import _no_collection
+    assert gc.isenabled()
+    _no_collection.__enter__()
+    with _no_collection:                                    # (another thread's, say)
+        assert not gc.isenabled()
+    assert not gc.isenabled()
+    _no_collection.__exit__(None, None, None)
+    assert gc.isenabled()
+    gc.disable()
+    try:
+        with pytest.raises(KeyError), _no_collection:
+            raise KeyError
+        assert not gc.isenabled()
+    finally:
+        gc.enable()
