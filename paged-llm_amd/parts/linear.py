@@ -8,9 +8,9 @@
   weights' tiled copy (``Weight``), with the same epilogues, or with float partial sums of ranges of K that the
   consuming norm adds; where it was measured slower than the library (the gated product and products with float
   results beyond 64 rows, the output head) the library stays.
-* bfloat16, more rows (prompt portions): the wide kernel where its tiles fill the compute units in one round, the tiled kernel for rotary products
-  up to 1536 rows, for gated ones up to 320 and, as partial sums, for small matrices up to 640; else the vendor's matrix-product library,
-  with bfloat16 or (logits) float results.
+* bfloat16, more rows (prompt portions): the wide kernel for gated products and, where its tiles fill the compute units in one round, for others; the tiled
+  kernel for rotary products up to 1536 rows, for some gated ones up to 320 and, as partial sums, for small matrices up to 640; else the vendor's
+  matrix-product library, with bfloat16 or (logits) float results.
 
 The choice depends on the number of rows and the sizes only, never on the rows' content.  ``x`` may
 be a tensor or a ``PendingNorm``; a weight may be a tensor [N, K] or a ``Weight``.
@@ -183,7 +183,7 @@ def _stream(x, weight: Weight, epi: int, rope: dict | None = None, partial_ok: b
 
 
 WIDE_MIN_ROWS = 129                              # rows from which the wide kernel is chosen (below, the streaming and tiled kernels are)
-WIDE_GATED_FROM_ROWS_WHEN_LARGE = 321            # ... for gated products in its large tiles, where the tiled kernel has them below
+WIDE_GATED_FROM_ROWS_WHEN_LARGE = 321            # ... for gated products of short K in its large tiles, where the tiled kernel has them below
 
 
 def _wide(x, weight, epi: int, beside_tiled: bool = False):
@@ -196,6 +196,10 @@ def _wide(x, weight, epi: int, beside_tiled: bool = False):
         return None
     if beside_tiled:
         return ops.wide_rotary_plan(rows, weight.shape[0], weight.shape[1], ops._num_compute_units(weight.plain.device))
+    if epi == ops.SL_GATED:
+        tile = ops.wide_gated_plan(rows, weight.shape[0], weight.shape[1], ops._num_compute_units(weight.plain.device))
+        if tile is not None:
+            return tile
     tile = ops.wide_linear_plan(rows, weight.shape[0], weight.shape[1], epi, ops._num_compute_units(weight.plain.device))
     if tile in ops.WIDE_GATED_TILES and rows < WIDE_GATED_FROM_ROWS_WHEN_LARGE:
         return None

@@ -170,6 +170,19 @@ def test_wide_products_fill_one_round():
                     assert 128 <= -(-rows // tile[0]) * -(-weight_rows // tile[1]) <= 256
 
 
+def test_gated_products_take_the_tile_of_the_least_estimate():
+    """From 129 rows and K = 1024 on, whatever the rounds; None where the tiled kernel's own tiles fill a round, for short K, and past 32-bit offsets."""
+    plan = ops.wide_gated_plan
+    assert plan(2048, 11264, 2048, 256) == (256, 352) and plan(1024, 16384, 2048, 256) == (256, 256) and plan(777, 11264, 2048, 256) == (160, 256)
+    assert plan(264, 28672, 4096, 256) == (288, 128) and plan(200, 16384, 2048, 256) == (128, 128) and plan(200, 4096, 1024, 256) == (64, 64)
+    assert plan(264, 16384, 2048, 256) is None and plan(160, 28672, 4096, 256) is None and plan(2048, 11264, 960, 256) is None
+    assert plan(2048, 11264, 2080, 256) is None and plan(2048, 11260, 2048, 256) is None and plan(1 << 17, 8192, 1024, 256) is None
+    for rows in (129, 161, 257, 500, 2000, 8192):
+        for weight_rows in (64, 1000, 2560, 11264, 28672):
+            tile = plan(rows, weight_rows, 2048, 256)
+            assert tile is None or tile in ops.WIDE_TILES + ops.WIDE_LARGE_TILES
+
+
 def test_experts_stay_with_the_staged_kernel_where_wide_tiles_were_behind():
     """Small experts of few rows (600 tokens with 8 of 64 of 512: 61 us staged, 86 in the wide tiles once chosen; of 1,536 at width 4,096 511 and 632)."""
     for case in ((4800, 64, 1024, 512, True), (4800, 64, 4096, 1536, True)):

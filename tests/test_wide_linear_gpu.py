@@ -108,6 +108,38 @@ def test_silu_to_float_accuracy():
         assert torch.equal(edge[ok].to(torch.bfloat16), exact[ok].to(torch.bfloat16)), (edge, exact)
 
 
+@pytest.mark.parametrize("m,n,k", [(257, 188, 64), (321, 364, 128), (130, 16, 320), (300, 520, 1088)])
+@pytest.mark.parametrize("activation", ["silu", "gelu_tanh"])
+def test_gated_products_in_large_tiles(m, n, k, activation):
+    """Every large tile where its last rows, blocks, stages and pieces of 16 bytes are whole or not: the bits of the smallest tile (the same chains of sums), also
+    of gates past the quick form's range and of rows that are no numbers, and nothing past the last row."""
+    o = ops()
+    x, w = bf(m, k, seed=31), bf(2 * n, k, seed=32) * 0.25
+    x[3] *= 64.0
+    x[m - 2, 0], x[m // 2, 1] = float("nan"), float("inf")
+    tiled, gx = o.tile_weight(w.cuda(), "gated"), x.cuda()
+    want = o.wide_linear(gx, tiled, (64, 64), o.SL_GATED, activation=activation).cpu()
+    for tile in o.WIDE_LARGE_TILES:
+        got = o.wide_linear(gx, tiled, tile, o.SL_GATED, activation=activation).cpu()
+        assert torch.equal(got.nan_to_num(7.0, 8.0, 9.0), want.nan_to_num(7.0, 8.0, 9.0)), tile
+
+
+@pytest.mark.parametrize("m,n,k,tile", [(1000, 5632, 1024, (256, 128)), (321, 512, 1024, (64, 64)), (290, 11264, 1024, (192, 128)), (2100, 5632, 1024, (192, 256)), (129, 2048, 1088, (64, 64))])
+def test_parts_take_the_wide_kernel_for_gated_products_of_long_k(m, n, k, tile, monkeypatch):
+    """n weight rows; within two roundings to bfloat16 of 64 bits."""
+    from paged_llm_amd.parts.linear import Weight, gated_linear
+    w = bf(n, k, seed=33) * 0.1
+    weight = Weight(w.cuda(), "gated")
+    for x, rows in rows_of_three_kinds(m, k):
+        tiles = taken(monkeypatch)
+        got = gated_linear(x, weight).cpu().double()
+        assert tiles == [tile]
+        sums = rows.double() @ w.cuda().double().T
+        want = (torch.nn.functional.silu(sums[:, :n // 2]) * sums[:, n // 2:]).cpu()
+        assert bool(((got - want).abs() <= 2.0 ** -7 * want.abs() + 1e-3 * want.abs().max()).all())
+        monkeypatch.undo()
+
+
 def taken(monkeypatch):
     """The tiles that the products of the parts go to in the wide kernel, from here on."""
     from paged_llm_amd.parts import linear as part
