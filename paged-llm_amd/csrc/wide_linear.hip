@@ -1,7 +1,7 @@
 // Products of prompt steps: y = x W^T for bfloat16 rows and a tiled weight matrix (ops.tile_weight), in tiles of 64 x 64 to 128 x 160
 // outputs, one workgroup of four wavefronts a tile, with bfloat16 or float results, act(gate) * up, or the rotation of q and k
-// with the write of k and v into their cache pages behind; gated products also in tiles of up to 320 x 256 and 256 x 352 by eight wavefronts
-// (big_linear_kernel).
+// with the write of k and v into their cache pages behind; gated products, and plain ones in fewer rounds than the library has, in tiles of up to 320 x 256
+// and 256 x 352 by eight wavefronts (big_linear_kernel).
 //
 // What bounds it: the matrix cores at the clock that they hold under such a load (1.3 to 1.4 PFLOP/s over the chip with nothing else in the
 // kernel), and for tiles of 128 x 128 and less a compute unit's way to the L2 (26 to 45 bytes a clock).  So every other
@@ -16,7 +16,7 @@
 //     them to and fro (96 to 248 moves a stage).
 // Measured (us, weights from memory; in brackets the library's product, with the kernel behind it where there is one): 896 rows x 2048 x 2048 14.0 (16.4),
 // 512 x 1024 x 1024 5.7 (8.4), 2048 x 2048 x 4096 39.5 (40.4), gated 512 rows of 5632 x 1024 13.4 (20.6), 320 rows of 11264 x 2048 25.4 (33.0).
-// Which tile a product takes, and whether it comes here, is the host's choice (ops.wide_linear_plan, ops.wide_gated_plan, ops.wide_rotary_plan).
+// Which tile a product takes, and whether it comes here, is the host's choice (ops.wide_linear_plan, ops.wide_gated_plan, ops.wide_plain_plan, ops.wide_rotary_plan).
 // An output is one chain in ascending k whatever its tile.
 // moe_wide.hip has the same stages, waits and held sums for the experts' products: what is mended in one belongs in the other.
 #include "common.h"
@@ -332,7 +332,8 @@ __device__ __forceinline__ void load_to_lds(__amdgpu_buffer_rsrc_t from, int lan
 //   * loads go through buffers whose moving part is scalar: one register a lane for all weights and one for each load of rows.
 // What bounds it now is power: 256 x 352 takes 1,590 cycles a step (1,408 of products) at 1.85 to 2.0 GHz, and the form of it with four wavefronts and 13 % more
 // cycles ran as long at 9 % more clock.  2048 rows of 11264 x 2048, with SiLU: 72 us (1.31 PFLOP/s; 97.7 in two rounds of 256 x 192 above, 94 in the
-// library with the activation behind); 777 rows 36 (40.6, 45), 1024 rows 41 (46.5, 56); 2048 / 8192 rows of 16384 x 2048 106 / 423 (library 122 / 483).
+// library with the activation behind); 777 rows 36 (40.6, 45), 1024 rows 41 (46.5, 56); 2048 / 8192 rows of 16384 x 2048 106 / 423 (library 122 / 483).  Plain: 2048 rows of 8512 x 2048 in 256 x 288 60 (library 79), 1178 of 32000 x 2048
+// with float results in 256 x 320 146 (168).
 template <int EPI, int WM, int MW, int NW, int RW, int RX>
 __global__ __launch_bounds__(512, 2) void big_linear_kernel(WideParams p) {
   constexpr int WN = 8 / WM, NB = WN * NW, XT = WM * MW;
@@ -570,7 +571,15 @@ static int launch_tile(const WideParams& p, int weight_rows, int rows, int weigh
     case 128128: return launch_wide<EPI, 2, 4, 4, 4>(p, weight_rows, stream);
     case 128160: return launch_wide<EPI, 2, 4, 5, 4>(p, weight_rows, stream);
   }
-  if constexpr (EPI == WL_GATED) {                                     // (plain products of so many outputs stay with the library)
+  if constexpr (EPI != WL_ROPE_KV) {                                   // (in one round where tiles of 256 x 256 need two: ops.wide_plain_plan)
+    switch (rows * 1000 + weights) {
+      case 256288: return launch_big<EPI, 4, 4, 9, 4, 2>(p, weight_rows, stream);
+      case 256320: return launch_big<EPI, 4, 4, 10, 4, 2>(p, weight_rows, stream);
+      case 256352: return launch_big<EPI, 4, 4, 11, 4, 2>(p, weight_rows, stream);
+      case 320256: return launch_big<EPI, 4, 5, 8, 4, 2>(p, weight_rows, stream);
+    }
+  }
+  if constexpr (EPI == WL_GATED) {
     switch (rows * 1000 + weights) {
       case 160256: return launch_big<EPI, 2, 5, 4, 5, 3>(p, weight_rows, stream);
       case 192128: return launch_big<EPI, 4, 3, 4, 10, 3>(p, weight_rows, stream);
@@ -582,12 +591,8 @@ static int launch_tile(const WideParams& p, int weight_rows, int rows, int weigh
       case 256192: return launch_big<EPI, 4, 4, 6, 4, 3>(p, weight_rows, stream);
       case 256224: return launch_big<EPI, 4, 4, 7, 5, 2>(p, weight_rows, stream);
       case 256256: return launch_big<EPI, 4, 4, 8, 4, 2>(p, weight_rows, stream);
-      case 256288: return launch_big<EPI, 4, 4, 9, 4, 2>(p, weight_rows, stream);
-      case 256320: return launch_big<EPI, 4, 4, 10, 4, 2>(p, weight_rows, stream);
-      case 256352: return launch_big<EPI, 4, 4, 11, 4, 2>(p, weight_rows, stream);
       case 288128: return launch_big<EPI, 2, 9, 2, 6, 3>(p, weight_rows, stream);
       case 320128: return launch_big<EPI, 4, 5, 4, 4, 3>(p, weight_rows, stream);
-      case 320256: return launch_big<EPI, 4, 5, 8, 4, 2>(p, weight_rows, stream);
     }
   }
   return -3;

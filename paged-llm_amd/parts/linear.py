@@ -203,6 +203,8 @@ def _wide(x, weight, epi: int, beside_tiled: bool = False):
     tile = ops.wide_linear_plan(rows, weight.shape[0], weight.shape[1], epi, ops._num_compute_units(weight.plain.device))
     if tile in ops.WIDE_GATED_TILES and rows < WIDE_GATED_FROM_ROWS_WHEN_LARGE:
         return None
+    if tile is None and epi in (ops.SL_BF16, ops.SL_F32):
+        tile = ops.wide_plain_plan(rows, weight.shape[0], weight.shape[1], ops._num_compute_units(weight.plain.device))
     return tile
 
 

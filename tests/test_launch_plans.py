@@ -183,6 +183,15 @@ def test_gated_products_take_the_tile_of_the_least_estimate():
             assert tile is None or tile in ops.WIDE_TILES + ops.WIDE_LARGE_TILES
 
 
+def test_plain_products_take_large_tiles_where_square_ones_begin_a_round():
+    """One round of 256 x 288 to 256 x 352 where 256 x 256 needs two, and so on; None in front of and behind that, for short K, and past 32-bit offsets."""
+    plan = ops.wide_plain_plan
+    assert plan(2048, 8512, 2048, 256) == (256, 288) and plan(2048, 8192, 2048, 256) is None and plan(2048, 10240, 1024, 256) == (256, 320)
+    assert plan(1777, 12288, 2048, 256) == (256, 352) and plan(2048, 12288, 2048, 256) is None and plan(1178, 32000, 2048, 256) == (256, 320)
+    assert plan(640, 32000, 2048, 256) == (320, 256) and plan(512, 32000, 2048, 256) is None and plan(777, 2048, 5632, 256) is None
+    assert plan(2048, 8512, 960, 256) is None and plan(2048, 8512, 2080, 256) is None and plan(2048, 8510, 2048, 256) is None and plan(70000, 8512, 2048, 256) is None
+
+
 def test_experts_stay_with_the_staged_kernel_where_wide_tiles_were_behind():
     """Small experts of few rows (600 tokens with 8 of 64 of 512: 61 us staged, 86 in the wide tiles once chosen; of 1,536 at width 4,096 511 and 632)."""
     for case in ((4800, 64, 1024, 512, True), (4800, 64, 4096, 1536, True)):

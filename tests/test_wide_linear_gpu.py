@@ -124,6 +124,18 @@ def test_gated_products_in_large_tiles(m, n, k, activation):
         assert torch.equal(got.nan_to_num(7.0, 8.0, 9.0), want.nan_to_num(7.0, 8.0, 9.0)), tile
 
 
+@pytest.mark.parametrize("m,n,k", [(257, 292, 64), (321, 364, 128), (130, 16, 320), (300, 520, 1088)])
+def test_plain_products_in_large_tiles(m, n, k):
+    """As ``test_plain_products``, and the bits of the smallest tile."""
+    o = ops()
+    x, w = bf(m, k, seed=34), bf(n, k, seed=35)
+    gx, tiled = x.cuda(), o.tile_weight(w.cuda())
+    want = o.wide_linear(gx, tiled, (64, 64), o.SL_F32)
+    for tile in o.WIDE_PLAIN_TILES:
+        assert torch.equal(o.wide_linear(gx, tiled, tile, o.SL_F32), want), tile
+        assert torch.equal(o.wide_linear(gx, tiled, tile, o.SL_BF16), want.to(torch.bfloat16)), tile
+
+
 @pytest.mark.parametrize("m,n,k,tile", [(1000, 5632, 1024, (256, 128)), (321, 512, 1024, (64, 64)), (290, 11264, 1024, (192, 128)), (2100, 5632, 1024, (192, 256)), (129, 2048, 1088, (64, 64))])
 def test_parts_take_the_wide_kernel_for_gated_products_of_long_k(m, n, k, tile, monkeypatch):
     """n weight rows; within two roundings to bfloat16 of 64 bits."""
