@@ -17,6 +17,11 @@
 // visible keys among themselves (the kept first positions' blocks, then the window's) and add their outputs through
 // LDS in wave order.  Weights are float and rounded to bfloat16 for the second product, as the softmax kernels round
 // their probabilities.  Values of keys that no column of the tile may see are zeroed (0 * stale data stays 0).
+//
+// What bounds it: prompts that fill the GPU the weights' four slow instructions a score (two exponentials, two reciprocals), shorter ones a tile's chain
+// of blocks, each a wait for memory and 64 keys of arithmetic: hence the wavefronts that share a tile (ops.sigmoid_attention_plan, with what was
+// measured) and the tiles with the most keys first.  32 heads on 4 key heads of 64, a window of 1,024, capped: 2,048 tokens 83 -> 78 us, 1,500 69 -> 62, 777 beside
+// their padding 74 -> 37, 256 behind 1,024 26 -> 22, 8 decoded tokens beside 200 89 -> 23.
 #include "common.h"
 #include <type_traits>
 
@@ -58,8 +63,9 @@ __global__ __launch_bounds__(WAVES * 64) void sigmoid_attention_kernel(
   const int q_begin = as_constant(cu_seqlens_q)[seq], num_q = as_constant(cu_seqlens_q)[seq + 1] - q_begin;
   const int len_k = as_constant(seq_lens_k)[seq];
   const int num_cols = num_q * G;
-  const int col0 = blockIdx.x * 16 * NCB;
-  if (col0 >= num_cols) return;
+  // (a sequence's last tile, which sees the most keys, starts first)
+  const int tile = (num_cols + 16 * NCB - 1) / (16 * NCB) - 1 - (int)blockIdx.x, col0 = tile * 16 * NCB;
+  if (tile < 0) return;
   const int last_col = min(col0 + 16 * NCB, num_cols) - 1;
   const int pos0 = len_k - num_q;                               // position of the sequence's first query
   const int qpos_min = pos0 + col0 / G, qpos_max = pos0 + last_col / G;
@@ -99,7 +105,7 @@ __global__ __launch_bounds__(WAVES * 64) void sigmoid_attention_kernel(
 #pragma unroll
     for (int db = 0; db < DBLOCKS; ++db) acc[cb][db] = floatx4{0.f, 0.f, 0.f, 0.f};
 
-  // the score in log2 units: log2(e) * cap(scale * s), with c tanh(x / c) = c (1 - 2 / (2^(2 log2(e) x / c) + 1))
+  // minus the score in log2 units: -log2(e) * cap(scale * s), with c tanh(x / c) = c (1 - 2 / (2^(2 log2(e) x / c) + 1))
   const bool capped = cap > 0.f;
   const float sl2 = scale * kLog2e, cap_l2 = cap * kLog2e, cap_in = capped ? 2.f * kLog2e * scale / cap : 0.f;
 
@@ -154,13 +160,19 @@ __global__ __launch_bounds__(WAVES * 64) void sigmoid_attention_kernel(
 #pragma unroll
           for (int s = 0; s < KSTEPS; ++s) s_t = __builtin_amdgcn_mfma_f32_16x16x32_bf16(blk.k[kt][s], qreg[cb][s], s_t, 0, 0, 0);
         }
+        // (the choice of form is the wavefront's: a selection would make both)
+        if (capped) {
+#pragma unroll
+          for (int i = 0; i < 4; ++i) s_t[i] = fmaf(2.f * cap_l2, __builtin_amdgcn_rcpf(__builtin_amdgcn_exp2f(s_t[i] * cap_in) + 1.f), -cap_l2);
+        } else {
+#pragma unroll
+          for (int i = 0; i < 4; ++i) s_t[i] *= -sl2;
+        }
 #pragma unroll
         for (int i = 0; i < 4; ++i) {
           const int n = n0 + kt * 16 + g * 4 + i;
           const bool vis = kAll || (blk.on[kt] && n <= my_qpos[cb] && (n >= my_first[cb] || n < keep_first));
-          float z = capped ? fmaf(-2.f * cap_l2, __builtin_amdgcn_rcpf(__builtin_amdgcn_exp2f(s_t[i] * cap_in) + 1.f), cap_l2) : s_t[i] * sl2;
-          z += my_bias[cb];
-          const float p = __builtin_amdgcn_rcpf(1.f + __builtin_amdgcn_exp2f(-z));
+          const float p = __builtin_amdgcn_rcpf(1.f + __builtin_amdgcn_exp2f(s_t[i] - my_bias[cb]));
           p_op[kt >> 1][cb][(kt & 1) * 4 + i] = (__bf16)(vis ? p : 0.f);
         }
       }

@@ -192,6 +192,15 @@ def test_plain_products_take_large_tiles_where_square_ones_begin_a_round():
     assert plan(2048, 8512, 960, 256) is None and plan(2048, 8512, 2080, 256) is None and plan(2048, 8510, 2048, 256) is None and plan(70000, 8512, 2048, 256) is None
 
 
+def test_sigmoid_attention_counts_the_columns_that_there_are():
+    """More wavefronts a tile where tiles are few; padding and short sequences beside a long one no longer count as long ones."""
+    plan = ops.sigmoid_attention_plan
+    assert plan(8, 64, 100) == plan(8, 64, 100, 800) == (1, 8, False)
+    assert plan(896 * 8, 64, 2 * 4) == (2, 1, False) and plan(896 * 8, 64, 2 * 4, 896 * 32) == (2, 4, False)
+    assert [plan(8 * t, 64, 4, 32 * t)[:2] for t in (64, 65, 384, 385, 960, 961, 1536, 1537)] == [(1, 8), (1, 4), (1, 4), (2, 4), (2, 4), (2, 2), (2, 2), (2, 1)]
+    assert plan(4 * 700, 128, 4, 16 * 700) == (1, 2, False) and plan(40, 256, 1, 40) == (1, 4, False)
+
+
 def test_experts_stay_with_the_staged_kernel_where_wide_tiles_were_behind():
     """Small experts of few rows (600 tokens with 8 of 64 of 512: 61 us staged, 86 in the wide tiles once chosen; of 1,536 at width 4,096 511 and 632)."""
     for case in ((4800, 64, 1024, 512, True), (4800, 64, 4096, 1536, True)):
