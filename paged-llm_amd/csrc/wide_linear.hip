@@ -136,15 +136,41 @@ __device__ __forceinline__ void finish(const WideParams& p, const floatx4 (&acc)
   const int row_bytes = p.ldo * (EPI == WL_F32 ? 4 : 2);
   const __amdgpu_buffer_rsrc_t out = __builtin_amdgcn_make_buffer_rsrc(p.out, 0, (int)((unsigned)p.M * (unsigned)row_bytes), 0x00027000);
   const int pair_row = (g & 1) * 4 + (g >> 1) * 2;                     // (of swap_halves)
+  // A rotation's operands are asked for together: one by one each waits for the memory, and for the stores in front of it (2048 rows of 2560 x 2048
+  // 35.2 -> 33 us, 777 of 3072 x 2048 23.7 -> 20.3, 26.7 and 16 without the rotation; the tiled kernel, with two blocks on a compute unit, gains nothing).
+  constexpr bool kTurns = EPI == WL_ROPE_KV;
+  int pos[kTurns ? MW : 1], slots[kTurns ? MW : 1];
+  f32x2 turn[kTurns ? MW : 1][kTurns ? NW : 1][2];
+  int heads[kTurns ? NW : 1], rows_in[kTurns ? NW : 1];                // a block's head, and this lane's first row in the head's half
+  if constexpr (kTurns) {
+#pragma unroll
+    for (int t = 0; t < MW; ++t) {
+      const int m = min(row0 + t * 16 + r, p.M - 1);
+      pos[t] = p.positions[m];
+      slots[t] = p.slots[m];
+    }
+    const int half = p.head_dim >> 1, per_head = half >> 3;
+    int head = unit0 / per_head, in_head = unit0 - head * per_head;
+#pragma unroll
+    for (int u = 0; u < NW; ++u) {
+      heads[u] = head;
+      rows_in[u] = in_head * 8 + pair_row;
+      if (++in_head == per_head) in_head = 0, ++head;
+    }
+#pragma unroll
+    for (int t = 0; t < MW; ++t)
+#pragma unroll
+      for (int u = 0; u < NW; ++u) {
+        const size_t at = (size_t)pos[t] * half + rows_in[u];
+        turn[t][u][0] = p.cos_t ? *reinterpret_cast<const f32x2*>(p.cos_t + at) : f32x2{1.f, 1.f};
+        turn[t][u][1] = p.cos_t ? *reinterpret_cast<const f32x2*>(p.sin_t + at) : f32x2{0.f, 0.f};
+      }
+    __builtin_amdgcn_sched_barrier(0);
+  }
 #pragma unroll
   for (int t = 0; t < MW; ++t) {
     const int m = row0 + t * 16 + r;
     const int at_row = m * row_bytes;
-    int pos = 0, slot_kv = -1;
-    if (EPI == WL_ROPE_KV && m < p.M) {
-      pos = p.positions[m];
-      slot_kv = p.slots[m];
-    }
     if constexpr (EPI == WL_GATED) {
       float z[2 * NW], y[2 * NW];
 #pragma unroll
@@ -157,7 +183,9 @@ __device__ __forceinline__ void finish(const WideParams& p, const floatx4 (&acc)
       }
       continue;
     }
-    const int page = EPI == WL_ROPE_KV && slot_kv >= 0 ? slot_kv / p.block_size : 0, off = slot_kv - page * p.block_size;
+    const int slot_kv = kTurns && m < p.M ? slots[kTurns ? t : 0] : -1;
+    int page = 0, off = 0;
+    if (kTurns && heads[kTurns ? NW - 1 : 0] >= p.num_heads && slot_kv >= 0) page = slot_kv / p.block_size, off = slot_kv - page * p.block_size;
 #pragma unroll
     for (int u = 0; u < NW; ++u) {
       const floatx4 a = acc[t][u];
@@ -171,15 +199,10 @@ __device__ __forceinline__ void finish(const WideParams& p, const floatx4 (&acc)
       } else {
         float x[2], y[2];
         swap_halves(a, x, y);
-        const int d = p.head_dim, half = d >> 1, per_head = half >> 3, nh = p.num_heads, nkv = p.num_kv_heads;
-        const int head = unit / per_head, ri = (unit - head * per_head) * 8 + pair_row;
+        const int d = p.head_dim, half = d >> 1, nh = p.num_heads, nkv = p.num_kv_heads, head = heads[u], ri = rows_in[u];
         if (head >= nh + 2 * nkv) continue;
         if (head < nh + nkv) {
-          f32x2 cs{1.f, 1.f}, sn{0.f, 0.f};
-          if (p.cos_t) {
-            cs = *reinterpret_cast<const f32x2*>(p.cos_t + (size_t)pos * half + ri);
-            sn = *reinterpret_cast<const f32x2*>(p.sin_t + (size_t)pos * half + ri);
-          }
+          const f32x2 cs = turn[t][u][0], sn = turn[t][u][1];
           float lo[2], hi[2];
 #pragma unroll
           for (int i = 0; i < 2; ++i)
