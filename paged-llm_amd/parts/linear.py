@@ -8,7 +8,8 @@
   weights' tiled copy (``Weight``), with the same epilogues, or with float partial sums of ranges of K that the
   consuming norm adds; where it was measured slower than the library (the gated product and products with float
   results beyond 64 rows, the output head) the library stays.
-* bfloat16, more rows (prompt portions): the wide kernel for gated products and, where its tiles fill the compute units in one round, for others; the tiled
+* bfloat16, more rows (prompt portions): the wide kernel for gated products, and for others where its tiles fill the compute units in one round or its large
+  ones take fewer rounds than the library's; the tiled
   kernel for rotary products up to 1536 rows, for some gated ones up to 320 and, as partial sums, for small matrices up to 640; else the vendor's
   matrix-product library, with bfloat16 or (logits) float results.
 
@@ -306,7 +307,7 @@ def _tiles_gated(x, weight, rows: int) -> bool:
     where the streaming kernel's workgroups of 32 to 64 weight rows draw the rows four times as often (28672 x 4096 at
     24 / 64 / 128 rows: 43 / 45 / 54 us against 50 / 57 us streaming at 32 and 64 and 53 / 53 / 59 us in the library with the activation
     kernel; 24576 x 2048 at 64 rows 27 against 33 and 30).  With two blocks of rows such matrices go in tiles of 256 weight rows
-    (264 rows: 81 us against 78 and 6 for the activation in the library).  A matrix whose tiles of 128 fill at most half of the compute
+    (264 rows: 81 us against 78 and 6 for the activation in the library; where those need more than a round, ``ops.wide_gated_plan`` has them, 71).  A matrix whose tiles of 128 fill at most half of the compute
     units is cut into tiles of 64 weight rows by the kernel when there is one block of rows, twice the workgroups (11264 x
     2048 at 64 / 96 / 128 / 160 rows: 14.0 / 16.1 / 19.0 / 21.7 us against 18.8 / 20.3 / 21.8 / 27.6 in the library with the
     activation kernel and 14.8 streaming at 64; 16384 x 2048 at 32 / 64 rows: 15.7 / 16.8 against 19.0 / 21.0 streaming; inside
