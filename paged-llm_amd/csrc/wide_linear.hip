@@ -573,6 +573,7 @@ static int launch_big(WideParams p, int weight_rows, hipStream_t stream) {
   constexpr int kRows = 16 * WM * MW, kWeights = 128 / WM * NW;
   constexpr size_t lds = (size_t)RW * (8 / WM * NW) * 1024 + (size_t)RX * (WM * MW) * 2048;
   static_assert(lds <= 160 * 1024, "LDS of one compute unit");
+  if (p.ldx >= 1 << 21 || p.ksteps >= 1 << 16) return -2;        // (a tile's 320 rows and 352 weight rows by 32-bit offsets)
   auto kernel = big_linear_kernel<EPI, WM, MW, NW, RW, RX>;
   hipError_t e = hipFuncSetAttribute(reinterpret_cast<const void*>(kernel), hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds);
   if (e != hipSuccess) return (int)e;

@@ -190,6 +190,7 @@ def test_plain_products_take_large_tiles_where_square_ones_begin_a_round():
     assert plan(1777, 12288, 2048, 256) == (256, 352) and plan(2048, 12288, 2048, 256) is None and plan(1178, 32000, 2048, 256) == (256, 320)
     assert plan(640, 32000, 2048, 256) == (320, 256) and plan(512, 32000, 2048, 256) is None and plan(777, 2048, 5632, 256) is None
     assert plan(2048, 8512, 960, 256) is None and plan(2048, 8512, 2080, 256) is None and plan(2048, 8510, 2048, 256) is None and plan(70000, 8512, 2048, 256) is None
+    assert plan(2048, 8512, 1 << 21, 256) is None and ops.wide_gated_plan(2048, 11264, 1 << 21, 256) is None
 
 
 def test_sigmoid_attention_counts_the_columns_that_there_are():

@@ -136,6 +136,17 @@ def test_plain_products_in_large_tiles(m, n, k):
         assert torch.equal(o.wide_linear(gx, tiled, tile, o.SL_BF16), want.to(torch.bfloat16)), tile
 
 
+def test_rows_of_a_very_wide_matrix():
+    """A tile's offsets have 32 bits: rows further apart than they reach are laid side by side first."""
+    o = ops()
+    x, w = bf(320, 64, seed=36), bf(512, 64, seed=37)
+    wide = torch.empty((320, o.WIDE_LARGE_OFFSETS * 2), dtype=torch.bfloat16, device="cuda")
+    wide[:, :64] = x.cuda()
+    tiled = o.tile_weight(w.cuda())
+    for tile in ((64, 64),) + o.WIDE_PLAIN_TILES:
+        assert torch.equal(o.wide_linear(wide[:, :64], tiled, tile), o.wide_linear(x.cuda(), tiled, tile)), tile
+
+
 @pytest.mark.parametrize("m,n,k,tile", [(1000, 5632, 1024, (256, 128)), (321, 512, 1024, (64, 64)), (290, 11264, 1024, (192, 128)), (2100, 5632, 1024, (192, 256)), (129, 2048, 1088, (64, 64))])
 def test_parts_take_the_wide_kernel_for_gated_products_of_long_k(m, n, k, tile, monkeypatch):
     """n weight rows; within two roundings to bfloat16 of 64 bits."""
